@@ -158,7 +158,7 @@ class AllReduce(Workload):
     ranks.  One launch folds each slice into the first output (eight inputs read once), a second copies it to the
     other seven, one output at a time."""
     dtype = "f32"
-    kernel = "hcclx::k_fold_wide<4, 0, 0, 4> + hcclx::(anonymous namespace)::k_phased_copy"
+    kernel = "hcclx::k_fold_wide<4, 0, 0, 4> + hcclx::(anonymous namespace)::k_phased_copy<hcclx::PhasedTable>"
     profile = "profiles/k_fold_wide_k_phased_copy_all_reduce_fp32_8x64MiB.txt"
 
     def __init__(self, torch, api, T, n=8, count=16 * 1024 * 1024, alg=None, step_mode=False, dtype=None, op=None,
@@ -205,7 +205,7 @@ class AllGather(Workload):
     """HcclAllGather fp16, 8 ranks x 33,554,432 elements (64 MiB per rank): every block lands in every
     output; each source byte is read once and written eight times."""
     dtype = "u8"
-    kernel = "hcclx::(anonymous namespace)::k_phased_copy_inline"
+    kernel = "hcclx::(anonymous namespace)::k_phased_copy<hcclx::PhasedInline>"
     profile = "profiles/k_phased_copy_all_gather_fp16_8x64MiB.txt"
 
     def __init__(self, torch, api, T, n=8, count=32 * 1024 * 1024):
@@ -234,7 +234,7 @@ class AllGatherV(Workload):
     """benchmark configuration 3: HcclAllGatherV fp16, 16 ranks, per-rank counts uniform in [0, 8,388,608] from a
     seed, displacements their prefix sum (so most blocks start at addresses that are only 2-byte aligned)."""
     dtype = "u8"
-    kernel = "hcclx::(anonymous namespace)::k_phased_copy_inline"
+    kernel = "hcclx::(anonymous namespace)::k_phased_copy<hcclx::PhasedInline>"
     profile = "profiles/k_phased_copy_all_gather_v_fp16_16_ranks_ragged.txt"
 
     def __init__(self, torch, api, T, n=16, seed=3):

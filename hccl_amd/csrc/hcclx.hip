@@ -128,8 +128,6 @@ void init_slot(DeviceSlot *s, int dev)
     }
     if (const char *v = std::getenv("HCCLX_FANOUT_FROM")) c.fanout_from = std::strtoull(v, nullptr, 10);
     if (const char *v = std::getenv("HCCLX_FANOUT_RUN")) {
-        // between 64 KiB and 1 GiB: a run is one job of a launch, and its tile count has to stay within the length
-        // classes the launches are grouped by
         const uint64_t b = std::min<uint64_t>(std::strtoull(v, nullptr, 10), 1ull << 30);
         if (b >= 65536) c.fanout_run = b & ~static_cast<uint64_t>(4095);
     }
@@ -266,15 +264,36 @@ uint32_t grid_for(const DeviceCtx *ctx, uint64_t total_tiles)
 // ---------------------------------------------------------------------------------------------------
 // copies that write one output at a time
 // ---------------------------------------------------------------------------------------------------
-size_t PhasedLaunch::jobs_bytes() const { return (jobs.size() * sizeof(PhasedJob) + 255) & ~static_cast<size_t>(255); }
-size_t PhasedLaunch::bytes() const { return jobs_bytes() + dsts.size() * sizeof(char *); }
+namespace {
+size_t align256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
+}  // namespace
+
+size_t PhasedLaunch::bytes() const
+{
+    return align256(sources.size() * sizeof(PhasedSource)) + align256(slabs.size() * sizeof(PhasedSlab)) + dsts.size() * sizeof(char *);
+}
+PhasedTable PhasedLaunch::table(const char *d) const
+{
+    PhasedTable t;
+    t.sources = reinterpret_cast<const PhasedSource *>(d);
+    d += align256(sources.size() * sizeof(PhasedSource));
+    t.slabs = reinterpret_cast<const PhasedSlab *>(d);
+    d += align256(slabs.size() * sizeof(PhasedSlab));
+    t.dsts = reinterpret_cast<char *const *>(d);
+    t.nd = grid.nd;
+    t.nslabs = static_cast<uint32_t>(slabs.size());
+    return t;
+}
 void PhasedLaunch::fill(char *h) const
 {
-    std::memcpy(h, jobs.data(), jobs.size() * sizeof(PhasedJob));
-    std::memcpy(h + jobs_bytes(), dsts.data(), dsts.size() * sizeof(char *));
+    std::memcpy(h, sources.data(), sources.size() * sizeof(PhasedSource));
+    h += align256(sources.size() * sizeof(PhasedSource));
+    std::memcpy(h, slabs.data(), slabs.size() * sizeof(PhasedSlab));
+    h += align256(slabs.size() * sizeof(PhasedSlab));
+    std::memcpy(h, dsts.data(), dsts.size() * sizeof(char *));
 }
 
-void build_phased(std::vector<PhasedStream> &streams, uint64_t run_bytes, std::vector<PhasedLaunch> *out)
+void build_phased(std::vector<PhasedStream> &streams, uint64_t batch_bytes, uint32_t max_slabs, std::vector<PhasedLaunch> *out)
 {
     // join streams that continue each other: the slices of a two-shot AllReduce lie back to back in every buffer
     std::vector<PhasedStream> joined;
@@ -289,65 +308,49 @@ void build_phased(std::vector<PhasedStream> &streams, uint64_t run_bytes, std::v
             joined.push_back(std::move(st));
         }
     }
-    struct Run {
-        const PhasedStream *st;
-        uint64_t at, len;
-        uint32_t tiles;
+    // the smallest slab size with which the sources need at most max_slabs slabs (or the largest, and several launches)
+    uint32_t tiles = kPhasedSlabTilesLeast;
+    auto slabs_at = [&](uint32_t t) {
+        uint64_t n = 0;
+        for (const PhasedStream &st : joined) n += phased_slabs_of(st.bytes, t);
+        return n;
     };
-    // runs of equal length per stream, a multiple of the tile size; then launches by length class (powers of four)
-    constexpr uint64_t kTile = 256ull * 16 * kPhasedUnroll;
-    run_bytes = std::min<uint64_t>(std::max<uint64_t>(run_bytes, kTile), 1ull << 30);   // every run falls into a class below
-    std::vector<Run> runs;
+    while (tiles < kPhasedSlabTilesMost && slabs_at(tiles) > max_slabs) tiles *= 2;
+    PhasedLaunch cur;
+    auto flush = [&]() {
+        if (cur.slabs.empty()) return;
+        const uint64_t n = cur.slabs.size();
+        const uint64_t most = std::max<uint64_t>(1, batch_bytes / (tiles * kPhasedTile));
+        const uint64_t batches = (n + most - 1) / most;
+        cur.grid.slab_tiles = tiles;
+        cur.grid.batches = static_cast<uint32_t>(batches);
+        cur.grid.per_batch = static_cast<uint32_t>((n + batches - 1) / batches);
+        // the pointer array is laid out once the source with the most places is known
+        std::vector<char *> flat(cur.sources.size() * cur.grid.nd, nullptr);
+        size_t at = 0;
+        for (size_t j = 0; j < cur.sources.size(); ++j) {
+            for (uint64_t d = 0; d < cur.sources[j].place; ++d) flat[j * cur.grid.nd + d] = cur.dsts[at++];
+        }
+        cur.dsts = std::move(flat);
+        out->push_back(std::move(cur));
+        cur = PhasedLaunch();
+    };
     for (const PhasedStream &st : joined) {
-        const uint64_t n = (st.bytes + run_bytes - 1) / run_bytes;
-        const uint64_t len = ((st.bytes + n - 1) / n + kTile - 1) / kTile * kTile;
-        for (uint64_t at = 0; at < st.bytes; at += len) {
-            Run r{&st, at, st.bytes - at < len ? st.bytes - at : len, 0};
-            r.tiles = static_cast<uint32_t>(v_tiles_of(r.len, reinterpret_cast<uint64_t>(st.dst[0]) + at, kPhasedUnroll));
-            runs.push_back(r);
+        const uint32_t nd = static_cast<uint32_t>(st.dst.size());
+        const uint64_t slabs = phased_slabs_of(st.bytes, tiles);
+        for (uint64_t k = 0; k < slabs; ++k) {
+            // a launch's tables stay inside one slice of the descriptor ring
+            const bool room = cur.slabs.size() < max_slabs && (cur.sources.size() + 1) * (sizeof(PhasedSource) + 8ull * std::max(cur.grid.nd, nd)) <= (1u << 19);
+            if (!room) flush();
+            if (k == 0 || !room) {
+                cur.sources.push_back({st.src, st.bytes, nd});
+                cur.dsts.insert(cur.dsts.end(), st.dst.begin(), st.dst.end());   // packed for now, see flush()
+                cur.grid.nd = std::max(cur.grid.nd, nd);
+            }
+            cur.slabs.push_back({static_cast<uint32_t>(cur.sources.size() - 1), static_cast<uint32_t>(k)});
         }
     }
-    constexpr size_t kMaxJobs = 4096;   // per launch: the table stays well inside one slice of the descriptor ring
-    for (int cls = 15; cls >= 0; --cls) {
-        PhasedLaunch cur;
-        auto flush = [&]() {
-            if (cur.jobs.empty()) return;
-            // Workgroups go to the eight XCDs in turn, each with an L2 of its own: with a multiple of eight slots per
-            // destination a tile is copied to all its destinations by the same XCD, whose L2 then serves the re-reads.
-            cur.slots = (cur.slots + 7) & ~7u;
-            // the pointer array is laid out once the widest job is known
-            std::vector<char *> flat(cur.jobs.size() * cur.nd, nullptr);
-            size_t at = 0;
-            for (size_t j = 0; j < cur.jobs.size(); ++j) {
-                for (uint32_t d = 0; d < cur.jobs[j].ndst; ++d) flat[j * cur.nd + d] = cur.dsts[at++];
-            }
-            cur.dsts = std::move(flat);
-            out->push_back(std::move(cur));
-            cur = PhasedLaunch();
-        };
-        for (const Run &r : runs) {
-            int c = 0;
-            for (uint32_t t = r.tiles; t > 1; t = (t + 3) / 4) ++c;
-            if (std::min(c, 15) != cls) continue;
-            const uint32_t nd = static_cast<uint32_t>(r.st->dst.size());
-            const uint64_t grid_x = (static_cast<uint64_t>(std::max(cur.slots, r.tiles)) + 7) * std::max(cur.nd, nd);
-            if (cur.jobs.size() == kMaxJobs || grid_x > 0x7fffffffull ||
-                (cur.jobs.size() + 1) * (sizeof(PhasedJob) + 8ull * std::max(cur.nd, nd)) > (1u << 19)) {
-                flush();
-            }
-            PhasedJob j;
-            j.src = r.st->src + r.at;
-            j.bytes = r.len;
-            j.dst0 = reinterpret_cast<uint64_t>(r.st->dst[0]) + r.at;
-            j.ndst = nd;
-            j.tiles = r.tiles;
-            cur.jobs.push_back(j);
-            for (char *p : r.st->dst) cur.dsts.push_back(p + r.at);   // packed for now, see flush()
-            cur.slots = std::max(cur.slots, r.tiles);
-            cur.nd = std::max(cur.nd, nd);
-        }
-        flush();
-    }
+    flush();
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -394,7 +397,7 @@ struct Batch {
     uint32_t xcd_remap = 0;      // wide kernels: contiguous tile ranges per XCD (pays with 16 or more destinations)
     std::vector<CopyBlock> blocks;   // instead of everything above: a list of blocks for the block copy kernel
     int block_unroll = 2;
-    PhasedLaunch phased;         // instead of everything above: jobs of the copy kernel that writes one output at a time
+    PhasedLaunch phased;         // instead of everything above: a launch of the copy kernel that writes one output at a time
     uint32_t store_policy = kStoreStream;   // how the fold kernels store (fold.h)
     uint32_t waves = 0;          // non-zero: the one-store-per-wavefront kernel, this many wavefronts per workgroup
     uint32_t pieces = 1;         // and this many 1 KiB pieces per source and workgroup
@@ -402,11 +405,10 @@ struct Batch {
     size_t nseg() const { return segs.size() + wide.size(); }
     size_t bytes() const
     {
-        if (!phased.jobs.empty()) return phased.bytes();
+        if (!phased.slabs.empty()) return phased.bytes();
         if (!blocks.empty()) return blocks.size() * sizeof(CopyBlock);
         return align256(tile_end.size() * 8) + segs.size() * sizeof(SegDev) + wide.size() * sizeof(SegWide);
     }
-    static size_t align256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 };
 
 struct Built {
@@ -651,11 +653,13 @@ bool split_fanout(const DeviceCtx *ctx, const SEG *segs, uint32_t nseg, int esz,
     return true;
 }
 
+constexpr uint32_t kPhasedTableSlabs = 4096;   // slabs of a fan-out launch at most: 32 KiB of table
+
 // Appends the second launch (or launches) of a split fold.
 void append_fanout(const DeviceCtx *ctx, std::vector<PhasedStream> &fan, Built *out)
 {
     std::vector<PhasedLaunch> launches;
-    build_phased(fan, ctx->fanout_run, &launches);
+    build_phased(fan, ctx->fanout_run, kPhasedTableSlabs, &launches);
     for (PhasedLaunch &l : launches) {
         Batch b;
         b.copy = true;
@@ -1010,7 +1014,7 @@ int build_wide_batches_impl(const hcclx_wide_seg_t *segs, uint32_t nseg, int dty
 
 void fill_table(const Batch &b, char *h)
 {
-    if (!b.phased.jobs.empty()) {
+    if (!b.phased.slabs.empty()) {
         b.phased.fill(h);
         return;
     }
@@ -1019,7 +1023,7 @@ void fill_table(const Batch &b, char *h)
         return;
     }
     std::memcpy(h, b.tile_end.data(), b.tile_end.size() * 8);
-    char *at = h + Batch::align256(b.tile_end.size() * 8);
+    char *at = h + align256(b.tile_end.size() * 8);
     if (!b.segs.empty()) std::memcpy(at, b.segs.data(), b.segs.size() * sizeof(SegDev));
     if (!b.wide.empty()) std::memcpy(at, b.wide.data(), b.wide.size() * sizeof(SegWide));
 }
@@ -1052,10 +1056,8 @@ hipError_t dispatch_fold(int dtype, int op, int maxn, int mode, const FoldLaunch
 
 int launch_batch(const DeviceCtx *ctx, const Batch &b, const char *d_table, hipStream_t stream)
 {
-    if (!b.phased.jobs.empty()) {
-        const hipError_t pe = launch_phased_copy(reinterpret_cast<const PhasedJob *>(d_table),
-                                                 reinterpret_cast<char *const *>(d_table + b.phased.jobs_bytes()),
-                                                 static_cast<uint32_t>(b.phased.jobs.size()), b.phased.slots, b.phased.nd, stream);
+    if (!b.phased.slabs.empty()) {
+        const hipError_t pe = launch_phased_copy(b.phased.table(d_table), b.phased.grid, stream);
         if (pe != hipSuccess) return fail_hip(pe, "phased copy kernel launch");
         return HCCL_SUCCESS;
     }
@@ -1067,7 +1069,7 @@ int launch_batch(const DeviceCtx *ctx, const Batch &b, const char *d_table, hipS
     }
     FoldLaunch l;
     l.tile_end = reinterpret_cast<const uint64_t *>(d_table);
-    l.segs = d_table + Batch::align256(b.tile_end.size() * 8);
+    l.segs = d_table + align256(b.tile_end.size() * 8);
     l.nseg = static_cast<uint32_t>(b.nseg());
     l.total_tiles = b.total_tiles;
     l.grid = grid_for(ctx, b.total_tiles);

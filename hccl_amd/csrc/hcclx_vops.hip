@@ -170,51 +170,27 @@ int hcclx_allgatherv(const void *const *send, void *const *recv, const uint64_t 
     if (!tables_on_device) {
         uint64_t payload = 0;
         for (uint32_t i = 0; i < n; ++i) payload += counts[i] * esz;
-        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(st, &capturing) != hipSuccess) (void)hipGetLastError();
-        // Large, and not being captured into a graph (the job table is uploaded at call time): the outputs of a run of
-        // a source are written one after the other.
-        if (n > 1 && ctx->agv_phased_from != 0 && payload >= ctx->agv_phased_from && capturing == hipStreamCaptureStatusNone) {
+        // Large: the outputs of a batch of slabs are written one after the other.  A source's places are one offset into
+        // every receive buffer and the tables fit the kernel arguments: nothing is copied in front of the kernel.
+        if (n > 1 && ctx->agv_phased_from != 0 && payload >= ctx->agv_phased_from) {
             std::vector<PhasedStream> streams;
+            streams.reserve(n);
             for (uint32_t i = 0; i < n; ++i) {
-                if (counts[i] == 0) continue;
-                PhasedStream s;
-                s.src = ptrs.send[i];
-                s.bytes = counts[i] * esz;
-                for (uint32_t d = 0; d < n; ++d) s.dst.push_back(ptrs.recv[d] + displs[i] * esz);
-                streams.push_back(std::move(s));
+                if (counts[i] != 0) streams.push_back({ptrs.send[i], counts[i] * esz, {ptrs.recv[0] + displs[i] * esz}});
             }
             std::vector<PhasedLaunch> launches;
-            build_phased(streams, ctx->fanout_run, &launches);
-            for (const PhasedLaunch &l : launches) {
-                // Among up to 16 ranks a job's places are one offset into every receive buffer, and the jobs of a
-                // launch usually fit the kernel arguments: no table in memory, nothing copied in front of the kernel.
-                if (n <= kPhasedInlineRanks && l.jobs.size() <= kPhasedInlineJobs && l.nd <= n) {
-                    PhasedInline tab;
-                    std::memset(&tab, 0, sizeof(tab));
-                    for (uint32_t d = 0; d < n; ++d) tab.base[d] = ptrs.recv[d];
-                    bool same_offset = true;
-                    for (size_t j = 0; j < l.jobs.size() && same_offset; ++j) {
-                        tab.jobs[j] = l.jobs[j];
-                        const uint64_t off = reinterpret_cast<uint64_t>(l.dsts[j * l.nd]) - reinterpret_cast<uint64_t>(ptrs.recv[0]);
-                        tab.jobs[j].dst0 = off;
-                        for (uint32_t d = 0; d < l.jobs[j].ndst; ++d) same_offset = same_offset && l.dsts[j * l.nd + d] == ptrs.recv[d] + off;
-                    }
-                    if (same_offset) {
-                        hipError_t e = launch_phased_copy_inline(tab, static_cast<uint32_t>(l.jobs.size()), l.slots, l.nd, st);
-                        if (e != hipSuccess) return fail_hip(e, "allgatherv kernel launch");
-                        continue;
-                    }
+            build_phased(streams, ctx->fanout_run, kPhasedInlineSlabs, &launches);
+            for (PhasedLaunch &l : launches) {
+                PhasedInline tab;
+                for (uint32_t d = 0; d < n; ++d) tab.base[d] = ptrs.recv[d];
+                for (size_t k = 0; k < l.sources.size(); ++k) {
+                    tab.sources[k] = l.sources[k];
+                    tab.sources[k].place = static_cast<uint64_t>(l.dsts[k] - ptrs.recv[0]);
                 }
-                char *h = nullptr;
-                char *d = nullptr;
-                rc = ring_reserve(ctx, l.bytes(), st, &h, &d);
-                if (rc != HCCL_SUCCESS) return rc;
-                l.fill(h);
-                HCCLX_HIP(hipMemcpyAsync(d, h, l.bytes(), hipMemcpyHostToDevice, st));
-                hipError_t e = launch_phased_copy(reinterpret_cast<const PhasedJob *>(d),
-                                                  reinterpret_cast<char *const *>(d + l.jobs_bytes()),
-                                                  static_cast<uint32_t>(l.jobs.size()), l.slots, l.nd, st);
+                for (size_t k = 0; k < l.slabs.size(); ++k) tab.slabs[k] = l.slabs[k].source | l.slabs[k].at << 6;
+                tab.nslabs = static_cast<uint32_t>(l.slabs.size());
+                l.grid.nd = n;
+                hipError_t e = launch_phased_copy_inline(tab, l.grid, st);
                 if (e != hipSuccess) return fail_hip(e, "allgatherv kernel launch");
             }
             return HCCL_SUCCESS;

@@ -20,11 +20,11 @@ constexpr uint32_t kMaxVRanks = 64;
 #endif
 constexpr int kA2avUnroll = HCCLX_A2AV_UNROLL;
 constexpr int kAgvUnroll = HCCLX_AGV_UNROLL;
-// The copies that write one output at a time (large AllGatherV, fan-out of a fold's result): 8 KiB tiles.
-#ifndef HCCLX_PHASED_UNROLL
-#define HCCLX_PHASED_UNROLL 2
-#endif
-constexpr int kPhasedUnroll = HCCLX_PHASED_UNROLL;
+// The copies that write one output at a time (large AllGatherV, fan-out of a fold's result): 4 KiB tiles, one vector
+// per thread.  A wavefront that issues one store and ends writes HBM faster than one that issues two or four (fills of
+// 1 GiB: 7.0 against 6.0 TB/s), and the same holds for these copies (8 x 64 MiB AllGather: 755 against 824 us).
+constexpr int kPhasedUnroll = 1;
+constexpr uint64_t kPhasedTile = 256ull * 16 * kPhasedUnroll;
 
 // Tiles of a block of `bytes` bytes whose first destination byte sits at address `dst`.  Stores are
 // aligned: the bytes before the first 16-byte boundary of dst (head) and after the last whole vector
@@ -95,24 +95,44 @@ struct AgvTablesPtr {
     __device__ uint64_t count(uint32_t i) const { return counts[i]; }
     __device__ uint64_t displ(uint32_t i) const { return displs[i]; }
 };
-// One job of the copy kernel that writes one output at a time: `bytes` bytes from src to ndst places (the
-// launch's pointer array holds them at [job * nd, job * nd + ndst)), cut into `tiles` tiles laid out for the
-// alignment of the first place, whose address is dst0.
-struct PhasedJob {
+// The copy kernel that writes one output at a time.  Its sources are cut into slabs of slab_tiles tiles each, a power of
+// two of at least eight (workgroups go to the eight XCDs in turn, each with an L2 of its own: a tile is then copied to
+// all its places by the same XCD); a batch of slabs, a few MiB, is copied to its first place, then to the second and so
+// on.  The last slab of a source is as long as what is left, so sources of any lengths share a launch and only those
+// ends leave workgroups that exit at once.
+struct PhasedSource {
     const char *src;
     uint64_t bytes;
-    uint64_t dst0;
-    uint32_t ndst;
-    uint32_t tiles;
+    uint64_t place;   // table in memory: ndst; tables in the kernel arguments: offset into every rank's receive buffer
 };
-// The same for an AllGather(V) among up to 16 ranks whose jobs fit the kernel arguments: every place a job goes to
-// is the same offset (the job's dst0) into the ranks' receive buffers, so the launch needs no table in memory.
-constexpr uint32_t kPhasedInlineJobs = 100;
-constexpr uint32_t kPhasedInlineRanks = 16;
+constexpr uint32_t kPhasedSlabTilesLeast = 8;
+constexpr uint32_t kPhasedSlabTilesMost = 1024;   // 4 MiB
+struct PhasedSlab {
+    uint32_t source;
+    uint32_t at;      // number of the slab inside its source
+};
+// A launch's tables in device memory: sources, slabs and nd places per source.
+struct PhasedTable {
+    const PhasedSource *sources;
+    const PhasedSlab *slabs;
+    char *const *dsts;
+    uint32_t nd;
+    uint32_t nslabs;
+};
+// The same for an AllGather(V), in the kernel arguments: every place of a source is the same offset into the ranks'
+// receive buffers.  Slab: source in the low six bits, its number above.
+constexpr uint32_t kPhasedInlineSlabs = 480;
 struct PhasedInline {
-    char *base[kPhasedInlineRanks];
-    PhasedJob jobs[kPhasedInlineJobs];
+    char *base[kMaxVRanks];
+    PhasedSource sources[kMaxVRanks];
+    uint32_t slabs[kPhasedInlineSlabs];
+    uint32_t nslabs;
 };
+// Slabs a source needs whatever the alignment of its places (their tile grids differ by less than a tile).
+__host__ __device__ inline uint64_t phased_slabs_of(uint64_t bytes, uint32_t slab_tiles)
+{
+    return bytes == 0 ? 0 : ((bytes / 16 + 63) / (kPhasedTile / 16) + slab_tiles) / slab_tiles;
+}
 struct AgvTablesInline {
     uint64_t counts[kMaxVRanks];
     uint64_t displs[kMaxVRanks];
@@ -122,11 +142,15 @@ struct AgvTablesInline {
 
 // blocks: device array of nblocks entries; unroll: 1, 2 or 4; grid = total number of tiles
 hipError_t launch_copy_blocks(const CopyBlock *blocks, uint32_t nblocks, uint32_t grid, int unroll, hipStream_t stream);
-// jobs, dsts: device arrays of njobs and njobs * nd entries; slots: tiles of the longest job; slots * nd < 2^31,
-// njobs < 65536
-hipError_t launch_phased_copy(const PhasedJob *jobs, char *const *dsts, uint32_t njobs, uint32_t slots, uint32_t nd,
-                              hipStream_t stream);
-hipError_t launch_phased_copy_inline(const PhasedInline &tab, uint32_t njobs, uint32_t slots, uint32_t nd, hipStream_t stream);
+// One batch after the other (grid z), each to one place after the other (grid y): per_batch slabs of slab_tiles tiles.
+struct PhasedGrid {
+    uint32_t slab_tiles;
+    uint32_t per_batch;
+    uint32_t batches;
+    uint32_t nd;
+};
+hipError_t launch_phased_copy(const PhasedTable &tab, const PhasedGrid &grid, hipStream_t stream);
+hipError_t launch_phased_copy_inline(const PhasedInline &tab, const PhasedGrid &grid, hipStream_t stream);
 // unroll: 1, 2 or 4 vectors per thread and tile; grid = total number of tiles
 hipError_t launch_alltoallv_direct(const VRankPtrs16 &ptrs, const A2avTablesDirect &tabs, uint32_t n, uint32_t esz,
                                    uint32_t grid, int unroll, hipStream_t stream);

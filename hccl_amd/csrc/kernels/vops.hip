@@ -220,25 +220,34 @@ k_copy_blocks(const CopyBlock *__restrict__ blocks, uint32_t nblocks)
     copy_tile<UNROLL>(src, reinterpret_cast<uint64_t>(dst), bytes, tl, 1, [=](uint32_t) { return dst; });
 }
 
-// One source run to several places, one place at a time.  Job blockIdx.y copies `bytes` bytes from src to its
-// destinations dsts[job * nd + 0 .. ndst): blockIdx.x = d * slots + tile, and workgroups start in the order of
-// their numbers, so a run (a few MiB) is written to its first destination, then to the second, and so on.  At any
-// moment the GPU therefore writes ONE output instead of n at once, which HBM takes a third faster (measured: one
-// source to eight outputs 4.8 -> 6.9 TB/s at the pins); the re-reads of the run come from the L2, not from HBM.
-// The place of a workgroup follows from its number by arithmetic and two independent scalar loads: a table search
-// in front of an 8 KiB tile costs a fifth of the kernel's time.  Jobs with fewer tiles or destinations than the
-// launch's widest leave workgroups that exit at once; the host groups jobs of similar length per launch.
-__global__ void __launch_bounds__(kThreads)
-k_phased_copy(const PhasedJob *__restrict__ jobs, char *const *__restrict__ dsts, uint32_t slots, uint32_t nd)
+__device__ __forceinline__ PhasedSlab phased_slab(const PhasedTable &t, uint32_t k) { return t.slabs[k]; }
+__device__ __forceinline__ PhasedSlab phased_slab(const PhasedInline &t, uint32_t k) { return {t.slabs[k] & 63u, t.slabs[k] >> 6}; }
+// null: the source has no such place
+__device__ __forceinline__ char *phased_dst(const PhasedTable &t, uint32_t source, uint32_t d)
 {
-    const uint32_t j = blockIdx.y;
-    const uint32_t d = blockIdx.x / slots;
-    const uint64_t tl = blockIdx.x - d * slots;
-    const PhasedJob job = jobs[j];
-    char *dst = dsts[static_cast<uint64_t>(j) * nd + d];
-    if (d >= job.ndst || tl >= job.tiles) return;
-    // tiles are laid out for the first destination's alignment; the others share it or lose only speed
-    copy_tile<kPhasedUnroll, true>(job.src, job.dst0, job.bytes, tl, 1, [=](uint32_t) { return dst; });
+    return d < t.sources[source].place ? t.dsts[static_cast<uint64_t>(source) * t.nd + d] : nullptr;
+}
+__device__ __forceinline__ char *phased_dst(const PhasedInline &t, uint32_t source, uint32_t d) { return t.base[d] + t.sources[source].place; }
+
+// Sources to several places, one place at a time.  Workgroups start in the order of their numbers (x: tile of the
+// batch, y: place, z: batch), so a batch is written to its first place, then to the second, and so on.  At any moment
+// the GPU writes ONE output instead of n at once, which HBM takes faster (one source to eight outputs, every workgroup
+// storing to all eight: 5.5 TB/s at the pins; this way 6.4-6.5); the re-reads of the batch come from the L2s, not from
+// HBM.  The place of a workgroup follows from its number with two dependent scalar loads: a table search in front of a
+// tile costs a fifth of the kernel's time.
+template <typename Tab>
+__global__ void __launch_bounds__(kThreads) k_phased_copy(Tab tab, uint32_t slab_shift, uint32_t per_batch)
+{
+    const uint32_t k = blockIdx.z * per_batch + (blockIdx.x >> slab_shift);
+    if (k >= tab.nslabs) return;
+    const PhasedSlab slab = phased_slab(tab, k);
+    const uint64_t tl = (static_cast<uint64_t>(slab.at) << slab_shift) + (blockIdx.x & ((1u << slab_shift) - 1u));
+    const PhasedSource &source = tab.sources[slab.source];
+    const char *src = source.src;
+    const uint64_t bytes = source.bytes;
+    char *dst = phased_dst(tab, slab.source, blockIdx.y);
+    if (dst == nullptr || tl >= v_tiles_of(bytes, reinterpret_cast<uint64_t>(dst), kPhasedUnroll)) return;
+    copy_tile<kPhasedUnroll, true>(src, reinterpret_cast<uint64_t>(dst), bytes, tl, 1, [=](uint32_t) { return dst; });
 }
 
 template <typename Tabs>
@@ -293,29 +302,23 @@ hipError_t launch_copy_blocks(const CopyBlock *blocks, uint32_t nblocks, uint32_
     return hipGetLastError();
 }
 
-__global__ void __launch_bounds__(kThreads) k_phased_copy_inline(PhasedInline tab, uint32_t slots, uint32_t nd)
+namespace {
+template <typename Tab> hipError_t launch_phased(const Tab &tab, const PhasedGrid &g, hipStream_t stream)
 {
-    const uint32_t j = blockIdx.y;
-    const uint32_t d = blockIdx.x / slots;
-    const uint64_t tl = blockIdx.x - d * slots;
-    const PhasedJob &job = tab.jobs[j];
-    if (d >= job.ndst || d >= nd || tl >= job.tiles) return;
-    char *dst = tab.base[d] + job.dst0;
-    copy_tile<kPhasedUnroll, true>(job.src, reinterpret_cast<uint64_t>(tab.base[0]) + job.dst0, job.bytes, tl, 1,
-                                   [=](uint32_t) { return dst; });
-}
-
-hipError_t launch_phased_copy_inline(const PhasedInline &tab, uint32_t njobs, uint32_t slots, uint32_t nd, hipStream_t stream)
-{
-    HCCLX_LAUNCH(k_phased_copy_inline, dim3(slots * nd, njobs), dim3(kThreads), 0, stream, tab, slots, nd);
+    const uint32_t shift = static_cast<uint32_t>(__builtin_ctz(g.slab_tiles));
+    HCCLX_LAUNCH((k_phased_copy<Tab>), dim3(g.per_batch << shift, g.nd, g.batches), dim3(kThreads), 0, stream, tab, shift, g.per_batch);
     return hipGetLastError();
 }
+}  // namespace
 
-hipError_t launch_phased_copy(const PhasedJob *jobs, char *const *dsts, uint32_t njobs, uint32_t slots, uint32_t nd,
-                              hipStream_t stream)
+hipError_t launch_phased_copy(const PhasedTable &tab, const PhasedGrid &grid, hipStream_t stream)
 {
-    HCCLX_LAUNCH(k_phased_copy, dim3(slots * nd, njobs), dim3(kThreads), 0, stream, jobs, dsts, slots, nd);
-    return hipGetLastError();
+    return launch_phased(tab, grid, stream);
+}
+
+hipError_t launch_phased_copy_inline(const PhasedInline &tab, const PhasedGrid &grid, hipStream_t stream)
+{
+    return launch_phased(tab, grid, stream);
 }
 
 hipError_t launch_alltoallv_direct(const VRankPtrs16 &ptrs, const A2avTablesDirect &tabs, uint32_t n, uint32_t esz,

@@ -218,6 +218,73 @@ def test_allgatherv_with_counts_and_displacements_that_never_leave_the_device():
         assert recv[j].guard_intact()
 
 
+SLAB = 32768    # the smallest slab of the copy kernel that writes one output at a time
+
+
+@pytest.mark.parametrize("n,sizes,pad", [
+    (2, [(4 << 20) + 1, 1], 0),                                                     # one long source, one of a byte
+    (5, [SLAB - 1, SLAB, SLAB + 1, 3 * SLAB + 1008, 4 << 20], 5),                   # around the slab edges, shifted places
+    (16, [300000 + 4099 * k for k in range(16)], 3),                                # no two sources of one length
+    (64, [(k % 7) * SLAB + (k * 37) % 1031 + (0 if k % 9 else -1) for k in range(64)], 2),   # most ranks, empty sources
+])
+def test_allgatherv_written_one_output_at_a_time(n, sizes, pad):
+    """From 4 MiB of payload: slabs of the sources, batch by batch to one receive buffer after the other; receive
+    buffers of different alignment, holes between the blocks."""
+    counts = [max(0, c) for c in sizes]
+    counts[0] += max(0, (4 << 20) - sum(counts))
+    displs = [sum(counts[:i]) + i * pad for i in range(n)]
+    rng = np.random.default_rng(n)
+    total = displs[-1] + counts[-1] + 7
+    ins = [rng.integers(0, 256, size=c, dtype=np.uint8) for c in counts]
+    want = T.run_allgatherv(ins, counts, displs, total, np.full(total, 0xA5, np.uint8))
+    send = [DevBuf(x, offset=i % 3) for i, x in enumerate(ins)]
+    recv = [DevBuf(nbytes=total, offset=(j * 5) % 48) for j in range(n)]
+    hcclx.allgatherv([b.ptr for b in send], [b.ptr for b in recv], np.array(counts, np.uint64), np.array(displs, np.uint64), T.INT8)
+    torch.cuda.synchronize()
+    for j in range(n):
+        assert np.array_equal(recv[j].get(np.uint8), want[j]), f"rank {j}"
+        assert recv[j].guard_intact()
+
+
+def test_allgatherv_payload_beyond_one_launch_of_the_largest_slabs():
+    counts = [(1 << 30) + 4099, (1 << 30) + 77]
+    g = torch.Generator(device="cuda:0")
+    g.manual_seed(4)
+    send = [torch.randint(0, 256, (c,), device="cuda:0", generator=g, dtype=torch.uint8) for c in counts]
+    recv = [torch.zeros(sum(counts), device="cuda:0", dtype=torch.uint8) for _ in counts]
+    torch.cuda.synchronize()
+    before = hcclx.kernels_launched()
+    hcclx.allgatherv([t.data_ptr() for t in send], [t.data_ptr() for t in recv], counts, [0, counts[0]], T.INT8)
+    assert hcclx.kernels_launched() - before == 2
+    torch.cuda.synchronize()
+    for t in recv:
+        assert torch.equal(t[:counts[0]], send[0]) and torch.equal(t[counts[0]:], send[1])
+
+
+@pytest.mark.parametrize("nseg", [1, 37, 200])
+def test_copies_to_several_places_of_different_number(nseg):
+    """The same kernel with its tables in memory: segments that only copy, 1 to 16 places each, 4 MiB and more."""
+    rng = np.random.default_rng(nseg)
+    counts = [int(c) for c in rng.integers(1, 2 * (5 << 20) // nseg, size=nseg)]
+    counts[0] += max(0, (5 << 20) - sum(counts))
+    fans = [int(f) for f in rng.integers(2, 17, size=nseg)]
+    if nseg > 1:
+        fans[1] = 1
+    ins = [rng.integers(0, 256, size=c, dtype=np.uint8) for c in counts]
+    src = [DevBuf(x, offset=i % 5) for i, x in enumerate(ins)]
+    dst = [[DevBuf(nbytes=c, offset=(3 * i + 7 * k) % 21) for k in range(f)] for i, (c, f) in enumerate(zip(counts, fans))]
+    segs = [(c, [s.ptr], [d.ptr for d in ds]) for c, s, ds in zip(counts, src, dst)]
+    plan = hcclx.Plan(segs, T.INT8)
+    for go in (lambda: hcclx.fold(segs, T.INT8), plan.launch):
+        go()
+        torch.cuda.synchronize()
+        for x, ds in zip(ins, dst):
+            for d in ds:
+                assert np.array_equal(d.get(np.uint8), x) and d.guard_intact()
+                d.t.fill_(0xA5)
+    plan.close()
+
+
 def test_v_ops_reject_bad_arguments():
     b = DevBuf(nbytes=64)
     with pytest.raises(HcclError) as e:
