@@ -110,7 +110,7 @@ void init_slot(DeviceSlot *s, int dev)
     if (const char *v = std::getenv("HCCLX_BLOCKS_PER_CU")) {
         c.blocks_per_cu = static_cast<uint32_t>(std::strtoul(v, nullptr, 10));
     }
-    if (const char *v = std::getenv("HCCLX_A2AV_DIRECT")) c.a2av_direct_unroll = static_cast<uint32_t>(std::strtoul(v, nullptr, 10));
+    if (const char *v = std::getenv("HCCLX_A2AV_DIRECT")) c.a2av_direct = std::strtoul(v, nullptr, 10) != 0;
     if (const char *v = std::getenv("HCCLX_WIDE_CHAIN_FROM")) c.wide_chain_from = static_cast<uint32_t>(std::strtoul(v, nullptr, 10));
     if (const char *v = std::getenv("HCCLX_WIDE_XCD_REMAP_FROM")) c.wide_xcd_remap_from = static_cast<uint32_t>(std::strtoul(v, nullptr, 10));
     c.wide_min_tiles = 2u * static_cast<uint32_t>(c.num_cus);
@@ -145,7 +145,7 @@ void init_slot(DeviceSlot *s, int dev)
     if (const char *v = std::getenv("HCCLX_MOE_SCATTER_ROWS")) c.moe_scatter_rows = static_cast<uint32_t>(std::strtoul(v, nullptr, 10));
     if (const char *v = std::getenv("HCCLX_STORE_THROUGH_UPTO")) c.store_through_upto = std::strtoull(v, nullptr, 10);
     c.ring_bytes = kSliceBytes * kSlices;
-    e = hipHostMalloc(reinterpret_cast<void **>(&c.h_ring), c.ring_bytes, hipHostMallocDefault);
+    e = hipHostMalloc(reinterpret_cast<void **>(&c.h_ring), c.ring_bytes, hipHostMallocCoherent);
     if (e != hipSuccess) {
         s->err = std::string("hipHostMalloc(descriptor ring): ") + hipGetErrorString(e);
         return;
@@ -253,6 +253,30 @@ int ring_reserve(DeviceCtx *ctx, size_t bytes, hipStream_t stream, char **h, cha
     return HCCL_SUCCESS;
 }
 
+// A launch table read out of pinned host memory by a kernel: what hipMemcpyAsync does with more than 16 KiB costs the
+// stream 18 to 33 us (24 to 256 KiB), this 3 to 7.  System-scope loads: the host rewrites the ring while the GPU runs.
+__global__ void __launch_bounds__(256) k_fetch_table(const uint64_t *h, uint64_t *d, uint32_t words)
+{
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i < words) d[i] = __hip_atomic_load(h + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+int upload_table(char *d, const char *h, size_t bytes, hipStream_t stream)
+{
+    constexpr size_t kInlineCopy = 16 * 1024;   // up to here the runtime copies inline: 2.8 us, the same as the kernel
+    if (bytes <= kInlineCopy) {
+        HCCLX_HIP(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, stream));
+        return HCCL_SUCCESS;
+    }
+    const uint32_t words = static_cast<uint32_t>((bytes + 7) / 8);   // both ends are 256-byte aligned slots
+    // not counted among the collective's kernels: it stands for a copy
+    hipLaunchKernelGGL(k_fetch_table, dim3((words + 255) / 256), dim3(256), 0, stream, reinterpret_cast<const uint64_t *>(h),
+                       reinterpret_cast<uint64_t *>(d), words);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail_hip(e, "launch table upload");
+    return HCCL_SUCCESS;
+}
+
 uint32_t grid_for(const DeviceCtx *ctx, uint64_t total_tiles)
 {
     uint64_t cap = static_cast<uint64_t>(ctx->num_cus) * ctx->blocks_per_cu;
@@ -270,15 +294,15 @@ size_t align256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 
 size_t PhasedLaunch::bytes() const
 {
-    return align256(sources.size() * sizeof(PhasedSource)) + align256(slabs.size() * sizeof(PhasedSlab)) + dsts.size() * sizeof(char *);
+    return align256(sources.size() * sizeof(PhasedSource)) + align256(slabs.size() * sizeof(CopySlab)) + dsts.size() * sizeof(char *);
 }
 PhasedTable PhasedLaunch::table(const char *d) const
 {
     PhasedTable t;
     t.sources = reinterpret_cast<const PhasedSource *>(d);
     d += align256(sources.size() * sizeof(PhasedSource));
-    t.slabs = reinterpret_cast<const PhasedSlab *>(d);
-    d += align256(slabs.size() * sizeof(PhasedSlab));
+    t.slabs = reinterpret_cast<const CopySlab *>(d);
+    d += align256(slabs.size() * sizeof(CopySlab));
     t.dsts = reinterpret_cast<char *const *>(d);
     t.nd = grid.nd;
     t.nslabs = static_cast<uint32_t>(slabs.size());
@@ -288,8 +312,8 @@ void PhasedLaunch::fill(char *h) const
 {
     std::memcpy(h, sources.data(), sources.size() * sizeof(PhasedSource));
     h += align256(sources.size() * sizeof(PhasedSource));
-    std::memcpy(h, slabs.data(), slabs.size() * sizeof(PhasedSlab));
-    h += align256(slabs.size() * sizeof(PhasedSlab));
+    std::memcpy(h, slabs.data(), slabs.size() * sizeof(CopySlab));
+    h += align256(slabs.size() * sizeof(CopySlab));
     std::memcpy(h, dsts.data(), dsts.size() * sizeof(char *));
 }
 
@@ -395,8 +419,9 @@ struct Batch {
     std::vector<SegWide> wide;   // instead of segs when maxn == kMaxWideFan
     int wide_unroll = 1;         // vectors per thread of the wide kernel
     uint32_t xcd_remap = 0;      // wide kernels: contiguous tile ranges per XCD (pays with 16 or more destinations)
-    std::vector<CopyBlock> blocks;   // instead of everything above: a list of blocks for the block copy kernel
-    int block_unroll = 2;
+    std::vector<CopyBlock> blocks;   // instead of everything above: a list of blocks for the block copy kernel,
+    std::vector<CopySlab> slabs;     // cut into these slabs
+    uint32_t slab_shift = 0;         // of 1 << slab_shift tiles
     PhasedLaunch phased;         // instead of everything above: a launch of the copy kernel that writes one output at a time
     uint32_t store_policy = kStoreStream;   // how the fold kernels store (fold.h)
     uint32_t waves = 0;          // non-zero: the one-store-per-wavefront kernel, this many wavefronts per workgroup
@@ -406,7 +431,7 @@ struct Batch {
     size_t bytes() const
     {
         if (!phased.slabs.empty()) return phased.bytes();
-        if (!blocks.empty()) return blocks.size() * sizeof(CopyBlock);
+        if (!blocks.empty()) return align256(blocks.size() * sizeof(CopyBlock)) + slabs.size() * sizeof(CopySlab);
         return align256(tile_end.size() * 8) + segs.size() * sizeof(SegDev) + wide.size() * sizeof(SegWide);
     }
 };
@@ -1020,6 +1045,7 @@ void fill_table(const Batch &b, char *h)
     }
     if (!b.blocks.empty()) {
         std::memcpy(h, b.blocks.data(), b.blocks.size() * sizeof(CopyBlock));
+        std::memcpy(h + align256(b.blocks.size() * sizeof(CopyBlock)), b.slabs.data(), b.slabs.size() * sizeof(CopySlab));
         return;
     }
     std::memcpy(h, b.tile_end.data(), b.tile_end.size() * 8);
@@ -1062,8 +1088,9 @@ int launch_batch(const DeviceCtx *ctx, const Batch &b, const char *d_table, hipS
         return HCCL_SUCCESS;
     }
     if (!b.blocks.empty()) {
-        const hipError_t be = launch_copy_blocks(reinterpret_cast<const CopyBlock *>(d_table), static_cast<uint32_t>(b.blocks.size()),
-                                                 static_cast<uint32_t>(b.total_tiles), b.block_unroll, stream);
+        const BlockTable tab{reinterpret_cast<const CopyBlock *>(d_table),
+                             reinterpret_cast<const CopySlab *>(d_table + align256(b.blocks.size() * sizeof(CopyBlock)))};
+        const hipError_t be = launch_copy_blocks(tab, static_cast<uint32_t>(b.slabs.size()), b.slab_shift, stream);
         if (be != hipSuccess) return fail_hip(be, "block copy kernel launch");
         return HCCL_SUCCESS;
     }
@@ -1147,7 +1174,8 @@ static int launch_built(DeviceCtx *ctx, const Built &built, hipStream_t st)
         int rc = ring_reserve(ctx, b.bytes(), st, &h, &d);
         if (rc != HCCL_SUCCESS) return rc;
         fill_table(b, h);
-        HCCLX_HIP(hipMemcpyAsync(d, h, b.bytes(), hipMemcpyHostToDevice, st));
+        rc = upload_table(d, h, b.bytes(), st);
+        if (rc != HCCL_SUCCESS) return rc;
         rc = launch_batch(ctx, b, d, st);
         if (rc != HCCL_SUCCESS) return rc;
     }
@@ -1343,10 +1371,10 @@ int hcclx_alltoallv_plan_create(const void *const *send, void *const *recv, cons
     Built built;
     Batch b;
     b.copy = true;
-    b.block_unroll = ctx->a2av_direct_unroll == 1 ? 1 : ctx->a2av_direct_unroll == 4 ? 4 : 2;
-    b.total_tiles = list_alltoallv_blocks(send, recv, send_counts, sdispls, rdispls, n, static_cast<uint32_t>(esz), b.block_unroll,
-                                          &b.blocks);
-    if (b.total_tiles > 0x7fffffffull) return fail(HCCL_E_PARA, "too much data for one launch");
+    list_alltoallv_blocks(send, recv, send_counts, sdispls, rdispls, n, static_cast<uint32_t>(esz), &b.blocks);
+    if (!b.blocks.empty() && !cut_slabs(b.blocks, kBlockTableSlabs, ~0u, &b.slabs, &b.slab_shift)) {
+        return fail(HCCL_E_PARA, "too much data for one launch");
+    }
     for (const CopyBlock &c : b.blocks) built.algo_bytes += 2 * c.bytes;
     if (!b.blocks.empty()) built.batches.push_back(std::move(b));
     return plan_from(ctx, built, plan);

@@ -41,7 +41,7 @@ struct DeviceCtx {
     // A single-destination chain launch that would have fewer four-vector tiles than this takes two vectors per
     // thread instead, to spread a small job over more CUs (HCCLX_WIDE_MIN_TILES; set from the CU count).
     uint32_t wide_min_tiles = 0;
-    uint32_t a2av_direct_unroll = 2;   // HCCLX_A2AV_DIRECT: 0 = off, 1 / 2 / 4 = vectors per thread and tile
+    bool a2av_direct = true;           // HCCLX_A2AV_DIRECT: AlltoAllV tables of up to 15 ranks in the kernel arguments (0 = off)
     // V kernels whose tables live on the device cannot know their tile count on the host and run as a
     // persistent grid of this many workgroups per CU.
     uint32_t v_blocks_per_cu = 2;
@@ -90,13 +90,12 @@ int ring_reserve(DeviceCtx *ctx, size_t bytes, hipStream_t stream, char **h, cha
 
 uint32_t grid_for(const DeviceCtx *ctx, uint64_t total_tiles);
 
-struct CopyBlock;
 
 // One launch of the copy kernel that writes one output at a time (kernels/vops.h).
 struct PhasedLaunch {
     std::vector<PhasedSource> sources;   // place = number of destinations
     std::vector<char *> dsts;            // sources.size() * grid.nd pointers, source s's at [s * nd, s * nd + ndst)
-    std::vector<PhasedSlab> slabs;
+    std::vector<CopySlab> slabs;
     PhasedGrid grid{};
     size_t bytes() const;       // the three arrays as they lie in the launch table
     void fill(char *h) const;
@@ -111,10 +110,14 @@ struct PhasedStream {
 // Turns streams into launches: streams that continue each other (source and every destination) are joined, and cut into
 // slabs as small as max_slabs of them allow; batches of up to batch_bytes are written to one place after the other.
 void build_phased(std::vector<PhasedStream> &streams, uint64_t batch_bytes, uint32_t max_slabs, std::vector<PhasedLaunch> *out);
-// The non-empty blocks of an AlltoAllV with host tables (row-major n x n, elements of esz bytes), with the
-// inclusive prefix of their tiles of `unroll` vectors per thread; returns the number of tiles.
-uint64_t list_alltoallv_blocks(const void *const *send, void *const *recv, const uint64_t *send_counts,
-                               const uint64_t *sdispls, const uint64_t *rdispls, uint32_t n, uint32_t esz, int unroll,
-                               std::vector<CopyBlock> *blocks);
+// The non-empty blocks of an AlltoAllV with host tables (row-major n x n, elements of esz bytes).
+void list_alltoallv_blocks(const void *const *send, void *const *recv, const uint64_t *send_counts, const uint64_t *sdispls,
+                           const uint64_t *rdispls, uint32_t n, uint32_t esz, std::vector<CopyBlock> *blocks);
+// Cuts blocks into slabs of 1 << shift tiles: the smallest power of two with which there are at most max_slabs of them,
+// numbered below max_at inside their block.  False when the launch would need more than 2^31 - 1 workgroups.
+bool cut_slabs(const std::vector<CopyBlock> &blocks, size_t max_slabs, uint32_t max_at, std::vector<CopySlab> *slabs, uint32_t *shift);
+
+// Queues the copy of a launch table from the pinned ring to its place in device memory.
+int upload_table(char *d, const char *h, size_t bytes, hipStream_t stream);
 
 }  // namespace hcclx

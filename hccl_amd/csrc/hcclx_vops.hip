@@ -48,27 +48,44 @@ int fill_ptrs(const void *const *send, void *const *recv, uint32_t n, VRankPtrs 
 
 namespace hcclx {
 
-uint64_t list_alltoallv_blocks(const void *const *send, void *const *recv, const uint64_t *send_counts,
-                               const uint64_t *sdispls, const uint64_t *rdispls, uint32_t n, uint32_t esz, int unroll,
-                               std::vector<CopyBlock> *blocks)
+void list_alltoallv_blocks(const void *const *send, void *const *recv, const uint64_t *send_counts, const uint64_t *sdispls,
+                           const uint64_t *rdispls, uint32_t n, uint32_t esz, std::vector<CopyBlock> *blocks)
 {
     blocks->clear();
     blocks->reserve(static_cast<size_t>(n) * n);
-    uint64_t tiles = 0;
     for (uint32_t i = 0; i < n; ++i) {
         for (uint32_t j = 0; j < n; ++j) {
             const uint64_t bytes = send_counts[i * n + j] * esz;
             if (bytes == 0) continue;
-            CopyBlock b;
-            b.src = static_cast<const char *>(send[i]) + sdispls[i * n + j] * esz;
-            b.dst = static_cast<char *>(recv[j]) + rdispls[j * n + i] * esz;
-            b.bytes = bytes;
-            tiles += v_tiles_of(bytes, reinterpret_cast<uint64_t>(b.dst), unroll);
-            b.tile_end = tiles;
-            blocks->push_back(b);
+            blocks->push_back({static_cast<const char *>(send[i]) + sdispls[i * n + j] * esz,
+                               static_cast<char *>(recv[j]) + rdispls[j * n + i] * esz, bytes});
         }
     }
-    return tiles;
+}
+
+bool cut_slabs(const std::vector<CopyBlock> &blocks, size_t max_slabs, uint32_t max_at, std::vector<CopySlab> *slabs, uint32_t *shift)
+{
+    std::vector<uint64_t> tiles(blocks.size());
+    uint64_t most = 0;
+    for (size_t b = 0; b < blocks.size(); ++b) {
+        tiles[b] = v_tiles_of(blocks[b].bytes, reinterpret_cast<uint64_t>(blocks[b].dst), 1);
+        most = tiles[b] > most ? tiles[b] : most;
+    }
+    if (max_slabs < blocks.size()) max_slabs = blocks.size();
+    uint64_t n = 0;
+    for (*shift = 0;; ++*shift) {
+        const uint64_t last = (1ull << *shift) - 1;
+        n = 0;
+        for (uint64_t t : tiles) n += (t + last) >> *shift;
+        if (n <= max_slabs && ((most + last) >> *shift) <= max_at) break;
+    }
+    if (n << *shift > 0x7fffffffull) return false;
+    slabs->clear();
+    slabs->reserve(n);
+    for (size_t b = 0; b < blocks.size(); ++b) {
+        for (uint64_t k = 0; k << *shift < tiles[b]; ++k) slabs->push_back({static_cast<uint32_t>(b), static_cast<uint32_t>(k)});
+    }
+    return true;
 }
 
 }  // namespace hcclx
@@ -89,56 +106,57 @@ int hcclx_alltoallv(const void *const *send, void *const *recv, const uint64_t *
     if (rc != HCCL_SUCCESS) return rc;
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (!tables_on_device) {
-        const int unroll = ctx->a2av_direct_unroll == 1 ? 1 : ctx->a2av_direct_unroll == 4 ? 4 : 2;
-        bool small = n <= kA2avDirectRanks && ctx->a2av_direct_unroll != 0;
+        std::vector<CopyBlock> blocks;
+        list_alltoallv_blocks(send, recv, send_counts, sdispls, rdispls, n, static_cast<uint32_t>(esz), &blocks);
+        if (blocks.empty()) return HCCL_SUCCESS;
+        std::vector<CopySlab> slabs;
+        uint32_t shift = 0;
+        bool small = n <= kA2avInlineRanks && ctx->a2av_direct;
         for (size_t k = 0; k < static_cast<size_t>(n) * n && small; ++k) {
             small = send_counts[k] <= 0xffffffffull && sdispls[k] <= 0xffffffffull && rdispls[k] <= 0xffffffffull;
         }
         if (small) {
-            // small host tables and their tile prefix ride in the kernel arguments: one small tile per workgroup,
-            // nothing is copied in front of the kernel
-            VRankPtrs16 p16;
-            A2avTablesDirect tabs;
-            std::memset(&p16, 0, sizeof(p16));
-            std::memset(&tabs, 0, sizeof(tabs));
+            // small host tables and their slabs ride in the kernel arguments: nothing is copied in front of the kernel
+            if (!cut_slabs(blocks, kA2avInlineSlabs, 256, &slabs, &shift)) return fail(HCCL_E_PARA, "too much data for one launch");
+            A2avInline tab;
+            tab.n = n;
+            tab.inv_n = 65536u / n + 1u;
+            tab.esz = static_cast<uint32_t>(esz);
+            uint8_t number[kA2avInlineBlocks];   // of the non-empty blocks in the n x n tables
+            uint32_t live = 0;
             for (uint32_t i = 0; i < n; ++i) {
-                p16.send[i] = ptrs.send[i];
-                p16.recv[i] = ptrs.recv[i];
-            }
-            uint64_t tiles = 0;
-            for (uint32_t i = 0; i < n; ++i) {
+                tab.send[i] = ptrs.send[i];
+                tab.recv[i] = ptrs.recv[i];
                 for (uint32_t j = 0; j < n; ++j) {
                     const uint32_t k = i * n + j;
-                    const uint64_t dst = reinterpret_cast<uint64_t>(ptrs.recv[j]) + rdispls[j * n + i] * esz;
-                    tiles += v_tiles_of(send_counts[k] * esz, dst, unroll);
-                    tabs.send_counts[k] = static_cast<uint32_t>(send_counts[k]);
-                    tabs.sdispls[k] = static_cast<uint32_t>(sdispls[k]);
-                    tabs.rdispls[k] = static_cast<uint32_t>(rdispls[j * n + i]);
-                    tabs.tile_end[k] = static_cast<uint32_t>(tiles);
+                    if (send_counts[k] != 0) number[live++] = static_cast<uint8_t>(k);
+                    tab.counts[k] = static_cast<uint32_t>(send_counts[k]);
+                    tab.sdispls[k] = static_cast<uint32_t>(sdispls[k]);
+                    tab.rdispls[k] = static_cast<uint32_t>(rdispls[j * n + i]);
                 }
             }
-            if (tiles == 0) return HCCL_SUCCESS;
-            if (tiles <= 0x7fffffffull) {
-                hipError_t e = launch_alltoallv_direct(p16, tabs, n, static_cast<uint32_t>(esz), static_cast<uint32_t>(tiles),
-                                                       unroll, st);
-                if (e != hipSuccess) return fail_hip(e, "alltoallv kernel launch");
-                return HCCL_SUCCESS;
+            for (size_t k = 0; k < slabs.size(); ++k) {
+                const uint32_t one = number[slabs[k].source] | slabs[k].at << 8;
+                tab.slabs[k >> 1] = (k & 1) ? (tab.slabs[k >> 1] | one << 16) : one;
             }
+            hipError_t e = launch_alltoallv_inline(tab, static_cast<uint32_t>(slabs.size()), shift, st);
+            if (e != hipSuccess) return fail_hip(e, "alltoallv kernel launch");
+            return HCCL_SUCCESS;
         }
-        // any other host table: the non-empty blocks as a list in device memory, one small tile per workgroup
-        std::vector<CopyBlock> blocks;
-        const uint64_t tiles = list_alltoallv_blocks(send, recv, send_counts, sdispls, rdispls, n, static_cast<uint32_t>(esz),
-                                                     unroll, &blocks);
-        if (blocks.empty()) return HCCL_SUCCESS;
-        if (tiles > 0x7fffffffull) return fail(HCCL_E_PARA, "too much data for one launch");
+        // any other host table: the non-empty blocks and their slabs in device memory
+        if (!cut_slabs(blocks, kBlockTableSlabs, ~0u, &slabs, &shift)) return fail(HCCL_E_PARA, "too much data for one launch");
+        const size_t block_bytes = (blocks.size() * sizeof(CopyBlock) + 255) & ~static_cast<size_t>(255);
+        const size_t bytes = block_bytes + slabs.size() * sizeof(CopySlab);
         char *h = nullptr;
         char *d = nullptr;
-        rc = ring_reserve(ctx, blocks.size() * sizeof(CopyBlock), st, &h, &d);
+        rc = ring_reserve(ctx, bytes, st, &h, &d);
         if (rc != HCCL_SUCCESS) return rc;
         std::memcpy(h, blocks.data(), blocks.size() * sizeof(CopyBlock));
-        HCCLX_HIP(hipMemcpyAsync(d, h, blocks.size() * sizeof(CopyBlock), hipMemcpyHostToDevice, st));
-        hipError_t e = launch_copy_blocks(reinterpret_cast<const CopyBlock *>(d), static_cast<uint32_t>(blocks.size()),
-                                          static_cast<uint32_t>(tiles), unroll, st);
+        std::memcpy(h + block_bytes, slabs.data(), slabs.size() * sizeof(CopySlab));
+        rc = upload_table(d, h, bytes, st);
+        if (rc != HCCL_SUCCESS) return rc;
+        const BlockTable tab{reinterpret_cast<const CopyBlock *>(d), reinterpret_cast<const CopySlab *>(d + block_bytes)};
+        hipError_t e = launch_copy_blocks(tab, static_cast<uint32_t>(slabs.size()), shift, st);
         if (e != hipSuccess) return fail_hip(e, "alltoallv kernel launch");
         return HCCL_SUCCESS;
     }

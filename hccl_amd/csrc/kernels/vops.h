@@ -57,7 +57,7 @@ struct VRankPtrs {
 
 // Count / displacement tables as the kernels read them.  Host tables of up to 15 ranks travel inside the kernel
 // arguments (no host-to-device copy is queued in front of the kernel); larger host tables become a list of
-// blocks in device memory; tables that already live on the device are read through pointers.
+// blocks and slabs in device memory; tables that already live on the device are read through pointers.
 struct A2avTablesPtr {
     const uint64_t *send_counts;
     const uint64_t *sdispls;
@@ -66,28 +66,39 @@ struct A2avTablesPtr {
     __device__ uint64_t sdispl(uint32_t p) const { return sdispls[p]; }
     __device__ uint64_t rdispl(uint32_t p) const { return rdispls[p]; }
 };
-// Host tables of up to 15 ranks with the tile prefix worked out by the host: a workgroup finds its block
-// with a binary search over kernel arguments (scalar loads), with no LDS table and no barrier, which is
-// what makes 4 KiB tiles affordable.  15 x 15 x 4 tables of uint32 = 3600 bytes of kernel arguments.
-constexpr uint32_t kA2avDirectRanks = 15;
-struct A2avTablesDirect {
-    uint32_t send_counts[kA2avDirectRanks * kA2avDirectRanks];
-    uint32_t sdispls[kA2avDirectRanks * kA2avDirectRanks];
-    uint32_t rdispls[kA2avDirectRanks * kA2avDirectRanks];   // indexed like send_counts: block (i, j) at i * n + j
-    uint32_t tile_end[kA2avDirectRanks * kA2avDirectRanks];  // inclusive prefix of tiles per block
-};
-// Base pointers for the launch with tables in the kernel arguments.
-struct VRankPtrs16 {
-    const char *send[16];
-    char *recv[16];
-};
-// One contiguous block to move, for host tables of any size: the host lists the non-empty blocks with the
-// inclusive prefix of their tiles; a workgroup finds its block with a binary search over that list (scalar loads).
+// Host tables.  A block of the exchange (source i to destination j) is cut into slabs of a power of two of 4 KiB tiles,
+// the last one as long as what is left, and a workgroup finds its slab by arithmetic and the block by the slab's
+// entry: two dependent scalar loads, where a search in a prefix of the blocks' tiles took 2 + log2(n * n).
 struct CopyBlock {
     const char *src;
     char *dst;
     uint64_t bytes;
-    uint64_t tile_end;
+};
+struct CopySlab {
+    uint32_t source;   // block (or source of a copy to several places)
+    uint32_t at;       // number of the slab inside it
+};
+// A launch's tables in device memory, for host tables of any size.
+struct BlockTable {
+    const CopyBlock *blocks;
+    const CopySlab *slabs;
+};
+constexpr uint32_t kBlockTableSlabs = 4096;   // at most, unless there are more blocks
+// The same in the kernel arguments, for up to 15 ranks and 32-bit counts: nothing is copied in front of the kernel.
+// Block b is source b / n, destination b % n.  A slab is 16 bits: block in the low eight, its number above.
+constexpr uint32_t kA2avInlineRanks = 15;
+constexpr uint32_t kA2avInlineBlocks = kA2avInlineRanks * kA2avInlineRanks;
+constexpr uint32_t kA2avInlineSlabs = 520;
+struct A2avInline {
+    const char *send[kA2avInlineRanks];
+    char *recv[kA2avInlineRanks];
+    uint32_t counts[kA2avInlineBlocks];
+    uint32_t sdispls[kA2avInlineBlocks];
+    uint32_t rdispls[kA2avInlineBlocks];
+    uint32_t slabs[kA2avInlineSlabs / 2];
+    uint32_t n;
+    uint32_t inv_n;   // 65536 / n + 1: b * inv_n >> 16 is b / n for every block number
+    uint32_t esz;
 };
 struct AgvTablesPtr {
     const uint64_t *counts;
@@ -107,14 +118,10 @@ struct PhasedSource {
 };
 constexpr uint32_t kPhasedSlabTilesLeast = 8;
 constexpr uint32_t kPhasedSlabTilesMost = 1024;   // 4 MiB
-struct PhasedSlab {
-    uint32_t source;
-    uint32_t at;      // number of the slab inside its source
-};
 // A launch's tables in device memory: sources, slabs and nd places per source.
 struct PhasedTable {
     const PhasedSource *sources;
-    const PhasedSlab *slabs;
+    const CopySlab *slabs;
     char *const *dsts;
     uint32_t nd;
     uint32_t nslabs;
@@ -140,8 +147,9 @@ struct AgvTablesInline {
     __device__ uint64_t displ(uint32_t i) const { return displs[i]; }
 };
 
-// blocks: device array of nblocks entries; unroll: 1, 2 or 4; grid = total number of tiles
-hipError_t launch_copy_blocks(const CopyBlock *blocks, uint32_t nblocks, uint32_t grid, int unroll, hipStream_t stream);
+// nslabs << slab_shift workgroups, slabs of 1 << slab_shift tiles
+hipError_t launch_copy_blocks(const BlockTable &tab, uint32_t nslabs, uint32_t slab_shift, hipStream_t stream);
+hipError_t launch_alltoallv_inline(const A2avInline &tab, uint32_t nslabs, uint32_t slab_shift, hipStream_t stream);
 // One batch after the other (grid z), each to one place after the other (grid y): per_batch slabs of slab_tiles tiles.
 struct PhasedGrid {
     uint32_t slab_tiles;
@@ -151,9 +159,6 @@ struct PhasedGrid {
 };
 hipError_t launch_phased_copy(const PhasedTable &tab, const PhasedGrid &grid, hipStream_t stream);
 hipError_t launch_phased_copy_inline(const PhasedInline &tab, const PhasedGrid &grid, hipStream_t stream);
-// unroll: 1, 2 or 4 vectors per thread and tile; grid = total number of tiles
-hipError_t launch_alltoallv_direct(const VRankPtrs16 &ptrs, const A2avTablesDirect &tabs, uint32_t n, uint32_t esz,
-                                   uint32_t grid, int unroll, hipStream_t stream);
 hipError_t launch_allgatherv_inline(const VRankPtrs &ptrs, const AgvTablesInline &tabs, uint32_t n, uint32_t esz,
                                     uint32_t grid, uint32_t tiles_per_block, hipStream_t stream);
 

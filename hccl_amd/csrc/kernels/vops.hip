@@ -87,7 +87,8 @@ __device__ __forceinline__ u32x4 ld16c(const char *p)
     }
 }
 
-template <int kCopyUnroll, bool kCached = false, typename DstFn>
+// kPolicy: how the vectors are stored (fold.h).
+template <int kCopyUnroll, bool kCached = false, uint32_t kPolicy = kStoreStream, typename DstFn>
 __device__ __forceinline__ void copy_tile(const char *src, uint64_t dst0, uint64_t bytes, uint64_t tl, uint32_t ndst,
                                           DstFn dst_of)
 {
@@ -107,7 +108,7 @@ __device__ __forceinline__ void copy_tile(const char *src, uint64_t dst0, uint64
         for (uint32_t d = 0; d < ndst; ++d) {
             char *db = dst_of(d) + head;
 #pragma unroll
-            for (int u = 0; u < kCopyUnroll; ++u) st16(db + (v0 + static_cast<uint64_t>(u) * kThreads) * 16, r[u]);
+            for (int u = 0; u < kCopyUnroll; ++u) st16x(db + (v0 + static_cast<uint64_t>(u) * kThreads) * 16, r[u], kPolicy);
         }
         return;
     }
@@ -131,7 +132,7 @@ __device__ __forceinline__ void copy_tile(const char *src, uint64_t dst0, uint64
 #pragma unroll
         for (int u = 0; u < kCopyUnroll; ++u) {
             const uint64_t vi = v0 + static_cast<uint64_t>(u) * kThreads;
-            if (vi < nvec) st16(dp + head + vi * 16, r[u]);
+            if (vi < nvec) st16x(dp + head + vi * 16, r[u], kPolicy);
         }
         if (has_edge) dp[edge_off] = edge;
     }
@@ -170,58 +171,39 @@ k_alltoallv(Ptrs ptrs, Tabs tabs, uint32_t n, uint32_t esz, uint32_t tiles_per_b
     }
 }
 
-// One tile per workgroup; the block of a tile is found in the host-made prefix that rides in the kernel
-// arguments.  Every index below is wave-uniform, so the table reads are scalar loads.
-template <int UNROLL>
-__global__ void __launch_bounds__(kThreads)
-k_alltoallv_direct(VRankPtrs16 ptrs, A2avTablesDirect tabs, uint32_t n, uint32_t esz)
+__device__ __forceinline__ CopySlab slab_of(const BlockTable &t, uint32_t k) { return t.slabs[k]; }
+__device__ __forceinline__ CopySlab slab_of(const A2avInline &t, uint32_t k)
 {
-    const uint32_t t = blockIdx.x;
-    uint32_t lo = 0;
-    uint32_t hi = n * n - 1;
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (tabs.tile_end[mid] > t) {
-            hi = mid;
-        } else {
-            lo = mid + 1;
-        }
-    }
-    const uint32_t p = lo;
-    const uint64_t tl = t - (p ? tabs.tile_end[p - 1] : 0);
-    const uint32_t i = p / n;
-    const uint32_t j = p - i * n;
-    const uint64_t bytes = static_cast<uint64_t>(tabs.send_counts[p]) * esz;
-    const char *src = ptrs.send[i] + static_cast<uint64_t>(tabs.sdispls[p]) * esz;
-    char *dst = ptrs.recv[j] + static_cast<uint64_t>(tabs.rdispls[p]) * esz;
-    copy_tile<UNROLL>(src, reinterpret_cast<uint64_t>(dst), bytes, tl, 1, [=](uint32_t) { return dst; });
+    const uint32_t two = t.slabs[k >> 1];
+    const uint32_t one = (k & 1u) ? two >> 16 : two & 0xffffu;
+    return {one & 255u, one >> 8};
+}
+__device__ __forceinline__ CopyBlock block_of(const BlockTable &t, uint32_t b) { return t.blocks[b]; }
+__device__ __forceinline__ CopyBlock block_of(const A2avInline &t, uint32_t b)
+{
+    const uint32_t i = b * t.inv_n >> 16;
+    const uint32_t j = b - i * t.n;
+    return {t.send[i] + static_cast<uint64_t>(t.sdispls[b]) * t.esz, t.recv[j] + static_cast<uint64_t>(t.rdispls[b]) * t.esz,
+            static_cast<uint64_t>(t.counts[b]) * t.esz};
 }
 
-// One tile per workgroup; its block is found in the host-made list (every index is wave-uniform: scalar loads).
-template <int UNROLL>
-__global__ void __launch_bounds__(kThreads)
-k_copy_blocks(const CopyBlock *__restrict__ blocks, uint32_t nblocks)
+// Blocks of any lengths, one 4 KiB tile per workgroup and one vector per thread, stored through the L2: bound by HBM.
+// A wavefront that loads and stores one vector per lane copies faster than one that moves two (1 GiB: 6.66 against
+// 6.22 TB/s with these stores, 6.54 streamed); 8 x 4096 x 7168 bf16 with two vectors, streamed, and the block searched
+// in a prefix: 151.3 us, this way 145.4.
+template <typename Tab>
+__global__ void __launch_bounds__(kThreads) k_copy_blocks(Tab tab, uint32_t slab_shift)
 {
-    const uint64_t t = blockIdx.x;
-    uint32_t lo = 0;
-    uint32_t hi = nblocks - 1;
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (blocks[mid].tile_end > t) {
-            hi = mid;
-        } else {
-            lo = mid + 1;
-        }
-    }
-    const uint64_t tl = t - (lo ? blocks[lo - 1].tile_end : 0);
-    const char *src = blocks[lo].src;
-    char *dst = blocks[lo].dst;
-    const uint64_t bytes = blocks[lo].bytes;
-    copy_tile<UNROLL>(src, reinterpret_cast<uint64_t>(dst), bytes, tl, 1, [=](uint32_t) { return dst; });
+    const CopySlab slab = slab_of(tab, blockIdx.x >> slab_shift);
+    const uint64_t tl = (static_cast<uint64_t>(slab.at) << slab_shift) + (blockIdx.x & ((1u << slab_shift) - 1u));
+    const CopyBlock b = block_of(tab, slab.source);
+    char *dst = b.dst;
+    if (tl >= v_tiles_of(b.bytes, reinterpret_cast<uint64_t>(dst), 1)) return;
+    copy_tile<1, false, kStoreThrough>(b.src, reinterpret_cast<uint64_t>(dst), b.bytes, tl, 1, [=](uint32_t) { return dst; });
 }
 
-__device__ __forceinline__ PhasedSlab phased_slab(const PhasedTable &t, uint32_t k) { return t.slabs[k]; }
-__device__ __forceinline__ PhasedSlab phased_slab(const PhasedInline &t, uint32_t k) { return {t.slabs[k] & 63u, t.slabs[k] >> 6}; }
+__device__ __forceinline__ CopySlab phased_slab(const PhasedTable &t, uint32_t k) { return t.slabs[k]; }
+__device__ __forceinline__ CopySlab phased_slab(const PhasedInline &t, uint32_t k) { return {t.slabs[k] & 63u, t.slabs[k] >> 6}; }
 // null: the source has no such place
 __device__ __forceinline__ char *phased_dst(const PhasedTable &t, uint32_t source, uint32_t d)
 {
@@ -240,7 +222,7 @@ __global__ void __launch_bounds__(kThreads) k_phased_copy(Tab tab, uint32_t slab
 {
     const uint32_t k = blockIdx.z * per_batch + (blockIdx.x >> slab_shift);
     if (k >= tab.nslabs) return;
-    const PhasedSlab slab = phased_slab(tab, k);
+    const CopySlab slab = phased_slab(tab, k);
     const uint64_t tl = (static_cast<uint64_t>(slab.at) << slab_shift) + (blockIdx.x & ((1u << slab_shift) - 1u));
     const PhasedSource &source = tab.sources[slab.source];
     const char *src = source.src;
@@ -290,15 +272,15 @@ hipError_t launch_alltoallv(const VRankPtrs &ptrs, const uint64_t *send_counts, 
     return hipGetLastError();
 }
 
-hipError_t launch_copy_blocks(const CopyBlock *blocks, uint32_t nblocks, uint32_t grid, int unroll, hipStream_t stream)
+hipError_t launch_copy_blocks(const BlockTable &tab, uint32_t nslabs, uint32_t slab_shift, hipStream_t stream)
 {
-    if (unroll == 1) {
-        HCCLX_LAUNCH((k_copy_blocks<1>), dim3(grid), dim3(kThreads), 0, stream, blocks, nblocks);
-    } else if (unroll == 2) {
-        HCCLX_LAUNCH((k_copy_blocks<2>), dim3(grid), dim3(kThreads), 0, stream, blocks, nblocks);
-    } else {
-        HCCLX_LAUNCH((k_copy_blocks<4>), dim3(grid), dim3(kThreads), 0, stream, blocks, nblocks);
-    }
+    HCCLX_LAUNCH((k_copy_blocks<BlockTable>), dim3(nslabs << slab_shift), dim3(kThreads), 0, stream, tab, slab_shift);
+    return hipGetLastError();
+}
+
+hipError_t launch_alltoallv_inline(const A2avInline &tab, uint32_t nslabs, uint32_t slab_shift, hipStream_t stream)
+{
+    HCCLX_LAUNCH((k_copy_blocks<A2avInline>), dim3(nslabs << slab_shift), dim3(kThreads), 0, stream, tab, slab_shift);
     return hipGetLastError();
 }
 
@@ -319,19 +301,6 @@ hipError_t launch_phased_copy(const PhasedTable &tab, const PhasedGrid &grid, hi
 hipError_t launch_phased_copy_inline(const PhasedInline &tab, const PhasedGrid &grid, hipStream_t stream)
 {
     return launch_phased(tab, grid, stream);
-}
-
-hipError_t launch_alltoallv_direct(const VRankPtrs16 &ptrs, const A2avTablesDirect &tabs, uint32_t n, uint32_t esz,
-                                   uint32_t grid, int unroll, hipStream_t stream)
-{
-    if (unroll == 1) {
-        HCCLX_LAUNCH((k_alltoallv_direct<1>), dim3(grid), dim3(kThreads), 0, stream, ptrs, tabs, n, esz);
-    } else if (unroll == 2) {
-        HCCLX_LAUNCH((k_alltoallv_direct<2>), dim3(grid), dim3(kThreads), 0, stream, ptrs, tabs, n, esz);
-    } else {
-        HCCLX_LAUNCH((k_alltoallv_direct<4>), dim3(grid), dim3(kThreads), 0, stream, ptrs, tabs, n, esz);
-    }
-    return hipGetLastError();
 }
 
 // One wavefront per row of n <= 64 counts: displs = exclusive prefix sum, totals[row] = the row's sum.

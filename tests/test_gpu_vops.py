@@ -108,6 +108,21 @@ def test_alltoallv_host_tables_of_any_rank_count_and_as_a_plan(n):
     plan.close()
 
 
+@pytest.mark.parametrize("n,least,most,hot", [
+    (2, 1, 9, 5 << 20),             # one block with more than 256 tiles and three of a few bytes
+    (3, 4095, 4097, 0),             # one or two tiles each
+    (15, 0, 60000, 3 << 20),        # the most ranks whose tables ride in the kernel arguments, 225 blocks
+    (16, 0, 60000, 3 << 20),        # the fewest whose tables lie in memory
+    (64, 0, 9000, 1 << 20),         # a table of more than 16 KiB, read by a kernel from pinned memory
+])
+def test_alltoallv_slabs_of_unequal_blocks(n, least, most, hot):
+    rng = np.random.default_rng(n)
+    m = rng.integers(least, most + 1, size=(n, n))
+    if hot:
+        m[n - 1][0] = hot + 13
+    run_a2av(m.tolist(), T.INT8, rng, send_pad=n % 7)
+
+
 def test_alltoallv_all_zero_and_single_rank():
     rng = np.random.default_rng(1)
     run_a2av([[0, 0], [0, 0]], T.FP32, rng)
