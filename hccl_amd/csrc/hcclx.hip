@@ -142,7 +142,10 @@ void init_slot(DeviceSlot *s, int dev)
         c.waves_pieces = b > kWavePieces ? static_cast<uint32_t>(kWavePieces) : static_cast<uint32_t>(b);
     }
     if (const char *v = std::getenv("HCCLX_AGV_PHASED_FROM")) c.agv_phased_from = std::strtoull(v, nullptr, 10);
-    if (const char *v = std::getenv("HCCLX_MOE_SCATTER_ROWS")) c.moe_scatter_rows = static_cast<uint32_t>(std::strtoul(v, nullptr, 10));
+    if (const char *v = std::getenv("HCCLX_MOE_SCATTER_ROWS")) {
+        const unsigned long b = std::strtoul(v, nullptr, 10);
+        if (b == 1 || b == 2) c.moe_scatter_rows = static_cast<uint32_t>(b);
+    }
     if (const char *v = std::getenv("HCCLX_STORE_THROUGH_UPTO")) c.store_through_upto = std::strtoull(v, nullptr, 10);
     c.ring_bytes = kSliceBytes * kSlices;
     e = hipHostMalloc(reinterpret_cast<void **>(&c.h_ring), c.ring_bytes, hipHostMallocCoherent);

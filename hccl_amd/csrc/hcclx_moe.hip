@@ -38,6 +38,13 @@ __device__ __forceinline__ const MoePtrs &as_mutable_dev(const MoeConstPtrs &c)
     return reinterpret_cast<const MoePtrs &>(c);   // same layout; the landing addresses are only read through
 }
 
+MoePtrs as_mutable(const MoeConstPtrs &c)
+{
+    MoePtrs m;
+    for (uint32_t i = 0; i < kMoeMaxRanks; ++i) m.p[i] = const_cast<void *>(c.p[i]);
+    return m;
+}
+
 // Workspace layout (uint32): base[n][n][chunks] (chunk fastest) -- first the per-chunk histogram, then,
 // in place, its exclusive prefix over the chunks -- followed by row_start[n][n].
 __host__ __device__ inline uint32_t chunks_of(uint32_t entries) { return (entries + kMoeChunk - 1) / kMoeChunk; }
@@ -387,163 +394,213 @@ k_moe_gather_combine(MoeConstPtrs expert, MoeConstPtrs dest, MoeConstPtrs perm, 
 }
 
 // ---- rows of at least kLongRow vectors ----------------------------------------------------------------------
-// A workgroup moves one run of ONE row, so the entry, its destination and where it lands are the same for every
-// thread: they are fetched with scalar loads, and no thread divides or looks anything up.
-constexpr uint32_t kLongRow = 128;
+// A wavefront moves one piece (64 vectors, 1 KiB) of ONE row, so the entry, its destination and where it lands are the
+// same for every lane: they are fetched with scalar loads, and no lane divides or looks anything up.  Pieces and not
+// runs of a workgroup's width: a row of 7168 bf16 is 14 whole pieces, but 3.5 runs of 256 vectors.
+// From 48 vectors on: 8 x 2000 tokens, top-2, routing and both directions with rows of 48 vectors 24.1 us against 32.6 for
+// the kernels above, with 32 (half of every wavefront idle) 23.7 against 24.9 and 8 x 2000 with 17 24.7 against 20.7.
+constexpr uint32_t kLongRow = 48;
+constexpr uint32_t kPieceVecs = 64;
+constexpr uint32_t kPiecesPerBlock = 4;
+constexpr uint32_t kXcds = 8;
 
-struct RowRuns {
-    uint32_t per_row;   // runs a row is cut into
-    uint32_t vecs;      // vectors per run (the last one may be shorter)
+struct RowPieces {
+    uint32_t per_row;   // pieces of a row
+    uint32_t total;     // pieces of all rows of a rank
+    uint32_t groups;    // dispatch: wavefronts that share a token's piece, S entries of it each
 };
-inline RowRuns row_runs(uint32_t vpr, uint32_t most)
+// A launch has at most 2^32 work-items along x: more rows than that take several launches, each with its pointers moved on.
+constexpr uint64_t kMostBlocks = 0xffff00;
+// Rows of one launch at most; 0: not even one row fits.
+inline uint32_t rows_per_launch(uint32_t vpr, uint32_t groups)
 {
-    RowRuns r;
-    r.per_row = (vpr + most - 1) / most;
-    r.vecs = (vpr + r.per_row - 1) / r.per_row;
-    return r;
+    const uint64_t per_row = (static_cast<uint64_t>(vpr) + kPieceVecs - 1) / kPieceVecs;
+    const uint64_t rows = kMostBlocks / kXcds / groups * kXcds * kPiecesPerBlock / per_row;
+    return rows > 0xffffffffull ? 0xffffffffu : static_cast<uint32_t>(rows);
+}
+inline RowPieces row_pieces(uint32_t rows, uint32_t vpr, uint32_t groups)
+{
+    const uint32_t per_row = static_cast<uint32_t>((static_cast<uint64_t>(vpr) + kPieceVecs - 1) / kPieceVecs);
+    return {per_row, rows * per_row, groups};
+}
+// The same arrays from `bytes` on.
+inline MoeConstPtrs moved_on(MoeConstPtrs a, uint32_t n, uint64_t bytes)
+{
+    for (uint32_t i = 0; i < n; ++i) a.p[i] = static_cast<const char *>(a.p[i]) + bytes;
+    return a;
 }
 
-// Scatter one row per entry straight to where the AlltoAllV would put it in recv[dest[e]].  Runs of up to 512
-// vectors, two per thread.
-__global__ void __launch_bounds__(256)
-k_moe_scatter_long(MoeConstPtrs tokens, MoeConstPtrs dest, MoeConstPtrs perm, MoePtrs dst, uint32_t n, uint32_t topk, uint32_t vpr,
-                   RowRuns runs, uint32_t esz, const uint64_t *sdispls, const uint64_t *rdispls)
-{
-    const uint32_t i = blockIdx.y;
-    const uint32_t e = blockIdx.x / runs.per_row;
-    const uint32_t c = blockIdx.x - e * runs.per_row;
-    const uint32_t p = static_cast<const uint32_t *>(perm.p[i])[e];
-    if (p == kDropped) return;
-    const uint32_t j = static_cast<uint32_t>(static_cast<const int32_t *>(dest.p[i])[e]);
-    if (j >= n) return;
-    char *base = landing(dst, i, j, n, esz, sdispls, rdispls);
-    const char *from = static_cast<const char *>(tokens.p[i]) + static_cast<uint64_t>(e / topk) * vpr * 16;
-    char *to = base + static_cast<uint64_t>(p) * vpr * 16;
-    const uint32_t lo = c * runs.vecs;
-    const uint32_t hi = lo + runs.vecs < vpr ? lo + runs.vecs : vpr;
-    const uint32_t v0 = lo + threadIdx.x;
-    const uint32_t v1 = v0 + 256;
-    u32x4 x0, x1;
-    if (v0 < hi) x0 = ld16(from + static_cast<uint64_t>(v0) * 16);
-    if (v1 < hi) x1 = ld16(from + static_cast<uint64_t>(v1) * 16);
-    if (v0 < hi) st16(to + static_cast<uint64_t>(v0) * 16, x0);
-    if (v1 < hi) st16(to + static_cast<uint64_t>(v1) * 16, x1);
-}
-
-// The same scatter with R consecutive entries per workgroup: the look-ups of all R rows (entry, destination, landing
-// offset: three dependent scalar loads each) are issued together and all 2 R vectors of a thread are loaded before
-// the first is stored.
-template <int R>
-__global__ void __launch_bounds__(256)
-k_moe_scatter_rows(MoeConstPtrs tokens, MoeConstPtrs dest, MoeConstPtrs perm, MoePtrs dst, uint32_t n, uint32_t entries, uint32_t topk,
-                   uint32_t vpr, RowRuns runs, uint32_t esz, const uint64_t *sdispls, const uint64_t *rdispls)
+// Dispatch: a piece of a token goes to S of its entries' rows, loaded once; what is left of topk / S goes to other
+// workgroups, eight apart, so that they run on the same XCD and find the piece in its L2 (kCached).  Bound: HBM.  8 x 4096
+// tokens, top-2, 7168 bf16 (1409 MB): 219 us where two vectors of two entries per thread, each read by itself, took 293;
+// 8 x 64 tokens, top-8: 11.5 against 22.5.
+template <int S, uint32_t kPolicy, bool kCached>
+__global__ void __launch_bounds__(kPieceVecs * kPiecesPerBlock)
+k_moe_scatter_pieces(MoeConstPtrs tokens, MoeConstPtrs dest, MoeConstPtrs perm, MoePtrs recv, uint32_t n, uint32_t topk, uint32_t vpr,
+                     RowPieces pieces, uint32_t esz, const uint64_t *sdispls, const uint64_t *rdispls)
 {
     const uint32_t i = blockIdx.y;
-    const uint32_t g = blockIdx.x / runs.per_row;
-    const uint32_t c = blockIdx.x - g * runs.per_row;
-    const uint32_t lo = c * runs.vecs;
-    const uint32_t hi = lo + runs.vecs < vpr ? lo + runs.vecs : vpr;
-    const uint32_t v0 = lo + threadIdx.x;
-    const uint32_t v1 = v0 + 256;
-    const uint32_t *pm = static_cast<const uint32_t *>(perm.p[i]);
-    const int32_t *dt = static_cast<const int32_t *>(dest.p[i]);
-    uint32_t p[R];
-    uint32_t j[R];
+    const uint32_t span = kXcds * pieces.groups;
+    const uint32_t hi = blockIdx.x / span;
+    const uint32_t in_span = blockIdx.x - hi * span;
+    const uint32_t block = hi * kXcds + in_span % kXcds;
+    const uint32_t piece = __builtin_amdgcn_readfirstlane(block * kPiecesPerBlock + threadIdx.x / kPieceVecs);
+    if (piece >= pieces.total) return;
+    const uint32_t t = piece / pieces.per_row;
+    const uint32_t v0 = (piece - t * pieces.per_row) * kPieceVecs;
+    const uint32_t lane = threadIdx.x % kPieceVecs;
+    const uint32_t lane_off = lane * 16;
+    const bool inside = lane < vpr - v0;
+    const char *from = static_cast<const char *>(tokens.p[i]) + (static_cast<uint64_t>(t) * vpr + v0) * 16;
+    u32x4 x = {0, 0, 0, 0};
+    if (inside) x = kCached ? ld16_cached(from + lane_off) : ld16(from + lane_off);
+    const uint32_t *pm = static_cast<const uint32_t *>(perm.p[i]) + static_cast<uint64_t>(t) * topk;
+    const int32_t *dt = static_cast<const int32_t *>(dest.p[i]) + static_cast<uint64_t>(t) * topk;
+    const uint32_t first = in_span / kXcds * S;
+    uint32_t p[S];
+    uint32_t j[S];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const uint32_t e = g * R + r;
-        const uint32_t at = e < entries ? e : entries - 1;   // a group behind the last entry repeats it and stores nothing
-        p[r] = pm[at];
-        j[r] = static_cast<uint32_t>(dt[at]);
-        if (e >= entries) p[r] = kDropped;
+    for (int s = 0; s < S; ++s) {
+        const uint32_t e = first + s;
+        const uint32_t at = e < topk ? e : topk - 1;   // an entry behind the token's last repeats it and stores nothing
+        p[s] = pm[at];
+        j[s] = static_cast<uint32_t>(dt[at]);
+        if (e >= topk) p[s] = kDropped;
     }
-    const char *from[R];
-    char *to[R];
-    bool ok[R];
+    char *to[S];
+    bool ok[S];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-        ok[r] = p[r] != kDropped && j[r] < n;
-        const uint32_t e = g * R + r;
-        char *base = landing(dst, i, ok[r] ? j[r] : 0u, n, esz, sdispls, rdispls);
-        from[r] = static_cast<const char *>(tokens.p[i]) + static_cast<uint64_t>((e < entries ? e : entries - 1) / topk) * vpr * 16;
-        to[r] = base + static_cast<uint64_t>(ok[r] ? p[r] : 0u) * vpr * 16;
-    }
-    u32x4 x[R][2];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        if (ok[r] && v0 < hi) x[r][0] = ld16(from[r] + static_cast<uint64_t>(v0) * 16);
-        if (ok[r] && v1 < hi) x[r][1] = ld16(from[r] + static_cast<uint64_t>(v1) * 16);
+    for (int s = 0; s < S; ++s) {
+        ok[s] = p[s] != kDropped && j[s] < n;
+        to[s] = landing(recv, i, ok[s] ? j[s] : 0u, n, esz, sdispls, rdispls) + (static_cast<uint64_t>(ok[s] ? p[s] : 0u) * vpr + v0) * 16;
     }
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-        if (ok[r] && v0 < hi) st16(to[r] + static_cast<uint64_t>(v0) * 16, x[r][0]);
-        if (ok[r] && v1 < hi) st16(to[r] + static_cast<uint64_t>(v1) * 16, x[r][1]);
+    for (int s = 0; s < S; ++s) {
+        if (ok[s] && inside) st16x(to[s] + lane_off, x, kPolicy);
     }
 }
 
-// Gather the rows of a token's entries from where dispatch put them in expert[dest[.]] and add them.  Runs of up
-// to 256 vectors, one per thread.  DT = int8 moves bytes (topk == 1).
+// Gather the rows of a token's entries from where dispatch put them in expert[dest[.]] and add them.  The entries one
+// after the other: the look-ups of several at once, by scalar loads or one lane each, measured no faster (8 x 4096,
+// top-2, 7168 bf16: 220 us, two at once 221 and 251, runs of 224 vectors in 256 threads 230).  DT = int8 moves bytes
+// (topk == 1).
 template <int DT>
-__global__ void __launch_bounds__(256)
-k_moe_gather_long(MoeConstPtrs rows, MoeConstPtrs dest, MoeConstPtrs perm, MoePtrs out, uint32_t n, uint32_t topk, uint32_t vpr,
-                  RowRuns runs, uint32_t esz, const uint64_t *sdispls, const uint64_t *rdispls)
+__global__ void __launch_bounds__(kPieceVecs * kPiecesPerBlock)
+k_moe_gather_pieces(MoeConstPtrs rows, MoeConstPtrs dest, MoeConstPtrs perm, MoePtrs out, uint32_t n, uint32_t topk, uint32_t vpr,
+                    RowPieces pieces, uint32_t esz, const uint64_t *sdispls, const uint64_t *rdispls)
 {
     using V = Vec16<DT>;
     using C = typename V::C;
     constexpr int NE = V::NE;
     const uint32_t i = blockIdx.y;
-    const uint32_t t = blockIdx.x / runs.per_row;
-    const uint32_t c = blockIdx.x - t * runs.per_row;
-    const uint32_t lo = c * runs.vecs;
-    const uint32_t hi = lo + runs.vecs < vpr ? lo + runs.vecs : vpr;
-    const uint32_t v = lo + threadIdx.x;
-    const uint32_t *pm = static_cast<const uint32_t *>(perm.p[i]);
-    const int32_t *dt = static_cast<const int32_t *>(dest.p[i]);
+    const uint32_t piece = __builtin_amdgcn_readfirstlane(blockIdx.x * kPiecesPerBlock + threadIdx.x / kPieceVecs);
+    if (piece >= pieces.total) return;
+    const uint32_t t = piece / pieces.per_row;
+    const uint32_t v0 = (piece - t * pieces.per_row) * kPieceVecs;
+    const uint32_t lane = threadIdx.x % kPieceVecs;
+    const uint32_t lane_off = lane * 16;
+    if (lane >= vpr - v0) return;
+    const uint32_t *pm = static_cast<const uint32_t *>(perm.p[i]) + static_cast<uint64_t>(t) * topk;
+    const int32_t *dt = static_cast<const int32_t *>(dest.p[i]) + static_cast<uint64_t>(t) * topk;
     C acc[NE];
     bool have = false;
 #pragma unroll
     for (int k = 0; k < NE; ++k) acc[k] = C(0);
-    for (uint32_t j = 0; j < topk; ++j) {
-        const uint64_t e = static_cast<uint64_t>(t) * topk + j;
+    for (uint32_t e = 0; e < topk; ++e) {
         const uint32_t p = pm[e];
-        if (p == kDropped) continue;
         const uint32_t d = static_cast<uint32_t>(dt[e]);
-        if (d >= n) continue;
-        const char *base = landing(as_mutable_dev(rows), i, d, n, esz, sdispls, rdispls);
-        if (v < hi) {
-            C x[NE];
-            V::unpack(ld16(base + (static_cast<uint64_t>(p) * vpr + v) * 16), x);
-            if (!have) {
+        if (p == kDropped || d >= n) continue;
+        const char *from = landing(as_mutable_dev(rows), i, d, n, esz, sdispls, rdispls) + (static_cast<uint64_t>(p) * vpr + v0) * 16;
+        C x[NE];
+        V::unpack(ld16(from + lane_off), x);
+        if (!have) {
 #pragma unroll
-                for (int k = 0; k < NE; ++k) acc[k] = x[k];
-            } else {
+            for (int k = 0; k < NE; ++k) acc[k] = x[k];
+        } else {
 #pragma unroll
-                for (int k = 0; k < NE; ++k) acc[k] = V::template combine<HCCL_REDUCE_SUM>(x[k], acc[k]);
-            }
+            for (int k = 0; k < NE; ++k) acc[k] = V::template combine<HCCL_REDUCE_SUM>(x[k], acc[k]);
         }
         have = true;
     }
-    if (v < hi) st16(static_cast<char *>(out.p[i]) + (static_cast<uint64_t>(t) * vpr + v) * 16, V::pack(acc));
+    st16(static_cast<char *>(out.p[i]) + (static_cast<uint64_t>(t) * vpr + v0) * 16 + lane_off, V::pack(acc));
 }
 
-hipError_t launch_gather_long(int kind, dim3 grid, hipStream_t st, const MoeConstPtrs &rows, const MoeConstPtrs &dest,
-                              const MoeConstPtrs &perm, const MoePtrs &out, uint32_t n, uint32_t topk, uint32_t vpr, RowRuns runs,
-                              uint32_t esz, const uint64_t *sdispls, const uint64_t *rdispls)
+// Which entries share a wavefront, and how rows are stored.  Tokens of up to kWarmTokens in all are usually still in the
+// Infinity Cache, just written by the layer in front, and stay there when the stores stream past it: with four entries
+// and more, two per wavefront (8 x 1024 tokens, top-8, 4096 bf16: 84 us; 131 with the caches flushed).  Everything else
+// reads each piece past the caches, once for up to four entries, and writes through the L2 (the same case: 104 and 106;
+// top-2 of 8 x 4096 x 7168: 222 against 235 to 240; 8 x 4096 x 4096, top-8: 403 against 481).
+constexpr uint64_t kWarmTokens = 128ull << 20;
+
+int launch_scatter_pieces(uint32_t per_wave, hipStream_t st, const MoeConstPtrs &tokens, const MoeConstPtrs &dest,
+                          const MoeConstPtrs &perm, const MoePtrs &recv, uint32_t n, uint32_t rows, uint32_t topk, uint32_t vpr,
+                          uint32_t esz, const uint64_t *sdispls, const uint64_t *rdispls)
 {
-    if (kind == HCCL_DATA_TYPE_FP32) {
-        HCCLX_LAUNCH(k_moe_gather_long<HCCL_DATA_TYPE_FP32>, grid, dim3(256), 0, st, rows, dest, perm, out, n, topk,
-                           vpr, runs, esz, sdispls, rdispls);
-    } else if (kind == HCCL_DATA_TYPE_FP16) {
-        HCCLX_LAUNCH(k_moe_gather_long<HCCL_DATA_TYPE_FP16>, grid, dim3(256), 0, st, rows, dest, perm, out, n, topk,
-                           vpr, runs, esz, sdispls, rdispls);
-    } else if (kind == HCCL_DATA_TYPE_BFP16) {
-        HCCLX_LAUNCH(k_moe_gather_long<HCCL_DATA_TYPE_BFP16>, grid, dim3(256), 0, st, rows, dest, perm, out, n, topk,
-                           vpr, runs, esz, sdispls, rdispls);
-    } else {
-        HCCLX_LAUNCH(k_moe_gather_long<HCCL_DATA_TYPE_INT8>, grid, dim3(256), 0, st, rows, dest, perm, out, n, topk,
-                           vpr, runs, esz, sdispls, rdispls);
+    const bool warm = per_wave == 0 && topk >= 4 && static_cast<uint64_t>(rows) * n <= kWarmTokens / 16 / vpr;
+    const uint32_t s = per_wave != 0 ? per_wave : warm ? 2u : topk >= 3 ? 4u : topk;
+    const uint32_t groups = (topk + s - 1) / s;
+    const uint32_t most = rows_per_launch(vpr, groups);
+    if (most == 0) return fail(HCCL_E_PARA, "too much data for one launch");
+    const dim3 block(kPieceVecs * kPiecesPerBlock);
+    for (uint32_t at = 0; at < rows;) {
+        const uint32_t take = rows - at < most ? rows - at : most;
+        const RowPieces pieces = row_pieces(take, vpr, groups);
+        const MoeConstPtrs tk = moved_on(tokens, n, static_cast<uint64_t>(at) * vpr * 16);
+        const MoeConstPtrs ds = moved_on(dest, n, static_cast<uint64_t>(at) * topk * 4);
+        const MoeConstPtrs pm = moved_on(perm, n, static_cast<uint64_t>(at) * topk * 4);
+        const dim3 grid((pieces.total + kPiecesPerBlock * kXcds - 1) / (kPiecesPerBlock * kXcds) * kXcds * groups, n);
+        if (warm) {
+            HCCLX_LAUNCH((k_moe_scatter_pieces<2, kStoreStream, true>), grid, block, 0, st, tk, ds, pm, recv, n, topk, vpr, pieces, esz,
+                         sdispls, rdispls);
+        } else if (s == 1) {
+            HCCLX_LAUNCH((k_moe_scatter_pieces<1, kStoreThrough, false>), grid, block, 0, st, tk, ds, pm, recv, n, topk, vpr, pieces,
+                         esz, sdispls, rdispls);
+        } else if (s == 2) {
+            HCCLX_LAUNCH((k_moe_scatter_pieces<2, kStoreThrough, false>), grid, block, 0, st, tk, ds, pm, recv, n, topk, vpr, pieces,
+                         esz, sdispls, rdispls);
+        } else {
+            HCCLX_LAUNCH((k_moe_scatter_pieces<4, kStoreThrough, false>), grid, block, 0, st, tk, ds, pm, recv, n, topk, vpr, pieces,
+                         esz, sdispls, rdispls);
+        }
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return fail_hip(e, "moe dispatch kernel");
+        at += take;
     }
-    return hipGetLastError();
+    return HCCL_SUCCESS;
+}
+
+int launch_gather_pieces(int kind, hipStream_t st, const MoeConstPtrs &rows, const MoeConstPtrs &dest, const MoeConstPtrs &perm,
+                         const MoeConstPtrs &out, uint32_t n, uint32_t tokens, uint32_t topk, uint32_t vpr, uint32_t esz,
+                         const uint64_t *sdispls, const uint64_t *rdispls)
+{
+    const uint32_t most = rows_per_launch(vpr, 1);
+    if (most == 0) return fail(HCCL_E_PARA, "too much data for one launch");
+    const dim3 block(kPieceVecs * kPiecesPerBlock);
+    for (uint32_t at = 0; at < tokens;) {
+        const uint32_t take = tokens - at < most ? tokens - at : most;
+        const RowPieces pieces = row_pieces(take, vpr, 1);
+        const MoePtrs to = as_mutable(moved_on(out, n, static_cast<uint64_t>(at) * vpr * 16));
+        const MoeConstPtrs ds = moved_on(dest, n, static_cast<uint64_t>(at) * topk * 4);
+        const MoeConstPtrs pm = moved_on(perm, n, static_cast<uint64_t>(at) * topk * 4);
+        const dim3 grid((pieces.total + kPiecesPerBlock - 1) / kPiecesPerBlock, n);
+        if (kind == HCCL_DATA_TYPE_FP32) {
+            HCCLX_LAUNCH(k_moe_gather_pieces<HCCL_DATA_TYPE_FP32>, grid, block, 0, st, rows, ds, pm, to, n, topk, vpr, pieces, esz,
+                         sdispls, rdispls);
+        } else if (kind == HCCL_DATA_TYPE_FP16) {
+            HCCLX_LAUNCH(k_moe_gather_pieces<HCCL_DATA_TYPE_FP16>, grid, block, 0, st, rows, ds, pm, to, n, topk, vpr, pieces, esz,
+                         sdispls, rdispls);
+        } else if (kind == HCCL_DATA_TYPE_BFP16) {
+            HCCLX_LAUNCH(k_moe_gather_pieces<HCCL_DATA_TYPE_BFP16>, grid, block, 0, st, rows, ds, pm, to, n, topk, vpr, pieces, esz,
+                         sdispls, rdispls);
+        } else {
+            HCCLX_LAUNCH(k_moe_gather_pieces<HCCL_DATA_TYPE_INT8>, grid, block, 0, st, rows, ds, pm, to, n, topk, vpr, pieces, esz,
+                         sdispls, rdispls);
+        }
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return fail_hip(e, "moe gather-combine kernel");
+        at += take;
+    }
+    return HCCL_SUCCESS;
 }
 
 int check_ranks(uint32_t n)
@@ -564,13 +621,6 @@ int fill(const void *const *in, uint32_t n, MoeConstPtrs *out, const char *what,
         out->p[i] = in[i];
     }
     return HCCL_SUCCESS;
-}
-
-MoePtrs as_mutable(const MoeConstPtrs &c)
-{
-    MoePtrs m;
-    for (uint32_t i = 0; i < kMoeMaxRanks; ++i) m.p[i] = const_cast<void *>(c.p[i]);
-    return m;
 }
 
 }  // namespace
@@ -715,25 +765,8 @@ int hcclx_moe_dispatch(const void *const *tokens, const int32_t *const *dest, co
     if (rc != HCCL_SUCCESS) return rc;
     const uint32_t vpr = static_cast<uint32_t>(row_bytes / 16);
     if (vpr >= kLongRow) {
-        const RowRuns runs = row_runs(vpr, 512);
-        const uint32_t rows = device_ctx()->moe_scatter_rows;
-        if (rows == 2) {   // two entries per workgroup: 162.2 against 165.4 us for route + dispatch of 8 x 4096 x 7168 bf16 (four: 281.6)
-            const uint64_t groups = (static_cast<uint64_t>(entries) + 1) / 2 * runs.per_row;
-            if (groups > 0x7fffffffull) return fail(HCCL_E_PARA, "too much data for one launch");
-            HCCLX_LAUNCH(k_moe_scatter_rows<2>, dim3(static_cast<uint32_t>(groups), n), dim3(256), 0, static_cast<hipStream_t>(stream),
-                         s, d, p, as_mutable(o), n, entries, topk, vpr, runs, static_cast<uint32_t>(esz), sdispls, rdispls);
-            hipError_t re = hipGetLastError();
-            if (re != hipSuccess) return fail_hip(re, "moe dispatch kernel");
-            return HCCL_SUCCESS;
-        }
-        const uint64_t long_blocks = static_cast<uint64_t>(entries) * runs.per_row;
-        if (long_blocks > 0x7fffffffull) return fail(HCCL_E_PARA, "too much data for one launch");
-        HCCLX_LAUNCH(k_moe_scatter_long, dim3(static_cast<uint32_t>(long_blocks), n), dim3(256), 0,
-                           static_cast<hipStream_t>(stream), s, d, p, as_mutable(o), n, topk, vpr, runs, static_cast<uint32_t>(esz),
-                           sdispls, rdispls);
-        hipError_t le = hipGetLastError();
-        if (le != hipSuccess) return fail_hip(le, "moe dispatch kernel");
-        return HCCL_SUCCESS;
+        return launch_scatter_pieces(device_ctx()->moe_scatter_rows, static_cast<hipStream_t>(stream), s, d, p, as_mutable(o), n,
+                                     entries / topk, topk, vpr, static_cast<uint32_t>(esz), sdispls, rdispls);
     }
     const uint64_t blocks = (static_cast<uint64_t>(entries) * vpr + 511) / 512;
     if (blocks > 0x7fffffffull) return fail(HCCL_E_PARA, "too much data for one launch");
@@ -774,13 +807,7 @@ int hcclx_moe_gather_combine(const void *const *expert, const int32_t *const *de
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int kind = topk == 1 ? HCCL_DATA_TYPE_INT8 : dtype;
     if (vpr >= kLongRow) {
-        const RowRuns runs = row_runs(vpr, 256);
-        const uint64_t long_blocks = static_cast<uint64_t>(tokens) * runs.per_row;
-        if (long_blocks > 0x7fffffffull) return fail(HCCL_E_PARA, "too much data for one launch");
-        const hipError_t le = launch_gather_long(kind, dim3(static_cast<uint32_t>(long_blocks), n), st, s, d, p, as_mutable(o), n,
-                                                       topk, vpr, runs, static_cast<uint32_t>(esz), sdispls, rdispls);
-        if (le != hipSuccess) return fail_hip(le, "moe gather-combine kernel");
-        return HCCL_SUCCESS;
+        return launch_gather_pieces(kind, st, s, d, p, o, n, tokens, topk, vpr, static_cast<uint32_t>(esz), sdispls, rdispls);
     }
     const uint64_t blocks = (static_cast<uint64_t>(tokens) * vpr + 255) / 256;
     if (blocks > 0x7fffffffull) return fail(HCCL_E_PARA, "too much data for one launch");

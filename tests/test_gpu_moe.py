@@ -258,3 +258,59 @@ def test_one_pass_round_trip_at_baseline_size():
             pos += mine.numel()
         assert pos == int(inbound[j]) * hidden
         assert bool((recv[j][pos:] == 0x2222).all())
+
+
+@pytest.mark.parametrize("topk,dtype,width,n,tokens", [(4, T.BFP16, 1024, 2, 37), (5, T.FP32, 516, 3, 65), (8, T.BFP16, 1536, 8, 16),
+                                                        (9, T.FP16, 1032, 2, 33), (2, T.FP32, 512, 64, 3), (6, T.BFP16, 1528, 1, 1),
+                                                        (3, T.BFP16, 376, 4, 50), (3, T.BFP16, 384, 4, 50), (2, T.FP16, 392, 2, 31)])
+def test_rows_cut_into_pieces(topk, dtype, width, n, tokens):
+    """Rows of 48 vectors and more are moved a piece of 64 vectors per wavefront: whole pieces, one vector more and one
+    less, rows around the 48 vectors, token numbers around the 32 pieces of eight workgroups, entries that do not divide by those of a wavefront."""
+    test_fused_dispatch_and_gather_combine_equal_the_two_pass_pipeline(topk, dtype, width, n, tokens)
+
+
+@pytest.mark.parametrize("topk,tokens,hidden", [(5, 4200, 8192), (3, 700, 7168)])
+def test_dispatch_of_tokens_beyond_the_cache(topk, tokens, hidden):
+    """The first: 264 MiB of tokens, four entries per wavefront and a rest of one, stored through the L2."""
+    n, entries = 2, tokens * topk
+    g = torch.Generator(device=DEV)
+    g.manual_seed(topk)
+    toks = [torch.randint(-2**31, 2**31 - 1, (tokens, hidden), device=DEV, dtype=torch.int32, generator=g) for _ in range(n)]
+    dest = [torch.randint(0, n + 1, (entries,), device=DEV, dtype=torch.int32, generator=g) for _ in range(n)]   # n = dropped
+    tabs, perm = route_on_gpu([d.cpu().numpy() for d in dest], n, entries, hidden)
+    inbound = [sum(int((d == j).sum()) for d in dest) for j in range(n)]
+    recv = [torch.full((r + 1, hidden), 7, device=DEV, dtype=torch.int32) for r in inbound]
+    ptrs = lambda ts: [t.data_ptr() for t in ts]
+    torch.cuda.synchronize()
+    hcclx.moe_dispatch(ptrs(toks), ptrs(dest), ptrs(perm), entries, topk, hidden, T.FP32, tabs[1].data_ptr(), tabs[3].data_ptr(), ptrs(recv))
+    torch.cuda.synchronize()
+    for j in range(n):
+        want = torch.cat([toks[i][(dest[i] == j).nonzero().reshape(-1) // topk] for i in range(n)])
+        assert torch.equal(recv[j][:-1], want), j
+        assert bool((recv[j][-1] == 7).all()), j
+
+
+def test_dispatch_and_gather_combine_in_several_launches():
+    """More work-items than one launch takes along x (2^32): 33000 tokens of two pieces, 4096 entries each, nearly all
+    dropped; the entries kept lie at both ends and around the first launch's last token."""
+    n, topk, tokens, width = 1, 4096, 33000, 512
+    tok = torch.arange(tokens * width, device=DEV, dtype=torch.float32).reshape(tokens, width)
+    dest = torch.full((tokens, topk), -1, device=DEV, dtype=torch.int32)
+    perm = torch.full((tokens, topk), -1, device=DEV, dtype=torch.int32)
+    kept = [(0, 0), (1, 4095), (32763, 17), (32764, 0), (32764, 4095), (32999, 2048)]
+    for row, (t, e) in enumerate(kept):
+        dest[t, e], perm[t, e] = 0, row
+    zero = torch.zeros(1, device=DEV, dtype=torch.int64)
+    recv = torch.full((len(kept) + 1, width), -1.0, device=DEV)
+    out = torch.full((tokens + 1, width), -1.0, device=DEV)
+    torch.cuda.synchronize()
+    hcclx.moe_dispatch([tok.data_ptr()], [dest.data_ptr()], [perm.data_ptr()], tokens * topk, topk, width, T.FP32, zero.data_ptr(),
+                       zero.data_ptr(), [recv.data_ptr()])
+    torch.cuda.synchronize()
+    rows = torch.tensor([t for t, _ in kept], device=DEV)
+    assert torch.equal(recv[:-1], tok[rows]) and bool((recv[-1] == -1).all())
+    hcclx.moe_gather_combine([recv.data_ptr()], [dest.data_ptr()], [perm.data_ptr()], tokens, topk, width, T.FP32, zero.data_ptr(),
+                             zero.data_ptr(), [out.data_ptr()])
+    torch.cuda.synchronize()
+    want = torch.zeros_like(tok).index_add_(0, rows, tok[rows])
+    assert torch.equal(out[:-1], want) and bool((out[-1] == -1).all())
