@@ -430,6 +430,7 @@ struct Batch {
     uint32_t waves = 0;          // non-zero: the one-store-per-wavefront kernel, this many wavefronts per workgroup
     uint32_t pieces = 1;         // and this many 1 KiB pieces per source and workgroup
     uint32_t waves_fixed = 0;    // and, when every segment has the same number of sources, that number
+    bool waves_team = false;     // chains: the wavefronts share the fold
     size_t nseg() const { return segs.size() + wide.size(); }
     size_t bytes() const
     {
@@ -633,11 +634,17 @@ bool make_segdev(const hcclx_seg_t &s, const SegProto &sp, int mode, SegDev *out
 // serves; segments that only copy go to that second launch whole (their source is the run).
 // Fills `one` (the segments of the first launch, one destination each) and `fan` (what the second launch copies)
 // and returns true; returns false when the launch stays as it is.  max_fan: the segment type's array size.
+// A fold of few places stays one pass: reading its result back is a large part of what it moves (AllReduce in two shots,
+// split : one pass: 2 x 400 MiB 343 : 267 us, 3 x 150 171 : 151, 4 x 128 185 : 166, 5 x 50 88.5 : 88.7; trees, which have
+// the register kernel only: 2 x 400 361 : 260, 3 x 250 279 : 251, 4 x 128 177 : 190).
+constexpr uint32_t kFanoutLeastPlaces = 5;
+constexpr uint32_t kFanoutLeastPlacesTree = 4;
 template <typename SEG>
-bool split_fanout(const DeviceCtx *ctx, const SEG *segs, uint32_t nseg, int esz, int mode, uint32_t max_fan,
+bool split_fanout(const DeviceCtx *ctx, const SEG *segs, uint32_t nseg, int esz, int mode, bool float_type, uint32_t max_fan,
                   std::vector<SEG> *one, std::vector<PhasedStream> *fan)
 {
     if (ctx == nullptr || mode == HCCLX_FOLD_SELF_FIRST || esz == 0) return false;
+    const uint32_t least = mode == HCCLX_FOLD_TREE && float_type ? kFanoutLeastPlacesTree : kFanoutLeastPlaces;
     uint64_t fold_traffic = 0;   // bytes read and written by the folds whose result goes to several places
     uint64_t copy_payload = 0;   // bytes of the sources that are only copied to several places
     for (uint32_t i = 0; i < nseg; ++i) {
@@ -651,7 +658,7 @@ bool split_fanout(const DeviceCtx *ctx, const SEG *segs, uint32_t nseg, int esz,
         const uint64_t bytes = g.count * static_cast<uint64_t>(esz);
         if (g.nsrc == 1) {
             copy_payload += bytes;
-        } else {
+        } else if (g.ndst >= least) {
             fold_traffic += bytes * (g.nsrc + g.ndst);
         }
     }
@@ -662,7 +669,7 @@ bool split_fanout(const DeviceCtx *ctx, const SEG *segs, uint32_t nseg, int esz,
     fan->clear();
     for (uint32_t i = 0; i < nseg; ++i) {
         const SEG &g = segs[i];
-        if (g.count == 0 || g.ndst < 2 || !(g.nsrc == 1 ? split_copies : split_folds)) {
+        if (g.count == 0 || g.ndst < (g.nsrc == 1 ? 2u : least) || !(g.nsrc == 1 ? split_copies : split_folds)) {
             one->push_back(g);
             continue;
         }
@@ -721,7 +728,7 @@ int build_batches(const hcclx_seg_t *segs, uint32_t nseg, int dtype, int op, int
     std::vector<hcclx_seg_t> one;
     std::vector<PhasedStream> fan;
     const DeviceCtx *fctx = device_ctx();
-    if (!split_fanout(fctx, segs, nseg, dtype_size(dtype), mode, HCCLX_MAX_FAN, &one, &fan)) {
+    if (!split_fanout(fctx, segs, nseg, dtype_size(dtype), mode, is_float_dtype(dtype), HCCLX_MAX_FAN, &one, &fan)) {
         return build_batches_impl(segs, nseg, dtype, op, mode, out);
     }
     const uint64_t algo_before = out->algo_bytes;
@@ -736,6 +743,8 @@ int build_batches(const hcclx_seg_t *segs, uint32_t nseg, int dtype, int op, int
     return HCCL_SUCCESS;
 }
 
+constexpr uint64_t kTeamFrom = 48ull << 20;
+
 // The n orders of a self-first fold take the kernel in which every wavefront issues one store (fold.h) when all
 // segments have the same number of ranks, at most waves_max_fan, and the launch writes waves_from bytes or more.
 // Measured against the register kernel on fp32 PROD (us, register : wavefronts): 4 ranks x 64 MiB 97.7 : 77.4,
@@ -749,13 +758,18 @@ int build_batches(const hcclx_seg_t *segs, uint32_t nseg, int dtype, int op, int
 // four from there on (12 x 64 MiB: 268.7 / 260.6 / 281.7).  Launches
 // whose segments differ in their number of ranks run on the instance that reads the count per segment, which only
 // wins up to eight ranks.  Chains whose value goes to several places (integer one-shot AllReduce, two-shot, NHR of
-// integers) take this kernel up to 256 KiB per place, where its prologue is the shorter one (12 ranks: 3.4-3.6
-// against 3.9-4.3 us for one segment, 5.0-6.2 against 5.9-6.8 for twelve slices; from 1 MiB per place on the register
-// kernels win: 4.9 against 5.5), and beyond only when asked for (waves_chains; as one pass the 8 x 64 MiB AllReduce
-// measured 189 to 245 us against 172 for fold + fan-out).
+// integers) take this kernel, the fold shared by the wavefronts from four of them on, while they are small: up to 2 MiB per
+// place among two to four ranks, 512 KiB among more (kernel times, bf16, register : this one: 2 x 2 MiB 5.06 : 4.24 us,
+// 4 x 256 KiB 6.3 : 3.5, 4 x 2 MiB 6.34 : 4.84, 8 x 512 KiB 5.44 : 4.40, 12 x 512 KiB 8.46 : 7.16, 16 x 512 KiB 6.68 : 5.76;
+// fp32 beyond: 4 x 4 MiB 5.42 : 5.92, 8 x 1 MiB 4.60 : 5.00, 12 x 1 MiB 7.24 : 7.90).  Among two to four ranks also, shared
+// and with four pieces, from kTeamFrom bytes written on (buffers that are not in the Infinity Cache, bf16: 2 x 25 MiB
+// 22.5 : 21.3, 2 x 400 277 : 267, 3 x 48 54.9 : 51.6, 3 x 150 162 : 151, 4 x 12 22.3 : 20.2, 4 x 128 181 : 166, 4 x 256
+// 375 : 337; below it 2 x 16 12.5 : 15.3, 3 x 12 14.1 : 15.5).  Otherwise only when asked for (waves_chains; 8 x 25 MiB
+// 78.7 : 74.7, fold + fan-out 70.7, and among 12 and more ranks no gain).
 // Returns the number of wavefronts per workgroup (the widest segment's sources or destinations), 0 = the register
 // kernels.
-uint32_t waves_for(const DeviceCtx *ctx, const hcclx_seg_t *segs, uint32_t nseg, int dtype, int mode, uint32_t *pieces)
+// *team: a chain whose fold the wavefronts share.
+uint32_t waves_for(const DeviceCtx *ctx, const hcclx_seg_t *segs, uint32_t nseg, int dtype, int mode, uint32_t *pieces, bool *team)
 {
     if (ctx == nullptr || ctx->waves_from == 0 || nseg == 0) return 0;
     if (mode != HCCLX_FOLD_SELF_FIRST && mode != HCCLX_FOLD_CHAIN) return 0;
@@ -780,16 +794,19 @@ uint32_t waves_for(const DeviceCtx *ctx, const hcclx_seg_t *segs, uint32_t nseg,
     const uint64_t per_place = written / most_dst;
     if (mode == HCCLX_FOLD_SELF_FIRST) {
         if (!same && widest > 8) return 0;
-    } else if (!ctx->waves_chains && per_place > (256ull << 10)) {
-        return 0;   // chains to several places: only the small ones by default (see above)
+    } else if (!ctx->waves_chains && per_place > (widest <= 4 ? 2048ull << 10 : 512ull << 10) && !(widest <= 4 && written >= kTeamFrom)) {
+        return 0;   // chains to several places: by default the small ones and, among few ranks, the large ones (see above)
     }
+    *team = mode == HCCLX_FOLD_CHAIN && (widest >= 4 || written >= kTeamFrom);
     uint32_t p = ctx->waves_pieces;
     if (p == 0) {   // the shipped policy; a forced piece count takes every launch that passed the tests above
         if (mode == HCCLX_FOLD_SELF_FIRST) {
             if (widest == 2 && per_place < (32ull << 20)) return 0;
             if ((widest == 7 || widest == 8) && per_place >= (3ull << 20) && per_place < (12ull << 20)) return 0;
         }
-        if (per_place < (2ull << 20) || widest <= 4) {
+        if (*team && written >= kTeamFrom) {
+            p = 4;
+        } else if (per_place < (2ull << 20) || widest <= 4) {
             p = 2;
         } else if (widest <= 8) {
             p = per_place < (32ull << 20) ? 4u : 2u;
@@ -808,7 +825,8 @@ int build_batches_impl(const hcclx_seg_t *segs, uint32_t nseg, int dtype, int op
     // the order a launch is asked for, and the one its kernel runs: integer folds are association-free
     const int kernel_mode = (mode != HCCLX_FOLD_CHAIN && !is_float_dtype(dtype)) ? HCCLX_FOLD_CHAIN : mode;
     uint32_t wave_pieces = 1;
-    const uint32_t waves = waves_for(device_ctx(), segs, nseg, dtype, kernel_mode, &wave_pieces);
+    bool waves_team = false;
+    const uint32_t waves = waves_for(device_ctx(), segs, nseg, dtype, kernel_mode, &wave_pieces, &waves_team);
     // Chains over many sources run faster on the wide chain kernel (sources in groups of eight, two vectors per
     // thread) than on the kernel that holds every source in registers.
     if (mode == HCCLX_FOLD_CHAIN && nseg != 0 && waves == 0) {
@@ -860,6 +878,7 @@ int build_batches_impl(const hcclx_seg_t *segs, uint32_t nseg, int dtype, int op
             same = same && segs[i].nsrc == common;
         }
         proto.waves_fixed = same ? common : 0;
+        proto.waves_team = waves_team;
     }
     proto.store_policy = store_policy_for(device_ctx(), segs, nseg, sp.copy ? 1 : dtype_size(dtype));
     Batch cur = proto;
@@ -891,7 +910,7 @@ int build_wide_batches(const hcclx_wide_seg_t *segs, uint32_t nseg, int dtype, i
     std::vector<hcclx_wide_seg_t> one;
     std::vector<PhasedStream> fan;
     const DeviceCtx *fctx = device_ctx();
-    if (!split_fanout(fctx, segs, nseg, dtype_size(dtype), mode, HCCLX_MAX_WIDE_FAN, &one, &fan)) {
+    if (!split_fanout(fctx, segs, nseg, dtype_size(dtype), mode, is_float_dtype(dtype), HCCLX_MAX_WIDE_FAN, &one, &fan)) {
         return build_wide_batches_impl(segs, nseg, dtype, op, mode, out);
     }
     const uint64_t algo_before = out->algo_bytes;
@@ -1110,6 +1129,7 @@ int launch_batch(const DeviceCtx *ctx, const Batch &b, const char *d_table, hipS
     l.waves = b.waves;
     l.pieces = b.pieces;
     l.waves_fixed = b.waves_fixed;
+    l.waves_team = b.waves_team;
     l.stream = stream;
     const hipError_t e = b.copy ? fold_dispatch_copy(l) : dispatch_fold(b.dtype, b.op, b.maxn, b.mode, l);
     if (e != hipSuccess) return fail_hip(e, "fold kernel launch");

@@ -50,13 +50,16 @@ struct DeviceCtx {
     // Writing n outputs at once runs HBM a third slower than writing them one after the other (the banks see n
     // streams of row misses).  A fold whose result goes to several places therefore stores it once and a second
     // launch copies it to the other places, one place at a time in batches of fanout_run bytes (HCCLX_FANOUT_RUN)
-    // whose re-reads the L2 serves: 8 x 64 MiB fp32 AllReduce 204 -> 175 us.  It pays from about 560 MiB read
-    // and written by such folds in one launch (HCCLX_FANOUT_FROM, 0 = never): below that the Infinity Cache
-    // (256 MiB) absorbs enough of the writes for the single pass to win (8 x 32 MiB: 84 against 90 us).
+    // whose re-reads the L2 serves: 8 x 64 MiB fp32 AllReduce 204 -> 175 us.  It pays from about 320 MiB read
+    // and written by such folds in one launch (HCCLX_FANOUT_FROM, 0 = never).  Buffers that are not in the Infinity Cache
+    // (256 MiB), one pass : split: 8 x 16 MiB bf16 52.4 : 48.5 us, 8 x 25 78.3 : 70.8, 8 x 32 99.4 : 88.3, 12 x 12
+    // 61.5 : 52.7, 32 x 6 80.9 : 71.7, 12 x 8 43.3 : 36.8, 6 x 24 55.9 : 53.9, 8 x 8 27.1 : 28.2.  The same buffers over and
+    // over, of which the cache holds what fits: 8 x 16 43.5 : 48.3, 8 x 25 65.7 : 71.0, 8 x 32 86.9 : 87.8, 12 x 12
+    // 51.1 : 52.9, 12 x 16 70.2 : 68.7.
     // A batch of 16 MiB is 2 MiB in each of the eight L2s (4 MiB each) while its copies are written: 8 x 64 MiB fp16
     // AllGather with batches of 4 / 8 / 12 / 16 / 20 / 24 MiB 801 / 761 / 753 / 740 / 744 / 732 us, and with 16 the
     // fan-out of a 12 x 1 GiB AllReduce 1930 us.
-    uint64_t fanout_from = 560ull << 20;
+    uint64_t fanout_from = 320ull << 20;
     uint64_t fanout_run = 16ull << 20;
     // AllGather(V) with host tables: from this many bytes of payload on (HCCLX_AGV_PHASED_FROM, 0 = never) the outputs
     // of a run of a source are written one after the other, each workgroup writing one output.

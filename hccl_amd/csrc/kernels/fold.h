@@ -555,7 +555,119 @@ __device__ __forceinline__ void waves_tile(u32x4 *s_piece, uint32_t waves, uint3
     }
 }
 
-// NFIX != 0: every segment of the launch has NFIX sources (the launcher checks); 0: the count is read per segment.
+// A chain has ONE value for all its places: the wavefronts of a workgroup share its fold instead of each folding the whole
+// piece.  A lane folds 4 bytes (8 of the 8-byte types) of every source piece and puts the result back into LDS; after a
+// second barrier wavefront w stores the piece of destination w.  LDS traffic is 3 n + 1 KiB per piece where folding in
+// every wavefront reads n * n, for one barrier more.  Kernel times among 4 / 8 / 12 / 16 ranks at 256 KiB per place, bf16:
+// 3.48 / 4.02 / 6.96 / 5.26 us against 3.68 / 4.84 / 8.64 / 8.12; with two wavefronts the barrier costs more than it saves
+// (fp32 2.9 against 2.6).  Large launches among two to four ranks are bound by HBM: see waves_for in hcclx.hip.
+template <int DT> struct TeamUnit {
+    using V = Vec16<DT>;
+    using C = typename V::C;
+    using S = typename V::S;
+    struct U {
+        uint32_t w[sizeof(S) == 8 ? 2 : 1];
+    };
+    static constexpr int E = V::NE * static_cast<int>(sizeof(U)) / 16;   // compute registers per unit
+    static __device__ __forceinline__ void unpack(const U &raw, C (&out)[E])
+    {
+        if constexpr (sizeof(C) * E == sizeof(U) && sizeof(S) != 2) {
+            __builtin_memcpy(out, &raw, sizeof(U));
+        } else {
+            S tmp[E];
+            __builtin_memcpy(tmp, &raw, sizeof(U));
+#pragma unroll
+            for (int e = 0; e < E; ++e) out[e] = V::D::widen(tmp[e]);
+        }
+    }
+    static __device__ __forceinline__ U pack(const C (&in)[E])
+    {
+        U raw;
+        if constexpr (sizeof(C) * E == sizeof(U) && sizeof(S) != 2) {
+            __builtin_memcpy(&raw, in, sizeof(U));
+        } else {
+            S tmp[E];
+#pragma unroll
+            for (int e = 0; e < E; ++e) tmp[e] = V::D::narrow(in[e]);
+            __builtin_memcpy(&raw, tmp, sizeof(U));
+        }
+        return raw;
+    }
+};
+
+// The sources four at a time, all four read before the first is combined; one that does not exist is read from slot 0 and
+// passed over.
+template <int DT, int OP>
+__device__ __forceinline__ void team_fold(const u32x4 *in, u32x4 *out, uint32_t nsrc, uint32_t flips)
+{
+    using T = TeamUnit<DT>;
+    using U = typename T::U;
+    using C = typename T::C;
+    constexpr int E = T::E;
+    constexpr int G = 4;
+    constexpr uint32_t kUnits = kWaveLanes * 16 / sizeof(U);
+    for (uint32_t at = threadIdx.x; at < kUnits; at += blockDim.x) {
+        const U *p = reinterpret_cast<const U *>(in) + at;
+        C acc[E];
+        T::unpack(p[0], acc);
+#pragma unroll
+        for (int base = 1; base < kMaxFan; base += G) {
+            if (base < static_cast<int>(nsrc)) {
+                U raw[G];
+#pragma unroll
+                for (int k = 0; k < G; ++k) {
+                    const uint32_t slot = static_cast<uint32_t>(base + k) < nsrc ? static_cast<uint32_t>(base + k) : 0u;
+                    raw[k] = p[slot * kUnits];
+                }
+#pragma unroll
+                for (int k = 0; k < G; ++k) {
+                    if (base + k < static_cast<int>(nsrc)) {
+                        C x[E];
+                        T::unpack(raw[k], x);
+                        const bool flip = OperandOrderMatters<DT, OP>::value && ((flips >> (base + k)) & 1u);
+#pragma unroll
+                        for (int e = 0; e < E; ++e) {
+                            acc[e] = flip ? Vec16<DT>::template combine<OP>(acc[e], x[e]) : Vec16<DT>::template combine<OP>(x[e], acc[e]);
+                        }
+                    }
+                }
+            }
+        }
+        reinterpret_cast<U *>(out)[at] = T::pack(acc);
+    }
+}
+
+// The pieces of one tile, as waves_tile.  One buffer of pieces and one of results are enough: a wavefront overwrites a piece
+// only behind the second barrier (all folds of it are done) and a result only behind the next first one (all have read it).
+template <int DT, int OP, bool CHECK>
+__device__ __forceinline__ void team_tile(u32x4 *s_piece, uint32_t waves, uint32_t w, uint32_t lane, const char *src, char *dst,
+                                          uint32_t nsrc, uint32_t ndst, uint64_t v_first, uint64_t nvec, uint64_t tile_first,
+                                          uint32_t shift, uint32_t pieces, uint32_t flips, uint32_t store_policy)
+{
+    const bool loads = w < nsrc;
+    const bool stores = w < ndst;
+    u32x4 *s_out = s_piece + waves * kWaveLanes;
+    u32x4 next = {0, 0, 0, 0};
+    if (loads) next = ld16(src + ((!CHECK || v_first < nvec) ? v_first : 0) * 16);
+#pragma unroll 1
+    for (uint32_t i = 0; i < pieces; ++i) {
+        const uint64_t v = v_first + static_cast<uint64_t>(i) * kWaveLanes;
+        if (CHECK && tile_first + static_cast<uint64_t>(i) * kWaveLanes >= nvec + shift) break;
+        if (loads) {
+            s_piece[w * kWaveLanes + lane] = next;
+            const uint64_t vn = v + kWaveLanes;
+            if (i + 1 < pieces) next = ld16(src + ((!CHECK || vn < nvec) ? vn : 0) * 16);
+        }
+        __syncthreads();
+        team_fold<DT, OP>(s_piece, s_out, nsrc, flips);
+        __syncthreads();
+        if (stores && (!CHECK || v < nvec)) st16x(dst + v * 16, s_out[lane], store_policy);
+    }
+}
+
+// NFIX > 1: every segment of the launch has NFIX sources (the launcher checks); 0 and kWavesTeam: the count is read per
+// segment; kWavesTeam: the wavefronts share the fold of a chain.
+constexpr int kWavesTeam = 1;
 template <int DT, int OP, int MODE, int NFIX>
 __global__ void __launch_bounds__(kMaxFan * kWaveLanes)
 k_fold_waves(const uint64_t *__restrict__ tile_end, const SegDev *__restrict__ segs, uint32_t nseg, uint32_t pieces,
@@ -584,7 +696,7 @@ k_fold_waves(const uint64_t *__restrict__ tile_end, const SegDev *__restrict__ s
     // entries and a workgroup at most as many wavefronts)
     const char *src_base = sd.src[w];
     char *dst_base = sd.dst[w];
-    const uint32_t nsrc = NFIX != 0 ? static_cast<uint32_t>(NFIX) : sd.nsrc;
+    const uint32_t nsrc = NFIX > 1 ? static_cast<uint32_t>(NFIX) : sd.nsrc;
     const uint32_t ndst = sd.ndst;
     const uint32_t head = sd.head;
     const uint32_t shift = sd.shift;
@@ -599,13 +711,23 @@ k_fold_waves(const uint64_t *__restrict__ tile_end, const SegDev *__restrict__ s
     const char *src = src_base + head_bytes;
     char *dst = dst_base + head_bytes;
     if (tl * TV >= shift && (tl + 1) * TV - shift <= nvec) {
-        waves_tile<DT, OP, MODE, NFIX, false>(s_piece, waves, w, lane, src, dst, nsrc, ndst, v_first, nvec, tl * TV, shift, pieces,
-                                              flips, store_policy);
+        if constexpr (NFIX == kWavesTeam) {
+            team_tile<DT, OP, false>(s_piece, waves, w, lane, src, dst, nsrc, ndst, v_first, nvec, tl * TV, shift, pieces, flips,
+                                     store_policy);
+        } else {
+            waves_tile<DT, OP, MODE, NFIX, false>(s_piece, waves, w, lane, src, dst, nsrc, ndst, v_first, nvec, tl * TV, shift, pieces,
+                                                  flips, store_policy);
+        }
         return;   // a tile inside the segment holds none of the elements outside the vector body
     }
     if (nvec != 0) {
-        waves_tile<DT, OP, MODE, NFIX, true>(s_piece, waves, w, lane, src, dst, nsrc, ndst, v_first, nvec, tl * TV, shift, pieces,
-                                             flips, store_policy);
+        if constexpr (NFIX == kWavesTeam) {
+            team_tile<DT, OP, true>(s_piece, waves, w, lane, src, dst, nsrc, ndst, v_first, nvec, tl * TV, shift, pieces, flips,
+                                    store_policy);
+        } else {
+            waves_tile<DT, OP, MODE, NFIX, true>(s_piece, waves, w, lane, src, dst, nsrc, ndst, v_first, nvec, tl * TV, shift, pieces,
+                                                 flips, store_policy);
+        }
     }
     // the last tile (the one that holds vector nvec + shift; said without a division, which takes hundreds of cycles
     // for 64-bit operands) also takes the elements in front of and behind the vector body, one per thread
@@ -904,6 +1026,7 @@ struct FoldLaunch {
     uint32_t waves = 0;        // non-zero: the one-store-per-wavefront kernel with this many wavefronts per workgroup
     uint32_t pieces = 1;       // and this many 1 KiB pieces per source and workgroup
     uint32_t waves_fixed = 0;  // non-zero: every segment of the launch has this many sources
+    bool waves_team = false;   // chains: the wavefronts share the fold
     hipStream_t stream;
 };
 

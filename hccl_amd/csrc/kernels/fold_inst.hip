@@ -25,8 +25,8 @@ static hipError_t launch_waves_n(const FoldLaunch &l)
     return hipGetLastError();
 }
 
-// The self-first orders get an instance per rank count up to twelve (the widest the launch policy takes by itself);
-// chains, and wider or mixed launches, run on the instance that reads the count per segment.
+// The self-first orders get an instance per rank count up to sixteen; mixed launches and chains run on instances that read
+// the count per segment.
 template <int DT, int OP, int MODE>
 static hipError_t launch_waves(const FoldLaunch &l)
 {
@@ -50,7 +50,8 @@ static hipError_t launch_waves(const FoldLaunch &l)
             default: return launch_waves_n<DT, OP, MODE, 0>(l);
         }
     } else if constexpr (MODE == kFoldChain) {
-        return launch_waves_n<DT, OP, MODE, 0>(l);
+        // from four wavefronts on they share the fold; large launches among two and three ranks do too (waves_team)
+        return l.waves_team ? launch_waves_n<DT, OP, MODE, kWavesTeam>(l) : launch_waves_n<DT, OP, MODE, 0>(l);
     } else {
         return hipErrorInvalidValue;
     }

@@ -223,3 +223,23 @@ def test_prod_allreduce_of_four_ranks_takes_the_wavefront_kernel_by_default():
     for r in range(n):
         assert torch.equal(results[0][r].view(torch.int32), results[1][r].view(torch.int32)), r
         assert_same_bits(results[0][r][idx].cpu().numpy(), want[r], T.FP32, f"rank {r}")
+
+
+@pytest.mark.parametrize("ranks,dtype,op", [(2, T.BFP16, T.SUM), (3, T.FP32, T.MAX), (4, T.INT8, T.SUM), (4, T.FP64, T.PROD), (2, T.INT16, T.MIN)])
+def test_large_chains_among_few_ranks_share_the_fold(ranks, dtype, op):
+    """48 MiB written and more among two to four ranks: one pass on the wavefront kernel, several pieces per workgroup, a
+    head, a tail and a partly filled last tile; against the register kernel."""
+    hcclx.init()
+    rng = np.random.default_rng(ranks + dtype)
+    esz = T.DTYPE_SIZE[dtype]
+    n = (48 << 20) // ranks // esz + 4099
+    xs = [payload(rng, dtype, n, "prod" if op == T.PROD else "normal") for _ in range(ranks)]
+    bufs = [DevBuf(x, offset=(k % 3) * esz) for k, x in enumerate(xs)]
+    outs = [DevBuf(nbytes=xs[0].nbytes, offset=(1 + k % 5) * esz) for k in range(ranks)]
+    before = hcclx.kernels_launched()
+    got, ref = fold_both([(n, [b.ptr for b in bufs], [o.ptr for o in outs])], dtype, op, hcclx.FOLD_CHAIN, outs)
+    assert hcclx.kernels_launched() - before == 2
+    want = chain_oracle(xs, dtype, op, [0] * ranks)
+    for r in range(ranks):
+        assert_same_bits(got[r], want, dtype, f"place {r}")
+        assert np.array_equal(got[r].view(np.uint8), ref[r].view(np.uint8)), f"place {r}: differs from the register kernel"
