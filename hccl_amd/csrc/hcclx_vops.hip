@@ -90,6 +90,37 @@ bool cut_slabs(const std::vector<CopyBlock> &blocks, size_t max_slabs, uint32_t 
 
 }  // namespace hcclx
 
+namespace {
+
+// Tables on the host that describe equal blocks, back to back in rank order: what HcclAlltoAll passes.
+bool equal_blocks(const uint64_t *send_counts, const uint64_t *sdispls, const uint64_t *rdispls, uint32_t n)
+{
+    const uint64_t count = send_counts[0];
+    uint64_t differ = 0;
+    for (uint32_t i = 0; i < n; ++i) {
+        const size_t row = static_cast<size_t>(i) * n;
+        uint64_t at = 0;
+        for (uint32_t j = 0; j < n; ++j) {
+            differ |= (send_counts[row + j] ^ count) | (sdispls[row + j] ^ at) | (rdispls[row + j] ^ at);
+            at += count;
+        }
+        if (differ != 0) return false;
+    }
+    return true;
+}
+
+bool is_capturing(hipStream_t stream)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+
+}  // namespace
+
 extern "C" {
 
 int hcclx_alltoallv(const void *const *send, void *const *recv, const uint64_t *send_counts,
@@ -106,6 +137,18 @@ int hcclx_alltoallv(const void *const *send, void *const *recv, const uint64_t *
     if (rc != HCCL_SUCCESS) return rc;
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (!tables_on_device) {
+        // Equal blocks need no table.  (A captured launch keeps to the tables, so that what can be captured stays as it
+        // is; and a grid has at most 2^32 work-items along x.)
+        const uint64_t block_bytes = send_counts[0] * esz;
+        if (block_bytes != 0 && block_bytes < (1ull << 35) && equal_blocks(send_counts, sdispls, rdispls, n) && !is_capturing(st)) {
+            EqualBlocks tab;
+            std::memcpy(tab.send, ptrs.send, sizeof(tab.send));
+            std::memcpy(tab.recv, ptrs.recv, sizeof(tab.recv));
+            tab.bytes = block_bytes;
+            const hipError_t e = launch_equal_blocks(tab, n, st);
+            if (e != hipSuccess) return fail_hip(e, "alltoall kernel launch");
+            return HCCL_SUCCESS;
+        }
         std::vector<CopyBlock> blocks;
         list_alltoallv_blocks(send, recv, send_counts, sdispls, rdispls, n, static_cast<uint32_t>(esz), &blocks);
         if (blocks.empty()) return HCCL_SUCCESS;
@@ -145,17 +188,17 @@ int hcclx_alltoallv(const void *const *send, void *const *recv, const uint64_t *
         }
         // any other host table: the non-empty blocks and their slabs in device memory
         if (!cut_slabs(blocks, kBlockTableSlabs, ~0u, &slabs, &shift)) return fail(HCCL_E_PARA, "too much data for one launch");
-        const size_t block_bytes = (blocks.size() * sizeof(CopyBlock) + 255) & ~static_cast<size_t>(255);
-        const size_t bytes = block_bytes + slabs.size() * sizeof(CopySlab);
+        const size_t list_bytes = (blocks.size() * sizeof(CopyBlock) + 255) & ~static_cast<size_t>(255);
+        const size_t bytes = list_bytes + slabs.size() * sizeof(CopySlab);
         char *h = nullptr;
         char *d = nullptr;
         rc = ring_reserve(ctx, bytes, st, &h, &d);
         if (rc != HCCL_SUCCESS) return rc;
         std::memcpy(h, blocks.data(), blocks.size() * sizeof(CopyBlock));
-        std::memcpy(h + block_bytes, slabs.data(), slabs.size() * sizeof(CopySlab));
+        std::memcpy(h + list_bytes, slabs.data(), slabs.size() * sizeof(CopySlab));
         rc = upload_table(d, h, bytes, st);
         if (rc != HCCL_SUCCESS) return rc;
-        const BlockTable tab{reinterpret_cast<const CopyBlock *>(d), reinterpret_cast<const CopySlab *>(d + block_bytes)};
+        const BlockTable tab{reinterpret_cast<const CopyBlock *>(d), reinterpret_cast<const CopySlab *>(d + list_bytes)};
         hipError_t e = launch_copy_blocks(tab, static_cast<uint32_t>(slabs.size()), shift, st);
         if (e != hipSuccess) return fail_hip(e, "alltoallv kernel launch");
         return HCCL_SUCCESS;

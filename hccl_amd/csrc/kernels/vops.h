@@ -100,6 +100,12 @@ struct A2avInline {
     uint32_t inv_n;   // 65536 / n + 1: b * inv_n >> 16 is b / n for every block number
     uint32_t esz;
 };
+// An exchange of equal blocks: block j of rank i's send buffer becomes block i of rank j's receive buffer.
+struct EqualBlocks {
+    const char *send[kMaxVRanks];
+    char *recv[kMaxVRanks];
+    uint64_t bytes;   // of a block
+};
 struct AgvTablesPtr {
     const uint64_t *counts;
     const uint64_t *displs;
@@ -149,6 +155,7 @@ struct AgvTablesInline {
 
 // nslabs << slab_shift workgroups, slabs of 1 << slab_shift tiles
 hipError_t launch_copy_blocks(const BlockTable &tab, uint32_t nslabs, uint32_t slab_shift, hipStream_t stream);
+hipError_t launch_equal_blocks(const EqualBlocks &tab, uint32_t n, hipStream_t stream);
 hipError_t launch_alltoallv_inline(const A2avInline &tab, uint32_t nslabs, uint32_t slab_shift, hipStream_t stream);
 // One batch after the other (grid z), each to one place after the other (grid y): per_batch slabs of slab_tiles tiles.
 struct PhasedGrid {

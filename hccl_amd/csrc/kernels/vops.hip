@@ -202,6 +202,18 @@ __global__ void __launch_bounds__(kThreads) k_copy_blocks(Tab tab, uint32_t slab
     copy_tile<1, false, kStoreThrough>(b.src, reinterpret_cast<uint64_t>(dst), b.bytes, tl, 1, [=](uint32_t) { return dst; });
 }
 
+// Equal blocks: nothing to look up and no table to bring, the block is the workgroup's place in the grid (x: tile, y:
+// destination, z: source).  32 ranks x 32 x 2049 bf16: 3.4 us of table upload in front of the copy less, and the host
+// builds no table of 1024 blocks.
+__global__ void __launch_bounds__(kThreads) k_equal_blocks(EqualBlocks tab)
+{
+    const uint64_t bytes = tab.bytes;
+    const char *src = tab.send[blockIdx.z] + blockIdx.y * bytes;
+    char *dst = tab.recv[blockIdx.y] + blockIdx.z * bytes;
+    if (blockIdx.x >= v_tiles_of(bytes, reinterpret_cast<uint64_t>(dst), 1)) return;
+    copy_tile<1, false, kStoreThrough>(src, reinterpret_cast<uint64_t>(dst), bytes, blockIdx.x, 1, [=](uint32_t) { return dst; });
+}
+
 __device__ __forceinline__ CopySlab phased_slab(const PhasedTable &t, uint32_t k) { return t.slabs[k]; }
 __device__ __forceinline__ CopySlab phased_slab(const PhasedInline &t, uint32_t k) { return {t.slabs[k] & 63u, t.slabs[k] >> 6}; }
 // null: the source has no such place
@@ -275,6 +287,14 @@ hipError_t launch_alltoallv(const VRankPtrs &ptrs, const uint64_t *send_counts, 
 hipError_t launch_copy_blocks(const BlockTable &tab, uint32_t nslabs, uint32_t slab_shift, hipStream_t stream)
 {
     HCCLX_LAUNCH((k_copy_blocks<BlockTable>), dim3(nslabs << slab_shift), dim3(kThreads), 0, stream, tab, slab_shift);
+    return hipGetLastError();
+}
+
+hipError_t launch_equal_blocks(const EqualBlocks &tab, uint32_t n, hipStream_t stream)
+{
+    // tiles of a block whatever the alignment of its place: up to 63 vectors in front of it in the tile grid
+    const uint64_t tiles = (tab.bytes / 16 + 63) / 256 + 1;
+    HCCLX_LAUNCH(k_equal_blocks, dim3(static_cast<uint32_t>(tiles), n, n), dim3(kThreads), 0, stream, tab);
     return hipGetLastError();
 }
 

@@ -300,6 +300,26 @@ def test_copies_to_several_places_of_different_number(nseg):
     plan.close()
 
 
+@pytest.mark.parametrize("n,count,dtype", [(1, 5, T.INT8), (2, 1, T.INT8), (3, 4095, T.INT8), (8, 2049, T.BFP16), (16, 4097, T.FP32),
+                                           (33, 1023, T.INT16), (64, 7, T.INT64), (5, 700001, T.INT8)])
+def test_alltoall_of_equal_blocks_needs_no_table(n, count, dtype):
+    """Equal blocks back to back: one launch, no upload; one byte, whole tiles and one element more or less, blocks at any
+    alignment."""
+    esz = T.DTYPE_SIZE[dtype]
+    rng = np.random.default_rng(n + count)
+    ins = [rng.integers(0, 256, size=n * count * esz, dtype=np.uint8) for _ in range(n)]
+    src = [DevBuf(x, offset=(i * esz) % 32) for i, x in enumerate(ins)]
+    dst = [DevBuf(nbytes=n * count * esz, offset=(3 * i * esz) % 40) for i in range(n)]
+    displs = [j * count for j in range(n)] * n
+    before = hcclx.kernels_launched()
+    hcclx.alltoallv([s.ptr for s in src], [d.ptr for d in dst], [count] * (n * n), displs, displs, dtype)
+    torch.cuda.synchronize()
+    assert hcclx.kernels_launched() - before == 1
+    for j in range(n):
+        want = np.concatenate([ins[i][j * count * esz:(j + 1) * count * esz] for i in range(n)])
+        assert np.array_equal(dst[j].get(np.uint8), want) and dst[j].guard_intact(), j
+
+
 def test_v_ops_reject_bad_arguments():
     b = DevBuf(nbytes=64)
     with pytest.raises(HcclError) as e:
