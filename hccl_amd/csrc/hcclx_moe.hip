@@ -245,6 +245,106 @@ k_moe_scan_perm(MoeConstPtrs dest, MoePtrs perm, uint32_t n, uint32_t entries, u
     }
 }
 
+// The whole routing in one launch, for so few entries per rank (kOneLaunchEntries) that every workgroup can count for
+// itself.  Workgroup (c, i): a pass over the destinations of rank i gives, per destination, its
+// entries and those in front of chunk c; then the permutation of chunk c as in k_moe_perm.  The workgroups of chunk 0 write
+// their rank's rows of the count and displacement tables and, from a pass over all ranks' destinations, what every rank
+// sends to rank i in front of which.  Bound by the latency of one launch and two rounds of loads.  Two launches : one, us: 8 ranks x 64
+// entries 5.95 : 4.44, x 512 6.16 : 4.61, x 1024 6.5 : 5.2, x 4096 7.6 : 9.4; 16 x 1024 8.3 : 7.3, x 2048 8.9 : 9.7; 64 x 1024
+// 26.3 : 20.5; 2 x 512 5.1 : 3.6, x 4096 6.2 : 7.3.
+constexpr uint32_t kOneLaunchEntries = 1024;
+
+__global__ void __launch_bounds__(kMoeChunk)
+k_moe_route_one(MoeConstPtrs dest, MoePtrs perm, uint32_t n, uint32_t entries, uint64_t row_elems, uint64_t *send_counts,
+                uint64_t *sdispls, uint64_t *recv_counts, uint64_t *rdispls)
+{
+    __shared__ uint32_t s_total[kMoeMaxRanks];
+    __shared__ uint32_t s_before[kMoeMaxRanks];
+    __shared__ uint32_t s_start[kMoeMaxRanks];
+    __shared__ uint32_t s_cnt[4][kMoeMaxRanks];
+    __shared__ uint32_t s_from[kMoeMaxRanks];   // chunk 0: entries of each rank for destination i
+    const uint32_t c = blockIdx.x;
+    const uint32_t i = blockIdx.y;
+    const uint32_t wave = threadIdx.x >> 6;
+    const uint32_t lane = threadIdx.x & 63;
+    const int32_t *mine = static_cast<const int32_t *>(dest.p[i]);
+    if (threadIdx.x < kMoeMaxRanks) {
+        s_total[threadIdx.x] = 0;
+        s_before[threadIdx.x] = 0;
+    }
+    __syncthreads();
+    // eight loads in flight; an entry behind the last repeats it and is not counted
+    for (uint32_t base = threadIdx.x; base < entries; base += 8 * kMoeChunk) {
+        uint32_t d[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const uint32_t e = base + u * kMoeChunk;
+            d[u] = static_cast<uint32_t>(mine[e < entries ? e : entries - 1]);
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const uint32_t e = base + u * kMoeChunk;
+            if (e < entries && d[u] < n) {
+                atomicAdd(&s_total[d[u]], 1u);
+                if (e < c * kMoeChunk) atomicAdd(&s_before[d[u]], 1u);
+            }
+        }
+    }
+    if (c == 0) {
+        for (uint32_t r = wave; r < n; r += 4) {
+            const int32_t *from = static_cast<const int32_t *>(dest.p[r]);
+            uint32_t count = 0;
+            for (uint32_t base = lane; base < entries; base += 8 * 64) {
+                uint32_t d[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const uint32_t e = base + u * 64;
+                    d[u] = static_cast<uint32_t>(from[e < entries ? e : entries - 1]);
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u) count += base + u * 64 < entries && d[u] == i ? 1u : 0u;
+            }
+            count = wave_sum_u32(count);
+            if (lane == 0) s_from[r] = count;
+        }
+    }
+    const uint32_t e = c * kMoeChunk + threadIdx.x;
+    uint32_t d = n;
+    if (e < entries) d = static_cast<uint32_t>(mine[e]);
+    uint32_t rank = 0;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    for (uint32_t dd = 0; dd < n; ++dd) {
+        const unsigned long long m = __ballot(d == dd);
+        if (d == dd) rank = __popcll(m & below);
+        if (lane == 0) s_cnt[wave][dd] = __popcll(m);
+    }
+    __syncthreads();
+    if (wave == 0) {
+        const uint32_t t = lane < n ? s_total[lane] : 0;
+        const uint32_t incl = wave_scan_u32(t);
+        s_start[lane] = incl - t;
+        if (c == 0) {
+            const uint32_t from = lane < n ? s_from[lane] : 0;
+            const uint32_t upto = wave_scan_u32(from);
+            if (lane < n) {
+                send_counts[i * n + lane] = static_cast<uint64_t>(t) * row_elems;
+                sdispls[i * n + lane] = static_cast<uint64_t>(incl - t) * row_elems;
+                recv_counts[i * n + lane] = static_cast<uint64_t>(from) * row_elems;
+                rdispls[i * n + lane] = static_cast<uint64_t>(upto - from) * row_elems;
+            }
+        }
+    }
+    __syncthreads();
+    if (e < entries) {
+        uint32_t out = kDropped;
+        if (d < n) {
+            out = s_start[d] + s_before[d] + rank;
+            for (uint32_t w = 0; w < wave; ++w) out += s_cnt[w][d];
+        }
+        static_cast<uint32_t *>(perm.p[i])[e] = out;
+    }
+}
+
 // Row gather / scatter: 512 vectors of 16 bytes per workgroup, rows of vpr vectors.
 //   PACK:    packed[perm[e]] = tokens[e / topk]      (g runs over entries x vpr)
 //   UNPACK:  out[t] = packed[perm[t]]                (topk == 1; g runs over tokens x vpr)
@@ -651,6 +751,13 @@ int hcclx_moe_route(const int32_t *const *dest, uint32_t n, uint32_t entries, ui
     const uint32_t chunks = chunks_of(entries);
     uint32_t *base = static_cast<uint32_t *>(workspace);
     uint32_t *row_start = base + static_cast<uint64_t>(n) * n * chunks;
+    if (entries <= kOneLaunchEntries) {
+        HCCLX_LAUNCH(k_moe_route_one, dim3(chunks, n), dim3(kMoeChunk), 0, st, d, as_mutable(p), n, entries, row_elems, send_counts,
+                     sdispls, recv_counts, rdispls);
+        const hipError_t oe = hipGetLastError();
+        if (oe != hipSuccess) return fail_hip(oe, "moe routing kernel");
+        return HCCL_SUCCESS;
+    }
     HCCLX_LAUNCH(k_moe_hist, dim3(chunks, n), dim3(kMoeChunk), 0, st, d, n, entries, chunks, base);
     if (chunks <= kFusedChunks && static_cast<uint64_t>(n) * n * chunks <= kFusedCells) {
         HCCLX_LAUNCH(k_moe_scan_perm, dim3(chunks, n), dim3(kMoeChunk), 0, st, d, as_mutable(p), n, entries, chunks,

@@ -314,3 +314,20 @@ def test_dispatch_and_gather_combine_in_several_launches():
     torch.cuda.synchronize()
     want = torch.zeros_like(tok).index_add_(0, rows, tok[rows])
     assert torch.equal(out[:-1], want) and bool((out[-1] == -1).all())
+
+
+@pytest.mark.parametrize("n,entries", [(1, 1), (8, 64), (8, 511), (8, 512), (4, 513), (64, 1024), (3, 1024), (3, 1025), (33, 257)])
+@pytest.mark.parametrize("skew", [0, 1])
+def test_route_in_one_launch(n, entries, skew):
+    """Up to 1024 entries per rank: around whole chunks of 256, whole rounds of eight loads and the size from which two
+    launches take over."""
+    before = hcclx.kernels_launched()
+    rng = np.random.default_rng(n + entries)
+    dests = [rng.integers(-1, n + 1, size=entries) for _ in range(n)]
+    tabs, perm = route_on_gpu(dests, n, entries, 8, skew)
+    assert hcclx.kernels_launched() - before == (1 if entries <= 1024 else 2)
+    sc, sd, rc, rd, perms = T.moe_route(dests, n, 8)
+    for got, want in zip(tabs, (sc, sd, rc, rd)):
+        assert np.array_equal(got.cpu().numpy().reshape(n, n), np.array(want, dtype=np.int64))
+    for i in range(n):
+        assert np.array_equal(perm[i].cpu().numpy().view(np.uint32), perms[i]), i
