@@ -1,6 +1,8 @@
 """Loader of the native library.  There is no fallback: every op in this package runs in
 libhccl_amd.so (HIP kernels for gfx950 behind a C ABI) or raises."""
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -112,6 +114,25 @@ def load():
                                      ctypes.c_int, ctypes.c_void_p]
     _lib = lib
     return lib
+
+
+_calls = None
+
+
+def native_call(name):
+    """The entry point as a callable that converts its arguments natively (csrc/python_calls.cc).  It returns
+    NotImplemented for arguments that ctypes has to convert; argtypes must have been set."""
+    global _calls
+    if _calls is None:
+        path = os.path.join(_HERE, "lib", "_hccl_calls.so")
+        if not os.path.exists(path):
+            raise RuntimeError(f"{path} is missing: build it with `make -C hccl_amd/csrc`")
+        loader = importlib.machinery.ExtensionFileLoader("_hccl_calls", path)
+        _calls = importlib.util.module_from_spec(importlib.util.spec_from_loader("_hccl_calls", loader))
+        loader.exec_module(_calls)
+    fn = getattr(load(), name)
+    kinds = "".join("p" if t is ctypes.c_void_p else "l" if t is ctypes.POINTER(ctypes.c_void_p) else "i" for t in fn.argtypes)
+    return _calls.Call(ctypes.cast(fn, ctypes.c_void_p).value, kinds, ctypes.Array)
 
 
 class HcclError(RuntimeError):

@@ -26,10 +26,14 @@ class CheckReport(ctypes.Structure):
 
 
 _bound = False
+# the collectives as native callables, set when the library is bound (a communicator exists only afterwards)
+_all_reduce = _reduce_scatter = _reduce_scatter_v = _all_gather = _all_gather_v = None
+_all_to_all_v = _all_to_all = _all_to_all_vc = None
 
 
 def lib():
-    global _bound
+    global _bound, _all_reduce, _reduce_scatter, _reduce_scatter_v, _all_gather, _all_gather_v
+    global _all_to_all_v, _all_to_all, _all_to_all_vc
     L = _lib.load()
     if not _bound:
         vp, u64, u32, ci = ctypes.c_void_p, ctypes.c_uint64, ctypes.c_uint32, ctypes.c_int
@@ -64,6 +68,9 @@ def lib():
             fn.argtypes = args
         L.hcclxCommGetLastTrace.restype = ctypes.c_uint64
         L.hcclxCommGetLastTrace.argtypes = [vp, ctypes.c_char_p, u64]
+        _all_reduce, _reduce_scatter, _reduce_scatter_v, _all_gather, _all_gather_v, _all_to_all_v, _all_to_all, _all_to_all_vc = (
+            _lib.native_call(name) for name in ("HcclAllReduce", "HcclReduceScatter", "HcclReduceScatterV", "HcclAllGather",
+                                                "HcclAllGatherV", "HcclAlltoAllV", "HcclAlltoAll", "HcclAlltoAllVC"))
         _bound = True
     return L
 
@@ -141,35 +148,60 @@ class World:
         return buf.value.decode()
 
     # ---- collectives: one call per rank, in any order; launched by the last one ----
+    # (ctypes converts what the native callable does not take)
     def all_reduce(self, rank, send, recv, count, dtype, op, stream):
+        rc = _all_reduce(send, recv, count, dtype, op, self.comms[rank], stream)
+        if rc is not NotImplemented:
+            return rc
         return lib().HcclAllReduce(send, recv, count, int(dtype), int(op), self.comms[rank], stream)
 
     def reduce_scatter(self, rank, send, recv, recv_count, dtype, op, stream):
+        rc = _reduce_scatter(send, recv, recv_count, dtype, op, self.comms[rank], stream)
+        if rc is not NotImplemented:
+            return rc
         return lib().HcclReduceScatter(send, recv, recv_count, int(dtype), int(op), self.comms[rank], stream)
 
     def reduce_scatter_v(self, rank, send, counts, displs, recv, recv_count, dtype, op, stream):
         c, d = _u64(counts), _u64(displs)
+        rc = _reduce_scatter_v(send, c, d, recv, recv_count, dtype, op, self.comms[rank], stream)
+        if rc is not NotImplemented:
+            return rc
         return lib().HcclReduceScatterV(send, ctypes.cast(c, ctypes.c_void_p), ctypes.cast(d, ctypes.c_void_p), recv,
                                         recv_count, int(dtype), int(op), self.comms[rank], stream)
 
     def all_gather(self, rank, send, recv, send_count, dtype, stream):
+        rc = _all_gather(send, recv, send_count, dtype, self.comms[rank], stream)
+        if rc is not NotImplemented:
+            return rc
         return lib().HcclAllGather(send, recv, send_count, int(dtype), self.comms[rank], stream)
 
     def all_gather_v(self, rank, send, send_count, recv, counts, displs, dtype, stream):
         c, d = _u64(counts), _u64(displs)
+        rc = _all_gather_v(send, send_count, recv, c, d, dtype, self.comms[rank], stream)
+        if rc is not NotImplemented:
+            return rc
         return lib().HcclAllGatherV(send, send_count, recv, ctypes.cast(c, ctypes.c_void_p),
                                     ctypes.cast(d, ctypes.c_void_p), int(dtype), self.comms[rank], stream)
 
     def all_to_all_v(self, rank, send, sc, sd, recv, rc, rd, dtype, stream):
         a, b, c, d = _u64(sc), _u64(sd), _u64(rc), _u64(rd)
+        ret = _all_to_all_v(send, a, b, dtype, recv, c, d, dtype, self.comms[rank], stream)
+        if ret is not NotImplemented:
+            return ret
         cast = lambda x: ctypes.cast(x, ctypes.c_void_p)
         return lib().HcclAlltoAllV(send, cast(a), cast(b), int(dtype), recv, cast(c), cast(d), int(dtype),
                                    self.comms[rank], stream)
 
     def all_to_all(self, rank, send, count, recv, dtype, stream):
+        rc = _all_to_all(send, count, dtype, recv, count, dtype, self.comms[rank], stream)
+        if rc is not NotImplemented:
+            return rc
         return lib().HcclAlltoAll(send, count, int(dtype), recv, count, int(dtype), self.comms[rank], stream)
 
     def all_to_all_vc(self, rank, send, matrix_flat, recv, dtype, stream):
         m = _u64(matrix_flat)
+        rc = _all_to_all_vc(send, m, dtype, recv, dtype, self.comms[rank], stream)
+        if rc is not NotImplemented:
+            return rc
         return lib().HcclAlltoAllVC(send, ctypes.cast(m, ctypes.c_void_p), int(dtype), recv, int(dtype),
                                     self.comms[rank], stream)

@@ -172,12 +172,30 @@ def displs_from_counts(counts, rows, n, displs, totals=0, stream=0):
                                                ctypes.c_void_p(totals) if totals else None, ctypes.c_void_p(stream)))
 
 
+_native = {}
+
+
+def _call(name, *args):
+    """Calls an entry point whose arguments are ints and lists of device addresses; False when ctypes has to convert one."""
+    fn = _native.get(name)
+    if fn is None:
+        fn = _native[name] = _lib.native_call(name)
+    rc = fn(*args)
+    if rc is NotImplemented:
+        return False
+    check(rc)
+    return True
+
+
 def moe_workspace_bytes(n, entries):
     return _lib.load().hcclx_moe_workspace_bytes(n, entries)
 
 
 def moe_route(dest, entries, row_elems, send_counts, sdispls, recv_counts, rdispls, perm, workspace, stream=0):
     """dest / perm: lists of n device addresses; the tables and the workspace are device addresses."""
+    if _call("hcclx_moe_route", dest, len(dest), entries, row_elems, send_counts, sdispls, recv_counts, rdispls, perm, workspace,
+             stream):
+        return
     check(_lib.load().hcclx_moe_route(_ptr_array(dest), len(dest), entries, row_elems, ctypes.c_void_p(send_counts),
                                       ctypes.c_void_p(sdispls), ctypes.c_void_p(recv_counts), ctypes.c_void_p(rdispls),
                                       _ptr_array(perm), ctypes.c_void_p(workspace), ctypes.c_void_p(stream)))
@@ -195,6 +213,8 @@ def moe_combine(packed, perm, tokens, topk, row_elems, dtype, out, stream=0):
 
 def moe_dispatch(tokens, dest, perm, entries, topk, row_elems, dtype, sdispls, rdispls, recv, stream=0):
     """Pack + AlltoAllV in one pass; sdispls / rdispls are the device tables moe_route wrote."""
+    if _call("hcclx_moe_dispatch", tokens, dest, perm, len(tokens), entries, topk, row_elems, dtype, sdispls, rdispls, recv, stream):
+        return
     check(_lib.load().hcclx_moe_dispatch(_ptr_array(tokens), _ptr_array(dest), _ptr_array(perm), len(tokens), entries, topk,
                                          row_elems, int(dtype), ctypes.c_void_p(sdispls), ctypes.c_void_p(rdispls),
                                          _ptr_array(recv), ctypes.c_void_p(stream)))
@@ -202,6 +222,9 @@ def moe_dispatch(tokens, dest, perm, entries, topk, row_elems, dtype, sdispls, r
 
 def moe_gather_combine(expert, dest, perm, tokens, topk, row_elems, dtype, sdispls, rdispls, out, stream=0):
     """AlltoAllV back + combine in one pass, reading the rows where moe_dispatch put them."""
+    if _call("hcclx_moe_gather_combine", expert, dest, perm, len(expert), tokens, topk, row_elems, dtype, sdispls, rdispls, out,
+             stream):
+        return
     check(_lib.load().hcclx_moe_gather_combine(_ptr_array(expert), _ptr_array(dest), _ptr_array(perm), len(expert), tokens,
                                                topk, row_elems, int(dtype), ctypes.c_void_p(sdispls),
                                                ctypes.c_void_p(rdispls), _ptr_array(out), ctypes.c_void_p(stream)))

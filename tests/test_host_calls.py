@@ -1,0 +1,82 @@
+"""The native callables behind the Python face (csrc/python_calls.cc) against ctypes: same results and codes, and what they do
+not take is left to ctypes.  Dry worlds: nothing here touches a GPU."""
+import ctypes
+import enum
+import threading
+
+import pytest
+
+from hccl_amd import _lib, api
+from hccl_amd import types as T
+
+
+class Kind(enum.IntEnum):
+    FP32 = T.FP32
+
+
+@pytest.fixture(scope="module")
+def world():
+    w = api.World(2, dry=True)
+    yield w
+    w.close()
+
+
+@pytest.mark.parametrize("args", [(0, 2, 10, 4, 0, "comm", 1), (1, 2, 10, 99, 0, "comm", 1), (1, 2, 10, 4, 9, "comm", 1),
+                                  (1, 2, 1 << 63, 4, 0, "comm", 1), (1, 2, -1, 4, 0, "comm", 1), (1, 2, 10, 4, 0, 0, 1),
+                                  (1, 2, 10, 4, 0, "comm", 0), (None, 2, 10, 4, 0, "comm", 1), (1, 2, (1 << 64) + 10, 4 + (1 << 32), 9, "comm", 1)])
+def test_codes_are_those_of_ctypes(world, args):
+    args = [world.comms[0] if a == "comm" else a for a in args]
+    native = api._all_reduce(*args)
+    assert native == api.lib().HcclAllReduce(*args) and native != 0
+
+
+@pytest.mark.parametrize("args", [(1.5, 2, 10, 4, 0, 7, 1), ([1, 2], 2, 10, 4, 0, 7, 1), (ctypes.c_void_p(5), 2, 10, 4, 0, 7, 1),
+                                  (1, 2, None, 4, 0, 7, 1), (1, 2, 10, None, 0, 7, 1), (1, 2, (ctypes.c_uint64 * 2)(), 4, 0, 7, 1),
+                                  (b"x", 2, 10, 4, 0, 7, 1)])
+def test_other_types_are_left_to_ctypes(world, args):
+    assert api._all_reduce(*args) is NotImplemented
+
+
+def test_what_ctypes_refuses_is_refused(world):
+    for bad in ([1, 2], 1.5):
+        with pytest.raises(ctypes.ArgumentError):
+            world.all_reduce(0, bad, 2 << 20, 10, T.FP32, T.SUM, 1)
+    with pytest.raises(ctypes.ArgumentError):
+        world.all_reduce(0, 1 << 20, 2 << 20, None, T.FP32, T.SUM, 1)
+    with pytest.raises(TypeError):
+        api._all_reduce(1, 2, 3)
+
+
+def test_enumerations_and_addresses_in_ctypes_objects(world):
+    for r in range(2):
+        assert world.all_reduce(r, ctypes.c_void_p((r + 1) << 20), (r + 10) << 20, 100, Kind.FP32, T.SUM, 1) == 0
+    assert world.last_info().algName
+
+
+def test_tables_as_lists_and_as_converted_arrays(world):
+    for table in (list, api.u64_table):
+        for r in range(2):
+            assert world.all_to_all_v(r, (r + 1) << 20, table([3, 4]), table([0, 3]), (r + 10) << 20, table([3 + r, 3 + r]),
+                                      table([0, 3 + r]), T.FP32, 1) == 0
+            assert world.all_gather_v(r, (r + 1) << 20, 5 + r, (r + 10) << 20, table([5, 6]), table([0, 5]), T.FP32, 1) == 0
+
+
+def test_the_callable_from_several_threads(world):
+    """The interpreter lock is given up during the call: ranks may call from threads of their own."""
+    codes = []
+    def rank(r):
+        for _ in range(50):
+            codes.append(world.all_reduce(r, (r + 1) << 20, (r + 10) << 20, 100, T.FP32, T.SUM, 1))
+    threads = [threading.Thread(target=rank, args=(r,)) for r in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert codes == [0] * 100
+
+
+def test_pointer_lists():
+    call = _lib.native_call("hcclx_moe_route")
+    assert call([1] * 65, 65, 8, 8, 1, 1, 1, 1, [1] * 65, 1, 0) is NotImplemented
+    assert call(1, 1, 8, 8, 1, 1, 1, 1, [1], 1, 0) is NotImplemented
+    assert call([1.5], 1, 8, 8, 1, 1, 1, 1, [1], 1, 0) is NotImplemented
