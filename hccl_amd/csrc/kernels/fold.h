@@ -254,9 +254,19 @@ __device__ __forceinline__ void fold_tail(const SEG &sd, uint32_t nsrc, uint32_t
     if constexpr (MODE == kFoldChain) {
         C acc = D::widen(reinterpret_cast<const S *>(sd.src[0])[idx]);
         const uint64_t flips = chain_flips(sd);
-        for (uint32_t k = 1; k < nsrc; ++k) {
-            const C x = D::widen(reinterpret_cast<const S *>(sd.src[k])[idx]);
-            acc = (OperandOrderMatters<DT, OP>::value && ((flips >> k) & 1u)) ? Op::run(acc, x) : Op::run(x, acc);
+        // eight loads in flight: one at a time, 32 sources keep a launch waiting for 15 us
+        for (uint32_t base = 1; base < nsrc; base += 8) {
+            S raw[8];
+#pragma unroll
+            for (uint32_t u = 0; u < 8; ++u) raw[u] = reinterpret_cast<const S *>(sd.src[base + u < nsrc ? base + u : 0])[idx];
+#pragma unroll
+            for (uint32_t u = 0; u < 8; ++u) {
+                const uint32_t k = base + u;
+                if (k < nsrc) {
+                    const C x = D::widen(raw[u]);
+                    acc = (OperandOrderMatters<DT, OP>::value && ((flips >> k) & 1u)) ? Op::run(acc, x) : Op::run(x, acc);
+                }
+            }
         }
         const S out = D::narrow(acc);
         for (uint32_t d = 0; d < ndst; ++d) reinterpret_cast<S *>(sd.dst[d])[idx] = out;
@@ -273,17 +283,6 @@ __device__ __forceinline__ void fold_tail(const SEG &sd, uint32_t nsrc, uint32_t
         }
         const S out = D::narrow(val[0][0]);
         for (uint32_t d = 0; d < ndst; ++d) reinterpret_cast<S *>(sd.dst[d])[idx] = out;
-    } else if constexpr (MAXN > kMaxFan) {
-        // The wide self-first order: the outputs of this entry's group, each from the sources as they lie in
-        // memory (no destination overlaps a source in this mode).
-        const uint32_t first = sd.first_dst;
-        for (uint32_t j = first; j < first + kMaxFan && j < nsrc; ++j) {
-            C acc = D::widen(reinterpret_cast<const S *>(sd.src[j])[idx]);
-            for (uint32_t k = 0; k < nsrc; ++k) {
-                if (k != j) acc = Op::run(D::widen(reinterpret_cast<const S *>(sd.src[k])[idx]), acc);
-            }
-            reinterpret_cast<S *>(sd.dst[j])[idx] = D::narrow(acc);
-        }
     } else {
         // Every source is read before the first destination is written: a destination may alias a source.
         C val[kMaxFan];
@@ -863,65 +862,156 @@ __device__ __forceinline__ void fold_tile_wide_tree(const SegWide &sd, uint32_t 
     }
 }
 
-// The self-first order among more than kMaxFan ranks: this segment entry computes the kMaxFan outputs
-// first_dst .. first_dst + kMaxFan - 1 (a segment of n ranks is entered once per such group).  Output j starts
-// from src[j] and takes the other sources in ascending order; the sources are loaded in groups of kMaxFan and every
-// loaded vector goes into all accumulators but its own.  Destinations must not overlap sources: other workgroups
-// still read what this one would overwrite.
-template <int DT, int OP, bool CHECK>
-__device__ __forceinline__ void fold_tile_wide_self(const SegWide &sd, uint32_t nsrc, uint64_t v, uint64_t nvec,
-                                                    uint32_t head_bytes)
+// The self-first order of the wide segments (17 to 64 ranks; up to 64 of any number): R outputs per wavefront of a workgroup
+// of sixteen.  Wavefront w loads a piece of the sources w, w + 16, ... into LDS; after the barrier it reads every piece once
+// and folds it into the outputs w, w + 16, ..., in source order, its own source first.  Bound by the N * N combines of N
+// orders (and 16 n KiB of LDS reads per n KiB of input).  The kernel before held 16 outputs per thread, read the sources once
+// for each group of 16, and folded each element outside the vector body in one thread that walked all sources 16 times over;
+// here those elements go through LDS as well.  One-shot AllReduce, fp32, before : now: 32 x 32770 elements 72.5 : 14.3 us (19 :
+// 13.8 with 32768), 64 x 32770 137 : 25, 32 x 8 MiB 195 : 142, 64 x 8 MiB 586 : 355; bf16 64 x 4 MiB 391 : 309.
+constexpr int kWideWaves = 16;
+
+// Four sources into the R outputs; MAYBE_OWN: source `own` of them is output own_q's own and passed over there.  (Without
+// the test in the groups that hold none: a quarter of the instructions for the 16-bit types.)
+template <int DT, int OP, int R, bool MAYBE_OWN>
+__device__ __forceinline__ void wide_waves_take(const u32x4 (&raw)[4], uint32_t left, uint32_t own, int own_q,
+                                                typename Vec16<DT>::C (&acc)[R][Vec16<DT>::NE])
 {
     using V = Vec16<DT>;
     using C = typename V::C;
     constexpr int NE = V::NE;
-    if (CHECK && v >= nvec) {
-        return;
-    }
-    const uint64_t off = head_bytes + v * 16;
-    const uint32_t first = sd.first_dst;
-    C acc[kMaxFan][NE];
-    {
-        u32x4 raw[kMaxFan];
 #pragma unroll
-        for (int j = 0; j < kMaxFan; ++j) {
-            if (first + j < nsrc) raw[j] = ld16(sd.src[first + j] + off);
-        }
+    for (uint32_t k = 0; k < 4; ++k) {
+        if (k < left) {
+            C x[NE];
+            V::unpack(raw[k], x);
 #pragma unroll
-        for (int j = 0; j < kMaxFan; ++j) {
-            if (first + j < nsrc) V::unpack(raw[j], acc[j]);
-        }
-    }
-    constexpr int G = 8;   // sources per load group: the unrolled body is G x kMaxFan updates
-    for (uint32_t base = 0; base < nsrc; base += G) {
-        u32x4 raw[G];
+            for (int q = 0; q < R; ++q) {
 #pragma unroll
-        for (int k = 0; k < G; ++k) {
-            if (base + k < nsrc) raw[k] = ld16(sd.src[base + k] + off);
-        }
-        // only the groups at first and first + G hold the outputs' own sources: source base + k is output
-        // j's own when j == k + (base - first)
-        const bool own_lo = (base == first);
-        const bool own_hi = (base == first + G);
-#pragma unroll
-        for (int k = 0; k < G; ++k) {
-            if (base + k < nsrc) {
-                C x[NE];
-                V::unpack(raw[k], x);
-#pragma unroll
-                for (int j = 0; j < kMaxFan; ++j) {
-                    const bool own = (own_lo && j == k) || (own_hi && j == k + G);
-                    if (first + j < nsrc && !own) {
-#pragma unroll
-                        for (int e = 0; e < NE; ++e) acc[j][e] = V::template combine<OP>(x[e], acc[j][e]);
-                    }
+                for (int e = 0; e < NE; ++e) {
+                    const C sum = V::template combine<OP>(x[e], acc[q][e]);
+                    acc[q][e] = MAYBE_OWN && q == own_q && k == own ? acc[q][e] : sum;
                 }
             }
         }
     }
+}
+
+template <int DT, int OP, int R>
+__global__ void __launch_bounds__(kWideWaves * kWaveLanes)
+k_fold_wide_waves(const uint64_t *__restrict__ tile_end, const SegWide *__restrict__ segs, uint32_t nseg, uint32_t rows, uint32_t pieces,
+                  uint32_t uniform_tiles)
+{
+    using D = DTypeOf<DT>;
+    using S = typename D::S;
+    using V = Vec16<DT>;
+    using C = typename V::C;
+    constexpr int NE = V::NE;
+    constexpr int NV = V::kElems;
+    constexpr uint32_t W = kWideWaves;
+    extern __shared__ u32x4 s_piece[];   // [rows][64], then the staged tile prefix when it is searched in LDS
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveLanes);
+    const uint32_t lane = threadIdx.x % kWaveLanes;
+    uint32_t seg = 0;
+    uint64_t tl = blockIdx.x;
+    if (nseg != 1) {
+        uint64_t *stage = reinterpret_cast<uint64_t *>(s_piece + rows * kWaveLanes);
+        const bool direct = nseg <= kFoldDirectSegs || uniform_tiles != 0;
+        if (!direct) {
+            for (uint32_t i = threadIdx.x; i < nseg; i += W * kWaveLanes) stage[i] = tile_end[i];
+            __syncthreads();
+        }
+        locate_tile(tile_end, stage, nseg, direct, uniform_tiles, blockIdx.x, &seg, &tl);
+    }
+    const SegWide &sd = segs[seg];
+    const uint32_t nsrc = sd.nsrc;
+    const uint32_t head = sd.head;
+    const uint32_t shift = sd.shift;
+    const uint64_t body = sd.count - head;
+    const uint64_t nvec = body / NV;
+    const uint32_t rem = static_cast<uint32_t>(body % NV);
+    const uint32_t head_bytes = head * (16 / NV);
+    const uint64_t TV = waves_tile_vecs(static_cast<int>(pieces));
+    const uint64_t v_first = tl * TV + lane - shift;
+    const bool full = tl * TV >= shift && (tl + 1) * TV - shift <= nvec;
+    const char *src[R];
+    char *dst[R];
 #pragma unroll
-    for (int j = 0; j < kMaxFan; ++j) {
-        if (first + j < nsrc) st16(sd.dst[first + j] + off, V::pack(acc[j]));
+    for (int q = 0; q < R; ++q) {
+        const uint32_t k = w + W * q < nsrc ? w + W * q : 0;
+        src[q] = sd.src[k] + head_bytes;
+        dst[q] = sd.dst[k] + head_bytes;
+    }
+    if (nvec != 0) {
+        // vectors in front of a shifted segment wrap below zero and fail the bound check like those behind its end; a
+        // lane outside the segment loads the segment's first vector and stores nothing
+        u32x4 next[R];
+#pragma unroll
+        for (int q = 0; q < R; ++q) next[q] = ld16(src[q] + (full || v_first < nvec ? v_first : 0) * 16);
+#pragma unroll 1
+        for (uint32_t i = 0; i < pieces; ++i) {
+            const uint64_t v = v_first + static_cast<uint64_t>(i) * kWaveLanes;
+            if (!full && tl * TV + static_cast<uint64_t>(i) * kWaveLanes >= nvec + shift) break;   // the same for all wavefronts
+            if (i != 0) __syncthreads();   // every wavefront has read the piece before
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                if (w + W * q < nsrc) s_piece[(w + W * q) * kWaveLanes + lane] = next[q];
+            }
+            if (i + 1 < pieces) {
+                const uint64_t vn = v + kWaveLanes;
+#pragma unroll
+                for (int q = 0; q < R; ++q) next[q] = ld16(src[q] + (full || vn < nvec ? vn : 0) * 16);
+            }
+            __syncthreads();
+            C acc[R][NE];
+#pragma unroll
+            for (int q = 0; q < R; ++q) V::unpack(s_piece[(w + W * q < nsrc ? w + W * q : 0) * kWaveLanes + lane], acc[q]);
+            // sources b * 16 .. b * 16 + 15: only output w + 16 b can have its own among them
+#pragma unroll
+            for (int b = 0; b < R; ++b) {
+#pragma unroll 1
+                for (uint32_t g = 0; g < W; g += 4) {
+                    const uint32_t base = W * b + g;
+                    if (base >= nsrc) break;
+                    u32x4 raw[4];
+#pragma unroll
+                    for (uint32_t k = 0; k < 4; ++k) raw[k] = s_piece[(base + k < nsrc ? base + k : base) * kWaveLanes + lane];
+                    if (g != (w & ~3u)) {
+                        wide_waves_take<DT, OP, R, false>(raw, nsrc - base, 0, b, acc);
+                    } else {
+                        wide_waves_take<DT, OP, R, true>(raw, nsrc - base, w & 3u, b, acc);
+                    }
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                if (w + W * q < nsrc && (full || v < nvec)) st16(dst[q] + v * 16, V::pack(acc[q]));
+            }
+        }
+    }
+    // the last tile also takes the elements in front of and behind the vector body: all of them into LDS, then one thread
+    // per element and output
+    const uint32_t edge = head + rem;
+    if (edge == 0 || tl * TV > nvec + shift || nvec + shift >= (tl + 1) * TV) return;
+    C *s_edge = reinterpret_cast<C *>(s_piece);   // [nsrc][edge], at most 14 elements of 4 bytes or 2 of 8 in a row's 1 KiB
+    __syncthreads();
+    for (uint32_t t = threadIdx.x; t < nsrc * edge; t += W * kWaveLanes) {
+        const uint32_t k = t / edge;
+        const uint32_t e = t - k * edge;
+        const uint64_t idx = e < head ? e : nvec * NV + e;
+        s_edge[t] = D::widen(reinterpret_cast<const S *>(sd.src[k])[idx]);
+    }
+    __syncthreads();
+    for (uint32_t t = threadIdx.x; t < nsrc * edge; t += W * kWaveLanes) {
+        const uint32_t j = t / edge;
+        const uint32_t e = t - j * edge;
+        C acc = s_edge[t];
+#pragma unroll 4
+        for (uint32_t k = 0; k < nsrc; ++k) {
+            const C sum = Combine<DT, OP>::run(s_edge[k * edge + e], acc);
+            acc = k == j ? acc : sum;
+        }
+        reinterpret_cast<S *>(sd.dst[j])[e < head ? e : nvec * NV + e] = D::narrow(acc);
     }
 }
 
@@ -932,7 +1022,8 @@ k_fold_wide(const uint64_t *__restrict__ tile_end, const SegWide *__restrict__ s
 {
     constexpr int NE = Vec16<DT>::kElems;
     const uint32_t policy = store_policy;
-    static_assert(MODE == kFoldChain || U == 1, "only the chain moves several vectors per thread");
+    static_assert(MODE == kFoldChain || (MODE == kFoldTree && U == 1), "the self-first order has a kernel of its own; only the chain "
+                                                                        "moves several vectors per thread");
     constexpr uint64_t TV = wide_tile_vecs(U);
     extern __shared__ uint64_t s_end[];
     const bool direct = nseg <= kFoldDirectSegs || uniform_tiles != 0;
@@ -959,16 +1050,12 @@ k_fold_wide(const uint64_t *__restrict__ tile_end, const SegWide *__restrict__ s
         if (tl * TV >= shift && (tl + 1) * TV - shift <= nvec) {
             if constexpr (MODE == kFoldTree) {
                 fold_tile_wide_tree<DT, OP, false>(sd, ndst, v, nvec, head_bytes, policy);
-            } else if constexpr (MODE == kFoldSelfFirst) {
-                fold_tile_wide_self<DT, OP, false>(sd, nsrc, v, nvec, head_bytes);
             } else {
                 fold_tile_wide<DT, OP, U, false>(sd, nsrc, ndst, v, nvec, head_bytes, policy);
             }
         } else {
             if constexpr (MODE == kFoldTree) {
                 fold_tile_wide_tree<DT, OP, true>(sd, ndst, v, nvec, head_bytes, policy);
-            } else if constexpr (MODE == kFoldSelfFirst) {
-                fold_tile_wide_self<DT, OP, true>(sd, nsrc, v, nvec, head_bytes);
             } else {
                 if (nvec != 0) fold_tile_wide<DT, OP, U, true>(sd, nsrc, ndst, v, nvec, head_bytes, policy);
             }
@@ -1024,6 +1111,7 @@ struct FoldLaunch {
     uint32_t store_policy;     // kStoreStream / kStoreThrough
     uint32_t uniform_tiles;    // non-zero: every segment has this many tiles, tile t belongs to segment t / uniform_tiles
     uint32_t waves = 0;        // non-zero: the one-store-per-wavefront kernel with this many wavefronts per workgroup
+                               // (wide self-first: sources of the widest segment)
     uint32_t pieces = 1;       // and this many 1 KiB pieces per source and workgroup
     uint32_t waves_fixed = 0;  // non-zero: every segment of the launch has this many sources
     bool waves_team = false;   // chains: the wavefronts share the fold

@@ -65,14 +65,38 @@ static hipError_t launch_wide_u(const FoldLaunch &l)
     return hipGetLastError();
 }
 
+// l.waves: sources of the widest segment
+template <int DT, int OP, int R>
+static hipError_t launch_wide_waves(const FoldLaunch &l)
+{
+    const bool direct = l.nseg <= kFoldDirectSegs || l.uniform_tiles != 0;
+    const size_t lds = static_cast<size_t>(l.waves) * kWaveLanes * 16 + (direct ? 0 : l.nseg * sizeof(uint64_t));
+    if (lds > 64 * 1024) {   // 64 sources and a staged prefix: more than a kernel gets unasked
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_fold_wide_waves<DT, OP, R>),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
+        if (e != hipSuccess) return e;
+    }
+    HCCLX_LAUNCH((k_fold_wide_waves<DT, OP, R>), dim3(static_cast<uint32_t>(l.total_tiles)), dim3(kWideWaves * kWaveLanes), lds, l.stream,
+                 l.tile_end, static_cast<const SegWide *>(l.segs), l.nseg, l.waves, l.pieces, l.uniform_tiles);
+    return hipGetLastError();
+}
+
 template <int DT, int OP, int MODE>
 static hipError_t launch_wide(const FoldLaunch &l)
 {
     if constexpr (MODE == kFoldChain) {
         return l.wide_unroll == kWideUnrollOne ? launch_wide_u<DT, OP, MODE, kWideUnrollOne>(l)
                                                : launch_wide_u<DT, OP, MODE, kWideUnrollMany>(l);
-    } else {
+    } else if constexpr (MODE == kFoldTree) {
         return launch_wide_u<DT, OP, MODE, 1>(l);
+    } else {
+        switch ((l.waves + kWideWaves - 1) / kWideWaves) {
+            case 1: return launch_wide_waves<DT, OP, 1>(l);
+            case 2: return launch_wide_waves<DT, OP, 2>(l);
+            case 3: return launch_wide_waves<DT, OP, 3>(l);
+            case 4: return launch_wide_waves<DT, OP, 4>(l);
+            default: return hipErrorInvalidValue;
+        }
     }
 }
 

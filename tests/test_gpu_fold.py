@@ -471,3 +471,46 @@ def test_errors_are_reported_not_launched():
     hcclx.fold([], T.FP32, T.SUM)           # nothing to do is fine
     hcclx.fold([(0, [0, 0], [0])], T.FP32)  # zero-size slices are skipped (LocalCopy/LocalReduce do the same)
     sync()
+
+
+@pytest.mark.parametrize("nsrc", [2, 16, 17, 31, 33, 49, 64])
+@pytest.mark.parametrize("dtype,op,counts", [(T.FP32, T.SUM, (1, 3, 257, 70001)), (T.BFP16, T.SUM, (5, 511, 1027)), (T.FP64, T.PROD, (1, 129, 300)),
+                                             (T.FP16, T.MIN, (7, 130000))])
+def test_wide_self_first_orders_one_piece_per_wavefront(nsrc, dtype, op, counts):
+    """Several segments in one launch, shorter than a vector up to many pieces, heads and tails; one to four outputs per
+    wavefront, the last ones of some wavefronts missing; one and two pieces per workgroup."""
+    rng = np.random.default_rng(nsrc * 7 + dtype + op)
+    esz = T.DTYPE_SIZE[dtype]
+    kind = "prod" if op == T.PROD else "uniform" if dtype in (T.FP32, T.FP64) else "normal"
+    if nsrc < 32:
+        counts += ((2 << 20) // esz + 11,)
+    xs = [[payload(rng, dtype, n, kind) for _ in range(nsrc)] for n in counts]
+    bufs = [[DevBuf(x, offset=(k % 3) * esz) for k, x in enumerate(seg)] for seg in xs]
+    outs = [[DevBuf(nbytes=seg[0].nbytes, offset=((k + i) % 5) * esz) for k in range(nsrc)] for i, seg in enumerate(xs)]
+    hcclx.fold_wide([(n, [b.ptr for b in bs], [o.ptr for o in os]) for n, bs, os in zip(counts, bufs, outs)], dtype, op,
+                    hcclx.FOLD_SELF_FIRST)
+    sync()
+    for seg, os in zip(xs, outs):
+        for r in sorted({0, 1, nsrc // 2, nsrc - 1}):
+            order = [r] + [k for k in range(nsrc) if k != r]
+            want = fold_oracle(seg, dtype, op, order, wide=fused_is_wide(dtype, op))
+            assert_same_bits(os[r].get(T.NP_STORAGE[dtype]), want, dtype, f"rank {r}")
+        assert all(o.guard_intact() for o in os)
+
+
+def test_wide_self_first_many_ragged_segments():
+    """More segments than the tile prefix is searched in place for, among 64 ranks: pieces and prefix are beyond 64 KiB of LDS."""
+    rng = np.random.default_rng(3)
+    counts = [int(c) for c in rng.integers(1, 700, size=80)]
+    xs = [[payload(rng, T.FP32, n, "uniform") for _ in range(64)] for n in counts]
+    whole = [np.concatenate([xs[i][k] for i in range(80)]) for k in range(64)]
+    bufs = [DevBuf(x) for x in whole]
+    outs = [DevBuf(nbytes=whole[0].nbytes) for _ in range(64)]
+    at = np.concatenate([[0], np.cumsum(counts)]) * 4
+    hcclx.fold_wide([(n, [b.ptr + int(at[i]) for b in bufs], [o.ptr + int(at[i]) for o in outs]) for i, n in enumerate(counts)], T.FP32,
+                    T.SUM, hcclx.FOLD_SELF_FIRST)
+    sync()
+    for r in (0, 17, 40, 63):
+        want = fold_oracle(whole, T.FP32, T.SUM, [r] + [k for k in range(64) if k != r], wide=False)
+        assert_same_bits(outs[r].get(np.float32), want, T.FP32, f"rank {r}")
+        assert outs[r].guard_intact()
