@@ -951,7 +951,7 @@ int build_wide_batches_impl(const hcclx_wide_seg_t *segs, uint32_t nseg, int dty
         }
         if (mode == HCCLX_FOLD_SELF_FIRST) {
             if (s.nsrc != s.ndst) return fail(HCCL_E_PARA, "self-first fold needs nsrc == ndst");
-            // the outputs are computed sixteen at a time by different workgroups: none may overwrite a source
+            // workgroups read the sources ahead of the outputs they store: none may overwrite a source
             // (integers have one value whatever the order and take the chain kernel: exempt)
             const uint64_t bytes = is_float_dtype(dtype) ? s.count * static_cast<uint64_t>(esz) : 0;
             for (uint32_t d = 0; d < s.ndst && bytes != 0; ++d) {

@@ -346,8 +346,8 @@ bool BuildFusedPlan(const std::vector<OpParam> &params, std::vector<Fold> &folds
             }
             if (!ok) continue;
             if (n > HCCLX_MAX_FAN) {
-                // the wide kernel computes the outputs sixteen at a time in different workgroups, so none of
-                // them may overwrite a source: an in-place collective writes to a staging buffer first
+                // the wide kernels take no destination that overlaps a source: an in-place collective writes to a
+                // staging buffer first
                 bool clash = false;
                 for (size_t j = 0; j < n && !clash; ++j) {
                     for (size_t k = 0; k < n && !clash; ++k) {

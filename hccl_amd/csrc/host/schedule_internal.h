@@ -236,9 +236,9 @@ struct FusedPlan {
     std::vector<hcclx_wide_seg_t> wideSegs;       // chains over more than HCCLX_MAX_FAN sources
     std::vector<hcclx_wide_seg_t> wideTreeSegs;   // trees with more leaves or levels than the 16-slot kernel holds
     std::vector<hcclx_wide_seg_t> wideSelfSegs;   // the per-rank orders of the one-shot templates among 17 .. 64 ranks
-    // The same in place (outputs overwrite inputs): the wide kernel computes its outputs sixteen at a time in
-    // different workgroups, so they go to a staging buffer first (dst[] hold byte offsets into it) and are copied
-    // to their places by a second launch.
+    // The same in place (outputs overwrite inputs): the wide kernels take no destination that overlaps a source, so
+    // they go to a staging buffer first (dst[] hold byte offsets into it) and are copied to their places by a second
+    // launch.
     struct StagedCopy {
         u64 offset;
         u64 dst;

@@ -68,8 +68,7 @@ typedef struct {
 /* A segment with up to HCCLX_MAX_WIDE_FAN sources and destinations, for communicators of more than
  * HCCLX_MAX_FAN ranks.  The modes are those of hcclx_seg_t; a floating-point tree may have up to six levels.
  * Aliasing rules as for hcclx_seg_t, except HCCLX_FOLD_SELF_FIRST over floating-point types: there no
- * destination may overlap a source (the outputs are computed sixteen at a time by different workgroups, each of
- * which reads every source; such a call is rejected). */
+ * destination may overlap a source (a workgroup reads ahead of the outputs it stores; such a call is rejected). */
 #define HCCLX_MAX_WIDE_FAN 64
 typedef struct {
     uint64_t count;
