@@ -750,9 +750,13 @@ constexpr uint64_t kTeamFrom = 48ull << 20;
 // Measured against the register kernel on fp32 PROD (us, register : wavefronts): 4 ranks x 64 MiB 97.7 : 77.4,
 // 8 x 64 MiB 210 : 175, 12 x 64 MiB 281 : 270, 12 x 256 MiB 1183 : 1056, 16 x 256 MiB 1582 : 1445, and at
 // 256 KiB per rank and below 4.6-5.6 : 3.2-3.5 among 8 to 12 ranks (at 4 KiB per rank: 4 ranks 3.9 : 3.1, 16 ranks
-// 5.3 : 3.9; the register kernel's threads each walk all the sources, here the wavefronts share them).  Where the register kernel measured
-// better it stays: two ranks below 32 MiB per rank (no difference), seven and eight ranks between 3 and 12 MiB per
-// rank (8 x 4 MiB: 10.6 : 12.1).  Pieces per workgroup: two for small launches and up to four ranks; five to eight
+// 5.3 : 3.9; the register kernel's threads each walk all the sources, here the wavefronts share them).  Where the register
+// kernel measured better it stays: two ranks below 32 MiB per rank (no difference); seven and eight ranks from 3 to 4.5 MiB
+// per rank of fp32 (8 x 3.5 MiB 12.4 : 12.8, 8 x 5 17.9 : 16.5, 8 x 11 37.7 : 30.6), to 6 MiB of fp16 (8 x 5 19.8 : 20.8, 8 x 8
+// 29.9 : 29.0), to 12 MiB of fp64, and never of bf16 (8 x 3.5 18.2 : 15.9, 8 x 8 33.0 : 29.6); and the 16-bit types among nine
+// and more ranks, where every wavefront widens every source for itself (bf16 SUM 12 x 1 MiB 16.6 : 10.6, 12 x 2 17.9 : 19.6,
+// 12 x 8 44 : 57, 16 x 2 26 : 30, 16 x 5 44 : 73, 16 x 16 110 : 204, 9 x 3.5 19.8 : 21.4, 9 x 8 34 : 42; 9 x 1.9 14.3 : 12.7 and
+// eight ranks x 16 56.8 : 55.7), from 2 MiB per rank.  Pieces per workgroup: two for small launches and up to four ranks; five to eight
 // ranks four below 32 MiB per rank (8 x 16 MiB: 47.9 / 43.0 us with 2 / 4) and two from there on (8 x 64 MiB:
 // 168.8 / 182.6); nine and more eight below 12 MiB per rank (12 x 8 MiB: 35.6 / 36.4 / 32.3 us with 2 / 4 / 8) and
 // four from there on (12 x 64 MiB: 268.7 / 260.6 / 281.7).  Launches
@@ -802,7 +806,11 @@ uint32_t waves_for(const DeviceCtx *ctx, const hcclx_seg_t *segs, uint32_t nseg,
     if (p == 0) {   // the shipped policy; a forced piece count takes every launch that passed the tests above
         if (mode == HCCLX_FOLD_SELF_FIRST) {
             if (widest == 2 && per_place < (32ull << 20)) return 0;
-            if ((widest == 7 || widest == 8) && per_place >= (3ull << 20) && per_place < (12ull << 20)) return 0;
+            if (widest == 7 || widest == 8) {
+                const uint64_t upto = esz == 8 ? 12ull << 20 : esz == 4 ? 9ull << 19 : dtype == HCCL_DATA_TYPE_FP16 ? 6ull << 20 : 0;
+                if (per_place >= (3ull << 20) && per_place < upto) return 0;
+            }
+            if (esz == 2 && widest >= 9 && per_place >= (2ull << 20)) return 0;
         }
         if (*team && written >= kTeamFrom) {
             p = 4;
