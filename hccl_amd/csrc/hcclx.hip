@@ -422,9 +422,7 @@ struct Batch {
     std::vector<SegWide> wide;   // instead of segs when maxn == kMaxWideFan
     int wide_unroll = 1;         // vectors per thread of the wide kernel
     uint32_t xcd_remap = 0;      // wide kernels: contiguous tile ranges per XCD (pays with 16 or more destinations)
-    std::vector<CopyBlock> blocks;   // instead of everything above: a list of blocks for the block copy kernel,
-    std::vector<CopySlab> slabs;     // cut into these slabs
-    uint32_t slab_shift = 0;         // of 1 << slab_shift tiles
+    BlockLaunch blocks;          // instead of everything above: a launch of the block copy kernel
     PhasedLaunch phased;         // instead of everything above: a launch of the copy kernel that writes one output at a time
     uint32_t store_policy = kStoreStream;   // how the fold kernels store (fold.h)
     uint32_t waves = 0;          // non-zero: the one-store-per-wavefront kernel, this many wavefronts per workgroup
@@ -435,7 +433,7 @@ struct Batch {
     size_t bytes() const
     {
         if (!phased.slabs.empty()) return phased.bytes();
-        if (!blocks.empty()) return align256(blocks.size() * sizeof(CopyBlock)) + slabs.size() * sizeof(CopySlab);
+        if (blocks.tiles != 0) return blocks.bytes();
         return align256(tile_end.size() * 8) + segs.size() * sizeof(SegDev) + wide.size() * sizeof(SegWide);
     }
 };
@@ -1078,9 +1076,8 @@ void fill_table(const Batch &b, char *h)
         b.phased.fill(h);
         return;
     }
-    if (!b.blocks.empty()) {
-        std::memcpy(h, b.blocks.data(), b.blocks.size() * sizeof(CopyBlock));
-        std::memcpy(h + align256(b.blocks.size() * sizeof(CopyBlock)), b.slabs.data(), b.slabs.size() * sizeof(CopySlab));
+    if (b.blocks.tiles != 0) {
+        b.blocks.fill(h);
         return;
     }
     std::memcpy(h, b.tile_end.data(), b.tile_end.size() * 8);
@@ -1122,10 +1119,8 @@ int launch_batch(const DeviceCtx *ctx, const Batch &b, const char *d_table, hipS
         if (pe != hipSuccess) return fail_hip(pe, "phased copy kernel launch");
         return HCCL_SUCCESS;
     }
-    if (!b.blocks.empty()) {
-        const BlockTable tab{reinterpret_cast<const CopyBlock *>(d_table),
-                             reinterpret_cast<const CopySlab *>(d_table + align256(b.blocks.size() * sizeof(CopyBlock)))};
-        const hipError_t be = launch_copy_blocks(tab, static_cast<uint32_t>(b.slabs.size()), b.slab_shift, stream);
+    if (b.blocks.tiles != 0) {
+        const hipError_t be = launch_copy_blocks(b.blocks.table(d_table), b.blocks.tiles, stream);
         if (be != hipSuccess) return fail_hip(be, "block copy kernel launch");
         return HCCL_SUCCESS;
     }
@@ -1407,12 +1402,13 @@ int hcclx_alltoallv_plan_create(const void *const *send, void *const *recv, cons
     Built built;
     Batch b;
     b.copy = true;
-    list_alltoallv_blocks(send, recv, send_counts, sdispls, rdispls, n, static_cast<uint32_t>(esz), &b.blocks);
-    if (!b.blocks.empty() && !cut_slabs(b.blocks, kBlockTableSlabs, ~0u, &b.slabs, &b.slab_shift)) {
-        return fail(HCCL_E_PARA, "too much data for one launch");
+    b.blocks.tiles = list_alltoallv_blocks(send, recv, send_counts, sdispls, rdispls, n, static_cast<uint32_t>(esz), &b.blocks.blocks);
+    if (b.blocks.tiles > 0x7fffffffull) return fail(HCCL_E_PARA, "too much data for one launch");
+    for (const CopyBlock &c : b.blocks.blocks) built.algo_bytes += 2 * c.bytes;
+    if (b.blocks.tiles != 0) {
+        b.blocks.index();
+        built.batches.push_back(std::move(b));
     }
-    for (const CopyBlock &c : b.blocks) built.algo_bytes += 2 * c.bytes;
-    if (!b.blocks.empty()) built.batches.push_back(std::move(b));
     return plan_from(ctx, built, plan);
 }
 

@@ -113,12 +113,24 @@ struct PhasedStream {
 // Turns streams into launches: streams that continue each other (source and every destination) are joined, and cut into
 // slabs as small as max_slabs of them allow; batches of up to batch_bytes are written to one place after the other.
 void build_phased(std::vector<PhasedStream> &streams, uint64_t batch_bytes, uint32_t max_slabs, std::vector<PhasedLaunch> *out);
-// The non-empty blocks of an AlltoAllV with host tables (row-major n x n, elements of esz bytes).
-void list_alltoallv_blocks(const void *const *send, void *const *recv, const uint64_t *send_counts, const uint64_t *sdispls,
-                           const uint64_t *rdispls, uint32_t n, uint32_t esz, std::vector<CopyBlock> *blocks);
-// Cuts blocks into slabs of 1 << shift tiles: the smallest power of two with which there are at most max_slabs of them,
-// numbered below max_at inside their block.  False when the launch would need more than 2^31 - 1 workgroups.
-bool cut_slabs(const std::vector<CopyBlock> &blocks, size_t max_slabs, uint32_t max_at, std::vector<CopySlab> *slabs, uint32_t *shift);
+// The non-empty blocks of an AlltoAllV with host tables (row-major n x n, elements of esz bytes), their tiles numbered
+// through; returns the number of tiles.
+uint64_t list_alltoallv_blocks(const void *const *send, void *const *recv, const uint64_t *send_counts, const uint64_t *sdispls,
+                               const uint64_t *rdispls, uint32_t n, uint32_t esz, std::vector<CopyBlock> *blocks);
+// The start table of blocks whose first tiles are begin[0 .. n): the block that holds tile g << *shift for every group g of
+// the `tiles` tiles, and behind them the block of the last tile.  The smallest groups of which there are at most max_groups.
+void index_tiles(const uint64_t *begin, size_t n, uint64_t tiles, uint32_t max_groups, std::vector<uint32_t> *starts, uint32_t *shift);
+// A launch's tables in device memory: blocks, start table.
+struct BlockLaunch {
+    std::vector<CopyBlock> blocks;
+    std::vector<uint32_t> starts;
+    uint32_t shift = 0;
+    uint64_t tiles = 0;
+    void index();           // once the blocks are listed
+    size_t bytes() const;
+    void fill(char *h) const;
+    BlockTable table(const char *d) const;   // the arrays of a launch table at d
+};
 
 // Queues the copy of a launch table from the pinned ring to its place in device memory.
 int upload_table(char *d, const char *h, size_t bytes, hipStream_t stream);

@@ -48,44 +48,63 @@ int fill_ptrs(const void *const *send, void *const *recv, uint32_t n, VRankPtrs 
 
 namespace hcclx {
 
-void list_alltoallv_blocks(const void *const *send, void *const *recv, const uint64_t *send_counts, const uint64_t *sdispls,
-                           const uint64_t *rdispls, uint32_t n, uint32_t esz, std::vector<CopyBlock> *blocks)
+uint64_t list_alltoallv_blocks(const void *const *send, void *const *recv, const uint64_t *send_counts, const uint64_t *sdispls,
+                               const uint64_t *rdispls, uint32_t n, uint32_t esz, std::vector<CopyBlock> *blocks)
 {
     blocks->clear();
     blocks->reserve(static_cast<size_t>(n) * n);
+    uint64_t tiles = 0;
     for (uint32_t i = 0; i < n; ++i) {
         for (uint32_t j = 0; j < n; ++j) {
             const uint64_t bytes = send_counts[i * n + j] * esz;
             if (bytes == 0) continue;
-            blocks->push_back({static_cast<const char *>(send[i]) + sdispls[i * n + j] * esz,
-                               static_cast<char *>(recv[j]) + rdispls[j * n + i] * esz, bytes});
+            char *dst = static_cast<char *>(recv[j]) + rdispls[j * n + i] * esz;
+            blocks->push_back({static_cast<const char *>(send[i]) + sdispls[i * n + j] * esz, dst, bytes, tiles});
+            tiles += v_tiles_of(bytes, reinterpret_cast<uint64_t>(dst), 1);
         }
+    }
+    return tiles;
+}
+
+void index_tiles(const uint64_t *begin, size_t n, uint64_t tiles, uint32_t max_groups, std::vector<uint32_t> *starts, uint32_t *shift)
+{
+    *shift = 0;
+    while ((tiles - 1) >> *shift >= max_groups) ++*shift;
+    starts->clear();
+    starts->reserve(((tiles - 1) >> *shift) + 2);
+    uint32_t b = 0;
+    for (uint64_t first = 0; first < tiles + (1ull << *shift); first += 1ull << *shift) {
+        const uint64_t tile = first < tiles ? first : tiles - 1;
+        while (b + 1 < n && begin[b + 1] <= tile) ++b;
+        starts->push_back(b);
     }
 }
 
-bool cut_slabs(const std::vector<CopyBlock> &blocks, size_t max_slabs, uint32_t max_at, std::vector<CopySlab> *slabs, uint32_t *shift)
+void BlockLaunch::index()
 {
-    std::vector<uint64_t> tiles(blocks.size());
-    uint64_t most = 0;
-    for (size_t b = 0; b < blocks.size(); ++b) {
-        tiles[b] = v_tiles_of(blocks[b].bytes, reinterpret_cast<uint64_t>(blocks[b].dst), 1);
-        most = tiles[b] > most ? tiles[b] : most;
-    }
-    if (max_slabs < blocks.size()) max_slabs = blocks.size();
-    uint64_t n = 0;
-    for (*shift = 0;; ++*shift) {
-        const uint64_t last = (1ull << *shift) - 1;
-        n = 0;
-        for (uint64_t t : tiles) n += (t + last) >> *shift;
-        if (n <= max_slabs && ((most + last) >> *shift) <= max_at) break;
-    }
-    if (n << *shift > 0x7fffffffull) return false;
-    slabs->clear();
-    slabs->reserve(n);
-    for (size_t b = 0; b < blocks.size(); ++b) {
-        for (uint64_t k = 0; k << *shift < tiles[b]; ++k) slabs->push_back({static_cast<uint32_t>(b), static_cast<uint32_t>(k)});
-    }
-    return true;
+    std::vector<uint64_t> begin(blocks.size());
+    for (size_t b = 0; b < blocks.size(); ++b) begin[b] = blocks[b].begin;
+    // four groups to a block, so that a small table stays small: what lies in front of the kernel is its upload
+    const uint64_t groups = 4 * static_cast<uint64_t>(blocks.size());
+    index_tiles(begin.data(), begin.size(), tiles, groups < kBlockTableGroups ? static_cast<uint32_t>(groups) : kBlockTableGroups, &starts,
+                &shift);
+}
+
+namespace {
+size_t list_bytes(size_t blocks) { return (blocks * sizeof(CopyBlock) + 255) & ~static_cast<size_t>(255); }
+}  // namespace
+
+size_t BlockLaunch::bytes() const { return list_bytes(blocks.size()) + starts.size() * sizeof(uint32_t); }
+
+void BlockLaunch::fill(char *h) const
+{
+    std::memcpy(h, blocks.data(), blocks.size() * sizeof(CopyBlock));
+    std::memcpy(h + list_bytes(blocks.size()), starts.data(), starts.size() * sizeof(uint32_t));
+}
+
+BlockTable BlockLaunch::table(const char *d) const
+{
+    return {reinterpret_cast<const CopyBlock *>(d), reinterpret_cast<const uint32_t *>(d + list_bytes(blocks.size())), shift};
 }
 
 }  // namespace hcclx
@@ -149,57 +168,56 @@ int hcclx_alltoallv(const void *const *send, void *const *recv, const uint64_t *
             if (e != hipSuccess) return fail_hip(e, "alltoall kernel launch");
             return HCCL_SUCCESS;
         }
-        std::vector<CopyBlock> blocks;
-        list_alltoallv_blocks(send, recv, send_counts, sdispls, rdispls, n, static_cast<uint32_t>(esz), &blocks);
-        if (blocks.empty()) return HCCL_SUCCESS;
-        std::vector<CopySlab> slabs;
-        uint32_t shift = 0;
         bool small = n <= kA2avInlineRanks && ctx->a2av_direct;
         for (size_t k = 0; k < static_cast<size_t>(n) * n && small; ++k) {
             small = send_counts[k] <= 0xffffffffull && sdispls[k] <= 0xffffffffull && rdispls[k] <= 0xffffffffull;
         }
         if (small) {
-            // small host tables and their slabs ride in the kernel arguments: nothing is copied in front of the kernel
-            if (!cut_slabs(blocks, kA2avInlineSlabs, 256, &slabs, &shift)) return fail(HCCL_E_PARA, "too much data for one launch");
+            // small host tables ride in the kernel arguments: nothing is copied in front of the kernel
             A2avInline tab;
             tab.n = n;
             tab.inv_n = 65536u / n + 1u;
             tab.esz = static_cast<uint32_t>(esz);
-            uint8_t number[kA2avInlineBlocks];   // of the non-empty blocks in the n x n tables
-            uint32_t live = 0;
+            uint64_t begin[kA2avInlineBlocks];
+            uint64_t tiles = 0;
             for (uint32_t i = 0; i < n; ++i) {
                 tab.send[i] = ptrs.send[i];
                 tab.recv[i] = ptrs.recv[i];
                 for (uint32_t j = 0; j < n; ++j) {
                     const uint32_t k = i * n + j;
-                    if (send_counts[k] != 0) number[live++] = static_cast<uint8_t>(k);
                     tab.counts[k] = static_cast<uint32_t>(send_counts[k]);
                     tab.sdispls[k] = static_cast<uint32_t>(sdispls[k]);
                     tab.rdispls[k] = static_cast<uint32_t>(rdispls[j * n + i]);
+                    begin[k] = tiles;
+                    tab.begin[k] = static_cast<uint32_t>(tiles);
+                    tiles += v_tiles_of(send_counts[k] * esz, reinterpret_cast<uint64_t>(ptrs.recv[j]) + rdispls[j * n + i] * esz, 1);
                 }
             }
-            for (size_t k = 0; k < slabs.size(); ++k) {
-                const uint32_t one = number[slabs[k].source] | slabs[k].at << 8;
-                tab.slabs[k >> 1] = (k & 1) ? (tab.slabs[k >> 1] | one << 16) : one;
+            if (tiles == 0) return HCCL_SUCCESS;
+            if (tiles <= 0x7fffffffull) {
+                std::vector<uint32_t> starts;
+                index_tiles(begin, static_cast<size_t>(n) * n, tiles, kA2avInlineGroups, &starts, &tab.shift);
+                std::memset(tab.starts, 0, sizeof(tab.starts));
+                for (size_t g = 0; g < starts.size(); ++g) tab.starts[g >> 2] |= starts[g] << (g & 3) * 8;
+                const hipError_t e = launch_alltoallv_inline(tab, tiles, st);
+                if (e != hipSuccess) return fail_hip(e, "alltoallv kernel launch");
+                return HCCL_SUCCESS;
             }
-            hipError_t e = launch_alltoallv_inline(tab, static_cast<uint32_t>(slabs.size()), shift, st);
-            if (e != hipSuccess) return fail_hip(e, "alltoallv kernel launch");
-            return HCCL_SUCCESS;
         }
-        // any other host table: the non-empty blocks and their slabs in device memory
-        if (!cut_slabs(blocks, kBlockTableSlabs, ~0u, &slabs, &shift)) return fail(HCCL_E_PARA, "too much data for one launch");
-        const size_t list_bytes = (blocks.size() * sizeof(CopyBlock) + 255) & ~static_cast<size_t>(255);
-        const size_t bytes = list_bytes + slabs.size() * sizeof(CopySlab);
+        // any other host table: the non-empty blocks and their start table in device memory
+        BlockLaunch l;
+        l.tiles = list_alltoallv_blocks(send, recv, send_counts, sdispls, rdispls, n, static_cast<uint32_t>(esz), &l.blocks);
+        if (l.tiles == 0) return HCCL_SUCCESS;
+        if (l.tiles > 0x7fffffffull) return fail(HCCL_E_PARA, "too much data for one launch");
+        l.index();
         char *h = nullptr;
         char *d = nullptr;
-        rc = ring_reserve(ctx, bytes, st, &h, &d);
+        rc = ring_reserve(ctx, l.bytes(), st, &h, &d);
         if (rc != HCCL_SUCCESS) return rc;
-        std::memcpy(h, blocks.data(), blocks.size() * sizeof(CopyBlock));
-        std::memcpy(h + list_bytes, slabs.data(), slabs.size() * sizeof(CopySlab));
-        rc = upload_table(d, h, bytes, st);
+        l.fill(h);
+        rc = upload_table(d, h, l.bytes(), st);
         if (rc != HCCL_SUCCESS) return rc;
-        const BlockTable tab{reinterpret_cast<const CopyBlock *>(d), reinterpret_cast<const CopySlab *>(d + list_bytes)};
-        hipError_t e = launch_copy_blocks(tab, static_cast<uint32_t>(slabs.size()), shift, st);
+        const hipError_t e = launch_copy_blocks(l.table(d), l.tiles, st);
         if (e != hipSuccess) return fail_hip(e, "alltoallv kernel launch");
         return HCCL_SUCCESS;
     }

@@ -57,7 +57,7 @@ struct VRankPtrs {
 
 // Count / displacement tables as the kernels read them.  Host tables of up to 15 ranks travel inside the kernel
 // arguments (no host-to-device copy is queued in front of the kernel); larger host tables become a list of
-// blocks and slabs in device memory; tables that already live on the device are read through pointers.
+// blocks in device memory; tables that already live on the device are read through pointers.
 struct A2avTablesPtr {
     const uint64_t *send_counts;
     const uint64_t *sdispls;
@@ -66,36 +66,38 @@ struct A2avTablesPtr {
     __device__ uint64_t sdispl(uint32_t p) const { return sdispls[p]; }
     __device__ uint64_t rdispl(uint32_t p) const { return rdispls[p]; }
 };
-// Host tables.  A block of the exchange (source i to destination j) is cut into slabs of a power of two of 4 KiB tiles,
-// the last one as long as what is left, and a workgroup finds its slab by arithmetic and the block by the slab's
-// entry: two dependent scalar loads, where a search in a prefix of the blocks' tiles took 2 + log2(n * n).
+// Host tables.  The 4 KiB tiles of all blocks of the exchange (source i to destination j) are numbered through, and a
+// workgroup moves one: there are as many workgroups as tiles, whatever the blocks' lengths.  Tiles come in groups of
+// 1 << shift, and starts[g] is the block that holds the first tile of group g: the block of a tile lies between starts[g] and
+// starts[g + 1].  With several groups to a block these are mostly one and the same, and two dependent scalar loads find
+// it, where a search in the whole prefix of the blocks' tiles takes 2 + log2(n * n).
 struct CopyBlock {
     const char *src;
     char *dst;
     uint64_t bytes;
-};
-struct CopySlab {
-    uint32_t source;   // block (or source of a copy to several places)
-    uint32_t at;       // number of the slab inside it
+    uint64_t begin;   // number of its first tile
 };
 // A launch's tables in device memory, for host tables of any size.
 struct BlockTable {
     const CopyBlock *blocks;
-    const CopySlab *slabs;
+    const uint32_t *starts;
+    uint32_t shift;
 };
-constexpr uint32_t kBlockTableSlabs = 4096;   // at most, unless there are more blocks
+constexpr uint32_t kBlockTableGroups = 4096;   // at most
 // The same in the kernel arguments, for up to 15 ranks and 32-bit counts: nothing is copied in front of the kernel.
-// Block b is source b / n, destination b % n.  A slab is 16 bits: block in the low eight, its number above.
+// Block b is source b / n, destination b % n, the empty ones among them (an empty block begins where the next one does).
 constexpr uint32_t kA2avInlineRanks = 15;
 constexpr uint32_t kA2avInlineBlocks = kA2avInlineRanks * kA2avInlineRanks;
-constexpr uint32_t kA2avInlineSlabs = 520;
+constexpr uint32_t kA2avInlineGroups = 128;
 struct A2avInline {
     const char *send[kA2avInlineRanks];
     char *recv[kA2avInlineRanks];
     uint32_t counts[kA2avInlineBlocks];
     uint32_t sdispls[kA2avInlineBlocks];
     uint32_t rdispls[kA2avInlineBlocks];
-    uint32_t slabs[kA2avInlineSlabs / 2];
+    uint32_t begin[kA2avInlineBlocks];
+    uint32_t starts[kA2avInlineGroups / 4 + 1];   // a byte each
+    uint32_t shift;
     uint32_t n;
     uint32_t inv_n;   // 65536 / n + 1: b * inv_n >> 16 is b / n for every block number
     uint32_t esz;
@@ -117,6 +119,10 @@ struct AgvTablesPtr {
 // all its places by the same XCD); a batch of slabs, a few MiB, is copied to its first place, then to the second and so
 // on.  The last slab of a source is as long as what is left, so sources of any lengths share a launch and only those
 // ends leave workgroups that exit at once.
+struct CopySlab {
+    uint32_t source;
+    uint32_t at;       // number of the slab inside it
+};
 struct PhasedSource {
     const char *src;
     uint64_t bytes;
@@ -153,10 +159,10 @@ struct AgvTablesInline {
     __device__ uint64_t displ(uint32_t i) const { return displs[i]; }
 };
 
-// nslabs << slab_shift workgroups, slabs of 1 << slab_shift tiles
-hipError_t launch_copy_blocks(const BlockTable &tab, uint32_t nslabs, uint32_t slab_shift, hipStream_t stream);
+// tiles: of all blocks
+hipError_t launch_copy_blocks(const BlockTable &tab, uint64_t tiles, hipStream_t stream);
 hipError_t launch_equal_blocks(const EqualBlocks &tab, uint32_t n, hipStream_t stream);
-hipError_t launch_alltoallv_inline(const A2avInline &tab, uint32_t nslabs, uint32_t slab_shift, hipStream_t stream);
+hipError_t launch_alltoallv_inline(const A2avInline &tab, uint64_t tiles, hipStream_t stream);
 // One batch after the other (grid z), each to one place after the other (grid y): per_batch slabs of slab_tiles tiles.
 struct PhasedGrid {
     uint32_t slab_tiles;

@@ -171,35 +171,43 @@ k_alltoallv(Ptrs ptrs, Tabs tabs, uint32_t n, uint32_t esz, uint32_t tiles_per_b
     }
 }
 
-__device__ __forceinline__ CopySlab slab_of(const BlockTable &t, uint32_t k) { return t.slabs[k]; }
-__device__ __forceinline__ CopySlab slab_of(const A2avInline &t, uint32_t k)
-{
-    const uint32_t two = t.slabs[k >> 1];
-    const uint32_t one = (k & 1u) ? two >> 16 : two & 0xffffu;
-    return {one & 255u, one >> 8};
-}
+__device__ __forceinline__ uint32_t start_of(const BlockTable &t, uint32_t g) { return t.starts[g]; }
+__device__ __forceinline__ uint32_t start_of(const A2avInline &t, uint32_t g) { return t.starts[g >> 2] >> (g & 3u) * 8 & 255u; }
+__device__ __forceinline__ uint64_t begin_of(const BlockTable &t, uint32_t b) { return t.blocks[b].begin; }
+__device__ __forceinline__ uint64_t begin_of(const A2avInline &t, uint32_t b) { return t.begin[b]; }
 __device__ __forceinline__ CopyBlock block_of(const BlockTable &t, uint32_t b) { return t.blocks[b]; }
 __device__ __forceinline__ CopyBlock block_of(const A2avInline &t, uint32_t b)
 {
     const uint32_t i = b * t.inv_n >> 16;
     const uint32_t j = b - i * t.n;
     return {t.send[i] + static_cast<uint64_t>(t.sdispls[b]) * t.esz, t.recv[j] + static_cast<uint64_t>(t.rdispls[b]) * t.esz,
-            static_cast<uint64_t>(t.counts[b]) * t.esz};
+            static_cast<uint64_t>(t.counts[b]) * t.esz, t.begin[b]};
 }
 
 // Blocks of any lengths, one 4 KiB tile per workgroup and one vector per thread, stored through the L2: bound by HBM.
 // A wavefront that loads and stores one vector per lane copies faster than one that moves two (1 GiB: 6.66 against
 // 6.22 TB/s with these stores, 6.54 streamed); 8 x 4096 x 7168 bf16 with two vectors, streamed, and the block searched
-// in a prefix: 151.3 us, this way 145.4.
+// in a prefix: 151.3 us, this way 145.4.  One workgroup per tile and none besides: an idle one costs 0.23 ns, and with blocks
+// cut into slabs of one size (two scalar loads without a search) 63 ranks that send 512 MiB, Zipf, launch fifteen for
+// every tile: 629 us, this way 205; 15 ranks 185 and 178, 32 ranks with blocks of nearly one size 114 and 101.
 template <typename Tab>
-__global__ void __launch_bounds__(kThreads) k_copy_blocks(Tab tab, uint32_t slab_shift)
+__global__ void __launch_bounds__(kThreads) k_copy_blocks(Tab tab)
 {
-    const CopySlab slab = slab_of(tab, blockIdx.x >> slab_shift);
-    const uint64_t tl = (static_cast<uint64_t>(slab.at) << slab_shift) + (blockIdx.x & ((1u << slab_shift) - 1u));
-    const CopyBlock b = block_of(tab, slab.source);
+    const uint64_t tile = blockIdx.x;
+    const uint32_t group = static_cast<uint32_t>(tile >> tab.shift);
+    uint32_t lo = start_of(tab, group);
+    uint32_t hi = start_of(tab, group + 1);
+    while (lo < hi) {   // the last block that begins at the tile or in front of it
+        const uint32_t mid = (lo + hi + 1) >> 1;
+        if (begin_of(tab, mid) <= tile) {
+            lo = mid;
+        } else {
+            hi = mid - 1;
+        }
+    }
+    const CopyBlock b = block_of(tab, lo);
     char *dst = b.dst;
-    if (tl >= v_tiles_of(b.bytes, reinterpret_cast<uint64_t>(dst), 1)) return;
-    copy_tile<1, false, kStoreThrough>(b.src, reinterpret_cast<uint64_t>(dst), b.bytes, tl, 1, [=](uint32_t) { return dst; });
+    copy_tile<1, false, kStoreThrough>(b.src, reinterpret_cast<uint64_t>(dst), b.bytes, tile - b.begin, 1, [=](uint32_t) { return dst; });
 }
 
 // Equal blocks: nothing to look up and no table to bring, the block is the workgroup's place in the grid (x: tile, y:
@@ -284,9 +292,9 @@ hipError_t launch_alltoallv(const VRankPtrs &ptrs, const uint64_t *send_counts, 
     return hipGetLastError();
 }
 
-hipError_t launch_copy_blocks(const BlockTable &tab, uint32_t nslabs, uint32_t slab_shift, hipStream_t stream)
+hipError_t launch_copy_blocks(const BlockTable &tab, uint64_t tiles, hipStream_t stream)
 {
-    HCCLX_LAUNCH((k_copy_blocks<BlockTable>), dim3(nslabs << slab_shift), dim3(kThreads), 0, stream, tab, slab_shift);
+    HCCLX_LAUNCH((k_copy_blocks<BlockTable>), dim3(static_cast<uint32_t>(tiles)), dim3(kThreads), 0, stream, tab);
     return hipGetLastError();
 }
 
@@ -298,9 +306,9 @@ hipError_t launch_equal_blocks(const EqualBlocks &tab, uint32_t n, hipStream_t s
     return hipGetLastError();
 }
 
-hipError_t launch_alltoallv_inline(const A2avInline &tab, uint32_t nslabs, uint32_t slab_shift, hipStream_t stream)
+hipError_t launch_alltoallv_inline(const A2avInline &tab, uint64_t tiles, hipStream_t stream)
 {
-    HCCLX_LAUNCH((k_copy_blocks<A2avInline>), dim3(nslabs << slab_shift), dim3(kThreads), 0, stream, tab, slab_shift);
+    HCCLX_LAUNCH((k_copy_blocks<A2avInline>), dim3(static_cast<uint32_t>(tiles)), dim3(kThreads), 0, stream, tab);
     return hipGetLastError();
 }
 

@@ -123,6 +123,28 @@ def test_alltoallv_slabs_of_unequal_blocks(n, least, most, hot):
     run_a2av(m.tolist(), T.INT8, rng, send_pad=n % 7)
 
 
+@pytest.mark.parametrize("n,hot", [(64, 16 << 20), (63, 9 << 20), (60, 3 << 20), (15, 16 << 20)])
+def test_alltoallv_one_long_block_among_many_short_ones(n, hot):
+    """No block empty: as many workgroups as there are tiles, also where one block has most of them; the call and the plan."""
+    rng = np.random.default_rng(n)
+    m = rng.integers(1, 300, size=(n, n))
+    m[n // 2][n - 1] = hot + 5
+    m = m.tolist()
+    run_a2av(m, T.INT8, rng, send_pad=1)
+    v = [T.alltoallvc_to_v(m, r) for r in range(n)]
+    ins = [rng.integers(0, 256, size=sum(m[i]), dtype=np.uint8) for i in range(n)]
+    want = T.run_alltoallv(ins, [x[0] for x in v], [x[1] for x in v], [x[2] for x in v], [x[3] for x in v], [sum(x[2]) for x in v])
+    send = [DevBuf(x) for x in ins]
+    recv = [DevBuf(nbytes=sum(x[2]), offset=j % 17) for j, x in enumerate(v)]
+    plan = hcclx.AlltoAllVPlan([s.ptr for s in send], [r.ptr for r in recv], np.array([x[0] for x in v], np.uint64).ravel(),
+                               np.array([x[1] for x in v], np.uint64).ravel(), np.array([x[3] for x in v], np.uint64).ravel(), T.INT8)
+    plan.launch()
+    torch.cuda.synchronize()
+    plan.close()
+    for j in range(n):
+        assert np.array_equal(recv[j].get(np.uint8), want[j]) and recv[j].guard_intact(), j
+
+
 def test_alltoallv_all_zero_and_single_rank():
     rng = np.random.default_rng(1)
     run_a2av([[0, 0], [0, 0]], T.FP32, rng)

@@ -1,0 +1,54 @@
+"""The launch tables of the copy kernels, checked tile by tile on the CPU by a program built against the library
+(tests/check_copy_tables.cpp): every tile is moved by exactly one workgroup, and no workgroup is launched without one."""
+import os
+import random
+import re
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIB = os.path.join(ROOT, "hccl_amd", "lib")
+
+
+@pytest.fixture(scope="module")
+def check(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("tables") / "check_copy_tables")
+    cmd = ["g++", "-std=c++17", "-O2", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", f"-I{ROOT}/include", f"-I{ROOT}/hccl_amd/csrc",
+           os.path.join(ROOT, "tests", "check_copy_tables.cpp"), "-o", exe, f"-L{LIB}", "-lhccl_amd", "-L/opt/rocm/lib", "-lamdhip64",
+           f"-Wl,-rpath,{LIB}", "-Wl,-rpath,/opt/rocm/lib"]
+    built = subprocess.run(cmd, capture_output=True, text=True)
+    assert built.returncode == 0, built.stderr[-3000:]
+
+    def run(*args):
+        r = subprocess.run([exe] + [str(a) for a in args], capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, r.stdout + r.stderr
+        return [int(x) for x in re.findall(r"\d+", r.stdout)]
+    return run
+
+
+def _matrix(kind, n):
+    rng = random.Random(n)
+    if kind == "equal":
+        return [[70001] * n for _ in range(n)]
+    if kind == "zipf":       # 2048 rows of 14336 bytes per rank, most of them for the first ranks
+        w = [(j + 1) ** -1.2 for j in range(n)]
+        return [[max(1, int(2048 * x / sum(w))) * 14336 for x in w] for _ in range(n)]
+    if kind == "empty":      # four blocks of five empty, at the ends too
+        return [[0 if (i * n + j) % 5 != 2 else rng.randint(1, 40000) for j in range(n)] for i in range(n)]
+    m = [[rng.randint(1, 200) for _ in range(n)] for _ in range(n)]
+    m[n - 1][0] = {"hot": 16 << 20, "huge": 2 << 30}[kind]
+    return m
+
+
+@pytest.mark.parametrize("kind", ["equal", "zipf", "hot", "huge", "empty"])
+@pytest.mark.parametrize("n", [2, 3, 8, 15, 16, 48, 60, 63, 64])
+def test_every_tile_of_an_alltoallv_is_found_once(check, n, kind):
+    m = _matrix(kind, n)
+    tiles, groups, size = check("blocks", n, *[c for row in m for c in row])
+    payload = sum(c for row in m for c in row)
+    live = sum(1 for row in m for c in row if c)
+    # the grid: a block's tiles are its vectors, shifted by up to 63 of them, and one more for the bytes outside them
+    assert tiles <= payload // 4096 + 2 * live
+    # what is uploaded in front of the kernel
+    assert groups <= 4096 and size <= 32 * live + 256 + 4 * (min(4096, 4 * live) + 1)
