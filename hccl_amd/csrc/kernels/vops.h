@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "launch.h"
+#include "segtab.h"
 
 namespace hcclx {
 
@@ -158,6 +159,9 @@ struct AgvTablesInline {
     __device__ uint64_t count(uint32_t i) const { return counts[i]; }
     __device__ uint64_t displ(uint32_t i) const { return displs[i]; }
 };
+
+// Workgroups of kThreads work-items that one launch takes along x: HIP allows fewer than 2^32 work-items there.
+constexpr uint64_t kMostBlocksX = 0xffffffffull / kThreads;
 
 // tiles: of all blocks
 hipError_t launch_copy_blocks(const BlockTable &tab, uint64_t tiles, hipStream_t stream);

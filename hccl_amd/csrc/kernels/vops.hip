@@ -191,9 +191,9 @@ __device__ __forceinline__ CopyBlock block_of(const A2avInline &t, uint32_t b)
 // cut into slabs of one size (two scalar loads without a search) 63 ranks that send 512 MiB, Zipf, launch fifteen for
 // every tile: 629 us, this way 205; 15 ranks 185 and 178, 32 ranks with blocks of nearly one size 114 and 101.
 template <typename Tab>
-__global__ void __launch_bounds__(kThreads) k_copy_blocks(Tab tab)
+__global__ void __launch_bounds__(kThreads) k_copy_blocks(Tab tab, uint64_t first)
 {
-    const uint64_t tile = blockIdx.x;
+    const uint64_t tile = first + blockIdx.x;
     const uint32_t group = static_cast<uint32_t>(tile >> tab.shift);
     uint32_t lo = start_of(tab, group);
     uint32_t hi = start_of(tab, group + 1);
@@ -292,11 +292,21 @@ hipError_t launch_alltoallv(const VRankPtrs &ptrs, const uint64_t *send_counts, 
     return hipGetLastError();
 }
 
-hipError_t launch_copy_blocks(const BlockTable &tab, uint64_t tiles, hipStream_t stream)
+namespace {
+// 64 GiB and more take several launches.
+template <typename Tab> hipError_t launch_tiles(const Tab &tab, uint64_t tiles, hipStream_t stream)
 {
-    HCCLX_LAUNCH((k_copy_blocks<BlockTable>), dim3(static_cast<uint32_t>(tiles)), dim3(kThreads), 0, stream, tab);
-    return hipGetLastError();
+    for (uint64_t first = 0; first < tiles; first += kMostBlocksX) {
+        const uint64_t take = tiles - first < kMostBlocksX ? tiles - first : kMostBlocksX;
+        HCCLX_LAUNCH((k_copy_blocks<Tab>), dim3(static_cast<uint32_t>(take)), dim3(kThreads), 0, stream, tab, first);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
+}  // namespace
+
+hipError_t launch_copy_blocks(const BlockTable &tab, uint64_t tiles, hipStream_t stream) { return launch_tiles(tab, tiles, stream); }
 
 hipError_t launch_equal_blocks(const EqualBlocks &tab, uint32_t n, hipStream_t stream)
 {
@@ -306,11 +316,7 @@ hipError_t launch_equal_blocks(const EqualBlocks &tab, uint32_t n, hipStream_t s
     return hipGetLastError();
 }
 
-hipError_t launch_alltoallv_inline(const A2avInline &tab, uint64_t tiles, hipStream_t stream)
-{
-    HCCLX_LAUNCH((k_copy_blocks<A2avInline>), dim3(static_cast<uint32_t>(tiles)), dim3(kThreads), 0, stream, tab);
-    return hipGetLastError();
-}
+hipError_t launch_alltoallv_inline(const A2avInline &tab, uint64_t tiles, hipStream_t stream) { return launch_tiles(tab, tiles, stream); }
 
 namespace {
 template <typename Tab> hipError_t launch_phased(const Tab &tab, const PhasedGrid &g, hipStream_t stream)

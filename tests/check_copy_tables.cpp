@@ -14,6 +14,8 @@ using namespace hcclx;
 
 namespace {
 
+static_assert((kMostBlocksX + 1) * kThreads > 0xffffffffull && kMostBlocksX * kThreads <= 0xffffffffull, "work-items along x of one launch");
+
 int wrong(const char *what, uint64_t at)
 {
     std::printf("wrong: %s at %llu\n", what, static_cast<unsigned long long>(at));

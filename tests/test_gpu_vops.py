@@ -145,6 +145,36 @@ def test_alltoallv_one_long_block_among_many_short_ones(n, hot):
         assert np.array_equal(recv[j].get(np.uint8), want[j]) and recv[j].guard_intact(), j
 
 
+@pytest.mark.parametrize("n,count", [(15, 78643201), (64, 4456449)])
+def test_alltoallv_of_more_tiles_than_one_launch_takes(n, count):
+    """More than 64 GiB (2^24 tiles) in two launches, tables in the kernel arguments and in memory.  All blocks are copies of
+    the same few MiB, and those of the first launch go to the same place; the blocks of the last rows, where the second launch
+    begins, each have a place of their own."""
+    own = n - (1 if n == 15 else 4)     # from this row on
+    g = torch.Generator(device="cuda:0")
+    g.manual_seed(n)
+    src = torch.randint(-2**31, 2**31 - 1, (count + 1,), device="cuda:0", generator=g, dtype=torch.int32)
+    rest = (n - own) * n
+    dst = torch.zeros((rest + 1) * count + 1, device="cuda:0", dtype=torch.int32)
+    sdispls = [1 if i >= own else 0 for i in range(n) for _ in range(n)]
+    rdispls = [(1 + (i - own) * n + j) * count if i >= own else 0 for j in range(n) for i in range(n)]
+    counts = [count] * (n * n)
+    torch.cuda.synchronize()
+    send, recv = [src.data_ptr()] * n, [dst.data_ptr()] * n
+    plan = hcclx.AlltoAllVPlan(send, recv, counts, sdispls, rdispls, T.FP32)
+    for go in (lambda: hcclx.alltoallv(send, recv, counts, sdispls, rdispls, T.FP32), plan.launch):
+        before = hcclx.kernels_launched()
+        go()
+        assert hcclx.kernels_launched() - before >= 2
+        torch.cuda.synchronize()
+        assert torch.equal(dst[:count], src[:-1])
+        for k in range(1, rest + 1):
+            assert torch.equal(dst[k * count:(k + 1) * count], src[1:]), k
+        assert int(dst[-1]) == 0
+        dst.zero_()
+    plan.close()
+
+
 def test_alltoallv_all_zero_and_single_rank():
     rng = np.random.default_rng(1)
     run_a2av([[0, 0], [0, 0]], T.FP32, rng)
