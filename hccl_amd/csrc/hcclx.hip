@@ -1120,7 +1120,7 @@ int launch_batch(const DeviceCtx *ctx, const Batch &b, const char *d_table, hipS
         return HCCL_SUCCESS;
     }
     if (b.blocks.tiles != 0) {
-        const hipError_t be = launch_copy_blocks(b.blocks.table(d_table), b.blocks.tiles, stream);
+        const hipError_t be = launch_copy_blocks(b.blocks.table(d_table), b.blocks.blocks.size(), b.blocks.tiles, stream);
         if (be != hipSuccess) return fail_hip(be, "block copy kernel launch");
         return HCCL_SUCCESS;
     }

@@ -217,7 +217,7 @@ int hcclx_alltoallv(const void *const *send, void *const *recv, const uint64_t *
         l.fill(h);
         rc = upload_table(d, h, l.bytes(), st);
         if (rc != HCCL_SUCCESS) return rc;
-        const hipError_t e = launch_copy_blocks(l.table(d), l.tiles, st);
+        const hipError_t e = launch_copy_blocks(l.table(d), l.blocks.size(), l.tiles, st);
         if (e != hipSuccess) return fail_hip(e, "alltoallv kernel launch");
         return HCCL_SUCCESS;
     }

@@ -164,7 +164,7 @@ struct AgvTablesInline {
 constexpr uint64_t kMostBlocksX = 0xffffffffull / kThreads;
 
 // tiles: of all blocks
-hipError_t launch_copy_blocks(const BlockTable &tab, uint64_t tiles, hipStream_t stream);
+hipError_t launch_copy_blocks(const BlockTable &tab, size_t blocks, uint64_t tiles, hipStream_t stream);
 hipError_t launch_equal_blocks(const EqualBlocks &tab, uint32_t n, hipStream_t stream);
 hipError_t launch_alltoallv_inline(const A2avInline &tab, uint64_t tiles, hipStream_t stream);
 // One batch after the other (grid z), each to one place after the other (grid y): per_batch slabs of slab_tiles tiles.

@@ -184,13 +184,13 @@ __device__ __forceinline__ CopyBlock block_of(const A2avInline &t, uint32_t b)
             static_cast<uint64_t>(t.counts[b]) * t.esz, t.begin[b]};
 }
 
-// Blocks of any lengths, one 4 KiB tile per workgroup and one vector per thread, stored through the L2: bound by HBM.
+// Blocks of any lengths, one 4 KiB tile per workgroup and one vector per thread, mostly stored through the L2: bound by HBM.
 // A wavefront that loads and stores one vector per lane copies faster than one that moves two (1 GiB: 6.66 against
 // 6.22 TB/s with these stores, 6.54 streamed); 8 x 4096 x 7168 bf16 with two vectors, streamed, and the block searched
 // in a prefix: 151.3 us, this way 145.4.  One workgroup per tile and none besides: an idle one costs 0.23 ns, and with blocks
 // cut into slabs of one size (two scalar loads without a search) 63 ranks that send 512 MiB, Zipf, launch fifteen for
 // every tile: 629 us, this way 205; 15 ranks 185 and 178, 32 ranks with blocks of nearly one size 114 and 101.
-template <typename Tab>
+template <typename Tab, uint32_t kPolicy>
 __global__ void __launch_bounds__(kThreads) k_copy_blocks(Tab tab, uint64_t first)
 {
     const uint64_t tile = first + blockIdx.x;
@@ -207,7 +207,7 @@ __global__ void __launch_bounds__(kThreads) k_copy_blocks(Tab tab, uint64_t firs
     }
     const CopyBlock b = block_of(tab, lo);
     char *dst = b.dst;
-    copy_tile<1, false, kStoreThrough>(b.src, reinterpret_cast<uint64_t>(dst), b.bytes, tile - b.begin, 1, [=](uint32_t) { return dst; });
+    copy_tile<1, false, kPolicy>(b.src, reinterpret_cast<uint64_t>(dst), b.bytes, tile - b.begin, 1, [=](uint32_t) { return dst; });
 }
 
 // Equal blocks: nothing to look up and no table to bring, the block is the workgroup's place in the grid (x: tile, y:
@@ -294,11 +294,11 @@ hipError_t launch_alltoallv(const VRankPtrs &ptrs, const uint64_t *send_counts, 
 
 namespace {
 // 64 GiB and more take several launches.
-template <typename Tab> hipError_t launch_tiles(const Tab &tab, uint64_t tiles, hipStream_t stream)
+template <uint32_t kPolicy, typename Tab> hipError_t launch_tiles(const Tab &tab, uint64_t tiles, hipStream_t stream)
 {
     for (uint64_t first = 0; first < tiles; first += kMostBlocksX) {
         const uint64_t take = tiles - first < kMostBlocksX ? tiles - first : kMostBlocksX;
-        HCCLX_LAUNCH((k_copy_blocks<Tab>), dim3(static_cast<uint32_t>(take)), dim3(kThreads), 0, stream, tab, first);
+        HCCLX_LAUNCH((k_copy_blocks<Tab, kPolicy>), dim3(static_cast<uint32_t>(take)), dim3(kThreads), 0, stream, tab, first);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
@@ -306,7 +306,18 @@ template <typename Tab> hipError_t launch_tiles(const Tab &tab, uint64_t tiles, 
 }
 }  // namespace
 
-hipError_t launch_copy_blocks(const BlockTable &tab, uint64_t tiles, hipStream_t stream) { return launch_tiles(tab, tiles, stream); }
+// Many blocks (more than 22 ranks) and more than the Infinity Cache takes up: streamed.  Plans, before the blocks were stored
+// through the L2 : through : streamed, us: 32 ranks with blocks of nearly one size 384 MiB in all 141 : 146 : 139, 256 MiB
+// 98.9 : 98.8 : 93; 48 x 192 MiB 72.9 : 74.7 : 72.2; 64 x 384 MiB 144 : 152 : 144, Zipf 256 MiB 94.1 : 103.5 : 96.1.  128 MiB and less
+// through the L2 (64 ranks 48.0 : 49.4 : 49.1, 32 ranks 48.0 : 46.2 : 47.8, 16 x 32 MiB 14.2 : 13.1 : 14.2), and few blocks at
+// every size (16 ranks, Zipf, 1 GiB 365 : 333 : 341; 8 ranks 351 : 328 : 333).
+hipError_t launch_copy_blocks(const BlockTable &tab, size_t blocks, uint64_t tiles, hipStream_t stream)
+{
+    constexpr size_t kStreamBlocks = 512;
+    constexpr uint64_t kStreamTiles = (160ull << 20) / 4096;
+    return blocks >= kStreamBlocks && tiles >= kStreamTiles ? launch_tiles<kStoreStream>(tab, tiles, stream)
+                                                            : launch_tiles<kStoreThrough>(tab, tiles, stream);
+}
 
 hipError_t launch_equal_blocks(const EqualBlocks &tab, uint32_t n, hipStream_t stream)
 {
@@ -316,7 +327,10 @@ hipError_t launch_equal_blocks(const EqualBlocks &tab, uint32_t n, hipStream_t s
     return hipGetLastError();
 }
 
-hipError_t launch_alltoallv_inline(const A2avInline &tab, uint64_t tiles, hipStream_t stream) { return launch_tiles(tab, tiles, stream); }
+hipError_t launch_alltoallv_inline(const A2avInline &tab, uint64_t tiles, hipStream_t stream)
+{
+    return launch_tiles<kStoreThrough>(tab, tiles, stream);
+}
 
 namespace {
 template <typename Tab> hipError_t launch_phased(const Tab &tab, const PhasedGrid &g, hipStream_t stream)

@@ -175,6 +175,15 @@ def test_alltoallv_of_more_tiles_than_one_launch_takes(n, count):
     plan.close()
 
 
+@pytest.mark.parametrize("n,rows", [(23, 168), (24, 144), (40, 56)])
+def test_alltoallv_of_many_blocks_and_160_mib_is_streamed(n, rows):
+    """529 and 576 blocks, 40960 tiles and more; blocks of half to one and a half KiB times rows, at any alignment."""
+    rng = np.random.default_rng(n)
+    m = rng.integers(rows * 1024, rows * 3072, size=(n, n))
+    assert m.sum() > 160 << 20 and (m > 0).sum() >= 512
+    run_a2av(m.tolist(), T.INT8, rng, send_pad=3)
+
+
 def test_alltoallv_all_zero_and_single_rank():
     rng = np.random.default_rng(1)
     run_a2av([[0, 0], [0, 0]], T.FP32, rng)
