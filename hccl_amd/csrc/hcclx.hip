@@ -335,14 +335,19 @@ void build_phased(std::vector<PhasedStream> &streams, uint64_t batch_bytes, uint
             joined.push_back(std::move(st));
         }
     }
-    // the smallest slab size with which the sources need at most max_slabs slabs (or the largest, and several launches)
+    // the smallest slab size with which the sources need at most max_slabs slabs (or the largest, and several launches); a
+    // smaller one, and more launches, where it would leave more than a quarter of the slabs' tiles empty: short sources beside
+    // a long one, or more of them than a launch has slabs (to eight places, slabs of the largest size : this way: 5000 x 64 KiB
+    // 15214 : 605 us, 64 MiB and 4090 x 4 KiB 12567 : 229)
     uint32_t tiles = kPhasedSlabTilesLeast;
     auto slabs_at = [&](uint32_t t) {
         uint64_t n = 0;
         for (const PhasedStream &st : joined) n += phased_slabs_of(st.bytes, t);
         return n;
     };
+    const uint64_t least = slabs_at(kPhasedSlabTilesLeast) * kPhasedSlabTilesLeast;
     while (tiles < kPhasedSlabTilesMost && slabs_at(tiles) > max_slabs) tiles *= 2;
+    while (tiles > kPhasedSlabTilesLeast && slabs_at(tiles) * tiles > least + least / 4) tiles /= 2;
     PhasedLaunch cur;
     auto flush = [&]() {
         if (cur.slabs.empty()) return;

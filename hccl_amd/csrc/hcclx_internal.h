@@ -110,8 +110,9 @@ struct PhasedStream {
     uint64_t bytes;
     std::vector<char *> dst;
 };
-// Turns streams into launches: streams that continue each other (source and every destination) are joined, and cut into
-// slabs as small as max_slabs of them allow; batches of up to batch_bytes are written to one place after the other.
+// Turns streams into launches of at most max_slabs slabs: streams that continue each other (source and every destination) are
+// joined, and cut into slabs, the smallest that need one launch, or smaller ones where those would mostly be empty; batches of
+// up to batch_bytes are written to one place after the other.
 void build_phased(std::vector<PhasedStream> &streams, uint64_t batch_bytes, uint32_t max_slabs, std::vector<PhasedLaunch> *out);
 // The non-empty blocks of an AlltoAllV with host tables (row-major n x n, elements of esz bytes), their tiles numbered
 // through; returns the number of tiles.

@@ -1,7 +1,11 @@
 // The tables that the copy kernels' launches are made of, checked tile by tile on the CPU (tests/test_host_copy_tables.py
 // builds it against the library and runs it; nothing here touches a GPU).
 //   blocks n  c00 c01 ...    an AlltoAllV's n x n counts (bytes): every tile of every block is found exactly once
-// Prints "tiles <blocks' own> groups <g> bytes <of the table>", or what is wrong.
+//       prints "tiles <blocks' own> groups <g> bytes <of the table>"
+//   copies max_slabs  bytes:places[xtimes] ...    sources that go to several places: every tile of every place is found exactly
+//       once; prints "tiles <of all places> workgroups <of all launches> launches <l> bytes <of the largest table>"
+// or what is wrong.
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -107,10 +111,74 @@ int blocks(int argc, char **argv)
     return 0;
 }
 
+int copies(int argc, char **argv)
+{
+    const uint32_t max_slabs = static_cast<uint32_t>(std::strtoul(argv[0], nullptr, 10));
+    std::vector<PhasedStream> streams;
+    for (int k = 1; k < argc; ++k) {
+        unsigned long long bytes = 0;
+        unsigned places = 0, times = 1;
+        if (std::sscanf(argv[k], "%llu:%ux%u", &bytes, &places, &times) < 2) return wrong("source", k);
+        for (unsigned t = 0; t < times; ++t) {
+            const uint64_t i = streams.size();
+            PhasedStream s{reinterpret_cast<const char *>((i + 1) << 33), bytes, {}};
+            for (unsigned d = 0; d < places; ++d) s.dst.push_back(reinterpret_cast<char *>((i + 1) << 33 | (1ull << 56) | (d + 1ull) << 50 | (3 * i + 7 * d) % 64));
+            streams.push_back(std::move(s));
+        }
+    }
+    const std::vector<PhasedStream> asked = streams;
+    std::vector<PhasedLaunch> launches;
+    build_phased(streams, 16ull << 20, max_slabs, &launches);
+    uint64_t own = 0, workgroups = 0, most_bytes = 0;
+    std::vector<std::vector<std::vector<bool>>> moved(asked.size());
+    for (size_t s = 0; s < asked.size(); ++s) {
+        for (char *dst : asked[s].dst) {
+            const uint64_t tiles = v_tiles_of(asked[s].bytes, reinterpret_cast<uint64_t>(dst), kPhasedUnroll);
+            own += tiles;
+            moved[s].push_back(std::vector<bool>(tiles));
+        }
+    }
+    for (const PhasedLaunch &l : launches) {
+        if (l.slabs.size() > max_slabs) return wrong("slabs of a launch", l.slabs.size());
+        if (l.bytes() > 1u << 20) return wrong("table of a launch", l.bytes());
+        most_bytes = std::max<uint64_t>(most_bytes, l.bytes());
+        const uint64_t x = static_cast<uint64_t>(l.grid.per_batch) * l.grid.slab_tiles;
+        if (x > kMostBlocksX || l.grid.nd > 65535 || l.grid.batches > 65535) return wrong("grid", x);
+        workgroups += x * l.grid.nd * l.grid.batches;
+        std::vector<char> table(l.bytes());
+        l.fill(table.data());
+        const PhasedTable t = l.table(table.data());
+        for (uint64_t k = 0; k < static_cast<uint64_t>(l.grid.per_batch) * l.grid.batches && k < t.nslabs; ++k) {
+            const CopySlab slab = t.slabs[k];
+            const PhasedSource &source = t.sources[slab.source];
+            const size_t s = (reinterpret_cast<uint64_t>(source.src) >> 33) - 1;
+            if (s >= asked.size() || source.bytes != asked[s].bytes || source.place != asked[s].dst.size()) return wrong("source of slab", k);
+            for (uint32_t d = 0; d < source.place; ++d) {
+                if (t.dsts[static_cast<uint64_t>(slab.source) * t.nd + d] != asked[s].dst[d]) return wrong("place of slab", k);
+                for (uint64_t tl = static_cast<uint64_t>(slab.at) * l.grid.slab_tiles; tl < (slab.at + 1ull) * l.grid.slab_tiles && tl < moved[s][d].size(); ++tl) {
+                    if (moved[s][d][tl]) return wrong("tile moved twice, source", s);
+                    moved[s][d][tl] = true;
+                }
+            }
+        }
+    }
+    for (size_t s = 0; s < asked.size(); ++s) {
+        for (const auto &tiles : moved[s]) {
+            for (bool m : tiles) {
+                if (!m) return wrong("tile not moved, source", s);
+            }
+        }
+    }
+    std::printf("tiles %llu workgroups %llu launches %zu bytes %llu\n", static_cast<unsigned long long>(own),
+                static_cast<unsigned long long>(workgroups), launches.size(), static_cast<unsigned long long>(most_bytes));
+    return 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
 {
+    if (argc > 3 && std::string(argv[1]) == "copies") return copies(argc - 2, argv + 2);
     if (argc > 2 && std::string(argv[1]) == "blocks") return blocks(argc - 2, argv + 2);
     return wrong("arguments", 0);
 }

@@ -52,3 +52,25 @@ def test_every_tile_of_an_alltoallv_is_found_once(check, n, kind):
     assert tiles <= payload // 4096 + 2 * live
     # what is uploaded in front of the kernel
     assert groups <= 4096 and size <= 32 * live + 256 + 4 * (min(4096, 4 * live) + 1)
+
+
+@pytest.mark.parametrize("max_slabs,sources,most_launches", [
+    (4096, ["65536:8x5000"], 4),                         # more sources than a launch has slabs
+    (4096, ["67108864:8", "4096:8x4090"], 4),            # one long source and nearly as many short ones as slabs
+    (4096, ["1073741824:2", "100:2x4000"], 8),
+    (4096, ["9000000:7x30", "70001:3x900", "1:2x50"], 2),
+    (4096, ["8388608:8x7"], 1),
+    (480, ["67108864:8", "1:8x63"], 2),                  # an AllGatherV in the kernel arguments
+    (480, ["8388608:16x16"], 1),
+    (480, ["33800:64x64"], 1),
+    (480, ["1073745923:2", "1073741901:2"], 2),
+])
+def test_copies_to_several_places_launch_few_idle_workgroups(check, max_slabs, sources, most_launches):
+    """A slab is at least eight tiles, and of the slabs' workgroups at most a quarter more than that are without a tile.  Sources
+    of fewer places than the launch's most leave more."""
+    tiles, workgroups, launches, _ = check("copies", max_slabs, *sources)
+    listed = [tuple(int(x) for x in (s if "x" in s else s + "x1").replace(":", "x").split("x")) for s in sources]
+    most = max(places for _, places, _ in listed)
+    least = sum(times * most * 8 * ((size // 4096 + 1) // 8 + 1) for size, _, times in listed)
+    assert workgroups <= 1.25 * least + most * 1024 * launches
+    assert launches <= most_launches
