@@ -793,7 +793,7 @@ uint32_t waves_for(const DeviceCtx *ctx, const hcclx_seg_t *segs, uint32_t nseg,
         least_src = segs[i].nsrc < least_src ? segs[i].nsrc : least_src;
         most_dst = segs[i].ndst > most_dst ? segs[i].ndst : most_dst;
         written += segs[i].count * esz * segs[i].ndst;
-        tiles += segs[i].count * esz / 1024 + 2;
+        tiles += segs[i].count * esz / 1024 + 2 + kWavePieces;   // 1 KiB pieces; a segment's last tile may hold one
     }
     const uint32_t widest = most_src > most_dst ? most_src : most_dst;
     if (most_src < 2 || most_dst < 2 || widest > ctx->waves_max_fan || written < ctx->waves_from || esz == 0) return 0;
@@ -825,7 +825,7 @@ uint32_t waves_for(const DeviceCtx *ctx, const hcclx_seg_t *segs, uint32_t nseg,
             p = per_place < (12ull << 20) ? 8u : 4u;
         }
     }
-    if (tiles / p > 0x7fffffffull) return 0;   // one workgroup per tile: the grid has to hold them
+    if (!waves_fit(tiles, p, widest)) return 0;
     *pieces = p;
     return widest;
 }

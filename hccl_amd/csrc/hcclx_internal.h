@@ -93,6 +93,13 @@ int ring_reserve(DeviceCtx *ctx, size_t bytes, hipStream_t stream, char **h, cha
 
 uint32_t grid_for(const DeviceCtx *ctx, uint64_t total_tiles);
 
+// Whether one launch of the wavefront kernel takes this many 1 KiB pieces per source, `per_tile` of them and `waves` wavefronts
+// of 64 to a workgroup: HIP allows fewer than 2^32 work-items along x.  (The register kernels' workgroups move more each.)
+inline bool waves_fit(uint64_t pieces, uint32_t per_tile, uint32_t waves)
+{
+    return pieces / per_tile + 1 <= 0xffffffffull / (64ull * waves);
+}
+
 
 // One launch of the copy kernel that writes one output at a time (kernels/vops.h).
 struct PhasedLaunch {

@@ -4,6 +4,7 @@
 //       prints "tiles <blocks' own> groups <g> bytes <of the table>"
 //   copies max_slabs  bytes:places[xtimes] ...    sources that go to several places: every tile of every place is found exactly
 //       once; prints "tiles <of all places> workgroups <of all launches> launches <l> bytes <of the largest table>"
+//   waves pieces per_tile waves    whether one launch of the wavefront fold takes them: prints 1 or 0
 // or what is wrong.
 #include <algorithm>
 #include <cstdio>
@@ -179,6 +180,10 @@ int copies(int argc, char **argv)
 int main(int argc, char **argv)
 {
     if (argc > 3 && std::string(argv[1]) == "copies") return copies(argc - 2, argv + 2);
+    if (argc == 5 && std::string(argv[1]) == "waves") {
+        std::printf("%d\n", waves_fit(std::strtoull(argv[2], nullptr, 10), std::atoi(argv[3]), std::atoi(argv[4])) ? 1 : 0);
+        return 0;
+    }
     if (argc > 2 && std::string(argv[1]) == "blocks") return blocks(argc - 2, argv + 2);
     return wrong("arguments", 0);
 }

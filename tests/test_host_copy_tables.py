@@ -74,3 +74,11 @@ def test_copies_to_several_places_launch_few_idle_workgroups(check, max_slabs, s
     least = sum(times * most * 8 * ((size // 4096 + 1) // 8 + 1) for size, _, times in listed)
     assert workgroups <= 1.25 * least + most * 1024 * launches
     assert launches <= most_launches
+
+
+@pytest.mark.parametrize("gib,per_tile,ranks,fits", [(63, 4, 4, 1), (64, 4, 4, 0), (127, 4, 2, 1), (128, 4, 2, 0), (86, 4, 3, 0), (31, 2, 4, 1),
+                                                     (32, 2, 4, 0), (15, 2, 8, 1), (16, 2, 8, 0), (22, 8, 16, 1), (33, 8, 16, 0)])
+def test_a_wavefront_fold_stays_below_2_to_the_32_work_items(check, gib, per_tile, ranks, fits):
+    """In place, 4 x 64 GiB or 2 x 128 GiB fit the memory, and the register kernel takes them."""
+    assert fits == (gib * 2**20 // per_tile * 64 * ranks < 2**32)
+    assert check("waves", gib * 2**20, per_tile, ranks) == [fits]
