@@ -751,7 +751,10 @@ int hcclx_moe_route(const int32_t *const *dest, uint32_t n, uint32_t entries, ui
     const uint32_t chunks = chunks_of(entries);
     uint32_t *base = static_cast<uint32_t *>(workspace);
     uint32_t *row_start = base + static_cast<uint64_t>(n) * n * chunks;
-    if (entries <= kOneLaunchEntries) {
+    // perm may lie on top of the destinations: then every entry is read a launch before, and by the thread that writes it
+    bool in_place = false;
+    for (uint32_t i = 0; i < n; ++i) in_place = in_place || d.p[i] == p.p[i];
+    if (entries <= kOneLaunchEntries && !in_place) {
         HCCLX_LAUNCH(k_moe_route_one, dim3(chunks, n), dim3(kMoeChunk), 0, st, d, as_mutable(p), n, entries, row_elems, send_counts,
                      sdispls, recv_counts, rdispls);
         const hipError_t oe = hipGetLastError();

@@ -201,7 +201,8 @@ uint64_t hcclx_moe_workspace_bytes(uint32_t n, uint32_t entries);
  *   send_counts[i*n + j], sdispls[i*n + j]   what rank i sends to rank j and where it starts in i's packed buffer
  *   rdispls[j*n + i]                         where that block lands in rank j's receive buffer (blocks in rank order)
  *   recv_counts[j*n + i] = send_counts[i*n + j]   (the send counts of the way back)
- * and perm[i] (device uint32[entries]): the row of rank i's packed buffer that entry e goes to.
+ * and perm[i] (device uint32[entries]): the row of rank i's packed buffer that entry e goes to.  perm[i] may be dest[i]
+ * itself; it overlaps no destinations otherwise.
  * The AlltoAllV of the way back uses (recv_counts, rdispls, sdispls) in the places of
  * (send_counts, sdispls, rdispls). */
 int hcclx_moe_route(const int32_t *const *dest, uint32_t n, uint32_t entries, uint64_t row_elems, uint64_t *send_counts,

@@ -331,3 +331,24 @@ def test_route_in_one_launch(n, entries, skew):
         assert np.array_equal(got.cpu().numpy().reshape(n, n), np.array(want, dtype=np.int64))
     for i in range(n):
         assert np.array_equal(perm[i].cpu().numpy().view(np.uint32), perms[i]), i
+
+
+@pytest.mark.parametrize("n,entries", [(1, 1), (8, 512), (64, 1024), (5, 300), (3, 1025), (3, 20000)])
+def test_route_with_perm_in_the_place_of_dest(n, entries):
+    """A caller that only packs and combines needs no destinations afterwards: the histogram runs a launch before the
+    permutation then, at every size."""
+    rng = np.random.default_rng(n + entries)
+    dests = [rng.integers(-1, n + 1, size=entries) for _ in range(n)]
+    both = [dev_i32(x) for x in dests]
+    tabs = [torch.full((n * n,), -1, dtype=torch.int64, device=DEV) for _ in range(4)]
+    ws = torch.empty(hcclx.moe_workspace_bytes(n, entries), dtype=torch.uint8, device=DEV)
+    torch.cuda.synchronize()
+    before = hcclx.kernels_launched()
+    hcclx.moe_route([b.data_ptr() for b in both], entries, 8, *[t.data_ptr() for t in tabs], [b.data_ptr() for b in both], ws.data_ptr())
+    assert hcclx.kernels_launched() - before >= 2
+    torch.cuda.synchronize()
+    sc, sd, rc, rd, perms = T.moe_route(dests, n, 8)
+    for got, want in zip(tabs, (sc, sd, rc, rd)):
+        assert np.array_equal(got.cpu().numpy().reshape(n, n), np.array(want, dtype=np.int64))
+    for i in range(n):
+        assert np.array_equal(both[i].cpu().numpy().view(np.uint32), perms[i]), i
