@@ -117,17 +117,19 @@ def load():
 
 
 _calls = None
+# named after the interpreter's ABI: a module built for another one is not loaded
+CALLS_PATH = os.path.join(_HERE, "lib", "_hccl_calls" + importlib.machinery.EXTENSION_SUFFIXES[0])
 
 
 def native_call(name):
     """The entry point as a callable that converts its arguments natively (csrc/python_calls.cc).  It returns
-    NotImplemented for arguments that ctypes has to convert; argtypes must have been set."""
+    NotImplemented for arguments that ctypes has to convert, for all of them where the module was not built (no Python
+    headers, another interpreter); argtypes must have been set."""
     global _calls
     if _calls is None:
-        path = os.path.join(_HERE, "lib", "_hccl_calls.so")
-        if not os.path.exists(path):
-            raise RuntimeError(f"{path} is missing: build it with `make -C hccl_amd/csrc`")
-        loader = importlib.machinery.ExtensionFileLoader("_hccl_calls", path)
+        if not os.path.exists(CALLS_PATH):
+            return lambda *args: NotImplemented
+        loader = importlib.machinery.ExtensionFileLoader("_hccl_calls", CALLS_PATH)
         _calls = importlib.util.module_from_spec(importlib.util.spec_from_loader("_hccl_calls", loader))
         loader.exec_module(_calls)
     fn = getattr(load(), name)

@@ -2,6 +2,10 @@
 not take is left to ctypes.  Dry worlds: nothing here touches a GPU."""
 import ctypes
 import enum
+import os
+import subprocess
+import sys
+import sysconfig
 import threading
 
 import pytest
@@ -80,3 +84,46 @@ def test_pointer_lists():
     assert call([1] * 65, 65, 8, 8, 1, 1, 1, 1, [1] * 65, 1, 0) is NotImplemented
     assert call(1, 1, 8, 8, 1, 1, 1, 1, [1], 1, 0) is NotImplemented
     assert call([1.5], 1, 8, 8, 1, 1, 1, 1, [1], 1, 0) is NotImplemented
+
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def test_without_the_module_the_calls_go_through_ctypes():
+    """The library alone is enough: the module may not have been built (no Python headers) or be another interpreter's."""
+    code = """
+from hccl_amd import _lib, api, types as T
+_lib.CALLS_PATH += ".missing"
+w = api.World(2, dry=True)
+assert api._all_reduce(1, 2, 10, T.FP32, T.SUM, w.comms[0], 1) is NotImplemented
+for r in range(2):
+    assert w.all_reduce(r, (r + 1) << 20, (r + 10) << 20, 100, T.FP32, T.SUM, 1) == 0
+    assert w.all_to_all(r, (r + 1) << 20, 5, (r + 10) << 20, T.FP32, 1) == 0
+    assert w.all_to_all_v(r, (r + 1) << 20, [3, 4], [0, 3], (r + 10) << 20, [3 + r, 3 + r], [0, 3 + r], T.FP32, 1) == 0
+assert w.last_info().algName
+w.close()
+"""
+    run = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=120)
+    assert run.returncode == 0, run.stderr[-2000:]
+
+
+def test_the_module_is_named_after_the_interpreter_it_was_built_for():
+    name = "_hccl_calls" + sysconfig.get_config_var("EXT_SUFFIX")
+    assert os.path.basename(_lib.CALLS_PATH) == name and os.path.exists(_lib.CALLS_PATH)
+
+
+@pytest.mark.parametrize("headers", [True, False])
+def test_the_build_needs_no_python_headers(tmp_path, headers):
+    """An interpreter that names a header directory: the module is built for its ABI where Python.h is in there."""
+    if headers:
+        (tmp_path / "Python.h").write_text("")
+    python = tmp_path / "python"
+    python.write_text(f"""#!/bin/sh
+case "$2" in *EXT_SUFFIX*) echo .cpython-399-test.so;; *) echo {tmp_path};; esac
+""")
+    python.chmod(0o755)
+    csrc = os.path.join(ROOT, "hccl_amd", "csrc")
+    run = subprocess.run(["make", "-n", "-C", csrc, f"PYTHON={python}", f"LIBDIR={tmp_path}/lib", "all"], capture_output=True, text=True)
+    assert run.returncode == 0, run.stderr[-2000:]
+    assert "libhccl_amd.so" in run.stdout
+    assert ("_hccl_calls.cpython-399-test.so" in run.stdout) == headers and ("python_calls.cc" in run.stdout) == headers
