@@ -746,7 +746,8 @@ int build_batches(const hcclx_seg_t *segs, uint32_t nseg, int dtype, int op, int
     return HCCL_SUCCESS;
 }
 
-constexpr uint64_t kTeamFrom = 48ull << 20;
+// Bytes written from which chains among two to four ranks share the fold (waves_for).
+uint64_t team_from(uint64_t esz) { return (esz <= 2 ? 136ull : 160ull) << 20; }
 
 // The n orders of a self-first fold take the kernel in which every wavefront issues one store (fold.h) when all
 // segments have the same number of ranks, at most waves_max_fan, and the launch writes waves_from bytes or more.
@@ -769,10 +770,12 @@ constexpr uint64_t kTeamFrom = 48ull << 20;
 // place among two to four ranks, 512 KiB among more (kernel times, bf16, register : this one: 2 x 2 MiB 5.06 : 4.24 us,
 // 4 x 256 KiB 6.3 : 3.5, 4 x 2 MiB 6.34 : 4.84, 8 x 512 KiB 5.44 : 4.40, 12 x 512 KiB 8.46 : 7.16, 16 x 512 KiB 6.68 : 5.76;
 // fp32 beyond: 4 x 4 MiB 5.42 : 5.92, 8 x 1 MiB 4.60 : 5.00, 12 x 1 MiB 7.24 : 7.90).  Among two to four ranks also, shared
-// and with four pieces, from kTeamFrom bytes written on (buffers that are not in the Infinity Cache, bf16: 2 x 25 MiB
-// 22.5 : 21.3, 2 x 400 277 : 267, 3 x 48 54.9 : 51.6, 3 x 150 162 : 151, 4 x 12 22.3 : 20.2, 4 x 128 181 : 166, 4 x 256
-// 375 : 337; below it 2 x 16 12.5 : 15.3, 3 x 12 14.1 : 15.5).  Otherwise only when asked for (waves_chains; 8 x 25 MiB
-// 78.7 : 74.7, fold + fan-out 70.7, and among 12 and more ranks no gain).
+// and with four pieces, from team_from bytes written on (AllReduce in two shots, 700 MiB of buffers that change, whole
+// vectors: fp32 2 x 100 MiB 71.8 : 70.2, 2 x 400 364 : 271, 3 x 56 63.7 : 62.6, 3 x 150 166 : 151, 4 x 44 66.4 : 65.8, 4 x 256
+// 366 : 345; bf16 2 x 72 54.6 : 52.5, 3 x 48 56.5 : 54.6, 4 x 36 57.8 : 56.2, 4 x 64 99.1 : 94.4; below it fp32 2 x 32 25.4 : 26.6,
+// 3 x 20 25.0 : 26.5, 4 x 12 18.9 : 21.8, 4 x 16 24.5 : 28.1, 4 x 32 48.1 : 51.7; bf16 4 x 16 25.4 : 28.9, 4 x 32 50.9 : 52.4, between
+// them within 3 % either way).  Otherwise only when asked for (waves_chains; 8 x 25 MiB 78.7 : 74.7, fold + fan-out 70.7, and
+// among 12 and more ranks no gain).
 // Returns the number of wavefronts per workgroup (the widest segment's sources or destinations), 0 = the register
 // kernels.
 // *team: a chain whose fold the wavefronts share.
@@ -801,10 +804,10 @@ uint32_t waves_for(const DeviceCtx *ctx, const hcclx_seg_t *segs, uint32_t nseg,
     const uint64_t per_place = written / most_dst;
     if (mode == HCCLX_FOLD_SELF_FIRST) {
         if (!same && widest > 8) return 0;
-    } else if (!ctx->waves_chains && per_place > (widest <= 4 ? 2048ull << 10 : 512ull << 10) && !(widest <= 4 && written >= kTeamFrom)) {
+    } else if (!ctx->waves_chains && per_place > (widest <= 4 ? 2048ull << 10 : 512ull << 10) && !(widest <= 4 && written >= team_from(esz))) {
         return 0;   // chains to several places: by default the small ones and, among few ranks, the large ones (see above)
     }
-    *team = mode == HCCLX_FOLD_CHAIN && (widest >= 4 || written >= kTeamFrom);
+    *team = mode == HCCLX_FOLD_CHAIN && (widest >= 4 || written >= team_from(esz));
     uint32_t p = ctx->waves_pieces;
     if (p == 0) {   // the shipped policy; a forced piece count takes every launch that passed the tests above
         if (mode == HCCLX_FOLD_SELF_FIRST) {
@@ -815,7 +818,7 @@ uint32_t waves_for(const DeviceCtx *ctx, const hcclx_seg_t *segs, uint32_t nseg,
             }
             if (esz == 2 && widest >= 9 && per_place >= (2ull << 20)) return 0;
         }
-        if (*team && written >= kTeamFrom) {
+        if (*team && written >= team_from(esz)) {
             p = 4;
         } else if (per_place < (2ull << 20) || widest <= 4) {
             p = 2;

@@ -243,3 +243,21 @@ def test_large_chains_among_few_ranks_share_the_fold(ranks, dtype, op):
     for r in range(ranks):
         assert_same_bits(got[r], want, dtype, f"place {r}")
         assert np.array_equal(got[r].view(np.uint8), ref[r].view(np.uint8)), f"place {r}: differs from the register kernel"
+
+
+@pytest.mark.parametrize("ranks,dtype,op,mib", [(2, T.BFP16, T.SUM, 136), (3, T.FP32, T.MAX, 160), (4, T.INT8, T.SUM, 136), (4, T.FP64, T.PROD, 160),
+                                                (3, T.INT32, T.MIN, 159)])
+def test_chains_among_few_ranks_around_the_size_from_which_they_share_the_fold(ranks, dtype, op, mib):
+    """So many bytes written and a little more; the last is the register kernel's."""
+    hcclx.init()
+    rng = np.random.default_rng(ranks + dtype)
+    esz = T.DTYPE_SIZE[dtype]
+    n = -(-(mib << 20) // ranks // esz) + 4099
+    xs = [payload(rng, dtype, n, "prod" if op == T.PROD else "normal") for _ in range(ranks)]
+    bufs = [DevBuf(x, offset=(k % 3) * esz) for k, x in enumerate(xs)]
+    outs = [DevBuf(nbytes=xs[0].nbytes, offset=(1 + k % 5) * esz) for k in range(ranks)]
+    got, ref = fold_both([(n, [b.ptr for b in bufs], [o.ptr for o in outs])], dtype, op, hcclx.FOLD_CHAIN, outs)
+    want = chain_oracle(xs, dtype, op, [0] * ranks)
+    for r in range(ranks):
+        assert_same_bits(got[r], want, dtype, f"place {r}")
+        assert np.array_equal(got[r].view(np.uint8), ref[r].view(np.uint8)), f"place {r}: differs from the register kernel"
