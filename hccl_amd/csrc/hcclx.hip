@@ -755,12 +755,24 @@ uint64_t team_from(uint64_t esz) { return (esz <= 2 ? 136ull : 160ull) << 20; }
 // 8 x 64 MiB 210 : 175, 12 x 64 MiB 281 : 270, 12 x 256 MiB 1183 : 1056, 16 x 256 MiB 1582 : 1445, and at
 // 256 KiB per rank and below 4.6-5.6 : 3.2-3.5 among 8 to 12 ranks (at 4 KiB per rank: 4 ranks 3.9 : 3.1, 16 ranks
 // 5.3 : 3.9; the register kernel's threads each walk all the sources, here the wavefronts share them).  Where the register
-// kernel measured better it stays: two ranks below 32 MiB per rank (no difference); seven and eight ranks from 3 to 4.5 MiB
-// per rank of fp32 (8 x 3.5 MiB 12.4 : 12.8, 8 x 5 17.9 : 16.5, 8 x 11 37.7 : 30.6), to 6 MiB of fp16 (8 x 5 19.8 : 20.8, 8 x 8
-// 29.9 : 29.0), to 12 MiB of fp64, and never of bf16 (8 x 3.5 18.2 : 15.9, 8 x 8 33.0 : 29.6); and the 16-bit types among nine
-// and more ranks, where every wavefront widens every source for itself (bf16 SUM 12 x 1 MiB 16.6 : 10.6, 12 x 2 17.9 : 19.6,
-// 12 x 8 44 : 57, 16 x 2 26 : 30, 16 x 5 44 : 73, 16 x 16 110 : 204, 9 x 3.5 19.8 : 21.4, 9 x 8 34 : 42; 9 x 1.9 14.3 : 12.7 and
-// eight ranks x 16 56.8 : 55.7), from 2 MiB per rank.  Pieces per workgroup: two for small launches and up to four ranks; five to eight
+// kernel measured better it stays: two ranks below 32 MiB per rank (no difference); seven and eight ranks in the middle, where
+// 256 CUs take its 8 KiB tiles in few whole rounds, and how far depends on whether there are elements outside the vectors,
+// which it folds one thread each (AllReduce in one shot, buffers that change, register : wavefronts).  Whole vectors:
+//   8 ranks fp32  3 MiB 12.2 : 11.0, 3.5 12.6 : 13.7, 4 13.6 : 15.9, 6 17.8 : 22.0, 8 24.1 : 30.3, 10 28.9 : 34.6, 11 40.8 : 38.3
+//           fp16  3 MiB 12.8 : 13.6, 4 14.2 : 17.1, 6 18.5 : 24.6, 8 29.9 : 31.6, 10 35.0 : 37.0, 11 42.2 : 39.5
+//           fp64  3 MiB 11.6 : 11.1, 4 13.9 : 16.1, 8 24.9 : 29.8, 11 37.4 : 37.4, 12 39.0 : 40.0
+//           bf16  4 MiB 17.6 : 17.5, 5 21.6 : 22.0, 6 22.1 : 24.2, 7 29.8 : 27.9, 8 33.4 : 32.0, 10 37.1 : 37.1
+//   7 ranks fp32  3 MiB 10.9 : 10.1, 4 12.4 : 13.5, 6 16.2 : 19.3, 8 21.4 : 25.3, 10 25.3 : 30.3, 11 35.3 : 34.0
+//           fp16  4 MiB 12.7 : 14.5, 6 16.4 : 22.0, 10 30.8 : 33.6, 11 37.2 : 36.7;  fp64  4 MiB 12.2 : 13.5, 8 22.0 : 25.3, 11 33.4 : 34.8
+//           bf16  4 MiB 15.5 : 14.5, 5 18.9 : 20.2, 6 19.2 : 21.5, 8 29.4 : 27.5
+// Elements outside them:
+//   8 ranks fp32  3.5 MiB 12.6 : 14.1, 4 16.4 : 16.9, 6 21.2 : 22.4, 7 28.0 : 26.6, 8 29.1 : 29.5, 11 40.4 : 37.5
+//           fp64  3.5 MiB 13.4 : 13.5, 6 25.1 : 23.1, 9 31.0 : 32.2, 11 37.5 : 37.2;  fp16  4 MiB 19.8 : 16.7, 6 26.5 : 24.4
+//           bf16  4 MiB 24.2 : 16.9, 8 34.0 : 30.4
+// And the 16-bit types among nine and more ranks, where every wavefront widens every source for itself, from 2 MiB per rank
+// (bf16 SUM, whole vectors: 9 x 2 MiB 10.8 : 16.4, 9 x 8 35.0 : 40.2, 12 x 2 14.3 : 20.0, 12 x 8 48.1 : 53.9, 16 x 2 19.3 : 27.0, 16 x 8
+// 64.9 : 98.9; 12 x 1 16.6 : 10.6; with elements outside them 9 x 2.5 15.9 : 20.3, 9 x 3 21.4 : 20.7, 12 x 2 21.2 : 19.8, 12 x 2.5
+// 22.1 : 27.7, 12 x 3 28.6 : 28.0, 12 x 5 33.0 : 41.3, 16 x 2 30.2 : 33.3).  Pieces per workgroup: two for small launches and up to four ranks; five to eight
 // ranks four below 32 MiB per rank (8 x 16 MiB: 47.9 / 43.0 us with 2 / 4) and two from there on (8 x 64 MiB:
 // 168.8 / 182.6); nine and more eight below 12 MiB per rank (12 x 8 MiB: 35.6 / 36.4 / 32.3 us with 2 / 4 / 8) and
 // four from there on (12 x 64 MiB: 268.7 / 260.6 / 281.7).  Launches
@@ -789,6 +801,7 @@ uint32_t waves_for(const DeviceCtx *ctx, const hcclx_seg_t *segs, uint32_t nseg,
     uint32_t least_src = ~0u;
     uint64_t written = 0;
     uint64_t tiles = 0;
+    bool edges = false;   // elements in front of or behind the vectors of 16 bytes
     for (uint32_t i = 0; i < nseg; ++i) {
         if (segs[i].nsrc == 0 || segs[i].nsrc > HCCLX_MAX_FAN || segs[i].ndst == 0 || segs[i].ndst > HCCLX_MAX_FAN) return 0;
         if (segs[i].count == 0) continue;
@@ -796,6 +809,7 @@ uint32_t waves_for(const DeviceCtx *ctx, const hcclx_seg_t *segs, uint32_t nseg,
         least_src = segs[i].nsrc < least_src ? segs[i].nsrc : least_src;
         most_dst = segs[i].ndst > most_dst ? segs[i].ndst : most_dst;
         written += segs[i].count * esz * segs[i].ndst;
+        edges = edges || segs[i].count * esz % 16 != 0 || reinterpret_cast<uint64_t>(segs[i].dst[0]) % 16 != 0;
         tiles += segs[i].count * esz / 1024 + 2 + kWavePieces;   // 1 KiB pieces; a segment's last tile may hold one
     }
     const uint32_t widest = most_src > most_dst ? most_src : most_dst;
@@ -812,9 +826,11 @@ uint32_t waves_for(const DeviceCtx *ctx, const hcclx_seg_t *segs, uint32_t nseg,
     if (p == 0) {   // the shipped policy; a forced piece count takes every launch that passed the tests above
         if (mode == HCCLX_FOLD_SELF_FIRST) {
             if (widest == 2 && per_place < (32ull << 20)) return 0;
+            const bool bf16 = dtype == HCCL_DATA_TYPE_BFP16;
             if (widest == 7 || widest == 8) {
-                const uint64_t upto = esz == 8 ? 12ull << 20 : esz == 4 ? 9ull << 19 : dtype == HCCL_DATA_TYPE_FP16 ? 6ull << 20 : 0;
-                if (per_place >= (3ull << 20) && per_place < upto) return 0;
+                const uint64_t from = bf16 ? 19ull << 18 : 3ull << 20;
+                const uint64_t upto = esz == 8 ? 12ull << 20 : edges ? (esz == 4 ? 13ull << 19 : 0) : bf16 ? 13ull << 19 : 21ull << 19;
+                if (per_place >= from && per_place < upto) return 0;
             }
             if (esz == 2 && widest >= 9 && per_place >= (2ull << 20)) return 0;
         }

@@ -261,3 +261,36 @@ def test_chains_among_few_ranks_around_the_size_from_which_they_share_the_fold(r
     for r in range(ranks):
         assert_same_bits(got[r], want, dtype, f"place {r}")
         assert np.array_equal(got[r].view(np.uint8), ref[r].view(np.uint8)), f"place {r}: differs from the register kernel"
+
+
+@pytest.mark.parametrize("ranks,dtype,mib,extra", [(8, T.FP32, 3, 0), (7, T.FP32, 6.5, 1), (8, T.FP32, 6.5, -1), (8, T.FP32, 10.5, 0), (7, T.FP16, 10.5, -8),
+                                                   (8, T.FP16, 4, 3), (8, T.BFP16, 4.75, 0), (7, T.BFP16, 6.5, 0), (8, T.FP64, 12, -2), (12, T.BFP16, 2, 0),
+                                                   (12, T.BFP16, 2, -5), (9, T.BFP16, 2, 3), (16, T.BFP16, 2, 1)])
+def test_self_first_orders_where_the_choice_of_the_kernel_changes(ranks, dtype, mib, extra):
+    """The sizes per rank at which the register kernel takes over or hands back, with and without elements outside the
+    vectors: the chosen kernel against both forced ones, the same bits, some of them against the oracle."""
+    hcclx.init()
+    esz = T.DTYPE_SIZE[dtype]
+    n = int(mib * 2**20) // esz + extra
+    td = {T.FP32: torch.float32, T.FP16: torch.float16, T.BFP16: torch.bfloat16, T.FP64: torch.float64}[dtype]
+    g = torch.Generator(device="cuda:0")
+    g.manual_seed(ranks * 31 + n)
+    xs = [torch.randn(n, device="cuda:0", generator=g, dtype=td) for _ in range(ranks)]
+    results = []
+    for tuned in (("waves_from", 1), ("waves_from", 0), ("waves_pieces", 4)):
+        hcclx.tune(*tuned)
+        outs = [torch.zeros_like(x) for x in xs]
+        torch.cuda.synchronize()
+        hcclx.fold([(n, [x.data_ptr() for x in xs], [o.data_ptr() for o in outs])], dtype, T.SUM, hcclx.FOLD_SELF_FIRST)
+        torch.cuda.synchronize()
+        for name, value in DEFAULTS.items():
+            hcclx.tune(name, value)
+        results.append(outs)
+    bits = {2: torch.int16, 4: torch.int32, 8: torch.int64}[esz]
+    cols = torch.cat([torch.arange(100), torch.randint(0, n, (500,)), torch.arange(n - 100, n)]).to("cuda:0")
+    sample = [x[cols].view(bits).cpu().numpy().view(T.NP_STORAGE[dtype]) for x in xs]
+    for r in range(ranks):
+        for other in results[1:]:
+            assert torch.equal(results[0][r].view(bits), other[r].view(bits)), r
+        want = fold_oracle(sample, dtype, T.SUM, [r] + [k for k in range(ranks) if k != r], wide=fused_is_wide(dtype, T.SUM))
+        assert_same_bits(results[0][r][cols].view(bits).cpu().numpy().view(T.NP_STORAGE[dtype]), want, dtype, f"rank {r}")
