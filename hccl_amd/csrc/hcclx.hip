@@ -1209,7 +1209,7 @@ int hcclx_tune(const char *name, uint64_t value)
     } else if (key == "fanout_from") {
         ctx->fanout_from = value;
     } else if (key == "moe_scatter_rows") {
-        if (value != 1 && value != 2) return fail(HCCL_E_PARA, "moe_scatter_rows is 1 or 2");
+        if (value > 2) return fail(HCCL_E_PARA, "moe_scatter_rows is 1, 2 or 0");
         ctx->moe_scatter_rows = static_cast<uint32_t>(value);
     } else if (key == "store_through_upto") {
         ctx->store_through_upto = value;

@@ -97,7 +97,7 @@ const char *hcclx_last_error(void);
  *                     launches for which the register kernel is otherwise kept)
  *   "fanout_from"     bytes read and written from which a fold with several destinations is split into fold + fan-out
  *   "store_through_upto"  bytes written up to which multi-destination folds store through the L2
- *   "moe_scatter_rows"  entries of a token per wavefront of the MoE dispatch of long rows (1 or 2; chosen per launch until set)
+ *   "moe_scatter_rows"  entries of a token per wavefront of the MoE dispatch of long rows (1 or 2; 0 = chosen per launch)
  * Plans made before the call keep the kernels they were made for.  The knobs are plain fields of the device's
  * context: set them while no other thread is planning a launch on that device.  Returns HCCL_E_PARA for an unknown
  * name or a value out of range.  No counterpart in the reference. */

@@ -352,3 +352,26 @@ def test_route_with_perm_in_the_place_of_dest(n, entries):
         assert np.array_equal(got.cpu().numpy().reshape(n, n), np.array(want, dtype=np.int64))
     for i in range(n):
         assert np.array_equal(both[i].cpu().numpy().view(np.uint32), perms[i]), i
+
+
+def test_the_scatter_knob_can_be_taken_back():
+    """1 and 2 entries per wavefront, then chosen per launch again: the same rows; anything else is refused."""
+    n, topk, tokens, width = 3, 4, 50, 512
+    rng = np.random.default_rng(8)
+    dests = [rng.integers(0, n, size=tokens * topk) for _ in range(n)]
+    tabs, perm = route_on_gpu(dests, n, tokens * topk, width)
+    dest = [dev_i32(d) for d in dests]
+    tok = [torch.arange(tokens * width, device=DEV, dtype=torch.int32) + i * 1000003 for i in range(n)]
+    ptrs = lambda ts: [t.data_ptr() for t in ts]
+    got = []
+    for value in (0, 1, 2, 0):
+        hcclx.tune("moe_scatter_rows", value)
+        recv = [torch.zeros(int(tabs[2].reshape(n, n)[j].sum()), device=DEV, dtype=torch.int32) for j in range(n)]
+        torch.cuda.synchronize()
+        hcclx.moe_dispatch(ptrs(tok), ptrs(dest), ptrs(perm), tokens * topk, topk, width, T.FP32, tabs[1].data_ptr(), tabs[3].data_ptr(), ptrs(recv))
+        torch.cuda.synchronize()
+        got.append(recv)
+    for recv in got[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(got[0], recv))
+    with pytest.raises(HcclError):
+        hcclx.tune("moe_scatter_rows", 3)
