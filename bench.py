@@ -268,7 +268,7 @@ class AllToAllV(Workload):
     """benchmark configuration 4: HcclAlltoAllV bf16, MoE dispatch: 8 ranks x 4096 tokens x hidden 7168,
     destination rank per token Zipf(s=1.2), tokens grouped by destination."""
     dtype = "u8"
-    kernel = "hcclx::(anonymous namespace)::k_copy_blocks<hcclx::A2avInline>"
+    kernel = "hcclx::(anonymous namespace)::k_copy_blocks<hcclx::A2avInline, 1u>"
 
     def __init__(self, torch, api, T, n=8, tokens=4096, hidden=7168, seed=0):
         import numpy as np

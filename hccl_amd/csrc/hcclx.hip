@@ -272,7 +272,7 @@ int upload_table(char *d, const char *h, size_t bytes, hipStream_t stream)
         return HCCL_SUCCESS;
     }
     const uint32_t words = static_cast<uint32_t>((bytes + 7) / 8);   // both ends are 256-byte aligned slots
-    // not counted among the collective's kernels: it stands for a copy
+    // not counted among the collective's kernels (launch.h)
     hipLaunchKernelGGL(k_fetch_table, dim3((words + 255) / 256), dim3(256), 0, stream, reinterpret_cast<const uint64_t *>(h),
                        reinterpret_cast<uint64_t *>(d), words);
     const hipError_t e = hipGetLastError();

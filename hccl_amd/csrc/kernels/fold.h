@@ -80,13 +80,15 @@ __device__ __forceinline__ u32x4 ld16(const char *p)
 __device__ __forceinline__ u32x4 ld16_cached(const char *p) { return *as_global(p); }
 // How results leave the CU.  Two ways to store, measured on MI355X against each other and against ordinary stores:
 //   stream   nontemporal: the line is marked for early eviction.  Best where many large output streams are
-//            written at once (the self-first orders) and for the copy kernels (AlltoAllV 154 us against 162).
+//            written at once (the self-first orders) and for copies to several places whose source the L2 keeps (these
+//            stores leave it there: AllGather of 8 x 64 MiB 741 us against 797).
 //   through  agent scope ("sc1"): written through the L2 instead of sitting there as a dirty line that has to be
 //            evicted later.  Best for a single output stream (8 sources of 64 MiB folded into one output: 97.2 us
 //            against 99.5 streamed and 96.8 ordinary; also when a second launch fans that output out: 174.6 us
 //            against 179.8 with ordinary stores for the 8 x 64 MiB AllReduce) and for every launch that writes
 //            several streams at once below the size where it is split into fold + fan-out (8 x 32 MiB AllReduce
-//            in one pass: 83.8 us against 96.3).
+//            in one pass: 83.8 us against 96.3).  Also for copies of blocks (AlltoAll(V); vops.hip says which ones are
+//            streamed) and the MoE dispatch of tokens that the caches do not hold.
 constexpr uint32_t kStoreStream = 0;
 constexpr uint32_t kStoreThrough = 1;
 __device__ __forceinline__ void st16(char *p, u32x4 v)

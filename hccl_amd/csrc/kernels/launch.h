@@ -1,5 +1,6 @@
-// Every kernel launch of the library goes through HCCLX_LAUNCH, which counts it for the calling host thread
-// (hcclx_kernels_launched): the host runtime reports how many kernels a collective took from that count.
+// Every kernel launch of the library but one goes through HCCLX_LAUNCH, which counts it for the calling host thread
+// (hcclx_kernels_launched): the host runtime reports how many kernels a collective took from that count.  The one is
+// the upload of a large launch table (upload_table), which stands for a copy and is not counted, as the copy is not.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

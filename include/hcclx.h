@@ -105,7 +105,9 @@ int hcclx_tune(const char *name, uint64_t value);
 
 /* Number of GPU kernels the calling host thread has launched through this library so far (a running count; take
  * the difference around a call to learn how many kernels it made -- a fold whose result fans out to many places is
- * two, an AllGatherV of about 2 GiB of payload or more several).  No counterpart in the reference. */
+ * two, an AllGatherV of about 2 GiB of payload or an AlltoAllV of 64 GiB or more several).  What brings a call's launch
+ * table to the device is not counted: the runtime's copy up to 16 KiB, a small kernel in front of the counted ones beyond.
+ * No counterpart in the reference. */
 uint64_t hcclx_kernels_launched(void);
 
 /* Size in bytes of an HcclDataType (0 if unknown).  DATATYPE_SIZE_TABLE, alg_param.h:43-45. */
