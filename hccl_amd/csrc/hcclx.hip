@@ -297,30 +297,31 @@ size_t align256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 
 size_t PhasedLaunch::bytes() const
 {
-    return align256(sources.size() * sizeof(PhasedSource)) + align256(slabs.size() * sizeof(CopySlab)) + dsts.size() * sizeof(char *);
+    return align256(sources.size() * sizeof(PhasedSource)) + align256(ranges.size() * sizeof(uint32_t)) + dsts.size() * sizeof(char *);
 }
 PhasedTable PhasedLaunch::table(const char *d) const
 {
     PhasedTable t;
     t.sources = reinterpret_cast<const PhasedSource *>(d);
     d += align256(sources.size() * sizeof(PhasedSource));
-    t.slabs = reinterpret_cast<const CopySlab *>(d);
-    d += align256(slabs.size() * sizeof(CopySlab));
+    t.ranges = reinterpret_cast<const uint32_t *>(d);
+    d += align256(ranges.size() * sizeof(uint32_t));
     t.dsts = reinterpret_cast<char *const *>(d);
     t.nd = grid.nd;
-    t.nslabs = static_cast<uint32_t>(slabs.size());
+    t.shift = shift;
+    t.tiles = static_cast<uint32_t>(tiles);
     return t;
 }
 void PhasedLaunch::fill(char *h) const
 {
     std::memcpy(h, sources.data(), sources.size() * sizeof(PhasedSource));
     h += align256(sources.size() * sizeof(PhasedSource));
-    std::memcpy(h, slabs.data(), slabs.size() * sizeof(CopySlab));
-    h += align256(slabs.size() * sizeof(CopySlab));
+    std::memcpy(h, ranges.data(), ranges.size() * sizeof(uint32_t));
+    h += align256(ranges.size() * sizeof(uint32_t));
     std::memcpy(h, dsts.data(), dsts.size() * sizeof(char *));
 }
 
-void build_phased(std::vector<PhasedStream> &streams, uint64_t batch_bytes, uint32_t max_slabs, std::vector<PhasedLaunch> *out)
+void build_phased(std::vector<PhasedStream> &streams, uint64_t batch_bytes, uint32_t max_groups, std::vector<PhasedLaunch> *out)
 {
     // join streams that continue each other: the slices of a two-shot AllReduce lie back to back in every buffer
     std::vector<PhasedStream> joined;
@@ -335,28 +336,24 @@ void build_phased(std::vector<PhasedStream> &streams, uint64_t batch_bytes, uint
             joined.push_back(std::move(st));
         }
     }
-    // the smallest slab size with which the sources need at most max_slabs slabs (or the largest, and several launches); a
-    // smaller one, and more launches, where it would leave more than a quarter of the slabs' tiles empty: short sources beside
-    // a long one, or more of them than a launch has slabs (to eight places, slabs of the largest size : this way: 5000 x 64 KiB
-    // 15214 : 605 us, 64 MiB and 4090 x 4 KiB 12567 : 229)
-    uint32_t tiles = kPhasedSlabTilesLeast;
-    auto slabs_at = [&](uint32_t t) {
-        uint64_t n = 0;
-        for (const PhasedStream &st : joined) n += phased_slabs_of(st.bytes, t);
-        return n;
-    };
-    const uint64_t least = slabs_at(kPhasedSlabTilesLeast) * kPhasedSlabTilesLeast;
-    while (tiles < kPhasedSlabTilesMost && slabs_at(tiles) > max_slabs) tiles *= 2;
-    while (tiles > kPhasedSlabTilesLeast && slabs_at(tiles) * tiles > least + least / 4) tiles /= 2;
+    const uint64_t most_tiles = static_cast<uint64_t>(max_groups) * kPhasedGroupTiles;
     PhasedLaunch cur;
     auto flush = [&]() {
-        if (cur.slabs.empty()) return;
-        const uint64_t n = cur.slabs.size();
-        const uint64_t most = std::max<uint64_t>(1, batch_bytes / (tiles * kPhasedTile));
-        const uint64_t batches = (n + most - 1) / most;
-        cur.grid.slab_tiles = tiles;
-        cur.grid.batches = static_cast<uint32_t>(batches);
-        cur.grid.per_batch = static_cast<uint32_t>((n + batches - 1) / batches);
+        if (cur.tiles == 0) return;
+        std::vector<uint64_t> begin(cur.sources.size());
+        for (size_t j = 1; j < begin.size(); ++j) begin[j] = cur.sources[j].begin;
+        std::vector<uint32_t> starts;
+        index_tiles(begin.data(), begin.size(), cur.tiles, static_cast<uint32_t>(std::min<uint64_t>(max_groups, 16 * begin.size())), &starts,
+                    &cur.shift);
+        // (the tables' size keeps the sources of a launch below 2^16)
+        for (size_t g = 0; g + 1 < starts.size(); ++g) cur.ranges.push_back(starts[g] | starts[g + 1] << 16);
+        // batches of equal length, up to a sixteenth longer than asked for rather than one more of them; at least eight tiles, at
+        // most 65535 batches (grid z)
+        const uint64_t want = std::max<uint64_t>(std::max<uint64_t>(8, batch_bytes / kPhasedTile), cur.tiles / 65534 + 1);
+        const uint64_t batches = (std::max<uint64_t>(cur.tiles - std::min(cur.tiles, want / 16), 1) + want - 1) / want;
+        const uint64_t per_batch = ((cur.tiles + batches - 1) / batches + 7) & ~7ull;
+        cur.grid.per_batch = static_cast<uint32_t>(per_batch);
+        cur.grid.batches = static_cast<uint32_t>((cur.tiles + per_batch - 1) / per_batch);
         // the pointer array is laid out once the source with the most places is known
         std::vector<char *> flat(cur.sources.size() * cur.grid.nd, nullptr);
         size_t at = 0;
@@ -369,17 +366,17 @@ void build_phased(std::vector<PhasedStream> &streams, uint64_t batch_bytes, uint
     };
     for (const PhasedStream &st : joined) {
         const uint32_t nd = static_cast<uint32_t>(st.dst.size());
-        const uint64_t slabs = phased_slabs_of(st.bytes, tiles);
-        for (uint64_t k = 0; k < slabs; ++k) {
+        const uint64_t tiles = phased_tiles_of(st.bytes);
+        for (uint64_t from = 0; from < tiles;) {
+            if (tiles >= kPhasedLongTiles) cur.tiles = (cur.tiles + 7) & ~7ull;   // left to the source in front, which has no such tiles
             // a launch's tables stay inside one slice of the descriptor ring
-            const bool room = cur.slabs.size() < max_slabs && (cur.sources.size() + 1) * (sizeof(PhasedSource) + 8ull * std::max(cur.grid.nd, nd)) <= (1u << 19);
-            if (!room) flush();
-            if (k == 0 || !room) {
-                cur.sources.push_back({st.src, st.bytes, nd});
-                cur.dsts.insert(cur.dsts.end(), st.dst.begin(), st.dst.end());   // packed for now, see flush()
-                cur.grid.nd = std::max(cur.grid.nd, nd);
-            }
-            cur.slabs.push_back({static_cast<uint32_t>(cur.sources.size() - 1), static_cast<uint32_t>(k)});
+            if (cur.tiles == most_tiles || (cur.sources.size() + 1) * (sizeof(PhasedSource) + 8ull * std::max(cur.grid.nd, nd)) > (1u << 19)) flush();
+            cur.sources.push_back({st.src, st.bytes, nd, static_cast<uint32_t>(cur.tiles - from), 0});
+            cur.dsts.insert(cur.dsts.end(), st.dst.begin(), st.dst.end());   // packed for now, see flush()
+            cur.grid.nd = std::max(cur.grid.nd, nd);
+            const uint64_t take = std::min(tiles - from, most_tiles - cur.tiles);
+            cur.tiles += take;
+            from += take;
         }
     }
     flush();
@@ -437,7 +434,7 @@ struct Batch {
     size_t nseg() const { return segs.size() + wide.size(); }
     size_t bytes() const
     {
-        if (!phased.slabs.empty()) return phased.bytes();
+        if (phased.tiles != 0) return phased.bytes();
         if (blocks.tiles != 0) return blocks.bytes();
         return align256(tile_end.size() * 8) + segs.size() * sizeof(SegDev) + wide.size() * sizeof(SegWide);
     }
@@ -691,13 +688,11 @@ bool split_fanout(const DeviceCtx *ctx, const SEG *segs, uint32_t nseg, int esz,
     return true;
 }
 
-constexpr uint32_t kPhasedTableSlabs = 4096;   // slabs of a fan-out launch at most: 32 KiB of table
-
 // Appends the second launch (or launches) of a split fold.
 void append_fanout(const DeviceCtx *ctx, std::vector<PhasedStream> &fan, Built *out)
 {
     std::vector<PhasedLaunch> launches;
-    build_phased(fan, ctx->fanout_run, kPhasedTableSlabs, &launches);
+    build_phased(fan, ctx->fanout_run, kPhasedTableGroups, &launches);
     for (PhasedLaunch &l : launches) {
         Batch b;
         b.copy = true;
@@ -1096,7 +1091,7 @@ int build_wide_batches_impl(const hcclx_wide_seg_t *segs, uint32_t nseg, int dty
 
 void fill_table(const Batch &b, char *h)
 {
-    if (!b.phased.slabs.empty()) {
+    if (b.phased.tiles != 0) {
         b.phased.fill(h);
         return;
     }
@@ -1138,7 +1133,7 @@ hipError_t dispatch_fold(int dtype, int op, int maxn, int mode, const FoldLaunch
 
 int launch_batch(const DeviceCtx *ctx, const Batch &b, const char *d_table, hipStream_t stream)
 {
-    if (!b.phased.slabs.empty()) {
+    if (b.phased.tiles != 0) {
         const hipError_t pe = launch_phased_copy(b.phased.table(d_table), b.phased.grid, stream);
         if (pe != hipSuccess) return fail_hip(pe, "phased copy kernel launch");
         return HCCL_SUCCESS;

@@ -105,7 +105,9 @@ inline bool waves_fit(uint64_t pieces, uint32_t per_tile, uint32_t waves)
 struct PhasedLaunch {
     std::vector<PhasedSource> sources;   // place = number of destinations
     std::vector<char *> dsts;            // sources.size() * grid.nd pointers, source s's at [s * nd, s * nd + ndst)
-    std::vector<CopySlab> slabs;
+    std::vector<uint32_t> ranges;
+    uint32_t shift = 0;
+    uint64_t tiles = 0;
     PhasedGrid grid{};
     size_t bytes() const;       // the three arrays as they lie in the launch table
     void fill(char *h) const;
@@ -117,10 +119,9 @@ struct PhasedStream {
     uint64_t bytes;
     std::vector<char *> dst;
 };
-// Turns streams into launches of at most max_slabs slabs: streams that continue each other (source and every destination) are
-// joined, and cut into slabs, the smallest that need one launch, or smaller ones where those would mostly be empty; batches of
-// up to batch_bytes are written to one place after the other.
-void build_phased(std::vector<PhasedStream> &streams, uint64_t batch_bytes, uint32_t max_slabs, std::vector<PhasedLaunch> *out);
+// Turns streams into launches of at most max_groups groups of kPhasedGroupTiles tiles: streams that continue each other (source
+// and every destination) are joined; batches of up to batch_bytes are written to one place after the other.
+void build_phased(std::vector<PhasedStream> &streams, uint64_t batch_bytes, uint32_t max_groups, std::vector<PhasedLaunch> *out);
 // The non-empty blocks of an AlltoAllV with host tables (row-major n x n, elements of esz bytes), their tiles numbered
 // through; returns the number of tiles.
 uint64_t list_alltoallv_blocks(const void *const *send, void *const *recv, const uint64_t *send_counts, const uint64_t *sdispls,

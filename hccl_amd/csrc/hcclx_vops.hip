@@ -249,7 +249,7 @@ int hcclx_allgatherv(const void *const *send, void *const *recv, const uint64_t 
     if (!tables_on_device) {
         uint64_t payload = 0;
         for (uint32_t i = 0; i < n; ++i) payload += counts[i] * esz;
-        // Large: the outputs of a batch of slabs are written one after the other.  A source's places are one offset into
+        // Large: the outputs of a batch of tiles are written one after the other.  A source's places are one offset into
         // every receive buffer and the tables fit the kernel arguments: nothing is copied in front of the kernel.
         if (n > 1 && ctx->agv_phased_from != 0 && payload >= ctx->agv_phased_from) {
             std::vector<PhasedStream> streams;
@@ -258,7 +258,7 @@ int hcclx_allgatherv(const void *const *send, void *const *recv, const uint64_t 
                 if (counts[i] != 0) streams.push_back({ptrs.send[i], counts[i] * esz, {ptrs.recv[0] + displs[i] * esz}});
             }
             std::vector<PhasedLaunch> launches;
-            build_phased(streams, ctx->fanout_run, kPhasedInlineSlabs, &launches);
+            build_phased(streams, ctx->fanout_run, kPhasedInlineGroups, &launches);
             for (PhasedLaunch &l : launches) {
                 PhasedInline tab;
                 for (uint32_t d = 0; d < n; ++d) tab.base[d] = ptrs.recv[d];
@@ -266,8 +266,10 @@ int hcclx_allgatherv(const void *const *send, void *const *recv, const uint64_t 
                     tab.sources[k] = l.sources[k];
                     tab.sources[k].place = static_cast<uint64_t>(l.dsts[k] - ptrs.recv[0]);
                 }
-                for (size_t k = 0; k < l.slabs.size(); ++k) tab.slabs[k] = l.slabs[k].source | l.slabs[k].at << 6;
-                tab.nslabs = static_cast<uint32_t>(l.slabs.size());
+                std::memset(tab.ranges, 0, sizeof(tab.ranges));
+                for (size_t g = 0; g < l.ranges.size(); ++g) tab.ranges[g >> 1] |= (l.ranges[g] & 255u) << (g & 1) * 16 | (l.ranges[g] >> 16) << ((g & 1) * 16 + 8);
+                tab.shift = l.shift;
+                tab.tiles = static_cast<uint32_t>(l.tiles);
                 l.grid.nd = n;
                 hipError_t e = launch_phased_copy_inline(tab, l.grid, st);
                 if (e != hipSuccess) return fail_hip(e, "allgatherv kernel launch");

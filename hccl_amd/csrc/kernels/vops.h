@@ -42,12 +42,15 @@ __host__ __device__ inline uint32_t v_shift_of(uint64_t head, uint64_t dst)
 {
     return static_cast<uint32_t>(((dst + head) & 1023) / 16);
 }
-__host__ __device__ inline uint64_t v_tiles_of(uint64_t bytes, uint64_t dst, int unroll)
+__host__ __device__ inline uint64_t v_last_tile_of(uint64_t bytes, uint64_t dst, int unroll)   // of a block that is not empty
 {
     const uint64_t kTileVecs = 256ull * unroll;
-    if (bytes == 0) return 0;
     const uint64_t head = v_head_of(bytes, dst);
-    return ((bytes - head) / 16 + v_shift_of(head, dst)) / kTileVecs + 1;
+    return ((bytes - head) / 16 + v_shift_of(head, dst)) / kTileVecs;
+}
+__host__ __device__ inline uint64_t v_tiles_of(uint64_t bytes, uint64_t dst, int unroll)
+{
+    return bytes == 0 ? 0 : v_last_tile_of(bytes, dst, unroll) + 1;
 }
 
 // Base pointers of every virtual rank's send and receive buffer, passed by value as a kernel argument.
@@ -115,43 +118,46 @@ struct AgvTablesPtr {
     __device__ uint64_t count(uint32_t i) const { return counts[i]; }
     __device__ uint64_t displ(uint32_t i) const { return displs[i]; }
 };
-// The copy kernel that writes one output at a time.  Its sources are cut into slabs of slab_tiles tiles each, a power of
-// two of at least eight (workgroups go to the eight XCDs in turn, each with an L2 of its own: a tile is then copied to
-// all its places by the same XCD); a batch of slabs, a few MiB, is copied to its first place, then to the second and so
-// on.  The last slab of a source is as long as what is left, so sources of any lengths share a launch and only those
-// ends leave workgroups that exit at once.
-struct CopySlab {
-    uint32_t source;
-    uint32_t at;       // number of the slab inside it
-};
+// The copy kernel that writes one output at a time.  The tiles of its sources are numbered through as those of the blocks
+// above, and a batch of tiles, a few MiB, is copied to its first place, then to the second and so on.  A batch is a multiple of
+// eight tiles: workgroups go to the eight XCDs in turn, each with an L2 of its own, and a tile is then copied to all its
+// places by the same XCD.
 struct PhasedSource {
     const char *src;
     uint64_t bytes;
     uint64_t place;   // table in memory: ndst; tables in the kernel arguments: offset into every rank's receive buffer
+    uint32_t begin;   // number of its first tile (of the first source of a launch: wrapped below zero when it begins inside)
+    uint32_t reserved;
 };
-constexpr uint32_t kPhasedSlabTilesLeast = 8;
-constexpr uint32_t kPhasedSlabTilesMost = 1024;   // 4 MiB
-// A launch's tables in device memory: sources, slabs and nd places per source.
+constexpr uint32_t kPhasedGroupTiles = 1024;   // at most: 4 MiB
+// A source of so many tiles begins at a multiple of eight of them: HBM is interleaved over its stacks by 4 KiB, and one XCD then
+// stays with the same stacks for all of them (100 x 1 MiB to eight places 149.7 us, 155.2 without; no difference for 33 tiles).
+constexpr uint32_t kPhasedLongTiles = 192;
+// A launch's tables in device memory: sources, start table (an entry and the next one in a word: one load) and nd places per
+// source.
 struct PhasedTable {
     const PhasedSource *sources;
-    const CopySlab *slabs;
+    const uint32_t *ranges;   // starts[g] | starts[g + 1] << 16
     char *const *dsts;
-    uint32_t nd;
-    uint32_t nslabs;
+    uint32_t shift : 8;   // in one word, so that both come with one load
+    uint32_t nd : 24;
+    uint32_t tiles;
 };
+constexpr uint32_t kPhasedTableGroups = 4096;
 // The same for an AllGather(V), in the kernel arguments: every place of a source is the same offset into the ranks'
-// receive buffers.  Slab: source in the low six bits, its number above.
-constexpr uint32_t kPhasedInlineSlabs = 480;
+// receive buffers.
+constexpr uint32_t kPhasedInlineGroups = 480;
 struct PhasedInline {
     char *base[kMaxVRanks];
     PhasedSource sources[kMaxVRanks];
-    uint32_t slabs[kPhasedInlineSlabs];
-    uint32_t nslabs;
+    uint32_t ranges[kPhasedInlineGroups / 2];   // sixteen bits each, starts[g] | starts[g + 1] << 8
+    uint32_t shift;
+    uint32_t tiles;
 };
-// Slabs a source needs whatever the alignment of its places (their tile grids differ by less than a tile).
-__host__ __device__ inline uint64_t phased_slabs_of(uint64_t bytes, uint32_t slab_tiles)
+// Tiles of a source whatever the alignment of its places (their tile grids differ by less than a tile).
+__host__ __device__ inline uint64_t phased_tiles_of(uint64_t bytes)
 {
-    return bytes == 0 ? 0 : ((bytes / 16 + 63) / (kPhasedTile / 16) + slab_tiles) / slab_tiles;
+    return bytes == 0 ? 0 : (bytes / 16 + 63) / (kPhasedTile / 16) + 1;
 }
 struct AgvTablesInline {
     uint64_t counts[kMaxVRanks];
@@ -167,9 +173,8 @@ constexpr uint64_t kMostBlocksX = 0xffffffffull / kThreads;
 hipError_t launch_copy_blocks(const BlockTable &tab, size_t blocks, uint64_t tiles, hipStream_t stream);
 hipError_t launch_equal_blocks(const EqualBlocks &tab, uint32_t n, hipStream_t stream);
 hipError_t launch_alltoallv_inline(const A2avInline &tab, uint64_t tiles, hipStream_t stream);
-// One batch after the other (grid z), each to one place after the other (grid y): per_batch slabs of slab_tiles tiles.
+// One batch after the other (grid z), each to one place after the other (grid y): per_batch tiles, a multiple of eight.
 struct PhasedGrid {
-    uint32_t slab_tiles;
     uint32_t per_batch;
     uint32_t batches;
     uint32_t nd;

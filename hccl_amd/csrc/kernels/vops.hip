@@ -171,8 +171,15 @@ k_alltoallv(Ptrs ptrs, Tabs tabs, uint32_t n, uint32_t esz, uint32_t tiles_per_b
     }
 }
 
-__device__ __forceinline__ uint32_t start_of(const BlockTable &t, uint32_t g) { return t.starts[g]; }
-__device__ __forceinline__ uint32_t start_of(const A2avInline &t, uint32_t g) { return t.starts[g >> 2] >> (g & 3u) * 8 & 255u; }
+// The first and the last block (or source) that a tile of group g can lie in.
+struct Range {
+    uint32_t lo, hi;
+};
+__device__ __forceinline__ Range range_of(const BlockTable &t, uint32_t g) { return {t.starts[g], t.starts[g + 1]}; }
+__device__ __forceinline__ Range range_of(const A2avInline &t, uint32_t g)
+{
+    return {t.starts[g >> 2] >> (g & 3u) * 8 & 255u, t.starts[(g + 1) >> 2] >> ((g + 1) & 3u) * 8 & 255u};
+}
 __device__ __forceinline__ uint64_t begin_of(const BlockTable &t, uint32_t b) { return t.blocks[b].begin; }
 __device__ __forceinline__ uint64_t begin_of(const A2avInline &t, uint32_t b) { return t.begin[b]; }
 __device__ __forceinline__ CopyBlock block_of(const BlockTable &t, uint32_t b) { return t.blocks[b]; }
@@ -182,6 +189,32 @@ __device__ __forceinline__ CopyBlock block_of(const A2avInline &t, uint32_t b)
     const uint32_t j = b - i * t.n;
     return {t.send[i] + static_cast<uint64_t>(t.sdispls[b]) * t.esz, t.recv[j] + static_cast<uint64_t>(t.rdispls[b]) * t.esz,
             static_cast<uint64_t>(t.counts[b]) * t.esz, t.begin[b]};
+}
+
+__device__ __forceinline__ Range range_of(const PhasedTable &t, uint32_t g) { return {t.ranges[g] & 0xffffu, t.ranges[g] >> 16}; }
+__device__ __forceinline__ Range range_of(const PhasedInline &t, uint32_t g)
+{
+    const uint32_t one = t.ranges[g >> 1] >> (g & 1u) * 16;
+    return {one & 255u, one >> 8 & 255u};
+}
+__device__ __forceinline__ uint32_t begin_of(const PhasedTable &t, uint32_t s) { return t.sources[s].begin; }
+__device__ __forceinline__ uint32_t begin_of(const PhasedInline &t, uint32_t s) { return t.sources[s].begin; }
+
+// The last block (or source) that begins at a tile or in front of it.
+template <typename Tab, typename N> __device__ __forceinline__ uint32_t at_tile(const Tab &tab, N tile)
+{
+    const Range r = range_of(tab, static_cast<uint32_t>(tile >> tab.shift));
+    uint32_t lo = r.lo;
+    uint32_t hi = r.hi;
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi + 1) >> 1;
+        if (begin_of(tab, mid) <= tile) {
+            lo = mid;
+        } else {
+            hi = mid - 1;
+        }
+    }
+    return lo;
 }
 
 // Blocks of any lengths, one 4 KiB tile per workgroup and one vector per thread, mostly stored through the L2: bound by HBM.
@@ -194,18 +227,7 @@ template <typename Tab, uint32_t kPolicy>
 __global__ void __launch_bounds__(kThreads) k_copy_blocks(Tab tab, uint64_t first)
 {
     const uint64_t tile = first + blockIdx.x;
-    const uint32_t group = static_cast<uint32_t>(tile >> tab.shift);
-    uint32_t lo = start_of(tab, group);
-    uint32_t hi = start_of(tab, group + 1);
-    while (lo < hi) {   // the last block that begins at the tile or in front of it
-        const uint32_t mid = (lo + hi + 1) >> 1;
-        if (begin_of(tab, mid) <= tile) {
-            lo = mid;
-        } else {
-            hi = mid - 1;
-        }
-    }
-    const CopyBlock b = block_of(tab, lo);
+    const CopyBlock b = block_of(tab, at_tile(tab, tile));
     char *dst = b.dst;
     copy_tile<1, false, kPolicy>(b.src, reinterpret_cast<uint64_t>(dst), b.bytes, tile - b.begin, 1, [=](uint32_t) { return dst; });
 }
@@ -222,34 +244,33 @@ __global__ void __launch_bounds__(kThreads) k_equal_blocks(EqualBlocks tab)
     copy_tile<1, false, kStoreThrough>(src, reinterpret_cast<uint64_t>(dst), bytes, blockIdx.x, 1, [=](uint32_t) { return dst; });
 }
 
-__device__ __forceinline__ CopySlab phased_slab(const PhasedTable &t, uint32_t k) { return t.slabs[k]; }
-__device__ __forceinline__ CopySlab phased_slab(const PhasedInline &t, uint32_t k) { return {t.slabs[k] & 63u, t.slabs[k] >> 6}; }
-// null: the source has no such place
-__device__ __forceinline__ char *phased_dst(const PhasedTable &t, uint32_t source, uint32_t d)
+// null: the source has no such place (the table has nd of them for every source)
+__device__ __forceinline__ char *phased_dst(const PhasedTable &t, uint32_t k, const PhasedSource &, uint32_t d)
 {
-    return d < t.sources[source].place ? t.dsts[static_cast<uint64_t>(source) * t.nd + d] : nullptr;
+    return t.dsts[k * t.nd + d];
 }
-__device__ __forceinline__ char *phased_dst(const PhasedInline &t, uint32_t source, uint32_t d) { return t.base[d] + t.sources[source].place; }
+__device__ __forceinline__ char *phased_dst(const PhasedInline &t, uint32_t, const PhasedSource &source, uint32_t d) { return t.base[d] + source.place; }
 
 // Sources to several places, one place at a time.  Workgroups start in the order of their numbers (x: tile of the
 // batch, y: place, z: batch), so a batch is written to its first place, then to the second, and so on.  At any moment
 // the GPU writes ONE output instead of n at once, which HBM takes faster (one source to eight outputs, every workgroup
 // storing to all eight: 5.5 TB/s at the pins; this way 6.4-6.5); the re-reads of the batch come from the L2s, not from
-// HBM.  The place of a workgroup follows from its number with two dependent scalar loads: a table search in front of a
-// tile costs a fifth of the kernel's time.
+// HBM.  The place of a workgroup follows from its number with mostly two dependent scalar loads: a table search in front
+// of a tile costs a fifth of the kernel's time.  No workgroup is idle but at the end of a batch and of a place that is aligned
+// better than the worst; with sources cut into slabs of one size, 5000 x 64 KiB to eight places took 15214 us (this way 565),
+// 64 MiB beside 4090 x 4 KiB 12567 (140), 900 x 70001 bytes to three 47.4 (40), and the AllGather of 8 x 64 MiB 754 (755).
 template <typename Tab>
-__global__ void __launch_bounds__(kThreads) k_phased_copy(Tab tab, uint32_t slab_shift, uint32_t per_batch)
+__global__ void __launch_bounds__(kThreads) k_phased_copy(Tab tab, uint32_t per_batch)
 {
-    const uint32_t k = blockIdx.z * per_batch + (blockIdx.x >> slab_shift);
-    if (k >= tab.nslabs) return;
-    const CopySlab slab = phased_slab(tab, k);
-    const uint64_t tl = (static_cast<uint64_t>(slab.at) << slab_shift) + (blockIdx.x & ((1u << slab_shift) - 1u));
-    const PhasedSource &source = tab.sources[slab.source];
-    const char *src = source.src;
-    const uint64_t bytes = source.bytes;
-    char *dst = phased_dst(tab, slab.source, blockIdx.y);
-    if (dst == nullptr || tl >= v_tiles_of(bytes, reinterpret_cast<uint64_t>(dst), kPhasedUnroll)) return;
-    copy_tile<kPhasedUnroll, true>(src, reinterpret_cast<uint64_t>(dst), bytes, tl, 1, [=](uint32_t) { return dst; });
+    const uint32_t tile = blockIdx.z * per_batch + blockIdx.x;
+    if (tile >= tab.tiles) return;
+    const uint32_t k = at_tile(tab, tile);
+    const PhasedSource source = tab.sources[k];
+    char *dst = phased_dst(tab, k, source, blockIdx.y);
+    const uint32_t tl = tile - source.begin;
+    // (one test: with a branch for each the look-ups would wait for one another)
+    if ((dst == nullptr) | (tl > v_last_tile_of(source.bytes, reinterpret_cast<uint64_t>(dst), kPhasedUnroll))) return;
+    copy_tile<kPhasedUnroll, true>(source.src, reinterpret_cast<uint64_t>(dst), source.bytes, tl, 1, [=](uint32_t) { return dst; });
 }
 
 template <typename Tabs>
@@ -335,8 +356,7 @@ hipError_t launch_alltoallv_inline(const A2avInline &tab, uint64_t tiles, hipStr
 namespace {
 template <typename Tab> hipError_t launch_phased(const Tab &tab, const PhasedGrid &g, hipStream_t stream)
 {
-    const uint32_t shift = static_cast<uint32_t>(__builtin_ctz(g.slab_tiles));
-    HCCLX_LAUNCH((k_phased_copy<Tab>), dim3(g.per_batch << shift, g.nd, g.batches), dim3(kThreads), 0, stream, tab, shift, g.per_batch);
+    HCCLX_LAUNCH((k_phased_copy<Tab>), dim3(g.per_batch, g.nd, g.batches), dim3(kThreads), 0, stream, tab, g.per_batch);
     return hipGetLastError();
 }
 }  // namespace

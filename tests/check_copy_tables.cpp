@@ -2,7 +2,7 @@
 // builds it against the library and runs it; nothing here touches a GPU).
 //   blocks n  c00 c01 ...    an AlltoAllV's n x n counts (bytes): every tile of every block is found exactly once
 //       prints "tiles <blocks' own> groups <g> bytes <of the table>"
-//   copies max_slabs  bytes:places[xtimes] ...    sources that go to several places: every tile of every place is found exactly
+//   copies max_groups  bytes:places[xtimes] ...    sources that go to several places: every tile of every place is found exactly
 //       once; prints "tiles <of all places> workgroups <of all launches> launches <l> bytes <of the largest table>"
 //   waves pieces per_tile waves    whether one launch of the wavefront fold takes them: prints 1 or 0
 // or what is wrong.
@@ -114,7 +114,7 @@ int blocks(int argc, char **argv)
 
 int copies(int argc, char **argv)
 {
-    const uint32_t max_slabs = static_cast<uint32_t>(std::strtoul(argv[0], nullptr, 10));
+    const uint32_t max_groups = static_cast<uint32_t>(std::strtoul(argv[0], nullptr, 10));
     std::vector<PhasedStream> streams;
     for (int k = 1; k < argc; ++k) {
         unsigned long long bytes = 0;
@@ -129,7 +129,7 @@ int copies(int argc, char **argv)
     }
     const std::vector<PhasedStream> asked = streams;
     std::vector<PhasedLaunch> launches;
-    build_phased(streams, 16ull << 20, max_slabs, &launches);
+    build_phased(streams, 16ull << 20, max_groups, &launches);
     uint64_t own = 0, workgroups = 0, most_bytes = 0;
     std::vector<std::vector<std::vector<bool>>> moved(asked.size());
     for (size_t s = 0; s < asked.size(); ++s) {
@@ -140,26 +140,36 @@ int copies(int argc, char **argv)
         }
     }
     for (const PhasedLaunch &l : launches) {
-        if (l.slabs.size() > max_slabs) return wrong("slabs of a launch", l.slabs.size());
+        if (l.ranges.size() > max_groups) return wrong("groups of a launch", l.ranges.size());
         if (l.bytes() > 1u << 20) return wrong("table of a launch", l.bytes());
         most_bytes = std::max<uint64_t>(most_bytes, l.bytes());
-        const uint64_t x = static_cast<uint64_t>(l.grid.per_batch) * l.grid.slab_tiles;
-        if (x > kMostBlocksX || l.grid.nd > 65535 || l.grid.batches > 65535) return wrong("grid", x);
+        const uint64_t x = l.grid.per_batch;
+        if (x > kMostBlocksX || x % 8 != 0 || l.grid.nd > 65535 || l.grid.batches > 65535) return wrong("grid", x);
         workgroups += x * l.grid.nd * l.grid.batches;
         std::vector<char> table(l.bytes());
         l.fill(table.data());
         const PhasedTable t = l.table(table.data());
-        for (uint64_t k = 0; k < static_cast<uint64_t>(l.grid.per_batch) * l.grid.batches && k < t.nslabs; ++k) {
-            const CopySlab slab = t.slabs[k];
-            const PhasedSource &source = t.sources[slab.source];
+        if (t.tiles > x * l.grid.batches) return wrong("tiles of a launch", t.tiles);
+        std::vector<uint32_t> starts;
+        for (size_t g = 0; g < l.ranges.size(); ++g) {
+            if (g != 0 && starts[g] != (t.ranges[g] & 0xffffu)) return wrong("range of group", g);
+            if (g == 0) starts.push_back(t.ranges[0] & 0xffffu);
+            starts.push_back(t.ranges[g] >> 16);
+        }
+        std::vector<uint64_t> begin;
+        for (size_t k = 0; k < l.sources.size(); ++k) begin.push_back(k == 0 ? 0 : t.sources[k].begin);
+        for (uint64_t tile = 0; tile < t.tiles; ++tile) {
+            if ((tile >> t.shift) + 1 >= starts.size()) return wrong("no group for tile", tile);
+            const size_t k = block_of(starts, t.shift, begin, tile);
+            const PhasedSource &source = t.sources[k];
             const size_t s = (reinterpret_cast<uint64_t>(source.src) >> 33) - 1;
-            if (s >= asked.size() || source.bytes != asked[s].bytes || source.place != asked[s].dst.size()) return wrong("source of slab", k);
+            if (s >= asked.size() || source.bytes != asked[s].bytes || source.place != asked[s].dst.size()) return wrong("source of tile", tile);
+            const uint32_t tl = static_cast<uint32_t>(tile) - source.begin;
             for (uint32_t d = 0; d < source.place; ++d) {
-                if (t.dsts[static_cast<uint64_t>(slab.source) * t.nd + d] != asked[s].dst[d]) return wrong("place of slab", k);
-                for (uint64_t tl = static_cast<uint64_t>(slab.at) * l.grid.slab_tiles; tl < (slab.at + 1ull) * l.grid.slab_tiles && tl < moved[s][d].size(); ++tl) {
-                    if (moved[s][d][tl]) return wrong("tile moved twice, source", s);
-                    moved[s][d][tl] = true;
-                }
+                if (t.dsts[static_cast<uint64_t>(k) * t.nd + d] != asked[s].dst[d]) return wrong("place of tile", tile);
+                if (tl >= moved[s][d].size()) continue;
+                if (moved[s][d][tl]) return wrong("tile moved twice, source", s);
+                moved[s][d][tl] = true;
             }
         }
     }

@@ -54,25 +54,28 @@ def test_every_tile_of_an_alltoallv_is_found_once(check, n, kind):
     assert groups <= 4096 and size <= 32 * live + 256 + 4 * (min(4096, 4 * live) + 1)
 
 
-@pytest.mark.parametrize("max_slabs,sources,most_launches", [
-    (4096, ["65536:8x5000"], 4),                         # more sources than a launch has slabs
-    (4096, ["67108864:8", "4096:8x4090"], 4),            # one long source and nearly as many short ones as slabs
-    (4096, ["1073741824:2", "100:2x4000"], 8),
-    (4096, ["9000000:7x30", "70001:3x900", "1:2x50"], 2),
+@pytest.mark.parametrize("max_groups,sources,most_launches", [
+    (4096, ["65536:8x5000"], 1),                         # more sources than a launch has groups
+    (4096, ["65536:8x6000"], 2),                         # more than its tables hold
+    (4096, ["67108864:8", "4096:8x4090"], 1),            # one long source and many short ones
+    (4096, ["100:2x4000", "1073741824:2"], 1),
+    (4096, ["9000000:7x30", "70001:3x900", "1:2x50"], 1),
     (4096, ["8388608:8x7"], 1),
-    (480, ["67108864:8", "1:8x63"], 2),                  # an AllGatherV in the kernel arguments
+    (480, ["67108864:8", "1:8x63"], 1),                  # an AllGatherV in the kernel arguments
     (480, ["8388608:16x16"], 1),
     (480, ["33800:64x64"], 1),
-    (480, ["1073745923:2", "1073741901:2"], 2),
+    (480, ["1073745923:2", "1073741901:2"], 2),          # a source that begins in one launch and ends in the next
+    (480, ["5368709120:3", "5:3"], 3),
 ])
-def test_copies_to_several_places_launch_few_idle_workgroups(check, max_slabs, sources, most_launches):
-    """A slab is at least eight tiles, and of the slabs' workgroups at most a quarter more than that are without a tile.  Sources
-    of fewer places than the launch's most leave more."""
-    tiles, workgroups, launches, _ = check("copies", max_slabs, *sources)
+def test_copies_to_several_places_launch_no_idle_workgroups(check, max_groups, sources, most_launches):
+    """Every tile of every place exactly once; and as many workgroups as the sources have tiles at the worst alignment, times the
+    launch's places, but for the last tiles of the batches and those in front of a source of 192 tiles or more."""
+    tiles, workgroups, launches, _ = check("copies", max_groups, *sources)
     listed = [tuple(int(x) for x in (s if "x" in s else s + "x1").replace(":", "x").split("x")) for s in sources]
     most = max(places for _, places, _ in listed)
-    least = sum(times * most * 8 * ((size // 4096 + 1) // 8 + 1) for size, _, times in listed)
-    assert workgroups <= 1.25 * least + most * 1024 * launches
+    own = sum(times * (size // 4096 + 2 + (7 if size // 4096 >= 190 else 0)) for size, _, times in listed)
+    batches = own // 4000 + launches
+    assert tiles <= workgroups <= most * (own + 8 * batches)
     assert launches <= most_launches
 
 
