@@ -297,17 +297,17 @@ def test_allgatherv_with_counts_and_displacements_that_never_leave_the_device():
         assert recv[j].guard_intact()
 
 
-SLAB = 32768    # the smallest slab of the copy kernel that writes one output at a time
+SLAB = 32768    # eight tiles, one for each XCD, of the copy kernel that writes one output at a time
 
 
 @pytest.mark.parametrize("n,sizes,pad", [
     (2, [(4 << 20) + 1, 1], 0),                                                     # one long source, one of a byte
-    (5, [SLAB - 1, SLAB, SLAB + 1, 3 * SLAB + 1008, 4 << 20], 5),                   # around the slab edges, shifted places
+    (5, [SLAB - 1, SLAB, SLAB + 1, 3 * SLAB + 1008, 4 << 20], 5),                   # around whole tiles, shifted places
     (16, [300000 + 4099 * k for k in range(16)], 3),                                # no two sources of one length
     (64, [(k % 7) * SLAB + (k * 37) % 1031 + (0 if k % 9 else -1) for k in range(64)], 2),   # most ranks, empty sources
 ])
 def test_allgatherv_written_one_output_at_a_time(n, sizes, pad):
-    """From 4 MiB of payload: slabs of the sources, batch by batch to one receive buffer after the other; receive
+    """From 4 MiB of payload: the tiles of the sources, batch by batch to one receive buffer after the other; receive
     buffers of different alignment, holes between the blocks."""
     counts = [max(0, c) for c in sizes]
     counts[0] += max(0, (4 << 20) - sum(counts))

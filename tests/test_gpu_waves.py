@@ -227,8 +227,8 @@ def test_prod_allreduce_of_four_ranks_takes_the_wavefront_kernel_by_default():
 
 @pytest.mark.parametrize("ranks,dtype,op", [(2, T.BFP16, T.SUM), (3, T.FP32, T.MAX), (4, T.INT8, T.SUM), (4, T.FP64, T.PROD), (2, T.INT16, T.MIN)])
 def test_large_chains_among_few_ranks_share_the_fold(ranks, dtype, op):
-    """48 MiB written and more among two to four ranks: one pass on the wavefront kernel, several pieces per workgroup, a
-    head, a tail and a partly filled last tile; against the register kernel."""
+    """48 MiB written among two to four ranks, a head, a tail and a partly filled last tile: one pass with the knob on and off
+    (the register kernel's size; the wavefronts share the fold from the sizes of the test below on)."""
     hcclx.init()
     rng = np.random.default_rng(ranks + dtype)
     esz = T.DTYPE_SIZE[dtype]
