@@ -422,7 +422,8 @@ struct Batch {
     std::vector<uint64_t> tile_end;
     std::vector<SegDev> segs;
     std::vector<SegWide> wide;   // instead of segs when maxn == kMaxWideFan
-    int wide_unroll = 1;         // vectors per thread of the wide kernel
+    int wide_shape = kWideMany;  // of the wide chain kernel (fold.h)
+    uint32_t per_cu = 0;         // non-zero: so many workgroups of the launch to a CU at most
     uint32_t xcd_remap = 0;      // wide kernels: contiguous tile ranges per XCD (pays with 16 or more destinations)
     BlockLaunch blocks;          // instead of everything above: a launch of the block copy kernel
     PhasedLaunch phased;         // instead of everything above: a launch of the copy kernel that writes one output at a time
@@ -949,6 +950,48 @@ int build_wide_batches(const hcclx_wide_seg_t *segs, uint32_t nseg, int dtype, i
     return HCCL_SUCCESS;
 }
 
+// The shape of a chain launch with one destination (fold.h) and how many of its workgroups share a CU.  Straddling: sources
+// that do not share the destination's alignment, so that loads straddle lines.  Kernels among 8 ranks unless said, us:
+//   many   fewer tiles of `one` than wide_min_tiles, unless they straddle and are 4 MiB or more: eight loads at a time hide more
+//          latency (many : small: 2 MiB bf16 6.9 : 7.5, 16 ranks x 4 MiB 13.9 : 16.0; 6 MiB odd 13.0 : 12.4).
+//   small  straddling below 32 MiB (one : small: 16 MiB bf16 31.0 : 27.9, 25 46.0 : 43.8; 40 MiB fp32 59.1 : 62.1).
+//   large  from 128 MiB on (one : large: 150 MiB bf16 246 : 229, 12 x 150 fp32 AllReduce 624 : 605, 12 x 1 GiB int32
+//          4395 : 4295; below it the last round of its 64 KiB tiles shows: 72 MiB 100.8 : 105.1), straddling elements of at
+//          least 4 bytes (200 MiB fp32 323 : 315; 400 MiB bf16 691 : 704).
+//   one    otherwise, three or four workgroups to a CU, whichever leaves less of the last round empty (three : four: 25 MiB
+//          40.2 : 38.8, 16 x 40 109.9 : 111.5, 24 x 20 AllReduce 157 : 168, 32 x 16 91.6 : 82.9; two, five and more: slower).
+int wide_shape_for(const DeviceCtx *ctx, const hcclx_wide_seg_t *segs, uint32_t nseg, int esz, uint32_t *per_cu)
+{
+    constexpr uint64_t kLargeFrom = 128ull << 20;
+    constexpr uint64_t kSmallFrom = 4ull << 20;
+    constexpr uint64_t kSmallUpto = 32ull << 20;
+    *per_cu = 0;
+    if (ctx == nullptr) return kWideMany;
+    const uint64_t tile_bytes = 16 * wide_tile_vecs(kWideOne, false);
+    uint64_t bytes = 0;
+    uint64_t tiles = 0;
+    bool straddling = false;
+    for (uint32_t i = 0; i < nseg; ++i) {
+        const uint64_t b = segs[i].count * static_cast<uint64_t>(esz);
+        bytes += b;
+        tiles += (b + tile_bytes - 1) / tile_bytes;
+        for (uint32_t k = 0; k < segs[i].nsrc && b != 0; ++k) {
+            straddling = straddling || (reinterpret_cast<uint64_t>(segs[i].src[k]) - reinterpret_cast<uint64_t>(segs[i].dst[0])) % 16 != 0;
+        }
+    }
+    if (straddling && bytes >= kSmallFrom && bytes < kSmallUpto) return kWideSmall;
+    if (bytes / tile_bytes < ctx->wide_min_tiles) return kWideMany;
+    if (bytes >= kLargeFrom && (!straddling || esz >= 4)) {
+        *per_cu = 1;
+        return kWideLarge;
+    }
+    const uint64_t cus = static_cast<uint64_t>(ctx->num_cus);
+    const uint64_t three = 3 * ((tiles + 3 * cus - 1) / (3 * cus));
+    const uint64_t four = 4 * ((tiles + 4 * cus - 1) / (4 * cus));
+    *per_cu = three <= four ? 3 : 4;
+    return kWideOne;
+}
+
 // Wide segments: chain order, up to kMaxWideFan sources and destinations, one kernel for every fan-in.
 int build_wide_batches_impl(const hcclx_wide_seg_t *segs, uint32_t nseg, int dtype, int op, int mode,
                             Built *out)
@@ -1008,15 +1051,10 @@ int build_wide_batches_impl(const hcclx_wide_seg_t *segs, uint32_t nseg, int dty
     proto.maxn = kMaxWideFan;
     uint32_t max_dst = 0;
     for (uint32_t i = 0; i < nseg; ++i) max_dst = segs[i].ndst > max_dst ? segs[i].ndst : max_dst;
-    proto.wide_unroll = proto.mode != HCCLX_FOLD_CHAIN ? 1 : max_dst <= 1 ? kWideUnrollOne : kWideUnrollMany;
     const DeviceCtx *dctx = device_ctx();
-    if (proto.wide_unroll == kWideUnrollOne && dctx) {
-        uint64_t bytes = 0;
-        for (uint32_t i = 0; i < nseg; ++i) bytes += segs[i].count * static_cast<uint64_t>(esz);
-        if (bytes / (16 * wide_tile_vecs(kWideUnrollOne)) < dctx->wide_min_tiles) proto.wide_unroll = kWideUnrollMany;
-    }
+    if (proto.mode == HCCLX_FOLD_CHAIN && max_dst <= 1) proto.wide_shape = wide_shape_for(dctx, segs, nseg, esz, &proto.per_cu);
     proto.xcd_remap = (dctx && max_dst >= dctx->wide_xcd_remap_from) ? 1u : 0u;
-    uint64_t tile_vecs = wide_tile_vecs(proto.wide_unroll);
+    uint64_t tile_vecs = wide_tile_vecs(proto.wide_shape, proto.mode == HCCLX_FOLD_TREE);
     if (proto.mode == HCCLX_FOLD_SELF_FIRST) {
         proto.waves = max_src;
         uint64_t bytes = 0;
@@ -1112,6 +1150,7 @@ uint32_t uniform_tiles_of(const uint64_t *tile_end, size_t nseg)
     for (size_t i = 1; i < nseg; ++i) {
         if (tile_end[i] != tile_end[0] * (i + 1)) return 0;
     }
+    if (tile_end[nseg - 1] > 0xffffffffull) return 0;   // tile numbers are divided in 32 bits
     return static_cast<uint32_t>(tile_end[0]);
 }
 
@@ -1149,7 +1188,8 @@ int launch_batch(const DeviceCtx *ctx, const Batch &b, const char *d_table, hipS
     l.nseg = static_cast<uint32_t>(b.nseg());
     l.total_tiles = b.total_tiles;
     l.grid = grid_for(ctx, b.total_tiles);
-    l.wide_unroll = b.wide_unroll;
+    l.wide_shape = b.wide_shape;
+    l.per_cu = b.per_cu;
     l.xcd_remap = b.xcd_remap;
     l.store_policy = b.store_policy;
     l.uniform_tiles = uniform_tiles_of(b.tile_end.data(), b.tile_end.size());
@@ -1350,7 +1390,6 @@ int hcclx_fold_static(const hcclx_seg_t *segs, uint32_t nseg, int dtype, int op,
     l.nseg = live;
     l.total_tiles = total;
     l.grid = grid_for(ctx, total);
-    l.wide_unroll = 1;
     l.xcd_remap = 0;
     l.store_policy = store_policy_for(ctx, segs, nseg, sp.copy ? 1 : dtype_size(dtype));
     l.uniform_tiles = uniform_tiles_of(tile_end, live);

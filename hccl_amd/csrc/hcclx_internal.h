@@ -39,7 +39,7 @@ struct DeviceCtx {
     // (HCCLX_WIDE_XCD_REMAP_FROM).
     uint32_t wide_xcd_remap_from = 16;
     // A single-destination chain launch that would have fewer four-vector tiles than this takes two vectors per
-    // thread instead, to spread a small job over more CUs (HCCLX_WIDE_MIN_TILES; set from the CU count).
+    // thread and eight sources at a time, to spread a small job over more CUs (HCCLX_WIDE_MIN_TILES; set from the CU count).
     uint32_t wide_min_tiles = 0;
     bool a2av_direct = true;           // HCCLX_A2AV_DIRECT: AlltoAllV tables of up to 15 ranks in the kernel arguments (0 = off)
     // V kernels whose tables live on the device cannot know their tile count on the host and run as a

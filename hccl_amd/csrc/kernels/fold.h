@@ -26,13 +26,20 @@ namespace hcclx {
 #define HCCLX_FOLD_THREADS 256
 #endif
 constexpr int kFoldThreads = HCCLX_FOLD_THREADS;
-// The wide chain kernel loads eight sources at a time for U vectors per thread.  U = 2 measured 24 % faster on a
-// 32-rank AllReduce than one vector with sixteen sources (the same loads outstanding, twice the contiguous run per
-// source); with a single destination (the ReduceScatter shape) U = 4 measured another 3 to 5 % faster, while it
-// costs 5 % where every result is written to many places.
-constexpr int kWideGroup = 8;
-constexpr int kWideUnrollMany = 2;   // several destinations
-constexpr int kWideUnrollOne = 4;    // one destination
+// Shapes of the wide chain kernel: U vectors per thread, G sources loaded before the first of them is folded in, T threads.
+//   many   several destinations.  U = 2 measured 24 % faster on a 32-rank AllReduce than one vector with sixteen sources
+//          (the same loads outstanding, twice the contiguous run per source); U = 4 costs 5 %.
+//   small, one, large   a single destination.  One source at a time leaves room for more workgroups than G = 8 does (one: 62
+//          registers of bf16 against 174), and fewer of them than would fit read and write HBM faster: the workgroups of a CU
+//          then read for a while together and write together, where many small ones mix the two (LDS that nobody uses holds
+//          the others off).  ReduceScatter among 8 ranks, us, G = 8 and U = 4 : these shapes, same run: small 6 MiB odd 12.9 :
+//          12.4, 16 MiB odd 31.3 : 27.9; one 64 MiB 95.2 : 92.1, 72 MiB 107.7 : 100.8; large 500 MiB bf16 821 : 749, fp32 888 :
+//          782.  Which one: wide_shape_for.
+constexpr int kWideGroup = 8;        // pointers fetched together
+enum WideShape : int { kWideMany, kWideSmall, kWideOne, kWideLarge };
+__host__ __device__ constexpr int wide_vecs(int shape) { return shape == kWideOne ? 4 : shape == kWideLarge ? 8 : 2; }
+__host__ __device__ constexpr int wide_group(int shape) { return shape == kWideMany ? kWideGroup : 1; }
+__host__ __device__ constexpr int wide_threads(int shape) { return shape == kWideLarge ? 512 : kFoldThreads; }
 constexpr uint32_t kFoldDirectSegs = 64;   // up to this many segments the tile prefix is searched in place
 #ifndef HCCLX_TREE16_UNROLL
 #define HCCLX_TREE16_UNROLL 1   // vectors per thread of the tree over up to 16 leaf slots
@@ -49,11 +56,10 @@ __host__ __device__ constexpr uint64_t fold_tile_vecs(int maxn, int mode)
 {
     return static_cast<uint64_t>(kFoldThreads) * fold_unroll(maxn, mode);
 }
-// Tiles of the wide kernels: `unroll` vectors per thread (the chain: kWideUnrollMany or kWideUnrollOne; the
-// self-first and tree orders: 1).
-__host__ __device__ constexpr uint64_t wide_tile_vecs(int unroll)
+// Tiles of the wide kernels (trees: one vector per thread).
+__host__ __device__ constexpr uint64_t wide_tile_vecs(int shape, bool tree)
 {
-    return static_cast<uint64_t>(kFoldThreads) * unroll;
+    return tree ? static_cast<uint64_t>(kFoldThreads) : static_cast<uint64_t>(wide_threads(shape)) * wide_vecs(shape);
 }
 
 #ifndef HCCLX_NT_LOAD
@@ -320,9 +326,10 @@ __device__ __forceinline__ void locate_tile(const uint64_t *__restrict__ tile_en
     if (uniform_tiles != 0) {
         // every segment has this many tiles (the slices of a two-shot, ring or NHR AllReduce): no table to search.
         // A search is a chain of dependent loads, which a launch of a few hundred workgroups cannot hide.
-        const uint64_t s = t / uniform_tiles;
-        *seg = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(s));
-        *tile_in_seg = uniform64(t - s * uniform_tiles);
+        const uint32_t t32 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(t));
+        const uint32_t s = __builtin_amdgcn_readfirstlane(t32 / uniform_tiles);
+        *seg = s;
+        *tile_in_seg = t32 - s * uniform_tiles;
         return;
     }
     uint32_t lo = 0;
@@ -738,55 +745,66 @@ k_fold_waves(const uint64_t *__restrict__ tile_end, const SegDev *__restrict__ s
     }
 }
 
-// More than kMaxFan sources or destinations, chain order: the sources are walked in groups of kMaxFan,
-// each group loaded before it is folded in, so the loads in flight per thread stay what the 16-source kernel
-// has.  One vector per thread and tile.
-template <int DT, int OP, int U, bool CHECK>
+// More than kMaxFan sources or destinations, or one destination, chain order: the sources are walked in groups of G, each
+// group loaded before it is folded in; the pointers of kWideGroup sources are fetched together, ahead of their loads.
+template <int DT, int OP, int U, int G, int T, bool CHECK>
 __device__ __forceinline__ void fold_tile_wide(const SegWide &sd, uint32_t nsrc, uint32_t ndst, uint64_t v0, uint64_t nvec,
                                                uint32_t head_bytes, uint32_t policy)
 {
     using V = Vec16<DT>;
     using C = typename V::C;
     constexpr int NE = V::NE;
-    constexpr int G = kWideGroup;
     bool ok[U];
     uint64_t off[U];
     C acc[U][NE];
+    const char *from[kWideGroup];
+#pragma unroll
+    for (int k = 0; k < kWideGroup; ++k) from[k] = sd.src[static_cast<uint32_t>(k) < nsrc ? k : 0];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-        const uint64_t v = v0 + static_cast<uint64_t>(u) * kFoldThreads;
+        const uint64_t v = v0 + static_cast<uint64_t>(u) * T;
         // A lane outside the segment loads the segment's first vector and stores nothing: the loads stay
         // unconditional, so all of a group are in flight at once as in the unchecked tile.
         ok[u] = !CHECK || v < nvec;
         off[u] = head_bytes + (ok[u] ? v : 0) * 16;
-        V::unpack(ld16(sd.src[0] + off[u]), acc[u]);
+        V::unpack(ld16(from[0] + off[u]), acc[u]);
     }
     const uint64_t flips = sd.leaf_mask;
-    for (uint32_t base = 1; base < nsrc; base += G) {
-        u32x4 raw[U][G];
+    for (uint32_t base = 0; base < nsrc; base += kWideGroup) {
+        if (base != 0) {
 #pragma unroll
-        for (int k = 0; k < G; ++k) {
-            if (base + k < nsrc) {
-#pragma unroll
-                for (int u = 0; u < U; ++u) raw[u][k] = ld16(sd.src[base + k] + off[u]);
-            }
+            for (int k = 0; k < kWideGroup; ++k) from[k] = sd.src[base + k < nsrc ? base + k : 0];
         }
 #pragma unroll
-        for (int k = 0; k < G; ++k) {
-            if (base + k < nsrc) {
+        for (int k0 = 0; k0 < kWideGroup; k0 += G) {
+            u32x4 raw[U][G];
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    C x[NE];
-                    V::unpack(raw[u][k], x);
-                    if (OperandOrderMatters<DT, OP>::value && ((flips >> (base + k)) & 1u)) {
+            for (int g = 0; g < G; ++g) {
+                const uint32_t k = base + k0 + g;
+                if (k != 0 && k < nsrc) {
 #pragma unroll
-                        for (int e = 0; e < NE; ++e) acc[u][e] = V::template combine<OP>(acc[u][e], x[e]);
-                    } else {
+                    for (int u = 0; u < U; ++u) raw[u][g] = ld16(from[k0 + g] + off[u]);
+                }
+            }
 #pragma unroll
-                        for (int e = 0; e < NE; ++e) acc[u][e] = V::template combine<OP>(x[e], acc[u][e]);
+            for (int g = 0; g < G; ++g) {
+                const uint32_t k = base + k0 + g;
+                if (k != 0 && k < nsrc) {
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        C x[NE];
+                        V::unpack(raw[u][g], x);
+                        if (OperandOrderMatters<DT, OP>::value && ((flips >> k) & 1u)) {
+#pragma unroll
+                            for (int e = 0; e < NE; ++e) acc[u][e] = V::template combine<OP>(acc[u][e], x[e]);
+                        } else {
+#pragma unroll
+                            for (int e = 0; e < NE; ++e) acc[u][e] = V::template combine<OP>(x[e], acc[u][e]);
+                        }
                     }
                 }
             }
+            if (G < kWideGroup) asm volatile("" ::: "memory");   // one step's loads at a time
         }
     }
     for (uint32_t base = 0; base < ndst; base += kMaxFan) {
@@ -1017,20 +1035,23 @@ k_fold_wide_waves(const uint64_t *__restrict__ tile_end, const SegWide *__restri
     }
 }
 
-template <int DT, int OP, int MODE, int U>
-__global__ void __launch_bounds__(kFoldThreads)
+template <int DT, int OP, int MODE, int SHAPE>
+__global__ void __launch_bounds__(wide_threads(SHAPE))
 k_fold_wide(const uint64_t *__restrict__ tile_end, const SegWide *__restrict__ segs, uint32_t nseg, uint64_t total_tiles,
             uint32_t xcd_remap, uint32_t store_policy, uint32_t uniform_tiles)
 {
     constexpr int NE = Vec16<DT>::kElems;
     const uint32_t policy = store_policy;
-    static_assert(MODE == kFoldChain || (MODE == kFoldTree && U == 1), "the self-first order has a kernel of its own; only the chain "
-                                                                        "moves several vectors per thread");
-    constexpr uint64_t TV = wide_tile_vecs(U);
+    static_assert(MODE == kFoldChain || (MODE == kFoldTree && SHAPE == kWideMany), "the self-first order has a kernel of its own; only "
+                                                                                   "chains come in several shapes");
+    constexpr int U = wide_vecs(SHAPE);
+    constexpr int G = wide_group(SHAPE);
+    constexpr int T = wide_threads(SHAPE);
+    constexpr uint64_t TV = wide_tile_vecs(SHAPE, MODE == kFoldTree);
     extern __shared__ uint64_t s_end[];
     const bool direct = nseg <= kFoldDirectSegs || uniform_tiles != 0;
     if (!direct) {
-        for (uint32_t i = threadIdx.x; i < nseg; i += kFoldThreads) {
+        for (uint32_t i = threadIdx.x; i < nseg; i += T) {
             s_end[i] = tile_end[i];
         }
         __syncthreads();
@@ -1053,13 +1074,13 @@ k_fold_wide(const uint64_t *__restrict__ tile_end, const SegWide *__restrict__ s
             if constexpr (MODE == kFoldTree) {
                 fold_tile_wide_tree<DT, OP, false>(sd, ndst, v, nvec, head_bytes, policy);
             } else {
-                fold_tile_wide<DT, OP, U, false>(sd, nsrc, ndst, v, nvec, head_bytes, policy);
+                fold_tile_wide<DT, OP, U, G, T, false>(sd, nsrc, ndst, v, nvec, head_bytes, policy);
             }
         } else {
             if constexpr (MODE == kFoldTree) {
                 fold_tile_wide_tree<DT, OP, true>(sd, ndst, v, nvec, head_bytes, policy);
             } else {
-                if (nvec != 0) fold_tile_wide<DT, OP, U, true>(sd, nsrc, ndst, v, nvec, head_bytes, policy);
+                if (nvec != 0) fold_tile_wide<DT, OP, U, G, T, true>(sd, nsrc, ndst, v, nvec, head_bytes, policy);
             }
             if (tl == (nvec + shift) / TV && threadIdx.x < head + rem) {
                 const uint64_t idx = threadIdx.x < head ? threadIdx.x : head + nvec * NE + (threadIdx.x - head);
@@ -1068,6 +1089,10 @@ k_fold_wide(const uint64_t *__restrict__ tile_end, const SegWide *__restrict__ s
         }
     }
 }
+
+// LDS of a CU, and the bytes that a workgroup asks for so that no more than `per_cu` of them share one.
+constexpr uint32_t kLdsPerCu = 160u * 1024;
+inline uint32_t lds_for(uint32_t per_cu) { return per_cu == 0 ? 0 : kLdsPerCu / per_cu * (per_cu == 1 ? 9 : 15) / 16 & ~1023u; }
 
 // Host-side geometry, used by the launcher to build tile_end[].
 // Elements of a segment in front of the first 16-byte boundary of its first destination.
@@ -1108,7 +1133,8 @@ struct FoldLaunch {
     uint32_t nseg;
     uint64_t total_tiles;
     uint32_t grid;
-    int wide_unroll;           // the wide chain kernel: vectors per thread (kWideUnrollMany or kWideUnrollOne)
+    int wide_shape = 0;        // the wide chain kernel: a WideShape
+    uint32_t per_cu = 0;       // non-zero: no more workgroups of the launch than this share a CU
     uint32_t xcd_remap;        // the wide kernels: give each XCD a contiguous eighth of the tiles
     uint32_t store_policy;     // kStoreStream / kStoreThrough
     uint32_t uniform_tiles;    // non-zero: every segment has this many tiles, tile t belongs to segment t / uniform_tiles

@@ -5,6 +5,8 @@
 // With -DHCCLX_COPY the unit holds the byte copy kernel instead (one source, many destinations).
 #include "fold.h"
 
+#include <algorithm>
+
 namespace hcclx {
 
 template <int DT, int OP, int MAXN, int MODE>
@@ -57,10 +59,16 @@ static hipError_t launch_waves(const FoldLaunch &l)
     }
 }
 
-template <int DT, int OP, int MODE, int U>
-static hipError_t launch_wide_u(const FoldLaunch &l)
+template <int DT, int OP, int MODE, int SHAPE>
+static hipError_t launch_wide_shape(const FoldLaunch &l)
 {
-    HCCLX_LAUNCH((k_fold_wide<DT, OP, MODE, U>), dim3(l.grid), dim3(kFoldThreads), l.nseg * sizeof(uint64_t), l.stream,
+    const size_t lds = std::max<size_t>(l.nseg * sizeof(uint64_t), lds_for(l.per_cu));
+    if (lds > 64 * 1024) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_fold_wide<DT, OP, MODE, SHAPE>),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
+        if (e != hipSuccess) return e;
+    }
+    HCCLX_LAUNCH((k_fold_wide<DT, OP, MODE, SHAPE>), dim3(l.grid), dim3(wide_threads(SHAPE)), lds, l.stream,
                        l.tile_end, static_cast<const SegWide *>(l.segs), l.nseg, l.total_tiles, l.xcd_remap, l.store_policy, l.uniform_tiles);
     return hipGetLastError();
 }
@@ -85,10 +93,14 @@ template <int DT, int OP, int MODE>
 static hipError_t launch_wide(const FoldLaunch &l)
 {
     if constexpr (MODE == kFoldChain) {
-        return l.wide_unroll == kWideUnrollOne ? launch_wide_u<DT, OP, MODE, kWideUnrollOne>(l)
-                                               : launch_wide_u<DT, OP, MODE, kWideUnrollMany>(l);
+        switch (l.wide_shape) {
+            case kWideSmall: return launch_wide_shape<DT, OP, MODE, kWideSmall>(l);
+            case kWideOne: return launch_wide_shape<DT, OP, MODE, kWideOne>(l);
+            case kWideLarge: return launch_wide_shape<DT, OP, MODE, kWideLarge>(l);
+            default: return launch_wide_shape<DT, OP, MODE, kWideMany>(l);
+        }
     } else if constexpr (MODE == kFoldTree) {
-        return launch_wide_u<DT, OP, MODE, 1>(l);
+        return launch_wide_shape<DT, OP, MODE, kWideMany>(l);
     } else {
         switch ((l.waves + kWideWaves - 1) / kWideWaves) {
             case 1: return launch_wide_waves<DT, OP, 1>(l);
