@@ -422,7 +422,7 @@ struct Batch {
     std::vector<uint64_t> tile_end;
     std::vector<SegDev> segs;
     std::vector<SegWide> wide;   // instead of segs when maxn == kMaxWideFan
-    int wide_shape = kWideMany;  // of the wide chain kernel (fold.h)
+    int wide_shape = 0;          // of the wide kernels: a WideShape or a TreeShape (fold.h)
     uint32_t per_cu = 0;         // non-zero: so many workgroups of the launch to a CU at most
     uint32_t xcd_remap = 0;      // wide kernels: contiguous tile ranges per XCD (pays with 16 or more destinations)
     BlockLaunch blocks;          // instead of everything above: a launch of the block copy kernel
@@ -907,6 +907,17 @@ int build_batches_impl(const hcclx_seg_t *segs, uint32_t nseg, int dtype, int op
         proto.waves_team = waves_team;
     }
     proto.store_policy = store_policy_for(device_ctx(), segs, nseg, sp.copy ? 1 : dtype_size(dtype));
+    // Trees over more than eight leaf slots to one place: from 64 MiB on four workgroups to a CU, as the chains (fold.h; fp32
+    // NHR AllReduce 12 x 64 MiB 256 : 252 us, ReduceScatter 16 x 64 191 : 186; 12 x 8 MiB 39.6 : 40.7)
+    if (sp.mode == HCCLX_FOLD_TREE && sp.maxn > 8) {
+        uint64_t bytes = 0;
+        bool one = true;
+        for (uint32_t i = 0; i < nseg; ++i) {
+            bytes += segs[i].count * static_cast<uint64_t>(sp.esz);
+            one = one && segs[i].ndst == 1;
+        }
+        if (one && bytes >= (64ull << 20)) proto.per_cu = 4;
+    }
     Batch cur = proto;
     for (uint32_t i = 0; i < nseg; ++i) {
         const hcclx_seg_t &s = segs[i];
@@ -967,7 +978,7 @@ int wide_shape_for(const DeviceCtx *ctx, const hcclx_wide_seg_t *segs, uint32_t 
     constexpr uint64_t kSmallUpto = 32ull << 20;
     *per_cu = 0;
     if (ctx == nullptr) return kWideMany;
-    const uint64_t tile_bytes = 16 * wide_tile_vecs(kWideOne, false);
+    const uint64_t tile_bytes = 16 * wide_tile_vecs(kWideOne);
     uint64_t bytes = 0;
     uint64_t tiles = 0;
     bool straddling = false;
@@ -1054,7 +1065,14 @@ int build_wide_batches_impl(const hcclx_wide_seg_t *segs, uint32_t nseg, int dty
     const DeviceCtx *dctx = device_ctx();
     if (proto.mode == HCCLX_FOLD_CHAIN && max_dst <= 1) proto.wide_shape = wide_shape_for(dctx, segs, nseg, esz, &proto.per_cu);
     proto.xcd_remap = (dctx && max_dst >= dctx->wide_xcd_remap_from) ? 1u : 0u;
-    uint64_t tile_vecs = wide_tile_vecs(proto.wide_shape, proto.mode == HCCLX_FOLD_TREE);
+    uint64_t tile_vecs = wide_tile_vecs(proto.wide_shape);
+    if (proto.mode == HCCLX_FOLD_TREE) {
+        const bool half = dtype == HCCL_DATA_TYPE_FP16 || dtype == HCCL_DATA_TYPE_BFP16;
+        uint64_t bytes = 0;
+        for (uint32_t i = 0; i < nseg; ++i) bytes += segs[i].count * static_cast<uint64_t>(esz);
+        proto.wide_shape = (half ? max_src > 32 : bytes >= kTreeLargeFrom) ? kTreeLarge : kTreePlain;
+        tile_vecs = tree_threads(proto.wide_shape, half);
+    }
     if (proto.mode == HCCLX_FOLD_SELF_FIRST) {
         proto.waves = max_src;
         uint64_t bytes = 0;

@@ -39,6 +39,15 @@ constexpr int kWideGroup = 8;        // pointers fetched together
 enum WideShape : int { kWideMany, kWideSmall, kWideOne, kWideLarge };
 __host__ __device__ constexpr int wide_vecs(int shape) { return shape == kWideOne ? 4 : shape == kWideLarge ? 8 : 2; }
 __host__ __device__ constexpr int wide_group(int shape) { return shape == kWideMany ? kWideGroup : 1; }
+// Shapes of the wide tree kernel (one vector per thread):
+//   plain   256 threads
+//   large   the 16-bit floats: two elements of every vector at a time, which holds 161 registers instead of 193 (three wavefronts
+//           to a SIMD); taken above 32 leaves (AllReduce NHR in us, plain : large: ReduceScatter 64 ranks x 30 MiB bf16 541 : 436,
+//           but 24 x 40 400 : 422).  The others: 512 threads, twice the contiguous run per source; from kTreeLargeFrom bytes of results on (fp32 32
+//           x 16 MiB 178 : 174, 64 x 16 356 : 347, ReduceScatter 32 x 64 366 : 355, but 24 x 10 90.0 : 91.7, 32 x 512 KiB 16.5 : 18.3).
+enum TreeShape : int { kTreePlain, kTreeLarge };
+constexpr uint64_t kTreeLargeFrom = 16ull << 20;
+__host__ __device__ constexpr int tree_threads(int shape, bool half_float) { return shape == kTreeLarge && !half_float ? 512 : kFoldThreads; }
 __host__ __device__ constexpr int wide_threads(int shape) { return shape == kWideLarge ? 512 : kFoldThreads; }
 constexpr uint32_t kFoldDirectSegs = 64;   // up to this many segments the tile prefix is searched in place
 #ifndef HCCLX_TREE16_UNROLL
@@ -56,10 +65,10 @@ __host__ __device__ constexpr uint64_t fold_tile_vecs(int maxn, int mode)
 {
     return static_cast<uint64_t>(kFoldThreads) * fold_unroll(maxn, mode);
 }
-// Tiles of the wide kernels (trees: one vector per thread).
-__host__ __device__ constexpr uint64_t wide_tile_vecs(int shape, bool tree)
+// Tiles of the wide chain kernel.
+__host__ __device__ constexpr uint64_t wide_tile_vecs(int shape)
 {
-    return tree ? static_cast<uint64_t>(kFoldThreads) : static_cast<uint64_t>(wide_threads(shape)) * wide_vecs(shape);
+    return static_cast<uint64_t>(wide_threads(shape)) * wide_vecs(shape);
 }
 
 #ifndef HCCLX_NT_LOAD
@@ -332,9 +341,10 @@ __device__ __forceinline__ void locate_tile(const uint64_t *__restrict__ tile_en
         *tile_in_seg = t32 - s * uniform_tiles;
         return;
     }
+    // (each search ends in its own load of the prefix: one load for both would be a FLAT one)
     uint32_t lo = 0;
     uint32_t hi = nseg - 1;
-    uint64_t before = 0;   // tiles of the segments in front of the one found
+    *tile_in_seg = t;
     if (direct) {
         while (lo < hi) {
             const uint32_t mid = (lo + hi) >> 1;
@@ -344,7 +354,7 @@ __device__ __forceinline__ void locate_tile(const uint64_t *__restrict__ tile_en
                 lo = mid + 1;
             }
         }
-        before = lo ? tile_end[lo - 1] : 0;
+        if (lo != 0) *tile_in_seg = uniform64(t - tile_end[lo - 1]);
     } else {
         while (lo < hi) {
             const uint32_t mid = (lo + hi) >> 1;
@@ -354,10 +364,9 @@ __device__ __forceinline__ void locate_tile(const uint64_t *__restrict__ tile_en
                 lo = mid + 1;
             }
         }
-        before = lo ? s_end[lo - 1] : 0;
+        if (lo != 0) *tile_in_seg = uniform64(t - s_end[lo - 1]);
     }
     *seg = __builtin_amdgcn_readfirstlane(lo);
-    *tile_in_seg = uniform64(t - before);
 }
 
 template <int DT, int OP, int MAXN, int MODE>
@@ -822,7 +831,7 @@ __device__ __forceinline__ void fold_tile_wide(const SegWide &sd, uint32_t nsrc,
 
 // The value of the subtree over leaf slots G * kMaxFan .. G * kMaxFan + kMaxFan - 1 (heap node
 // kMaxWideFan / kMaxFan + G); nothing is loaded and `out` is left alone when no leaf of it is present.
-template <int DT, int OP, int G>
+template <int DT, int OP, int G, bool PAIRS>
 __device__ __forceinline__ void wide_subtree(const SegWide &sd, uint64_t off, uint64_t mask,
                                              typename Vec16<DT>::C (&out)[Vec16<DT>::NE])
 {
@@ -833,26 +842,56 @@ __device__ __forceinline__ void wide_subtree(const SegWide &sd, uint64_t off, ui
     if (present == 0) {
         return;
     }
+    // The sixteen pointers in one batch: fetched behind the test of their slot, each would be a round trip of its own.  (The
+    // empty asm statements keep the compiler from moving them there.)
+    const char *src[kMaxFan];
+#pragma unroll
+    for (int k = 0; k < kMaxFan; ++k) src[k] = sd.src[G * kMaxFan + k];
+#pragma unroll
+    for (int k = 0; k < kMaxFan; k += 8) {
+        asm volatile("" : "+s"(src[k]), "+s"(src[k + 1]), "+s"(src[k + 2]), "+s"(src[k + 3]), "+s"(src[k + 4]), "+s"(src[k + 5]),
+                     "+s"(src[k + 6]), "+s"(src[k + 7]));
+    }
     u32x4 raw[kMaxFan];
 #pragma unroll
     for (int k = 0; k < kMaxFan; ++k) {
-        if ((present >> k) & 1u) raw[k] = ld16(sd.src[G * kMaxFan + k] + off);
+        if ((present >> k) & 1u) raw[k] = ld16(src[k] + off);
     }
-    C val[kMaxFan][NE];
+    auto code = [&sd](int node) { return (sd.tree_codes[node / 16] >> (2 * (node % 16))) & 3u; };
+    constexpr int kRoot = kMaxWideFan / kMaxFan + G;
+    if constexpr (PAIRS) {
+        using S = typename V::S;
+        static_assert(sizeof(S) == 2 && NE == 8, "two elements in each of four registers");
 #pragma unroll
-    for (int k = 0; k < kMaxFan; ++k) {
-        if ((present >> k) & 1u) V::unpack(raw[k], val[k]);
+        for (int q = 0; q < 4; ++q) {
+            C val[kMaxFan][2];
+#pragma unroll
+            for (int k = 0; k < kMaxFan; ++k) {
+                if ((present >> k) & 1u) {
+                    val[k][0] = V::D::widen(static_cast<S>(raw[k][q] & 0xffffu));
+                    val[k][1] = V::D::widen(static_cast<S>(raw[k][q] >> 16));
+                }
+            }
+            tree_eval_at<DT, OP, kMaxFan, kRoot, C, 2>(val, code);
+            out[2 * q] = val[0][0];
+            out[2 * q + 1] = val[0][1];
+        }
+    } else {
+        C val[kMaxFan][NE];
+#pragma unroll
+        for (int k = 0; k < kMaxFan; ++k) {
+            if ((present >> k) & 1u) V::unpack(raw[k], val[k]);
+        }
+        tree_eval_at<DT, OP, kMaxFan, kRoot, C, NE>(val, code);
+#pragma unroll
+        for (int e = 0; e < NE; ++e) out[e] = val[0][e];
     }
-    tree_eval_at<DT, OP, kMaxFan, kMaxWideFan / kMaxFan + G, C, NE>(
-        val, [&sd](int node) { return (sd.tree_codes[node / 16] >> (2 * (node % 16))) & 3u; });
-#pragma unroll
-    for (int e = 0; e < NE; ++e) out[e] = val[0][e];
 }
 
 // A tree over up to kMaxWideFan leaf slots: the four subtrees of kMaxFan slots below heap nodes 4 .. 7 are
 // evaluated one after the other, each with its leaves loaded first as in the 16-slot kernel, and their values go
 // through the two top levels.
-template <int DT, int OP, bool CHECK>
+template <int DT, int OP, bool PAIRS, bool CHECK>
 __device__ __forceinline__ void fold_tile_wide_tree(const SegWide &sd, uint32_t ndst, uint64_t v, uint64_t nvec,
                                                     uint32_t head_bytes, uint32_t policy)
 {
@@ -867,10 +906,10 @@ __device__ __forceinline__ void fold_tile_wide_tree(const SegWide &sd, uint32_t 
     const uint64_t mask = sd.leaf_mask;
     auto code = [&sd](int node) { return (sd.tree_codes[node / 16] >> (2 * (node % 16))) & 3u; };
     C part[kGroups][NE];
-    wide_subtree<DT, OP, 0>(sd, off, mask, part[0]);
-    wide_subtree<DT, OP, 1>(sd, off, mask, part[1]);
-    wide_subtree<DT, OP, 2>(sd, off, mask, part[2]);
-    wide_subtree<DT, OP, 3>(sd, off, mask, part[3]);
+    wide_subtree<DT, OP, 0, PAIRS>(sd, off, mask, part[0]);
+    wide_subtree<DT, OP, 1, PAIRS>(sd, off, mask, part[1]);
+    wide_subtree<DT, OP, 2, PAIRS>(sd, off, mask, part[2]);
+    wide_subtree<DT, OP, 3, PAIRS>(sd, off, mask, part[3]);
     static_assert(kMaxFan == 16 && kGroups == 4, "the subtree roots above are heap nodes 4 .. 7");
     tree_eval_at<DT, OP, kGroups, 1, C, NE>(part, code);
     const u32x4 out = V::pack(part[0]);
@@ -1036,18 +1075,20 @@ k_fold_wide_waves(const uint64_t *__restrict__ tile_end, const SegWide *__restri
 }
 
 template <int DT, int OP, int MODE, int SHAPE>
-__global__ void __launch_bounds__(wide_threads(SHAPE))
+__global__ void __launch_bounds__(MODE == kFoldTree ? tree_threads(SHAPE, DTypeOf<DT>::kHalfFloat) : wide_threads(SHAPE))
 k_fold_wide(const uint64_t *__restrict__ tile_end, const SegWide *__restrict__ segs, uint32_t nseg, uint64_t total_tiles,
             uint32_t xcd_remap, uint32_t store_policy, uint32_t uniform_tiles)
 {
     constexpr int NE = Vec16<DT>::kElems;
     const uint32_t policy = store_policy;
-    static_assert(MODE == kFoldChain || (MODE == kFoldTree && SHAPE == kWideMany), "the self-first order has a kernel of its own; only "
-                                                                                   "chains come in several shapes");
-    constexpr int U = wide_vecs(SHAPE);
+    static_assert(MODE == kFoldChain || MODE == kFoldTree, "the self-first order has a kernel of its own");
+    // SHAPE: a WideShape or a TreeShape
+    constexpr bool kTree = MODE == kFoldTree;
+    constexpr int U = kTree ? 1 : wide_vecs(SHAPE);
     constexpr int G = wide_group(SHAPE);
-    constexpr int T = wide_threads(SHAPE);
-    constexpr uint64_t TV = wide_tile_vecs(SHAPE, MODE == kFoldTree);
+    constexpr int T = kTree ? tree_threads(SHAPE, DTypeOf<DT>::kHalfFloat) : wide_threads(SHAPE);
+    constexpr bool kPairs = kTree && SHAPE == kTreeLarge && DTypeOf<DT>::kHalfFloat;
+    constexpr uint64_t TV = static_cast<uint64_t>(T) * U;
     extern __shared__ uint64_t s_end[];
     const bool direct = nseg <= kFoldDirectSegs || uniform_tiles != 0;
     if (!direct) {
@@ -1072,13 +1113,13 @@ k_fold_wide(const uint64_t *__restrict__ tile_end, const SegWide *__restrict__ s
         const uint64_t v = tl * TV + threadIdx.x - shift;   // wraps in front of a shifted segment: fails the check
         if (tl * TV >= shift && (tl + 1) * TV - shift <= nvec) {
             if constexpr (MODE == kFoldTree) {
-                fold_tile_wide_tree<DT, OP, false>(sd, ndst, v, nvec, head_bytes, policy);
+                fold_tile_wide_tree<DT, OP, kPairs, false>(sd, ndst, v, nvec, head_bytes, policy);
             } else {
                 fold_tile_wide<DT, OP, U, G, T, false>(sd, nsrc, ndst, v, nvec, head_bytes, policy);
             }
         } else {
             if constexpr (MODE == kFoldTree) {
-                fold_tile_wide_tree<DT, OP, true>(sd, ndst, v, nvec, head_bytes, policy);
+                fold_tile_wide_tree<DT, OP, kPairs, true>(sd, ndst, v, nvec, head_bytes, policy);
             } else {
                 if (nvec != 0) fold_tile_wide<DT, OP, U, G, T, true>(sd, nsrc, ndst, v, nvec, head_bytes, policy);
             }
@@ -1133,7 +1174,7 @@ struct FoldLaunch {
     uint32_t nseg;
     uint64_t total_tiles;
     uint32_t grid;
-    int wide_shape = 0;        // the wide chain kernel: a WideShape
+    int wide_shape = 0;        // the wide kernels: a WideShape or a TreeShape
     uint32_t per_cu = 0;       // non-zero: no more workgroups of the launch than this share a CU
     uint32_t xcd_remap;        // the wide kernels: give each XCD a contiguous eighth of the tiles
     uint32_t store_policy;     // kStoreStream / kStoreThrough

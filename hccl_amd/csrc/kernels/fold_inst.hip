@@ -12,7 +12,8 @@ namespace hcclx {
 template <int DT, int OP, int MAXN, int MODE>
 static hipError_t launch_one(const FoldLaunch &l)
 {
-    HCCLX_LAUNCH((k_fold<DT, OP, MAXN, MODE>), dim3(l.grid), dim3(kFoldThreads), l.nseg * sizeof(uint64_t), l.stream,
+    const size_t lds = std::max<size_t>(l.nseg * sizeof(uint64_t), lds_for(l.per_cu));
+    HCCLX_LAUNCH((k_fold<DT, OP, MAXN, MODE>), dim3(l.grid), dim3(kFoldThreads), lds, l.stream,
                        l.tile_end, static_cast<const SegDev *>(l.segs), l.nseg, l.total_tiles, l.store_policy, l.uniform_tiles);
     return hipGetLastError();
 }
@@ -62,13 +63,14 @@ static hipError_t launch_waves(const FoldLaunch &l)
 template <int DT, int OP, int MODE, int SHAPE>
 static hipError_t launch_wide_shape(const FoldLaunch &l)
 {
+    constexpr int kThreads = MODE == kFoldTree ? tree_threads(SHAPE, DTypeOf<DT>::kHalfFloat) : wide_threads(SHAPE);
     const size_t lds = std::max<size_t>(l.nseg * sizeof(uint64_t), lds_for(l.per_cu));
     if (lds > 64 * 1024) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_fold_wide<DT, OP, MODE, SHAPE>),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
         if (e != hipSuccess) return e;
     }
-    HCCLX_LAUNCH((k_fold_wide<DT, OP, MODE, SHAPE>), dim3(l.grid), dim3(wide_threads(SHAPE)), lds, l.stream,
+    HCCLX_LAUNCH((k_fold_wide<DT, OP, MODE, SHAPE>), dim3(l.grid), dim3(kThreads), lds, l.stream,
                        l.tile_end, static_cast<const SegWide *>(l.segs), l.nseg, l.total_tiles, l.xcd_remap, l.store_policy, l.uniform_tiles);
     return hipGetLastError();
 }
@@ -100,7 +102,7 @@ static hipError_t launch_wide(const FoldLaunch &l)
             default: return launch_wide_shape<DT, OP, MODE, kWideMany>(l);
         }
     } else if constexpr (MODE == kFoldTree) {
-        return launch_wide_shape<DT, OP, MODE, kWideMany>(l);
+        return l.wide_shape == kTreeLarge ? launch_wide_shape<DT, OP, MODE, kTreeLarge>(l) : launch_wide_shape<DT, OP, MODE, kTreePlain>(l);
     } else {
         switch ((l.waves + kWideWaves - 1) / kWideWaves) {
             case 1: return launch_wide_waves<DT, OP, 1>(l);

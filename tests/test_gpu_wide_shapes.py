@@ -64,3 +64,57 @@ def test_chain_to_one_destination(nsrc, mib, straddle, dtype, op):
         got, want = (torch.where(v.isnan(), torch.zeros_like(v), v).view(torch.int32) for v in (got, want))
     assert torch.equal(got, want)
     assert bool((out[at:] == 77).all())
+
+
+def nhr_like_tree(n):
+    """The steps (dst, src) of a tree over n registers in which each round halves what is left: ceil(log2 n) levels."""
+    steps, left = [], list(range(n))
+    while len(left) > 1:
+        half = (len(left) + 1) // 2
+        steps += [(left[k], left[half + k]) for k in range(len(left) - half)]
+        left = left[:half]
+    return steps
+
+
+@pytest.mark.parametrize("dtype,nsrc,mib", [(T.FP32, 17, 16), (T.FP32, 33, 15), (T.FP64, 20, 17), (T.BFP16, 32, 4), (T.BFP16, 33, 4),
+                                            (T.FP16, 64, 1)])
+def test_wide_tree_shapes(dtype, nsrc, mib):
+    """Both shapes of the wide tree kernel (by size; the 16-bit floats by their number of leaves): partial tiles at both ends of
+    unequal segments, against the same tree in torch."""
+    esz = T.DTYPE_SIZE[dtype]
+    whole = mib * MIB // esz
+    edge = 512 * 16 // esz                    # elements of the larger tile
+    lengths = [edge - 1, whole, edge + 1, 3]
+    xs = [device_payload(dtype, sum(lengths) + 8, 100 * k + mib) for k in range(nsrc)]
+    out = torch.full((sum(lengths) + 8,), 77, device="cuda:0", dtype=TORCH_STORAGE[dtype])
+    torch.cuda.synchronize()
+    steps = nhr_like_tree(nsrc)
+    prog = [r for st in steps for r in st]
+    segs, at = [], 1
+    for n in lengths:
+        segs.append((n, [x.data_ptr() + at * esz for x in xs], [out.data_ptr() + at * esz], prog))
+        at += n
+    hcclx.fold_wide(segs, dtype, T.SUM, hcclx.FOLD_TREE)
+    torch.cuda.synchronize()
+    val = [x.float() if esz == 2 else x.clone() for x in xs]
+    for d, s in steps:
+        val[d] = val[s] + val[d]
+    want = val[0].to(TORCH_STORAGE[dtype])
+    bits = {2: torch.int16, 4: torch.int32, 8: torch.int64}[esz]
+    assert torch.equal(out[1:at].view(bits), want[1:at].view(bits))
+    assert bool((out[at:] == 77).all()) and bool((out[:1] == 77).all())
+
+
+@pytest.mark.parametrize("nsrc,mib", [(12, 64), (16, 63)])
+def test_tree_to_one_destination_with_fewer_workgroups(nsrc, mib):
+    """Trees over more than eight slots: from 64 MiB on fewer workgroups share a CU, the tiles are the same."""
+    n = mib * MIB // 4 + 5
+    xs = [device_payload(T.FP32, n, k) for k in range(nsrc)]
+    out = torch.zeros(n, device="cuda:0")
+    torch.cuda.synchronize()
+    steps = nhr_like_tree(nsrc)
+    hcclx.fold([(n, [x.data_ptr() for x in xs], [out.data_ptr()], [r for st in steps for r in st])], T.FP32, T.SUM, hcclx.FOLD_TREE)
+    torch.cuda.synchronize()
+    for d, s in steps:
+        xs[d] = xs[s] + xs[d]
+    assert torch.equal(out.view(torch.int32), xs[0].view(torch.int32))
