@@ -137,6 +137,23 @@ def native_call(name):
     return _calls.Call(ctypes.cast(fn, ctypes.c_void_p).value, kinds, ctypes.Array)
 
 
+COMM = 255   # native_method: the communicator's place
+
+
+def table(place):
+    """native_method: an argument that has to be a ctypes array for the native call."""
+    return place + 64
+
+
+def native_method(call, function, places):
+    """The method `function` of a class with a list `comms` of communicators, in native code (csrc/python_calls.cc): `call`
+    gets the method's arguments at `places` (the object is 0, the rank 1); what it does not take goes to `function`.  None
+    where the module was not built."""
+    if _calls is None or not isinstance(call, _calls.Call):
+        return None
+    return _calls.Method(call, function, bytes(places), function.__code__.co_argcount)
+
+
 class HcclError(RuntimeError):
     def __init__(self, code, text):
         super().__init__(f"HcclResult {code}: {text}")

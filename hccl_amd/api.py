@@ -71,6 +71,19 @@ def lib():
         _all_reduce, _reduce_scatter, _reduce_scatter_v, _all_gather, _all_gather_v, _all_to_all_v, _all_to_all, _all_to_all_vc = (
             _lib.native_call(name) for name in ("HcclAllReduce", "HcclReduceScatter", "HcclReduceScatterV", "HcclAllGather",
                                                 "HcclAllGatherV", "HcclAlltoAllV", "HcclAlltoAll", "HcclAlltoAllVC"))
+        t = _lib.table
+        for call, function, places in (
+                (_all_reduce, World.all_reduce, (2, 3, 4, 5, 6, _lib.COMM, 7)),
+                (_reduce_scatter, World.reduce_scatter, (2, 3, 4, 5, 6, _lib.COMM, 7)),
+                (_reduce_scatter_v, World.reduce_scatter_v, (2, t(3), t(4), 5, 6, 7, 8, _lib.COMM, 9)),
+                (_all_gather, World.all_gather, (2, 3, 4, 5, _lib.COMM, 6)),
+                (_all_gather_v, World.all_gather_v, (2, 3, 4, t(5), t(6), 7, _lib.COMM, 8)),
+                (_all_to_all_v, World.all_to_all_v, (2, t(3), t(4), 8, 5, t(6), t(7), 8, _lib.COMM, 9)),
+                (_all_to_all, World.all_to_all, (2, 3, 5, 4, 3, 5, _lib.COMM, 6)),
+                (_all_to_all_vc, World.all_to_all_vc, (2, t(3), 5, 4, 5, _lib.COMM, 6))):
+            method = _lib.native_method(call, function, places)
+            if method is not None:
+                setattr(World, function.__name__, method)
         _bound = True
     return L
 
@@ -148,7 +161,8 @@ class World:
         return buf.value.decode()
 
     # ---- collectives: one call per rank, in any order; launched by the last one ----
-    # (ctypes converts what the native callable does not take)
+    # (Where the native module was built these become native methods when the library is bound, and what is written here
+    # takes what those do not; ctypes converts what the native callable does not take.)
     def all_reduce(self, rank, send, recv, count, dtype, op, stream):
         rc = _all_reduce(send, recv, count, dtype, op, self.comms[rank], stream)
         if rc is not NotImplemented:

@@ -140,6 +140,32 @@ bool is_capturing(hipStream_t stream)
 
 }  // namespace
 
+namespace hcclx {
+
+// An exchange of equal blocks of `count` elements needs no table.  *launched: false where it goes by the tables after all (a
+// captured launch, so that what can be captured stays as it is; a grid has at most 2^32 work-items along x).
+int alltoall_equal(const void *const *send, void *const *recv, uint64_t count, uint32_t n, int dtype, void *stream, bool *launched)
+{
+    *launched = false;
+    if (!device_ctx()) return HCCL_E_RUNTIME;
+    const uint64_t block_bytes = count * dtype_size(dtype);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (block_bytes == 0 || block_bytes >= (1ull << 35) || is_capturing(st)) return HCCL_SUCCESS;
+    VRankPtrs ptrs;
+    const int rc = fill_ptrs(send, recv, n, &ptrs);
+    if (rc != HCCL_SUCCESS) return rc;
+    EqualBlocks tab;
+    std::memcpy(tab.send, ptrs.send, sizeof(tab.send));
+    std::memcpy(tab.recv, ptrs.recv, sizeof(tab.recv));
+    tab.bytes = block_bytes;
+    const hipError_t e = launch_equal_blocks(tab, n, st);
+    if (e != hipSuccess) return fail_hip(e, "alltoall kernel launch");
+    *launched = true;
+    return HCCL_SUCCESS;
+}
+
+}  // namespace hcclx
+
 extern "C" {
 
 int hcclx_alltoallv(const void *const *send, void *const *recv, const uint64_t *send_counts,
@@ -156,17 +182,10 @@ int hcclx_alltoallv(const void *const *send, void *const *recv, const uint64_t *
     if (rc != HCCL_SUCCESS) return rc;
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (!tables_on_device) {
-        // Equal blocks need no table.  (A captured launch keeps to the tables, so that what can be captured stays as it
-        // is; and a grid has at most 2^32 work-items along x.)
-        const uint64_t block_bytes = send_counts[0] * esz;
-        if (block_bytes != 0 && block_bytes < (1ull << 35) && equal_blocks(send_counts, sdispls, rdispls, n) && !is_capturing(st)) {
-            EqualBlocks tab;
-            std::memcpy(tab.send, ptrs.send, sizeof(tab.send));
-            std::memcpy(tab.recv, ptrs.recv, sizeof(tab.recv));
-            tab.bytes = block_bytes;
-            const hipError_t e = launch_equal_blocks(tab, n, st);
-            if (e != hipSuccess) return fail_hip(e, "alltoall kernel launch");
-            return HCCL_SUCCESS;
+        if (equal_blocks(send_counts, sdispls, rdispls, n)) {
+            bool launched = false;
+            rc = alltoall_equal(send, recv, send_counts[0], n, dtype, stream, &launched);
+            if (rc != HCCL_SUCCESS || launched) return rc;
         }
         bool small = n <= kA2avInlineRanks && ctx->a2av_direct;
         for (size_t k = 0; k < static_cast<size_t>(n) * n && small; ++k) {

@@ -89,11 +89,10 @@ HcclResult SingleRankProc(const OpParam &param, u64 len, World *w)
     return static_cast<HcclResult>(hcclx_fold(&s, 1, HCCL_DATA_TYPE_INT8, 0, HCCLX_FOLD_CHAIN, param.stream));
 }
 
-void FillCommon(OpParam &p, RankComm *rc, const char *opName, HcclCMDType type, aclrtStream stream, const void *in,
-                const void *out)
+// (The tag is filled in when a template gets to see it.)
+void FillCommon(OpParam &p, RankComm *rc, HcclCMDType type, aclrtStream stream, const void *in, const void *out)
 {
     p.hcclComm = rc;
-    p.tag = std::string(opName) + "_vworld";
     p.stream = stream;
     p.inputPtr = const_cast<void *>(in);
     p.outputPtr = const_cast<void *>(out);
@@ -119,7 +118,7 @@ HcclResult AlltoAllCommon(RankComm *rc, OpParam &p, const void *sendBuf, const v
     (void)sendBuf;
     (void)recvBuf;
     if (n == 1) return SingleRankProc(p, d.sendCounts[0] * esz, rc->world);
-    return SubmitOp(rc, p);
+    return SubmitOp(rc, std::move(p));
 }
 
 }  // namespace
@@ -316,14 +315,14 @@ HcclResult HcclAllReduce(void *sendBuf, void *recvBuf, uint64_t count, HcclDataT
     CHK_RET(CheckDataType(dataType, true));
     CHK_RET(CheckReduceOp(dataType, op));
     OpParam p;
-    FillCommon(p, rc, "AllReduce", HcclCMDType::HCCL_CMD_ALLREDUCE, stream, sendBuf, recvBuf);
+    FillCommon(p, rc, HcclCMDType::HCCL_CMD_ALLREDUCE, stream, sendBuf, recvBuf);
     p.inputSize = count * DATATYPE_SIZE_TABLE[dataType];
     p.outputSize = p.inputSize;
     p.reduceType = op;
     p.DataDes.count = count;
     p.DataDes.dataType = dataType;
     if (rc->world->rankSize == 1) return SingleRankProc(p, p.inputSize, rc->world);
-    return SubmitOp(rc, p);
+    return SubmitOp(rc, std::move(p));
 }
 
 HcclResult HcclReduceScatter(void *sendBuf, void *recvBuf, uint64_t recvCount, HcclDataType dataType, HcclReduceOp op,
@@ -340,14 +339,14 @@ HcclResult HcclReduceScatter(void *sendBuf, void *recvBuf, uint64_t recvCount, H
     CHK_RET(CheckDataType(dataType, true));
     CHK_RET(CheckReduceOp(dataType, op));
     OpParam p;
-    FillCommon(p, rc, "ReduceScatter", HcclCMDType::HCCL_CMD_REDUCE_SCATTER, stream, sendBuf, recvBuf);
+    FillCommon(p, rc, HcclCMDType::HCCL_CMD_REDUCE_SCATTER, stream, sendBuf, recvBuf);
     p.outputSize = recvCount * DATATYPE_SIZE_TABLE[dataType];
     p.inputSize = p.outputSize * rc->world->rankSize;
     p.reduceType = op;
     p.DataDes.count = recvCount;
     p.DataDes.dataType = dataType;
     if (rc->world->rankSize == 1) return SingleRankProc(p, p.outputSize, rc->world);
-    return SubmitOp(rc, p);
+    return SubmitOp(rc, std::move(p));
 }
 
 HcclResult HcclReduceScatterV(void *sendBuf, const void *sendCounts, const void *sendDispls, void *recvBuf,
@@ -373,7 +372,7 @@ HcclResult HcclReduceScatterV(void *sendBuf, const void *sendCounts, const void 
     CHK_PRT_RET(counts[rc->rank] != recvCount, HCCL_ERROR("[HcclReduceScatterV] recvCount != sendCounts[rank]"),
                 HCCL_E_PARA);
     OpParam p;
-    FillCommon(p, rc, "ReduceScatterV", HcclCMDType::HCCL_CMD_REDUCE_SCATTER_V, stream, sendBuf, recvBuf);
+    FillCommon(p, rc, HcclCMDType::HCCL_CMD_REDUCE_SCATTER_V, stream, sendBuf, recvBuf);
     const u64 esz = DATATYPE_SIZE_TABLE[dataType];
     p.reduceType = op;
     p.vDataDes.counts.assign(counts, counts + n);
@@ -386,7 +385,7 @@ HcclResult HcclReduceScatterV(void *sendBuf, const void *sendCounts, const void 
     p.inputSize = inElems * esz;
     p.outputSize = recvCount * esz;
     if (n == 1) return SingleRankProc(p, counts[0] * esz, rc->world);
-    return SubmitOp(rc, p);
+    return SubmitOp(rc, std::move(p));
 }
 
 HcclResult HcclAllGather(void *sendBuf, void *recvBuf, uint64_t sendCount, HcclDataType dataType, HcclComm comm,
@@ -402,13 +401,13 @@ HcclResult HcclAllGather(void *sendBuf, void *recvBuf, uint64_t sendCount, HcclD
     CHK_RET(CheckCount(sendCount));
     CHK_RET(CheckDataType(dataType, false));
     OpParam p;
-    FillCommon(p, rc, "AllGather", HcclCMDType::HCCL_CMD_ALLGATHER, stream, sendBuf, recvBuf);
+    FillCommon(p, rc, HcclCMDType::HCCL_CMD_ALLGATHER, stream, sendBuf, recvBuf);
     p.inputSize = sendCount * DATATYPE_SIZE_TABLE[dataType];
     p.outputSize = p.inputSize * rc->world->rankSize;
     p.DataDes.count = sendCount;
     p.DataDes.dataType = dataType;
     if (rc->world->rankSize == 1) return SingleRankProc(p, p.inputSize, rc->world);
-    return SubmitOp(rc, p);
+    return SubmitOp(rc, std::move(p));
 }
 
 HcclResult HcclAllGatherV(void *sendBuf, uint64_t sendCount, void *recvBuf, const void *recvCounts,
@@ -431,7 +430,7 @@ HcclResult HcclAllGatherV(void *sendBuf, uint64_t sendCount, void *recvBuf, cons
     CHK_PRT_RET(counts[rc->rank] != sendCount, HCCL_ERROR("[HcclAllGatherV] sendCount != recvCounts[rank]"),
                 HCCL_E_PARA);
     OpParam p;
-    FillCommon(p, rc, "AllGatherV", HcclCMDType::HCCL_CMD_ALLGATHER_V, stream, sendBuf, recvBuf);
+    FillCommon(p, rc, HcclCMDType::HCCL_CMD_ALLGATHER_V, stream, sendBuf, recvBuf);
     const u64 esz = DATATYPE_SIZE_TABLE[dataType];
     p.vDataDes.counts.assign(counts, counts + n);
     p.vDataDes.displs.assign(displs, displs + n);
@@ -442,7 +441,7 @@ HcclResult HcclAllGatherV(void *sendBuf, uint64_t sendCount, void *recvBuf, cons
     for (u32 i = 0; i < n; ++i) outElems = std::max(outElems, displs[i] + counts[i]);
     p.outputSize = outElems * esz;
     if (n == 1) return SingleRankProc(p, counts[0] * esz, rc->world);
-    return SubmitOp(rc, p);
+    return SubmitOp(rc, std::move(p));
 }
 
 HcclResult HcclAlltoAllV(const void *sendBuf, const void *sendCounts, const void *sdispls, HcclDataType sendType,
@@ -470,7 +469,7 @@ HcclResult HcclAlltoAllV(const void *sendBuf, const void *sendCounts, const void
     CHK_RET(CheckDataType(recvType, false));
     CHK_PRT_RET(sendType != recvType, HCCL_ERROR("[HcclAlltoAllV] sendType != recvType"), HCCL_E_PARA);
     OpParam p;
-    FillCommon(p, rc, "ALLTOALLV", HcclCMDType::HCCL_CMD_ALLTOALLV, stream, sendBuf, recvBuf);
+    FillCommon(p, rc, HcclCMDType::HCCL_CMD_ALLTOALLV, stream, sendBuf, recvBuf);
     p.all2AllVDataDes.sendCounts.assign(sc, sc + n);
     p.all2AllVDataDes.recvCounts.assign(rcv, rcv + n);
     p.all2AllVDataDes.sdispls.assign(static_cast<const u64 *>(sdispls), static_cast<const u64 *>(sdispls) + n);
@@ -495,21 +494,17 @@ HcclResult HcclAlltoAll(const void *sendBuf, uint64_t sendCount, HcclDataType se
     CHK_RET(CheckDataType(recvType, false));
     const u32 n = rc->world->rankSize;
     OpParam p;
-    FillCommon(p, rc, "ALLTOALL", HcclCMDType::HCCL_CMD_ALLTOALL, stream, sendBuf, recvBuf);
+    FillCommon(p, rc, HcclCMDType::HCCL_CMD_ALLTOALL, stream, sendBuf, recvBuf);
+    // equal blocks back to back (ConvertAlltoAllParam, all_to_all_v_op.cc:385-394); the tables that say so are made where a
+    // template or a key needs them (FillEqualTables)
     p.all2AllDataDes.sendCount = sendCount;
     p.all2AllDataDes.recvCount = recvCount;
-    auto &d = p.all2AllVDataDes;
-    d.sendCounts.assign(n, sendCount);
-    d.recvCounts.assign(n, recvCount);
-    d.sdispls.resize(n);
-    d.rdispls.resize(n);
-    u64 off = 0;  // ConvertAlltoAllParam, all_to_all_v_op.cc:385-394
-    for (u32 i = 0; i < n; ++i) {
-        d.sdispls[i] = off;
-        d.rdispls[i] = off;
-        off += recvCount;
-    }
-    return AlltoAllCommon(rc, p, sendBuf, recvBuf, recvType);
+    p.all2AllVDataDes.sendType = sendType;
+    p.all2AllVDataDes.recvType = recvType;
+    p.inputSize = n * sendCount * DATATYPE_SIZE_TABLE[recvType];
+    p.outputSize = p.inputSize;
+    if (n == 1) return SingleRankProc(p, p.inputSize, rc->world);
+    return SubmitOp(rc, std::move(p));
 }
 
 HcclResult HcclAlltoAllVC(const void *sendBuf, const void *sendCountMatrix, HcclDataType sendType, const void *recvBuf,
@@ -528,7 +523,7 @@ HcclResult HcclAlltoAllVC(const void *sendBuf, const void *sendCountMatrix, Hccl
     CHK_RET(CheckDataType(recvType, false));
     CHK_PRT_RET(sendType != recvType, HCCL_ERROR("[HcclAlltoAllVC] sendType != recvType"), HCCL_E_PARA);
     OpParam p;
-    FillCommon(p, rc, "ALLTOALLVC", HcclCMDType::HCCL_CMD_ALLTOALLVC, stream, sendBuf, recvBuf);
+    FillCommon(p, rc, HcclCMDType::HCCL_CMD_ALLTOALLVC, stream, sendBuf, recvBuf);
     auto &d = p.all2AllVDataDes;
     d.sendCounts.resize(n);
     d.recvCounts.resize(n);

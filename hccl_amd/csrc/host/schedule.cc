@@ -15,6 +15,11 @@
 #include "schedule_internal.h"
 #include "selector.h"
 
+namespace hcclx {
+// hcclx_vops.hip
+int alltoall_equal(const void *const *send, void *const *recv, uint64_t count, uint32_t n, int dtype, void *stream, bool *launched);
+}  // namespace hcclx
+
 namespace ops_hccl {
 
 void SetForcedAlgorithm(World *w, HcclCMDType type, const std::string &algName)
@@ -75,9 +80,38 @@ bool IsDataMove(HcclCMDType t)
            t == HcclCMDType::HCCL_CMD_ALLTOALLVC;
 }
 
+// The tables of an AlltoAll of equal blocks, which the call itself does not carry.
+void FillEqualTables(OpParam &p, size_t n)
+{
+    auto &d = p.all2AllVDataDes;
+    d.sendCounts.assign(n, p.all2AllDataDes.sendCount);
+    d.recvCounts.assign(n, p.all2AllDataDes.recvCount);
+    d.sdispls.resize(n);
+    d.rdispls.resize(n);
+    for (size_t i = 0; i < n; ++i) d.sdispls[i] = d.rdispls[i] = i * p.all2AllDataDes.recvCount;
+}
+void FillEqualTables(std::vector<OpParam> &params)
+{
+    for (OpParam &p : params) FillEqualTables(p, params.size());
+}
+
+const char *OpTag(HcclCMDType t)
+{
+    switch (t) {
+        case HcclCMDType::HCCL_CMD_ALLREDUCE: return "AllReduce_vworld";
+        case HcclCMDType::HCCL_CMD_REDUCE_SCATTER: return "ReduceScatter_vworld";
+        case HcclCMDType::HCCL_CMD_REDUCE_SCATTER_V: return "ReduceScatterV_vworld";
+        case HcclCMDType::HCCL_CMD_ALLGATHER: return "AllGather_vworld";
+        case HcclCMDType::HCCL_CMD_ALLGATHER_V: return "AllGatherV_vworld";
+        case HcclCMDType::HCCL_CMD_ALLTOALL: return "ALLTOALL_vworld";
+        case HcclCMDType::HCCL_CMD_ALLTOALLVC: return "ALLTOALLVC_vworld";
+        default: return "ALLTOALLV_vworld";
+    }
+}
+
 // Pure data movement has no fold order to preserve: in FUSED mode the contract itself is launched on the
 // ragged-copy kernels (one read and one write per delivered byte), with the tables of all ranks.
-HcclResult LaunchDataMove(World *w, const std::vector<OpParam> &params, void *stream)
+HcclResult LaunchDataMove(World *w, std::vector<OpParam> &params, void *stream)
 {
     const u32 n = w->rankSize;
     std::vector<const void *> send(n);
@@ -102,6 +136,13 @@ HcclResult LaunchDataMove(World *w, const std::vector<OpParam> &params, void *st
         const int dt = (t == HcclCMDType::HCCL_CMD_ALLGATHER) ? params[0].DataDes.dataType : params[0].vDataDes.dataType;
         return static_cast<HcclResult>(
             hcclx_allgatherv(send.data(), recv.data(), counts.data(), displs.data(), n, dt, 0, stream));
+    }
+    if (t == HcclCMDType::HCCL_CMD_ALLTOALL) {
+        bool launched = false;
+        const int rc = hcclx::alltoall_equal(send.data(), recv.data(), params[0].all2AllDataDes.sendCount, n,
+                                             params[0].all2AllVDataDes.sendType, stream, &launched);
+        if (rc != HCCL_SUCCESS || launched) return static_cast<HcclResult>(rc);
+        FillEqualTables(params);
     }
     std::vector<u64> sc(static_cast<size_t>(n) * n);
     std::vector<u64> sd(static_cast<size_t>(n) * n);
@@ -170,7 +211,13 @@ HcclResult RunCollectiveOnStream(World *w, std::vector<OpParam> &params)
                     HCCL_ERROR("[RunCollective] rank %u issued a different collective than rank 0", r), HCCL_E_PARA);
     }
     const HcclCMDType type = params[0].opType;
-    if (IsDataMove(type)) {
+    if (type == HcclCMDType::HCCL_CMD_ALLTOALL) {
+        // a rank sends and expects one count for all: they have to be the same
+        for (u32 r = 1; r < n; ++r) {
+            CHK_PRT_RET(params[r].all2AllDataDes.sendCount != params[0].all2AllDataDes.sendCount,
+                        HCCL_ERROR("[RunCollective] sendCounts[%u][%u] != recvCounts[%u][%u]", 0u, r, r, 0u), HCCL_E_PARA);
+        }
+    } else if (IsDataMove(type)) {
         // what i sends to j must be what j expects from i
         for (u32 i = 0; i < n && type != HcclCMDType::HCCL_CMD_ALLGATHER && type != HcclCMDType::HCCL_CMD_ALLGATHER_V;
              ++i) {
@@ -196,6 +243,7 @@ HcclResult RunCollectiveOnStream(World *w, std::vector<OpParam> &params)
         topo.topoLevelNums = w->topoLevels;
         topo.level0Topo = w->topoShape;
         topo.localNetInsSizeOfLayer0 = w->devicesPerServer ? w->devicesPerServer : n;
+        if (type == HcclCMDType::HCCL_CMD_ALLTOALL) FillEqualTables(params[0], n);   // a selector may look at them
         CHK_RET(ExecuteSelector().Run(params[0], &topo, algName));
     }
     w->lastAlgName = algName;
@@ -212,6 +260,7 @@ HcclResult RunCollectiveOnStream(World *w, std::vector<OpParam> &params)
         w->lastWasFused = true;
         return LaunchDataMove(w, params, stream);
     }
+    if (type == HcclCMDType::HCCL_CMD_ALLTOALL) FillEqualTables(params);
     std::vector<u64> shape;
     std::vector<u64> key;
     bool separate = false;
@@ -284,6 +333,7 @@ HcclResult RunCollectiveOnStream(World *w, std::vector<OpParam> &params)
         w->ResetRecording();
         for (u32 r = 0; r < n; ++r) {
             params[r].algName = algName;
+            params[r].tag = OpTag(type);
             std::unique_ptr<InsCollAlgBase> exec = CollAlgExecRegistryV2::Instance().GetAlgExec(type, algName);
             CHK_PRT_RET(exec == nullptr, HCCL_ERROR("[RunCollective] no executor named %s", algName.c_str()),
                         HCCL_E_NOT_SUPPORT);
@@ -322,6 +372,7 @@ HcclResult RunCollectiveOnStream(World *w, std::vector<OpParam> &params)
         std::unique_ptr<InsCollAlgBase> exec = CollAlgExecRegistryV2::Instance().GetAlgExec(type, algName);
         std::vector<ClosedFold> closed;
         params[0].algName = algName;
+        params[0].tag = OpTag(type);
         if (exec != nullptr && exec->ClosedForm(params[0], n, w->cclBytes, closed)) {
             if (FoldsFromClosedForm(closed, params, dtype, op, folds, text)) {
                 haveFolds = true;

@@ -18,17 +18,24 @@ HcclResult SelectorRegistry::RegisterByOpType(HcclCMDType opType, u32 priority, 
     return HCCL_SUCCESS;
 }
 
-std::map<u32, AutoSelectorBase *> SelectorRegistry::GetSelectorsByOpType(HcclCMDType opType)
+AutoSelectorBase *SelectorRegistry::Next(HcclCMDType opType, bool first, u32 &priority)
 {
     std::lock_guard<std::mutex> lock(mu_);
-    return opTypeImpls_[opType];
+    const std::map<u32, AutoSelectorBase *> &impls = opTypeImpls_[opType];
+    const auto it = first ? impls.begin() : impls.upper_bound(priority);
+    if (it == impls.end()) return nullptr;
+    priority = it->first;
+    return it->second;
 }
 
 HcclResult ExecuteSelector::Run(OpParam &opParam, TopoInfoWithNetLayerDetails *topoInfo,
                                 std::string &selectAlgName) const
 {
-    for (auto &kv : SelectorRegistry::Global()->GetSelectorsByOpType(opParam.opType)) {
-        if (kv.second->Select(opParam, topoInfo, selectAlgName) == SelectorStatus::MATCH) return HCCL_SUCCESS;
+    SelectorRegistry *registry = SelectorRegistry::Global();
+    u32 priority = 0;
+    for (AutoSelectorBase *s = registry->Next(opParam.opType, true, priority); s != nullptr;
+         s = registry->Next(opParam.opType, false, priority)) {
+        if (s->Select(opParam, topoInfo, selectAlgName) == SelectorStatus::MATCH) return HCCL_SUCCESS;
     }
     HCCL_ERROR("[Algo][Selector] No selector is matched.");
     return HCCL_E_NOT_SUPPORT;

@@ -262,22 +262,22 @@ void FillResources(World *w, u32 rank, u32 threadNum, AlgResourceCtxSerializable
     }
 }
 
-HcclResult SubmitOp(RankComm *rc, const OpParam &param)
+HcclResult SubmitOp(RankComm *rc, OpParam &&param)
 {
     World *w = rc->world;
     std::unique_lock<std::mutex> lock(w->mu);
-    QueuedOp q;
-    q.param = param;
-    w->queue[rc->rank].push_back(std::move(q));
-    const u64 myTicket = w->launched[rc->rank] + w->queue[rc->rank].size();  // collective number of this call
+    RankQueue &mine = w->queue[rc->rank];
+    if (mine.empty()) ++w->waiting;
+    mine.Push(std::move(param));
+    const u64 myTicket = w->launched[rc->rank] + mine.size();  // collective number of this call
 
-    bool all = true;
-    for (u32 r = 0; r < w->rankSize; ++r) all = all && !w->queue[r].empty();
-    while (all) {
-        std::vector<OpParam> params;
+    while (w->waiting == w->rankSize) {
+        std::vector<OpParam> &params = w->current;
+        params.clear();
+        params.reserve(w->rankSize);
         for (u32 r = 0; r < w->rankSize; ++r) {
-            params.push_back(std::move(w->queue[r].front().param));
-            w->queue[r].pop_front();
+            params.push_back(w->queue[r].Take());
+            if (w->queue[r].empty()) --w->waiting;
         }
         const HcclResult res = RunCollective(w, params);
         for (u32 r = 0; r < w->rankSize; ++r) {
@@ -285,8 +285,6 @@ HcclResult SubmitOp(RankComm *rc, const OpParam &param)
             w->lastResult[r] = res;
         }
         w->cv.notify_all();
-        all = true;
-        for (u32 r = 0; r < w->rankSize; ++r) all = all && !w->queue[r].empty();
     }
     if (w->launched[rc->rank] >= myTicket) return w->lastResult[rc->rank];
     if (!w->blocking) return HCCL_SUCCESS;  // queued; the last rank to arrive launches

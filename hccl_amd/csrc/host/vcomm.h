@@ -6,7 +6,6 @@
 // and the recorded steps are launched on the GPU (schedule.h).
 #pragma once
 #include <condition_variable>
-#include <deque>
 #include <list>
 #include <map>
 #include <memory>
@@ -67,9 +66,25 @@ struct RankComm {
     u32 rank = 0;
 };
 
-struct QueuedOp {
-    OpParam param;
-    hipEvent_t ready = nullptr;  // recorded on the caller's stream when it differs from the launch stream
+// The calls of one rank that wait for the other ranks' (mostly one: the vector keeps its memory).
+struct RankQueue {
+    std::vector<OpParam> ops;
+    size_t head = 0;   // ops[0 .. head) have been taken
+    size_t size() const { return ops.size() - head; }
+    bool empty() const { return head == ops.size(); }
+    void Push(OpParam &&p) { ops.push_back(std::move(p)); }
+    OpParam Take()
+    {
+        OpParam p = std::move(ops[head++]);
+        if (head == ops.size()) {
+            ops.clear();
+            head = 0;
+        } else if (head >= 64) {   // a rank far ahead of the others
+            ops.erase(ops.begin(), ops.begin() + static_cast<std::ptrdiff_t>(head));
+            head = 0;
+        }
+        return p;
+    }
 };
 
 struct CachedPlan {
@@ -161,7 +176,9 @@ struct World {
 
     std::mutex mu;
     std::condition_variable cv;
-    std::vector<std::deque<QueuedOp>> queue;  // per rank
+    std::vector<RankQueue> queue;             // per rank
+    u32 waiting = 0;                          // ranks whose queue is not empty
+    std::vector<OpParam> current;             // the calls of the collective being run, by rank
     std::vector<u64> launched;                // per rank: collectives completed so far
     std::vector<HcclResult> lastResult;
 
@@ -209,6 +226,6 @@ RankComm *AsRankComm(HcclComm comm);
 void FillResources(World *w, u32 rank, u32 threadNum, AlgResourceCtxSerializable &resCtx);
 
 // Queues one rank's call; launches the collective when all ranks have one queued.
-HcclResult SubmitOp(RankComm *rc, const OpParam &param);
+HcclResult SubmitOp(RankComm *rc, OpParam &&param);
 
 }  // namespace ops_hccl

@@ -127,3 +127,50 @@ case "$2" in *EXT_SUFFIX*) echo .cpython-399-test.so;; *) echo {tmp_path};; esac
     assert run.returncode == 0, run.stderr[-2000:]
     assert "libhccl_amd.so" in run.stdout
     assert ("_hccl_calls.cpython-399-test.so" in run.stdout) == headers and ("python_calls.cc" in run.stdout) == headers
+
+
+@pytest.mark.parametrize("how", ["plain", "keywords", "unbound", "kind", "boolean rank", "subclass"])
+def test_the_native_methods_and_what_they_leave_to_python(how):
+    """The collectives of api.World as native methods: the same calls and codes as the methods written in Python."""
+    class Sub(api.World):
+        def all_reduce(self, *args):
+            return super().all_reduce(*args)
+    w = (Sub if how == "subclass" else api.World)(2, dry=True)
+    assert type(api.World.__dict__["all_reduce"]).__name__ == "Method"
+    for r in range(2):
+        rank = bool(r) if how == "boolean rank" else r
+        args = ((r + 1) << 20, (r + 10) << 20, 100, Kind.FP32 if how == "kind" else T.FP32, T.SUM, 1)
+        if how == "keywords":
+            names = ("send", "recv", "count", "dtype", "op", "stream")
+            assert w.all_reduce(rank, **dict(zip(names, args))) == 0
+        elif how == "unbound":
+            assert api.World.all_reduce(w, rank, *args) == 0
+        else:
+            assert w.all_reduce(rank, *args) == 0
+    assert w.last_info().algName
+    w.close()
+
+
+def test_what_a_method_refuses(world):
+    args = (1 << 20, 2 << 20, 10, T.FP32, T.SUM, 1)
+    for bad, kind in (((2,) + args, IndexError), ((1.5,) + args, TypeError), ((0,) + args[:-1], TypeError), ((1 << 70,) + args, IndexError)):
+        with pytest.raises(kind):
+            world.all_reduce(*bad)
+    for table in (5, None):   # an address in the place of a table is not taken for one
+        with pytest.raises(TypeError):
+            world.all_gather_v(0, 1 << 20, 5, 2 << 20, table, [0, 5], T.FP32, 1)
+    assert world.all_reduce(0, 1 << 20, 2 << 20, 10, 99, T.SUM, 1) != 0
+    closed = api.World(2, dry=True)
+    closed.close()
+    with pytest.raises(IndexError):
+        closed.all_reduce(0, *args)
+
+
+def test_ranks_that_run_ahead(world):
+    """One rank's calls wait, in order, for the other's; counts that differ are found out at their own collective."""
+    counts = [3 + k % 5 for k in range(200)]
+    for c in counts:
+        assert world.all_to_all(0, 1 << 20, c, 10 << 20, T.FP32, 1) == 0
+    for k, c in enumerate(counts):
+        wrong = k in (70, 199)
+        assert (world.all_to_all(1, 2 << 20, c + wrong, 11 << 20, T.FP32, 1) != 0) == wrong
