@@ -249,7 +249,7 @@ k_moe_scan_perm(MoeConstPtrs dest, MoePtrs perm, uint32_t n, uint32_t entries, u
 // itself.  Workgroup (c, i): a pass over the destinations of rank i gives, per destination, its
 // entries and those in front of chunk c; then the permutation of chunk c as in k_moe_perm.  The workgroups of chunk 0 write
 // their rank's rows of the count and displacement tables and, from a pass over all ranks' destinations, what every rank
-// sends to rank i in front of which.  Bound by the latency of one launch and two rounds of loads.  Two launches : one, us: 8 ranks x 64
+// sends to rank i in front of which.  Bound by the latency of one launch and its rounds of loads.  Two launches : one, us: 8 ranks x 64
 // entries 5.95 : 4.44, x 512 6.16 : 4.61, x 1024 6.5 : 5.2, x 4096 7.6 : 9.4; 16 x 1024 8.3 : 7.3, x 2048 8.9 : 9.7; 64 x 1024
 // 26.3 : 20.5; 2 x 512 5.1 : 3.6, x 4096 6.2 : 7.3.
 constexpr uint32_t kOneLaunchEntries = 1024;
@@ -268,49 +268,64 @@ k_moe_route_one(MoeConstPtrs dest, MoePtrs perm, uint32_t n, uint32_t entries, u
     const uint32_t wave = threadIdx.x >> 6;
     const uint32_t lane = threadIdx.x & 63;
     const int32_t *mine = static_cast<const int32_t *>(dest.p[i]);
+    // Every load that does not depend on another is issued here: the launch is little more than these round trips.  An entry
+    // behind the last repeats it and is not counted.
+    const uint32_t e = c * kMoeChunk + threadIdx.x;
+    uint32_t d = static_cast<uint32_t>(mine[e < entries ? e : entries - 1]);
+    constexpr int kPerThread = kOneLaunchEntries / kMoeChunk;
+    uint32_t all[kPerThread];
+#pragma unroll
+    for (int u = 0; u < kPerThread; ++u) {
+        const uint32_t at = u * kMoeChunk + threadIdx.x;
+        all[u] = static_cast<uint32_t>(mine[at < entries ? at : entries - 1]);
+    }
+    // chunk 0: entries of rank r for rank i, a wavefront per rank, the loads of its next rank ahead of the count of this one
+    constexpr int kAhead = 8;
+    auto load_from = [&](uint32_t r, uint32_t first, uint32_t (&f)[kAhead]) {
+        const int32_t *from = static_cast<const int32_t *>(dest.p[r]);
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const uint32_t at = first + u * 64 + lane;
+            f[u] = static_cast<uint32_t>(from[at < entries ? at : entries - 1]);
+        }
+    };
+    auto count_from = [&](uint32_t first, const uint32_t (&f)[kAhead]) {
+        uint32_t count = 0;
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) count += first + u * 64 + lane < entries && f[u] == i ? 1u : 0u;
+        return count;
+    };
+    uint32_t f[kAhead];
+    if (c == 0) load_from(wave < n ? wave : 0, 0, f);
     if (threadIdx.x < kMoeMaxRanks) {
         s_total[threadIdx.x] = 0;
         s_before[threadIdx.x] = 0;
     }
     __syncthreads();
-    // eight loads in flight; an entry behind the last repeats it and is not counted
-    for (uint32_t base = threadIdx.x; base < entries; base += 8 * kMoeChunk) {
-        uint32_t d[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const uint32_t e = base + u * kMoeChunk;
-            d[u] = static_cast<uint32_t>(mine[e < entries ? e : entries - 1]);
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const uint32_t e = base + u * kMoeChunk;
-            if (e < entries && d[u] < n) {
-                atomicAdd(&s_total[d[u]], 1u);
-                if (e < c * kMoeChunk) atomicAdd(&s_before[d[u]], 1u);
-            }
+    for (int u = 0; u < kPerThread; ++u) {
+        const uint32_t at = u * kMoeChunk + threadIdx.x;
+        if (at < entries && all[u] < n) {
+            atomicAdd(&s_total[all[u]], 1u);
+            if (at < c * kMoeChunk) atomicAdd(&s_before[all[u]], 1u);
         }
     }
     if (c == 0) {
         for (uint32_t r = wave; r < n; r += 4) {
-            const int32_t *from = static_cast<const int32_t *>(dest.p[r]);
-            uint32_t count = 0;
-            for (uint32_t base = lane; base < entries; base += 8 * 64) {
-                uint32_t d[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    const uint32_t e = base + u * 64;
-                    d[u] = static_cast<uint32_t>(from[e < entries ? e : entries - 1]);
-                }
-#pragma unroll
-                for (int u = 0; u < 8; ++u) count += base + u * 64 < entries && d[u] == i ? 1u : 0u;
+            uint32_t ahead[kAhead];
+            load_from(r + 4 < n ? r + 4 : r, 0, ahead);
+            uint32_t count = count_from(0, f);
+            for (uint32_t first = kAhead * 64; first < entries; first += kAhead * 64) {
+                load_from(r, first, f);
+                count += count_from(first, f);
             }
             count = wave_sum_u32(count);
             if (lane == 0) s_from[r] = count;
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) f[u] = ahead[u];
         }
     }
-    const uint32_t e = c * kMoeChunk + threadIdx.x;
-    uint32_t d = n;
-    if (e < entries) d = static_cast<uint32_t>(mine[e]);
+    if (e >= entries) d = n;
     uint32_t rank = 0;
     const unsigned long long below = (1ull << lane) - 1ull;
     for (uint32_t dd = 0; dd < n; ++dd) {
@@ -580,11 +595,11 @@ k_moe_scatter_pieces(MoeConstPtrs tokens, MoeConstPtrs dest, MoeConstPtrs perm, 
     }
 }
 
-// Gather the rows of a token's entries from where dispatch put them in expert[dest[.]] and add them.  The entries one
-// after the other: the look-ups of several at once, by scalar loads or one lane each, measured no faster (8 x 4096,
-// top-2, 7168 bf16: 220 us, two at once 221 and 251, runs of 224 vectors in 256 threads 230).  DT = int8 moves bytes
-// (topk == 1).
-template <int DT>
+// Gather the rows of a token's entries from where dispatch put them in expert[dest[.]] and add them, K entries at a time: their
+// look-ups and then their rows are in flight together.  Whatever an entry is, its lanes load from somewhere (a dropped one
+// from the result's own place): a branch per entry would make the compiler wait for every load before the next.  K by
+// gather_entries.  DT = int8 moves bytes (topk == 1).
+template <int DT, int K>
 __global__ void __launch_bounds__(kPieceVecs * kPiecesPerBlock)
 k_moe_gather_pieces(MoeConstPtrs rows, MoeConstPtrs dest, MoeConstPtrs perm, MoePtrs out, uint32_t n, uint32_t topk, uint32_t vpr,
                     RowPieces pieces, uint32_t esz, const uint64_t *sdispls, const uint64_t *rdispls)
@@ -606,23 +621,55 @@ k_moe_gather_pieces(MoeConstPtrs rows, MoeConstPtrs dest, MoeConstPtrs perm, Moe
     bool have = false;
 #pragma unroll
     for (int k = 0; k < NE; ++k) acc[k] = C(0);
-    for (uint32_t e = 0; e < topk; ++e) {
-        const uint32_t p = pm[e];
-        const uint32_t d = static_cast<uint32_t>(dt[e]);
-        if (p == kDropped || d >= n) continue;
-        const char *from = landing(as_mutable_dev(rows), i, d, n, esz, sdispls, rdispls) + (static_cast<uint64_t>(p) * vpr + v0) * 16;
-        C x[NE];
-        V::unpack(ld16(from + lane_off), x);
-        if (!have) {
+    char *to = static_cast<char *>(out.p[i]) + (static_cast<uint64_t>(t) * vpr + v0) * 16 + lane_off;
+    for (uint32_t first = 0; first < topk; first += K) {
+        uint32_t p[K];
+        uint32_t d[K];
+        bool ok[K];
 #pragma unroll
-            for (int k = 0; k < NE; ++k) acc[k] = x[k];
-        } else {
-#pragma unroll
-            for (int k = 0; k < NE; ++k) acc[k] = V::template combine<HCCL_REDUCE_SUM>(x[k], acc[k]);
+        for (int k = 0; k < K; ++k) {
+            const uint32_t e = first + k < topk ? first + k : topk - 1;   // an entry behind the last repeats it and is not added
+            p[k] = pm[e];
+            d[k] = static_cast<uint32_t>(dt[e]);
         }
-        have = true;
+        u32x4 raw[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            ok[k] = first + k < topk && p[k] != kDropped && d[k] < n;
+            const char *row = landing(as_mutable_dev(rows), i, ok[k] ? d[k] : 0u, n, esz, sdispls, rdispls) +
+                              (static_cast<uint64_t>(ok[k] ? p[k] : 0u) * vpr + v0) * 16 + lane_off;
+            raw[k] = ld16(ok[k] ? row : to);
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            if (!ok[k]) continue;
+            C x[NE];
+            V::unpack(raw[k], x);
+            if (!have) {
+#pragma unroll
+                for (int q = 0; q < NE; ++q) acc[q] = x[q];
+            } else {
+#pragma unroll
+                for (int q = 0; q < NE; ++q) acc[q] = V::template combine<HCCL_REDUCE_SUM>(x[q], acc[q]);
+            }
+            have = true;
+        }
     }
-    st16(static_cast<char *>(out.p[i]) + (static_cast<uint64_t>(t) * vpr + v0) * 16 + lane_off, V::pack(acc));
+    st16(to, V::pack(acc));
+}
+
+// Entries of a token that the gather takes at a time.  Two of two (8 x 4096 tokens of 7168 bf16, dispatch and gather, one : two
+// entries at a time, us: 462 : 454, 16 x 695 153.8 : 152.5, 4 x 300 26.3 : 25.4).  Of more entries: four while all wavefronts
+// fit the chip with room to spare and the launch is bound by its round trips (top-8, 8 x 16 tokens 18.8 : 16.0, 16 x 52 26.7 :
+// 25.5; top-4, 8 x 32 15.9 : 14.1; eight at a time 16.0, 25.7 and 14.7), two up to the wavefronts that fit (8 x 64 30.4 : 30.0), and one
+// beyond, where more of them open more rows at once than HBM likes (top-8, 8 x 1024 191 : 199 with four, 8 x 4096 586 : 611;
+// top-4, 4 x 3683 211 : 218).
+inline int gather_entries(const DeviceCtx *ctx, uint32_t topk, uint64_t waves)
+{
+    if (topk == 1) return 1;
+    if (topk == 2) return 2;
+    const uint64_t cus = ctx ? static_cast<uint64_t>(ctx->num_cus) : 256;
+    return waves <= 20 * cus ? 4 : waves <= 32 * cus ? 2 : 1;
 }
 
 // Which entries share a wavefront, and how rows are stored.  Tokens of up to kWarmTokens in all are usually still in the
@@ -669,6 +716,20 @@ int launch_scatter_pieces(uint32_t per_wave, hipStream_t st, const MoeConstPtrs 
     return HCCL_SUCCESS;
 }
 
+template <int DT>
+void launch_gather_k(int k, dim3 grid, dim3 block, hipStream_t st, const MoeConstPtrs &rows, const MoeConstPtrs &dest, const MoeConstPtrs &perm,
+                     const MoePtrs &out, uint32_t n, uint32_t topk, uint32_t vpr, const RowPieces &pieces, uint32_t esz,
+                     const uint64_t *sdispls, const uint64_t *rdispls)
+{
+    if (k == 4) {
+        HCCLX_LAUNCH((k_moe_gather_pieces<DT, 4>), grid, block, 0, st, rows, dest, perm, out, n, topk, vpr, pieces, esz, sdispls, rdispls);
+    } else if (k == 2) {
+        HCCLX_LAUNCH((k_moe_gather_pieces<DT, 2>), grid, block, 0, st, rows, dest, perm, out, n, topk, vpr, pieces, esz, sdispls, rdispls);
+    } else {
+        HCCLX_LAUNCH((k_moe_gather_pieces<DT, 1>), grid, block, 0, st, rows, dest, perm, out, n, topk, vpr, pieces, esz, sdispls, rdispls);
+    }
+}
+
 int launch_gather_pieces(int kind, hipStream_t st, const MoeConstPtrs &rows, const MoeConstPtrs &dest, const MoeConstPtrs &perm,
                          const MoeConstPtrs &out, uint32_t n, uint32_t tokens, uint32_t topk, uint32_t vpr, uint32_t esz,
                          const uint64_t *sdispls, const uint64_t *rdispls)
@@ -683,17 +744,15 @@ int launch_gather_pieces(int kind, hipStream_t st, const MoeConstPtrs &rows, con
         const MoeConstPtrs ds = moved_on(dest, n, static_cast<uint64_t>(at) * topk * 4);
         const MoeConstPtrs pm = moved_on(perm, n, static_cast<uint64_t>(at) * topk * 4);
         const dim3 grid((pieces.total + kPiecesPerBlock - 1) / kPiecesPerBlock, n);
+        const int k = gather_entries(device_ctx(), topk, static_cast<uint64_t>(pieces.total) * n);
         if (kind == HCCL_DATA_TYPE_FP32) {
-            HCCLX_LAUNCH(k_moe_gather_pieces<HCCL_DATA_TYPE_FP32>, grid, block, 0, st, rows, ds, pm, to, n, topk, vpr, pieces, esz,
-                         sdispls, rdispls);
+            launch_gather_k<HCCL_DATA_TYPE_FP32>(k, grid, block, st, rows, ds, pm, to, n, topk, vpr, pieces, esz, sdispls, rdispls);
         } else if (kind == HCCL_DATA_TYPE_FP16) {
-            HCCLX_LAUNCH(k_moe_gather_pieces<HCCL_DATA_TYPE_FP16>, grid, block, 0, st, rows, ds, pm, to, n, topk, vpr, pieces, esz,
-                         sdispls, rdispls);
+            launch_gather_k<HCCL_DATA_TYPE_FP16>(k, grid, block, st, rows, ds, pm, to, n, topk, vpr, pieces, esz, sdispls, rdispls);
         } else if (kind == HCCL_DATA_TYPE_BFP16) {
-            HCCLX_LAUNCH(k_moe_gather_pieces<HCCL_DATA_TYPE_BFP16>, grid, block, 0, st, rows, ds, pm, to, n, topk, vpr, pieces, esz,
-                         sdispls, rdispls);
+            launch_gather_k<HCCL_DATA_TYPE_BFP16>(k, grid, block, st, rows, ds, pm, to, n, topk, vpr, pieces, esz, sdispls, rdispls);
         } else {
-            HCCLX_LAUNCH(k_moe_gather_pieces<HCCL_DATA_TYPE_INT8>, grid, block, 0, st, rows, ds, pm, to, n, topk, vpr, pieces, esz,
+            HCCLX_LAUNCH((k_moe_gather_pieces<HCCL_DATA_TYPE_INT8, 1>), grid, block, 0, st, rows, ds, pm, to, n, topk, vpr, pieces, esz,
                          sdispls, rdispls);
         }
         const hipError_t e = hipGetLastError();
