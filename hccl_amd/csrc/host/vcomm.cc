@@ -266,7 +266,7 @@ HcclResult SubmitOp(RankComm *rc, OpParam &&param)
 {
     World *w = rc->world;
     std::unique_lock<std::mutex> lock(w->mu);
-    RankQueue &mine = w->queue[rc->rank];
+    CallQueue<OpParam> &mine = w->queue[rc->rank];
     if (mine.empty()) ++w->waiting;
     mine.Push(std::move(param));
     const u64 myTicket = w->launched[rc->rank] + mine.size();  // collective number of this call

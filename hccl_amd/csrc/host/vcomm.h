@@ -17,6 +17,7 @@
 
 #include "alg_env_config.h"
 #include "alg_param.h"
+#include "call_queue.h"
 
 #include "hcclx.h"
 
@@ -64,27 +65,6 @@ enum class ExecMode {
 struct RankComm {
     World *world = nullptr;
     u32 rank = 0;
-};
-
-// The calls of one rank that wait for the other ranks' (mostly one: the vector keeps its memory).
-struct RankQueue {
-    std::vector<OpParam> ops;
-    size_t head = 0;   // ops[0 .. head) have been taken
-    size_t size() const { return ops.size() - head; }
-    bool empty() const { return head == ops.size(); }
-    void Push(OpParam &&p) { ops.push_back(std::move(p)); }
-    OpParam Take()
-    {
-        OpParam p = std::move(ops[head++]);
-        if (head == ops.size()) {
-            ops.clear();
-            head = 0;
-        } else if (head >= 64) {   // a rank far ahead of the others
-            ops.erase(ops.begin(), ops.begin() + static_cast<std::ptrdiff_t>(head));
-            head = 0;
-        }
-        return p;
-    }
 };
 
 struct CachedPlan {
@@ -176,7 +156,7 @@ struct World {
 
     std::mutex mu;
     std::condition_variable cv;
-    std::vector<RankQueue> queue;             // per rank
+    std::vector<CallQueue<OpParam>> queue;    // per rank
     u32 waiting = 0;                          // ranks whose queue is not empty
     std::vector<OpParam> current;             // the calls of the collective being run, by rank
     std::vector<u64> launched;                // per rank: collectives completed so far
