@@ -267,8 +267,8 @@ HcclResult SubmitOp(RankComm *rc, OpParam &&param)
     World *w = rc->world;
     std::unique_lock<std::mutex> lock(w->mu);
     CallQueue<OpParam> &mine = w->queue[rc->rank];
-    if (mine.empty()) ++w->waiting;
-    mine.Push(std::move(param));
+    mine.Push(std::move(param));   // counted only once it is in the queue: there may be no memory for it
+    if (mine.size() == 1) ++w->waiting;
     const u64 myTicket = w->launched[rc->rank] + mine.size();  // collective number of this call
 
     while (w->waiting == w->rankSize) {

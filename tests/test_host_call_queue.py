@@ -25,3 +25,11 @@ def test_a_call_is_moved_a_bounded_number_of_times(queue, waiting):
     # least doubles: 2
     assert moves <= 5 * out
     assert most <= 4 * max(64, waiting) and left <= 64
+
+
+def test_a_call_that_could_not_be_queued_does_not_count(tmp_path):
+    exe = str(tmp_path / "check_failed_push")
+    subprocess.run(["g++", "-std=c++17", "-O1", f"-I{ROOT}/include", os.path.join(ROOT, "tests", "check_failed_push.cpp"), "-o", exe,
+                    f"-L{LIB}", "-lhccl_amd", f"-Wl,-rpath,{LIB}"], check=True)
+    run = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert run.returncode == 0 and run.stdout == "ok\n", (run.returncode, run.stderr[-2000:])
