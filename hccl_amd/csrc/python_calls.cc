@@ -160,6 +160,7 @@ struct Method {
     PyObject *comms;   // the attribute's name
     Py_ssize_t nargs;  // of the method
     unsigned char order[kMaxArgs];
+    PyObject *weakrefs;
     vectorcallfunc vectorcall;
 };
 
@@ -236,6 +237,7 @@ PyObject *make_method(PyTypeObject *type, PyObject *args, PyObject *)
 void drop_method(PyObject *self)
 {
     Method *m = reinterpret_cast<Method *>(self);
+    if (m->weakrefs != nullptr) PyObject_ClearWeakRefs(self);
     Py_XDECREF(reinterpret_cast<PyObject *>(m->call));
     Py_XDECREF(m->function);
     Py_XDECREF(m->comms);
@@ -251,7 +253,41 @@ PyObject *bind_method(PyObject *self, PyObject *object, PyObject *)
     return PyMethod_New(self, object);
 }
 
-// what inspect, help() and the like look at
+// What a program asks of a method is what the function says: its name, module, documentation, code and class, and attributes of
+// the program's own.
+PyObject *method_attribute(PyObject *self, PyObject *name)
+{
+    PyObject *found = PyObject_GenericGetAttr(self, name);
+    if (found != nullptr || !PyErr_ExceptionMatches(PyExc_AttributeError)) return found;
+    PyErr_Clear();
+    return PyObject_GetAttr(reinterpret_cast<Method *>(self)->function, name);
+}
+
+int set_method_attribute(PyObject *self, PyObject *name, PyObject *value)
+{
+    return PyObject_SetAttr(reinterpret_cast<Method *>(self)->function, name, value);
+}
+
+PyObject *repr_method(PyObject *self) { return PyObject_Repr(reinterpret_cast<Method *>(self)->function); }
+
+// (these two the type of any object has, so the lookup above would end there)
+PyObject *of_the_function(PyObject *self, void *name)
+{
+    return PyObject_GetAttrString(reinterpret_cast<Method *>(self)->function, static_cast<const char *>(name));
+}
+char g_doc[] = "__doc__";
+char g_class[] = "__class__";
+PyGetSetDef g_method_getset[] = {{g_doc, of_the_function, nullptr, nullptr, g_doc},
+                                 {g_class, of_the_function, nullptr, nullptr, g_class},
+                                 {nullptr, nullptr, nullptr, nullptr, nullptr}};
+
+// pickled and copied by name, as a function is
+PyObject *reduce_method(PyObject *self, PyObject *)
+{
+    return PyObject_GetAttrString(reinterpret_cast<Method *>(self)->function, "__qualname__");
+}
+PyMethodDef g_method_methods[] = {{"__reduce__", reduce_method, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
+
 PyMemberDef g_method_members[] = {{"__wrapped__", T_OBJECT, offsetof(Method, function), READONLY, nullptr},
                                   {nullptr, 0, 0, 0, nullptr}};
 
@@ -281,6 +317,12 @@ PyMODINIT_FUNC PyInit__hccl_calls(void)
     g_method_type.tp_dealloc = drop_method;
     g_method_type.tp_descr_get = bind_method;
     g_method_type.tp_members = g_method_members;
+    g_method_type.tp_getset = g_method_getset;
+    g_method_type.tp_methods = g_method_methods;
+    g_method_type.tp_getattro = method_attribute;
+    g_method_type.tp_setattro = set_method_attribute;
+    g_method_type.tp_repr = repr_method;
+    g_method_type.tp_weaklistoffset = offsetof(Method, weakrefs);
     if (PyType_Ready(&g_method_type) < 0) return nullptr;
     PyObject *m = PyModule_Create(&g_module);
     if (m == nullptr) return nullptr;

@@ -1,12 +1,18 @@
 """The native callables behind the Python face (csrc/python_calls.cc) against ctypes: same results and codes, and what they do
 not take is left to ctypes.  Dry worlds: nothing here touches a GPU."""
+import copy
 import ctypes
 import enum
+import functools
+import inspect
 import os
+import pickle
 import subprocess
 import sys
 import sysconfig
 import threading
+import types
+import weakref
 
 import pytest
 
@@ -174,3 +180,24 @@ def test_ranks_that_run_ahead(world):
     for k, c in enumerate(counts):
         wrong = k in (70, 199)
         assert (world.all_to_all(1, 2 << 20, c + wrong, 11 << 20, T.FP32, 1) != 0) == wrong
+
+
+@pytest.mark.parametrize("name", ["all_reduce", "reduce_scatter", "reduce_scatter_v", "all_gather", "all_gather_v", "all_to_all_v", "all_to_all",
+                                  "all_to_all_vc"])
+def test_a_native_method_is_a_function_to_a_program(world, name):
+    """What tracing decorators, documentation tools and pickle ask of a method."""
+    for m in (getattr(api.World, name), getattr(world, name)):
+        assert (m.__name__, m.__qualname__, m.__module__) == (name, "World." + name, "hccl_amd.api")
+        assert m.__doc__ is None and m.__code__.co_varnames[:2] == ("self", "rank")
+        assert name in repr(m) and weakref.ref(m)() is m
+    m = getattr(api.World, name)
+    assert type(m).__name__ == "Method" and inspect.isfunction(m) and inspect.isroutine(m) and isinstance(m, types.FunctionType)
+    assert name in dict(inspect.getmembers(api.World, inspect.isfunction)) and inspect.ismethod(getattr(world, name))
+    assert list(inspect.signature(m).parameters)[:2] == ["self", "rank"] and "rank" in inspect.signature(getattr(world, name)).parameters
+    assert pickle.loads(pickle.dumps(m)) is m and copy.copy(m) is m and copy.deepcopy(m) is m
+    assert weakref.WeakMethod(getattr(world, name))() == getattr(world, name)
+    assert functools.wraps(m)(lambda *a: None).__name__ == name
+    m.seen = 5
+    assert getattr(world, name).seen == 5
+    del m.seen
+    assert not hasattr(m, "seen") and not hasattr(m, "no_such_name")
