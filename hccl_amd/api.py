@@ -71,19 +71,19 @@ def lib():
         _all_reduce, _reduce_scatter, _reduce_scatter_v, _all_gather, _all_gather_v, _all_to_all_v, _all_to_all, _all_to_all_vc = (
             _lib.native_call(name) for name in ("HcclAllReduce", "HcclReduceScatter", "HcclReduceScatterV", "HcclAllGather",
                                                 "HcclAllGatherV", "HcclAlltoAllV", "HcclAlltoAll", "HcclAlltoAllVC"))
-        t = _lib.table
-        for call, function, places in (
-                (_all_reduce, World.all_reduce, (2, 3, 4, 5, 6, _lib.COMM, 7)),
-                (_reduce_scatter, World.reduce_scatter, (2, 3, 4, 5, 6, _lib.COMM, 7)),
-                (_reduce_scatter_v, World.reduce_scatter_v, (2, t(3), t(4), 5, 6, 7, 8, _lib.COMM, 9)),
-                (_all_gather, World.all_gather, (2, 3, 4, 5, _lib.COMM, 6)),
-                (_all_gather_v, World.all_gather_v, (2, 3, 4, t(5), t(6), 7, _lib.COMM, 8)),
-                (_all_to_all_v, World.all_to_all_v, (2, t(3), t(4), 8, 5, t(6), t(7), 8, _lib.COMM, 9)),
-                (_all_to_all, World.all_to_all, (2, 3, 5, 4, 3, 5, _lib.COMM, 6)),
-                (_all_to_all_vc, World.all_to_all_vc, (2, t(3), 5, 4, 5, _lib.COMM, 6))):
-            method = _lib.native_method(call, function, places)
-            if method is not None:
-                setattr(World, function.__name__, method)
+        for call, name, places in (
+                (_all_reduce, "all_reduce", (2, 3, 4, 5, 6, _lib.COMM, 7)),
+                (_reduce_scatter, "reduce_scatter", (2, 3, 4, 5, 6, _lib.COMM, 7)),
+                (_reduce_scatter_v, "reduce_scatter_v", (2, _t(3), _t(4), 5, 6, 7, 8, _lib.COMM, 9)),
+                (_all_gather, "all_gather", (2, 3, 4, 5, _lib.COMM, 6)),
+                (_all_gather_v, "all_gather_v", (2, 3, 4, _t(5), _t(6), 7, _lib.COMM, 8)),
+                (_all_to_all_v, "all_to_all_v", (2, _t(3), _t(4), 8, 5, _t(6), _t(7), 8, _lib.COMM, 9)),
+                (_all_to_all, "all_to_all", (2, 3, 5, 4, 3, 5, _lib.COMM, 6)),
+                (_all_to_all_vc, "all_to_all_vc", (2, _t(3), 5, 4, 5, _lib.COMM, 6))):
+            method = _lib.native_method(call, _written[name], places)
+            # (a program may have put a method of its own in the place of one before it made a communicator: that one stays)
+            if method is not None and World.__dict__.get(name) is _written[name]:
+                setattr(World, name, method)
         _bound = True
     return L
 
@@ -102,6 +102,7 @@ def u64_table(seq):
 
 
 _u64 = u64_table
+_t = _lib.table
 
 
 class World:
@@ -219,3 +220,8 @@ class World:
             return rc
         return lib().HcclAlltoAllVC(send, ctypes.cast(m, ctypes.c_void_p), int(dtype), recv, int(dtype),
                                     self.comms[rank], stream)
+
+
+# World's collectives as written above, whatever a program puts in their places
+_written = {name: World.__dict__[name] for name in ("all_reduce", "reduce_scatter", "reduce_scatter_v", "all_gather", "all_gather_v",
+                                                    "all_to_all_v", "all_to_all", "all_to_all_vc")}

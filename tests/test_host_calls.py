@@ -201,3 +201,27 @@ def test_a_native_method_is_a_function_to_a_program(world, name):
     assert getattr(world, name).seen == 5
     del m.seen
     assert not hasattr(m, "seen") and not hasattr(m, "no_such_name")
+
+
+PATCHED = """
+from hccl_amd import api
+seen = []
+def traced(of):
+    def call(*args, **kw):
+        seen.append(of.__name__)
+        return of(*args, **kw)
+    return call
+for name in ("all_reduce", "all_gather_v"):
+    setattr(api.World, name, traced(getattr(api.World, name)))
+w = api.World(2, dry=True)
+for r in range(2):
+    assert w.all_reduce(r, (r + 1) << 20, (r + 10) << 20, 100, 4, 0, 1) == 0
+    assert w.all_gather(r, (r + 1) << 20, (r + 10) << 20, 100, 4, 1) == 0
+assert seen == ["all_reduce"] * 2, seen
+assert type(api.World.__dict__["all_gather"]).__name__ == "Method"
+"""
+
+
+def test_methods_replaced_before_the_first_communicator_stay():
+    run = subprocess.run([sys.executable, "-c", PATCHED], cwd=ROOT, capture_output=True, text=True, timeout=60)
+    assert run.returncode == 0, run.stderr[-2000:]
