@@ -174,11 +174,14 @@ PyObject *call_method(PyObject *self, PyObject *const *args, size_t nargsf, PyOb
         const Py_ssize_t rank = PyLong_AsSsize_t(args[1]);
         if (rank == -1 && PyErr_Occurred()) PyErr_Clear();
         if (comms != nullptr && PyList_CheckExact(comms) && rank >= 0 && rank < PyList_GET_SIZE(comms)) {
+            // (held: asking an argument for its class may run code that empties the list)
+            PyObject *comm = PyList_GET_ITEM(comms, rank);
+            Py_INCREF(comm);
             PyObject *a[kMaxArgs];
             bool fits = true;
             for (Py_ssize_t k = 0; fits && k < m->call->nargs; ++k) {
                 if (m->order[k] == kTheComm) {
-                    a[k] = PyList_GET_ITEM(comms, rank);
+                    a[k] = comm;
                     continue;
                 }
                 a[k] = args[m->order[k] & (kTable - 1)];
@@ -190,6 +193,7 @@ PyObject *call_method(PyObject *self, PyObject *const *args, size_t nargsf, PyOb
             } else if (PyErr_Occurred()) {
                 PyErr_Clear();
             }
+            Py_DECREF(comm);
             Py_DECREF(comms);
             if (fits && result != Py_NotImplemented) return result;
             Py_XDECREF(result);

@@ -225,3 +225,25 @@ assert type(api.World.__dict__["all_gather"]).__name__ == "Method"
 def test_methods_replaced_before_the_first_communicator_stay():
     run = subprocess.run([sys.executable, "-c", PATCHED], cwd=ROOT, capture_output=True, text=True, timeout=60)
     assert run.returncode == 0, run.stderr[-2000:]
+
+
+EMPTIED_MEANWHILE = """
+import ctypes
+from hccl_amd import api
+w = api.World(2, dry=True)
+class Table(bytearray):
+    @property
+    def __class__(self):
+        w.comms.clear()
+        return type(api.u64_table([1]))
+try:
+    w.reduce_scatter_v(0, 1 << 20, Table(16), Table(16), 2 << 20, 0, 4, 0, 1)   # a call of the rank it was made for, or an error
+except (IndexError, TypeError):
+    pass
+print("ended")
+"""
+
+
+def test_an_argument_that_empties_the_communicators_while_it_is_looked_at():
+    run = subprocess.run([sys.executable, "-c", EMPTIED_MEANWHILE], cwd=ROOT, capture_output=True, text=True, timeout=60)
+    assert run.returncode == 0 and run.stdout == "ended\n", (run.returncode, run.stdout, run.stderr[-2000:])
