@@ -89,7 +89,7 @@ HcclResult SingleRankProc(const OpParam &param, u64 len, World *w)
     return static_cast<HcclResult>(hcclx_fold(&s, 1, HCCL_DATA_TYPE_INT8, 0, HCCLX_FOLD_CHAIN, param.stream));
 }
 
-// (The tag is filled in when a template gets to see it.)
+// (The tag is filled in when a selector or a template gets to see it.)
 void FillCommon(OpParam &p, RankComm *rc, HcclCMDType type, aclrtStream stream, const void *in, const void *out)
 {
     p.hcclComm = rc;

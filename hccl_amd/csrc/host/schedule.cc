@@ -243,7 +243,9 @@ HcclResult RunCollectiveOnStream(World *w, std::vector<OpParam> &params)
         topo.topoLevelNums = w->topoLevels;
         topo.level0Topo = w->topoShape;
         topo.localNetInsSizeOfLayer0 = w->devicesPerServer ? w->devicesPerServer : n;
-        if (type == HcclCMDType::HCCL_CMD_ALLTOALL) FillEqualTables(params[0], n);   // a selector may look at them
+        // a selector may look at the tag, and at the tables that an AlltoAll of equal counts does not carry
+        params[0].tag = OpTag(type);
+        if (type == HcclCMDType::HCCL_CMD_ALLTOALL) FillEqualTables(params[0], n);
         CHK_RET(ExecuteSelector().Run(params[0], &topo, algName));
     }
     w->lastAlgName = algName;

@@ -18,6 +18,12 @@ HcclResult SelectorRegistry::RegisterByOpType(HcclCMDType opType, u32 priority, 
     return HCCL_SUCCESS;
 }
 
+std::map<u32, AutoSelectorBase *> SelectorRegistry::GetSelectorsByOpType(HcclCMDType opType)
+{
+    std::lock_guard<std::mutex> lock(mu_);
+    return opTypeImpls_[opType];
+}
+
 AutoSelectorBase *SelectorRegistry::Next(HcclCMDType opType, bool first, u32 &priority)
 {
     std::lock_guard<std::mutex> lock(mu_);

@@ -46,6 +46,7 @@ class SelectorRegistry {
 public:
     static SelectorRegistry *Global();
     HcclResult RegisterByOpType(HcclCMDType opType, u32 priority, AutoSelectorBase *selector);
+    std::map<u32, AutoSelectorBase *> GetSelectorsByOpType(HcclCMDType opType);   // by priority number, lowest first
     // The selector of lowest priority number (first), or of the lowest beyond `priority`, which is set to its number; null
     // behind the last.
     AutoSelectorBase *Next(HcclCMDType opType, bool first, u32 &priority);

@@ -3,6 +3,7 @@ is added through the plugin API from a separately compiled shared object."""
 import ctypes
 import os
 import subprocess
+import sys
 
 import pytest
 
@@ -351,3 +352,64 @@ def test_strict_determinism_selects_the_order_preserved_reduce_scatter(monkeypat
     with pytest.raises(_lib.HcclError) as e:
         api.World(2, ccl_bytes=SMALL_CCL, dry=True)
     assert e.value.code == 1
+
+
+SELECTOR = r'''
+// A selector from outside the library that looks at what it is given and leaves the choice to the next one.
+#include "host/selector.h"
+using namespace ops_hccl;
+static std::string g_seen;
+class LookingSelector : public AutoSelectorBase {
+protected:
+    SelectorStatus SelectAicpuAlgo(const TopoInfoWithNetLayerDetails *, const OpParam &p, std::string &) const override
+    {
+        g_seen = p.tag + " " + std::to_string(p.all2AllVDataDes.sendCounts.size()) + " " + std::to_string(p.all2AllVDataDes.rdispls.size());
+        return SelectorStatus::NOT_MATCH;
+    }
+};
+extern "C" const char *seen() { return g_seen.c_str(); }
+extern "C" int others(int type)   // selectors of a type, this one among them
+{
+    return static_cast<int>(SelectorRegistry::Global()->GetSelectorsByOpType(static_cast<HcclCMDType>(type)).size());
+}
+extern "C" int add(int type) { return SelectorRegistry::Global()->RegisterByOpType(static_cast<HcclCMDType>(type), 1, new LookingSelector()); }
+'''
+
+
+def test_a_selector_from_outside_sees_the_tag_and_the_tables(tmp_path):
+    src = tmp_path / "selector.cc"
+    src.write_text(SELECTOR)
+    lib_dir = os.path.dirname(_lib.LIB_PATH)
+    subprocess.check_call(["g++", "-std=c++17", "-shared", "-fPIC", "-O1", "-I", os.path.join(ROOT, "include"), "-I",
+                           os.path.join(ROOT, "hccl_amd", "csrc"), str(src), "-o", str(tmp_path / "libselector.so"), "-L", lib_dir,
+                           "-lhccl_amd", "-Wl,-rpath," + lib_dir])
+    code = """
+import ctypes, sys
+from hccl_amd import _lib, api
+_lib.load()
+so = ctypes.CDLL(sys.argv[1])
+so.seen.restype = ctypes.c_char_p
+n = 3
+w = api.World(n, dry=True)
+at = lambda r, k: ((16 * k + r + 1) << 24)
+t = [0, 5, 10]
+calls = {
+    api.CMD_ALLREDUCE: (lambda r: w.all_reduce(r, at(r, 0), at(r, 1), 100, 4, 0, 1), "AllReduce_vworld 0 0"),
+    api.CMD_REDUCE_SCATTER: (lambda r: w.reduce_scatter(r, at(r, 0), at(r, 1), 100, 4, 0, 1), "ReduceScatter_vworld 0 0"),
+    api.CMD_REDUCE_SCATTER_V: (lambda r: w.reduce_scatter_v(r, at(r, 0), [5] * n, t, at(r, 1), 5, 4, 0, 1), "ReduceScatterV_vworld 0 0"),
+    api.CMD_ALLGATHER: (lambda r: w.all_gather(r, at(r, 0), at(r, 1), 100, 4, 1), "AllGather_vworld 0 0"),
+    api.CMD_ALLGATHER_V: (lambda r: w.all_gather_v(r, at(r, 0), 5, at(r, 1), [5] * n, t, 4, 1), "AllGatherV_vworld 0 0"),
+    api.CMD_ALLTOALL: (lambda r: w.all_to_all(r, at(r, 0), 5, at(r, 1), 4, 1), "ALLTOALL_vworld 3 3"),
+    api.CMD_ALLTOALLV: (lambda r: w.all_to_all_v(r, at(r, 0), [5] * n, t, at(r, 1), [5] * n, t, 4, 1), "ALLTOALLV_vworld 3 3"),
+    api.CMD_ALLTOALLVC: (lambda r: w.all_to_all_vc(r, at(r, 0), [5] * n * n, at(r, 1), 4, 1), "ALLTOALLVC_vworld 3 3"),
+}
+for cmd, (call, want) in calls.items():
+    before = so.others(cmd)
+    assert so.add(cmd) == 0 and so.others(cmd) == before + 1
+    for r in range(n):
+        assert call(r) == 0, cmd
+    assert so.seen().decode() == want, (so.seen(), want)
+    assert w.last_info().algName
+"""
+    run = subprocess.run([sys.executable, "-c", code, str(tmp_path / "libselector.so")], cwd=ROOT, capture_output=True, text=True, timeout=60)
+    assert run.returncode == 0, run.stderr[-2000:]
