@@ -596,9 +596,9 @@ k_moe_scatter_pieces(MoeConstPtrs tokens, MoeConstPtrs dest, MoeConstPtrs perm, 
 }
 
 // Gather the rows of a token's entries from where dispatch put them in expert[dest[.]] and add them, K entries at a time: their
-// look-ups and then their rows are in flight together.  Whatever an entry is, its lanes load from somewhere (a dropped one
-// from the result's own place): a branch per entry would make the compiler wait for every load before the next.  K by
-// gather_entries.  DT = int8 moves bytes (topk == 1).
+// look-ups are in flight together, and their rows too where all K are there.  (A branch per entry makes the compiler wait for
+// every load before the next.)  Where one is dropped or behind the last, those that are left are read one after the other, so
+// that what is dropped costs no bytes.  K by gather_entries.  DT = int8 moves bytes (topk == 1).
 template <int DT, int K>
 __global__ void __launch_bounds__(kPieceVecs * kPiecesPerBlock)
 k_moe_gather_pieces(MoeConstPtrs rows, MoeConstPtrs dest, MoeConstPtrs perm, MoePtrs out, uint32_t n, uint32_t topk, uint32_t vpr,
@@ -622,37 +622,48 @@ k_moe_gather_pieces(MoeConstPtrs rows, MoeConstPtrs dest, MoeConstPtrs perm, Moe
 #pragma unroll
     for (int k = 0; k < NE; ++k) acc[k] = C(0);
     char *to = static_cast<char *>(out.p[i]) + (static_cast<uint64_t>(t) * vpr + v0) * 16 + lane_off;
+    auto row = [&](uint32_t d, uint32_t p) {
+        return ld16(landing(as_mutable_dev(rows), i, d, n, esz, sdispls, rdispls) + (static_cast<uint64_t>(p) * vpr + v0) * 16 + lane_off);
+    };
+    auto add = [&](u32x4 raw) {
+        C x[NE];
+        V::unpack(raw, x);
+        if (!have) {
+#pragma unroll
+            for (int q = 0; q < NE; ++q) acc[q] = x[q];
+        } else {
+#pragma unroll
+            for (int q = 0; q < NE; ++q) acc[q] = V::template combine<HCCL_REDUCE_SUM>(x[q], acc[q]);
+        }
+        have = true;
+    };
     for (uint32_t first = 0; first < topk; first += K) {
         uint32_t p[K];
         uint32_t d[K];
         bool ok[K];
+        bool all = true;
 #pragma unroll
         for (int k = 0; k < K; ++k) {
             const uint32_t e = first + k < topk ? first + k : topk - 1;   // an entry behind the last repeats it and is not added
             p[k] = pm[e];
             d[k] = static_cast<uint32_t>(dt[e]);
         }
-        u32x4 raw[K];
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-            ok[k] = first + k < topk && p[k] != kDropped && d[k] < n;
-            const char *row = landing(as_mutable_dev(rows), i, ok[k] ? d[k] : 0u, n, esz, sdispls, rdispls) +
-                              (static_cast<uint64_t>(ok[k] ? p[k] : 0u) * vpr + v0) * 16 + lane_off;
-            raw[k] = ld16(ok[k] ? row : to);
+            ok[k] = (first + k < topk) & (p[k] != kDropped) & (d[k] < n);   // without branches between the look-ups
+            all = all & ok[k];
         }
+        if (K > 1 && all) {
+            u32x4 raw[K];
 #pragma unroll
-        for (int k = 0; k < K; ++k) {
-            if (!ok[k]) continue;
-            C x[NE];
-            V::unpack(raw[k], x);
-            if (!have) {
+            for (int k = 0; k < K; ++k) raw[k] = row(d[k], p[k]);
 #pragma unroll
-                for (int q = 0; q < NE; ++q) acc[q] = x[q];
-            } else {
+            for (int k = 0; k < K; ++k) add(raw[k]);
+        } else {
 #pragma unroll
-                for (int q = 0; q < NE; ++q) acc[q] = V::template combine<HCCL_REDUCE_SUM>(x[q], acc[q]);
+            for (int k = 0; k < K; ++k) {
+                if (ok[k]) add(row(d[k], p[k]));
             }
-            have = true;
         }
     }
     st16(to, V::pack(acc));

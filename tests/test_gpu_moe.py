@@ -280,6 +280,37 @@ def test_entries_of_a_token_in_flight_together(topk, dtype, width, n, tokens):
     test_fused_dispatch_and_gather_combine_equal_the_two_pass_pipeline(topk, dtype, width, n, tokens)
 
 
+def gather_time(n, tokens, topk, hidden, dropped):
+    """us of a gather in which this share of the entries is dropped, the least of several groups of launches."""
+    entries = tokens * topk
+    rng = np.random.default_rng(5)
+    dests = [np.where(rng.random(entries) < dropped, n, rng.integers(0, n, size=entries)) for _ in range(n)]
+    tabs, perm = route_on_gpu(dests, n, entries, hidden)
+    d = [dev_i32(x) for x in dests]
+    landed = (tabs[2].view(n, n).sum(1) // hidden).tolist()
+    rows = [torch.zeros(max(1, r) * hidden, dtype=torch.int16, device=DEV) for r in landed]
+    out = [torch.zeros(tokens * hidden, dtype=torch.int16, device=DEV) for _ in range(n)]
+    ptrs = [[x.data_ptr() for x in t] for t in (rows, d, perm, out)]
+    start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    times = []
+    for _ in range(8):
+        torch.cuda.synchronize()
+        start.record()
+        for _ in range(5):
+            hcclx.moe_gather_combine(*ptrs[:3], tokens, topk, hidden, T.BFP16, tabs[1].data_ptr(), tabs[3].data_ptr(), ptrs[3])
+        end.record()
+        torch.cuda.synchronize()
+        times.append(start.elapsed_time(end) / 5e-3)
+    return min(times)
+
+
+@pytest.mark.parametrize("topk,share", [(1, 0.75), (2, 0.62)])
+def test_entries_that_are_dropped_cost_no_bytes(topk, share):
+    """A gather of which every entry is dropped only writes.  Measured 0.48 and 0.52 of the time with none dropped; 0.95 and 0.75
+    when a dropped entry read something from HBM."""
+    assert gather_time(8, 4096, topk, 7168, 1.0) < share * gather_time(8, 4096, topk, 7168, 0.0)
+
+
 @pytest.mark.parametrize("topk,tokens,hidden", [(5, 4200, 8192), (3, 700, 7168)])
 def test_dispatch_of_tokens_beyond_the_cache(topk, tokens, hidden):
     """The first: 264 MiB of tokens, four entries per wavefront and a rest of one, stored through the L2."""
