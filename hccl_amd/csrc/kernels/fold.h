@@ -35,7 +35,7 @@ constexpr int kFoldThreads = HCCLX_FOLD_THREADS;
 //          the others off).  ReduceScatter among 8 ranks, us, G = 8 and U = 4 : these shapes, same run: small 6 MiB odd 12.9 :
 //          12.4, 16 MiB odd 31.3 : 27.9; one 64 MiB 95.2 : 92.1, 72 MiB 107.7 : 100.8; large 500 MiB bf16 821 : 749, fp32 888 :
 //          782.  Which one: wide_shape_for.
-constexpr int kWideGroup = 8;        // pointers fetched together
+constexpr int kWideGroup = 8;        // sources whose loads (many) or pointers (the others) are fetched together
 enum WideShape : int { kWideMany, kWideSmall, kWideOne, kWideLarge };
 __host__ __device__ constexpr int wide_vecs(int shape) { return shape == kWideOne ? 4 : shape == kWideLarge ? 8 : 2; }
 __host__ __device__ constexpr int wide_group(int shape) { return shape == kWideMany ? kWideGroup : 1; }
@@ -754,8 +754,11 @@ k_fold_waves(const uint64_t *__restrict__ tile_end, const SegDev *__restrict__ s
     }
 }
 
-// More than kMaxFan sources or destinations, or one destination, chain order: the sources are walked in groups of G, each
-// group loaded before it is folded in; the pointers of kWideGroup sources are fetched together, ahead of their loads.
+// More than kMaxFan sources or destinations, or one destination, chain order.  G = kWideGroup: the sources behind the first are
+// walked in groups, each group loaded before it is folded in.  G = 1: one source at a time, the pointers of kWideGroup sources
+// fetched together, ahead of their loads.  (Groups that fetch their pointers first and begin at source 0 are slower, the more
+// sources the more: int32, this way : that way, us: 9 x 256 KiB to nine places 3.5 : 3.9, 32 x 256 KiB 10.7 : 12.6, 64 x 1 MiB
+// 27.3 : 32.6, fp32 33 x 512 KiB to one 8.7 : 11.4; only from 2 MiB x 16 on up to a tenth faster, 24 x 4 MiB 31.9 : 29.0.)
 template <int DT, int OP, int U, int G, int T, bool CHECK>
 __device__ __forceinline__ void fold_tile_wide(const SegWide &sd, uint32_t nsrc, uint32_t ndst, uint64_t v0, uint64_t nvec,
                                                uint32_t head_bytes, uint32_t policy)
@@ -763,12 +766,15 @@ __device__ __forceinline__ void fold_tile_wide(const SegWide &sd, uint32_t nsrc,
     using V = Vec16<DT>;
     using C = typename V::C;
     constexpr int NE = V::NE;
+    static_assert(G == 1 || G == kWideGroup, "one source at a time, or a group");
     bool ok[U];
     uint64_t off[U];
     C acc[U][NE];
     const char *from[kWideGroup];
+    if constexpr (G == 1) {
 #pragma unroll
-    for (int k = 0; k < kWideGroup; ++k) from[k] = sd.src[static_cast<uint32_t>(k) < nsrc ? k : 0];
+        for (int k = 0; k < kWideGroup; ++k) from[k] = sd.src[static_cast<uint32_t>(k) < nsrc ? k : 0];
+    }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const uint64_t v = v0 + static_cast<uint64_t>(u) * T;
@@ -776,44 +782,54 @@ __device__ __forceinline__ void fold_tile_wide(const SegWide &sd, uint32_t nsrc,
         // unconditional, so all of a group are in flight at once as in the unchecked tile.
         ok[u] = !CHECK || v < nvec;
         off[u] = head_bytes + (ok[u] ? v : 0) * 16;
-        V::unpack(ld16(from[0] + off[u]), acc[u]);
+        V::unpack(ld16((G == 1 ? from[0] : sd.src[0]) + off[u]), acc[u]);
     }
     const uint64_t flips = sd.leaf_mask;
-    for (uint32_t base = 0; base < nsrc; base += kWideGroup) {
-        if (base != 0) {
+    auto fold_in = [&](uint32_t k, const u32x4 (&raw)[U]) {
 #pragma unroll
-            for (int k = 0; k < kWideGroup; ++k) from[k] = sd.src[base + k < nsrc ? base + k : 0];
+        for (int u = 0; u < U; ++u) {
+            C x[NE];
+            V::unpack(raw[u], x);
+            if (OperandOrderMatters<DT, OP>::value && ((flips >> k) & 1u)) {
+#pragma unroll
+                for (int e = 0; e < NE; ++e) acc[u][e] = V::template combine<OP>(acc[u][e], x[e]);
+            } else {
+#pragma unroll
+                for (int e = 0; e < NE; ++e) acc[u][e] = V::template combine<OP>(x[e], acc[u][e]);
+            }
         }
+    };
+    if constexpr (G == 1) {
+        for (uint32_t base = 0; base < nsrc; base += kWideGroup) {
+            if (base != 0) {
 #pragma unroll
-        for (int k0 = 0; k0 < kWideGroup; k0 += G) {
-            u32x4 raw[U][G];
+                for (int k = 0; k < kWideGroup; ++k) from[k] = sd.src[base + k < nsrc ? base + k : 0];
+            }
 #pragma unroll
-            for (int g = 0; g < G; ++g) {
-                const uint32_t k = base + k0 + g;
-                if (k != 0 && k < nsrc) {
+            for (int k = 0; k < kWideGroup; ++k) {
+                if (base + k != 0 && base + k < nsrc) {
+                    u32x4 raw[U];
 #pragma unroll
-                    for (int u = 0; u < U; ++u) raw[u][g] = ld16(from[k0 + g] + off[u]);
+                    for (int u = 0; u < U; ++u) raw[u] = ld16(from[k] + off[u]);
+                    fold_in(base + k, raw);
+                }
+                asm volatile("" ::: "memory");   // one source's loads at a time
+            }
+        }
+    } else {
+        for (uint32_t base = 1; base < nsrc; base += G) {
+            u32x4 raw[G][U];
+#pragma unroll
+            for (int k = 0; k < G; ++k) {
+                if (base + k < nsrc) {
+#pragma unroll
+                    for (int u = 0; u < U; ++u) raw[k][u] = ld16(sd.src[base + k] + off[u]);
                 }
             }
 #pragma unroll
-            for (int g = 0; g < G; ++g) {
-                const uint32_t k = base + k0 + g;
-                if (k != 0 && k < nsrc) {
-#pragma unroll
-                    for (int u = 0; u < U; ++u) {
-                        C x[NE];
-                        V::unpack(raw[u][g], x);
-                        if (OperandOrderMatters<DT, OP>::value && ((flips >> k) & 1u)) {
-#pragma unroll
-                            for (int e = 0; e < NE; ++e) acc[u][e] = V::template combine<OP>(acc[u][e], x[e]);
-                        } else {
-#pragma unroll
-                            for (int e = 0; e < NE; ++e) acc[u][e] = V::template combine<OP>(x[e], acc[u][e]);
-                        }
-                    }
-                }
+            for (int k = 0; k < G; ++k) {
+                if (base + k < nsrc) fold_in(base + k, raw[k]);
             }
-            if (G < kWideGroup) asm volatile("" ::: "memory");   // one step's loads at a time
         }
     }
     for (uint32_t base = 0; base < ndst; base += kMaxFan) {

@@ -118,3 +118,24 @@ def test_tree_to_one_destination_with_fewer_workgroups(nsrc, mib):
     for d, s in steps:
         xs[d] = xs[s] + xs[d]
     assert torch.equal(out.view(torch.int32), xs[0].view(torch.int32))
+
+
+@pytest.mark.parametrize("nsrc", [9, 10, 16, 17, 18, 25, 33, 57, 64])
+@pytest.mark.parametrize("ndst", [1, 3])
+def test_chain_in_groups_of_sources(nsrc, ndst):
+    """Small chains take eight sources at a time behind the first: last groups of one, of eight and in between, with the operands of
+    every third step turned round."""
+    n = 5003
+    xs = [device_payload(T.FP32, n + 8, 100 + k) for k in range(nsrc)]
+    for k, x in enumerate(xs):
+        x[k::11] = -0.0
+        x[k + 1::11] = 0.0
+    flips = [k % 3 == 2 for k in range(nsrc)]
+    outs = [torch.full((n + 8,), 77.0, device="cuda:0") for _ in range(ndst)]
+    torch.cuda.synchronize()
+    hcclx.fold_wide([(n, [x.data_ptr() + 4 for x in xs], [o.data_ptr() + 4 for o in outs], [int(f) for f in flips])], T.FP32, T.MAX)
+    torch.cuda.synchronize()
+    want = chain([x[1:n + 1] for x in xs], T.FP32, T.MAX, flips)
+    for o in outs:
+        assert torch.equal(o[1:n + 1].view(torch.int32), want.view(torch.int32))
+        assert bool((o[n + 1:] == 77).all()) and bool((o[:1] == 77).all())
