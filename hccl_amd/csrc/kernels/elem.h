@@ -117,8 +117,12 @@ template <int DT, int OP> struct Combine {
             return s + d;
         } else {
             C p = s * d;
-            if constexpr (D::kHalfFloat) {
-                p = D::widen(D::narrow(p));  // the CPU path narrows after every product
+            if constexpr (DT == HCCL_DATA_TYPE_FP16) {
+                // the CPU path narrows after every product.  A product of two halves is exact in fp32, so narrowing it is this
+                // half product; left to itself the compiler makes a fused multiply-add of +0 of the two, and -0 becomes +0
+                p = static_cast<C>(static_cast<_Float16>(s) * static_cast<_Float16>(d));
+            } else if constexpr (D::kHalfFloat) {
+                p = D::widen(D::narrow(p));
             }
             return p;
         }

@@ -514,3 +514,36 @@ def test_wide_self_first_many_ragged_segments():
         want = fold_oracle(whole, T.FP32, T.SUM, [r] + [k for k in range(64) if k != r], wide=False)
         assert_same_bits(outs[r].get(np.float32), want, T.FP32, f"rank {r}")
         assert outs[r].guard_intact()
+
+
+@pytest.mark.parametrize("nsrc", [2, 3, 4, 8, 9, 16, 17, 24, 40, 64])
+@pytest.mark.parametrize("how", ["chain to one", "chain to many", "self-first", "self-first in registers", "tree"])
+def test_products_of_halves_keep_the_sign_of_zero(nsrc, how):
+    """Every product of two halves is narrowed by itself: -0 stays -0 in every kernel, and products below the smallest half become
+    a zero of their sign."""
+    rng = np.random.default_rng(nsrc)
+    vals = np.array([0.0, -0.0, 1.0, -1.0, 0.5, -2.0, 1.5, 2.0**-24, -(2.0**-24), 2.0**-10, -(2.0**-12), 60000.0], dtype=np.float16)
+    n = (4 << 20) // 2 + 13 if how == "chain to one" and nsrc in (8, 9, 24) else 4096 + 13   # (the larger: another shape of kernel)
+    xs = [vals[rng.integers(0, vals.size if k < 3 else 7, size=n)].view(np.uint16) for k in range(nsrc)]
+    bufs = [DevBuf(x, offset=2 * (k % 3)) for k, x in enumerate(xs)]
+    outs = [DevBuf(nbytes=2 * n, offset=2 * (k % 5)) for k in range({"chain to one": 1, "chain to many": 3, "tree": 2}.get(how, nsrc))]
+    fold = hcclx.fold if nsrc <= 16 else hcclx.fold_wide
+    ptrs, dsts = [b.ptr for b in bufs], [o.ptr for o in outs]
+    orders = [list(range(nsrc))] * len(outs)
+    if how.startswith("self-first"):
+        orders = [[j] + [k for k in range(nsrc) if k != j] for j in range(nsrc)]
+        hcclx.tune("waves_from", 0 if how.endswith("registers") else 1)
+        try:
+            fold([(n, ptrs, dsts)], T.FP16, T.PROD, hcclx.FOLD_SELF_FIRST)
+        finally:
+            hcclx.tune("waves_from", 1)
+    elif how == "tree":
+        prog = split_tree(rng, nsrc, 6) if nsrc > 16 else split_tree(rng, nsrc, 4)
+        fold([(n, ptrs, dsts, prog)], T.FP16, T.PROD, hcclx.FOLD_TREE)
+    else:
+        fold([(n, ptrs, dsts)], T.FP16, T.PROD)
+    sync()
+    for o, order in zip(outs, orders):
+        want = tree_oracle(xs, T.FP16, T.PROD, prog, False) if how == "tree" else fold_oracle(xs, T.FP16, T.PROD, order, wide=False)
+        assert_same_bits(o.get(np.uint16), want, T.FP16, how)
+        assert o.guard_intact()
