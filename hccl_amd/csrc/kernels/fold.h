@@ -807,12 +807,14 @@ __device__ __forceinline__ void fold_tile_wide(const SegWide &sd, uint32_t nsrc,
             }
 #pragma unroll
             for (int k = 0; k < kWideGroup; ++k) {
+                // (two branches: the compiler then folds the last of a source's vectors in behind the first loads of the next;
+                // one branch: 8 ranks x 64 MiB fp32 90.0 -> 91.5 us, 12 x 100 int32 208 -> 214)
+                u32x4 raw[U];
                 if (base + k != 0 && base + k < nsrc) {
-                    u32x4 raw[U];
 #pragma unroll
                     for (int u = 0; u < U; ++u) raw[u] = ld16(from[k] + off[u]);
-                    fold_in(base + k, raw);
                 }
+                if (base + k != 0 && base + k < nsrc) fold_in(base + k, raw);
                 asm volatile("" ::: "memory");   // one source's loads at a time
             }
         }
