@@ -147,6 +147,7 @@ void init_slot(DeviceSlot *s, int dev)
         if (b == 1 || b == 2) c.moe_scatter_rows = static_cast<uint32_t>(b);
     }
     if (const char *v = std::getenv("HCCLX_STORE_THROUGH_UPTO")) c.store_through_upto = std::strtoull(v, nullptr, 10);
+    if (const char *v = std::getenv("HCCLX_FOLD_LDS_HOLD")) c.fold_lds_hold = std::strtoul(v, nullptr, 10) != 0;
     c.ring_bytes = kSliceBytes * kSlices;
     e = hipHostMalloc(reinterpret_cast<void **>(&c.h_ring), c.ring_bytes, hipHostMallocCoherent);
     if (e != hipSuccess) {
@@ -423,7 +424,7 @@ struct Batch {
     std::vector<SegDev> segs;
     std::vector<SegWide> wide;   // instead of segs when maxn == kMaxWideFan
     int wide_shape = 0;          // of the wide kernels: a WideShape or a TreeShape (fold.h)
-    uint32_t per_cu = 0;         // non-zero: so many workgroups of the launch to a CU at most
+    uint32_t per_cu = 0;         // non-zero: LDS holds more workgroups of the launch than this off a CU
     uint32_t xcd_remap = 0;      // wide kernels: contiguous tile ranges per XCD (pays with 16 or more destinations)
     BlockLaunch blocks;          // instead of everything above: a launch of the block copy kernel
     PhasedLaunch phased;         // instead of everything above: a launch of the copy kernel that writes one output at a time
@@ -907,9 +908,11 @@ int build_batches_impl(const hcclx_seg_t *segs, uint32_t nseg, int dtype, int op
         proto.waves_team = waves_team;
     }
     proto.store_policy = store_policy_for(device_ctx(), segs, nseg, sp.copy ? 1 : dtype_size(dtype));
-    // Trees over more than eight leaf slots to one place: from 64 MiB on four workgroups to a CU, as the chains (fold.h; fp32
-    // NHR AllReduce 12 x 64 MiB 256 : 252 us, ReduceScatter 16 x 64 191 : 186; 12 x 8 MiB 39.6 : 40.7)
-    if (sp.mode == HCCLX_FOLD_TREE && sp.maxn > 8) {
+    // Trees over more than eight leaf slots to one place: from 64 MiB on LDS holds them to four workgroups to a CU (fp32 NHR
+    // AllReduce 12 x 64 MiB 256 : 252 us, ReduceScatter 16 x 64 191 : 186; 12 x 8 MiB 39.6 : 40.7).  Beside work on another stream
+    // nothing is lost (16 AllReduces of 16 x 64 MiB with a kernel of 64 KiB LDS 8584 : 8453, with matrix products 10266 : 10200).
+    const DeviceCtx *ctx = device_ctx();
+    if (sp.mode == HCCLX_FOLD_TREE && sp.maxn > 8 && ctx && ctx->fold_lds_hold) {
         uint64_t bytes = 0;
         bool one = true;
         for (uint32_t i = 0; i < nseg; ++i) {
@@ -961,24 +964,26 @@ int build_wide_batches(const hcclx_wide_seg_t *segs, uint32_t nseg, int dtype, i
     return HCCL_SUCCESS;
 }
 
-// The shape of a chain launch with one destination (fold.h) and how many of its workgroups share a CU.  Straddling: sources
-// that do not share the destination's alignment, so that loads straddle lines.  Kernels among 8 ranks unless said, us:
-//   many   fewer tiles of `one` than wide_min_tiles, unless they straddle and are 4 MiB or more: eight loads at a time hide more
+}  // namespace
+
+// The shape of a chain launch with one destination (fold.h).  Straddling: sources that do not share the destination's
+// alignment, so that loads straddle lines.  Kernels among 8 ranks unless said, us:
+//   many   fewer tiles of `three` than wide_min_tiles, unless they straddle and are 4 MiB or more: eight loads at a time hide more
 //          latency (many : small: 2 MiB bf16 6.9 : 7.5, 16 ranks x 4 MiB 13.9 : 16.0; 6 MiB odd 13.0 : 12.4).
-//   small  straddling below 32 MiB (one : small: 16 MiB bf16 31.0 : 27.9, 25 46.0 : 43.8; 40 MiB fp32 59.1 : 62.1).
-//   large  from 128 MiB on (one : large: 150 MiB bf16 246 : 229, 12 x 150 fp32 AllReduce 624 : 605, 12 x 1 GiB int32
+//   small  straddling below 32 MiB (three or four : small: 16 MiB bf16 31.0 : 27.9, 25 46.0 : 43.8; 40 MiB fp32 59.1 : 62.1).
+//   large  from 128 MiB on (three or four : large: 150 MiB bf16 246 : 229, 12 x 150 fp32 AllReduce 624 : 605, 12 x 1 GiB int32
 //          4395 : 4295; below it the last round of its 64 KiB tiles shows: 72 MiB 100.8 : 105.1), straddling elements of at
 //          least 4 bytes (200 MiB fp32 323 : 315; 400 MiB bf16 691 : 704).
-//   one    otherwise, three or four workgroups to a CU, whichever leaves less of the last round empty (three : four: 25 MiB
-//          40.2 : 38.8, 16 x 40 109.9 : 111.5, 24 x 20 AllReduce 157 : 168, 32 x 16 91.6 : 82.9; two, five and more: slower).
-int wide_shape_for(const DeviceCtx *ctx, const hcclx_wide_seg_t *segs, uint32_t nseg, int esz, uint32_t *per_cu)
+//   three, four   otherwise, whichever leaves less of the last round empty (three : four: 25 MiB 40.2 : 38.8, 16 x 40 109.9 :
+//          111.5, 24 x 20 AllReduce 157 : 168, 32 x 16 91.6 : 82.9; two, five and more to a CU: slower).
+WideShape wide_shape_for(const DeviceCtx *ctx, const hcclx_wide_seg_t *segs, uint32_t nseg, int esz, uint32_t *per_cu)
 {
     constexpr uint64_t kLargeFrom = 128ull << 20;
     constexpr uint64_t kSmallFrom = 4ull << 20;
     constexpr uint64_t kSmallUpto = 32ull << 20;
     *per_cu = 0;
     if (ctx == nullptr) return kWideMany;
-    const uint64_t tile_bytes = 16 * wide_tile_vecs(kWideOne);
+    const uint64_t tile_bytes = 16 * wide_tile_vecs(kWideThree);
     uint64_t bytes = 0;
     uint64_t tiles = 0;
     bool straddling = false;
@@ -992,16 +997,17 @@ int wide_shape_for(const DeviceCtx *ctx, const hcclx_wide_seg_t *segs, uint32_t 
     }
     if (straddling && bytes >= kSmallFrom && bytes < kSmallUpto) return kWideSmall;
     if (bytes / tile_bytes < ctx->wide_min_tiles) return kWideMany;
-    if (bytes >= kLargeFrom && (!straddling || esz >= 4)) {
+    if (ctx->fold_lds_hold && bytes >= kLargeFrom && (!straddling || esz >= 4)) {
         *per_cu = 1;
         return kWideLarge;
     }
     const uint64_t cus = static_cast<uint64_t>(ctx->num_cus);
     const uint64_t three = 3 * ((tiles + 3 * cus - 1) / (3 * cus));
     const uint64_t four = 4 * ((tiles + 4 * cus - 1) / (4 * cus));
-    *per_cu = three <= four ? 3 : 4;
-    return kWideOne;
+    return three <= four ? kWideThree : kWideFour;
 }
+
+namespace {
 
 // Wide segments: chain order, up to kMaxWideFan sources and destinations, one kernel for every fan-in.
 int build_wide_batches_impl(const hcclx_wide_seg_t *segs, uint32_t nseg, int dtype, int op, int mode,
@@ -1266,6 +1272,8 @@ int hcclx_tune(const char *name, uint64_t value)
         ctx->moe_scatter_rows = static_cast<uint32_t>(value);
     } else if (key == "store_through_upto") {
         ctx->store_through_upto = value;
+    } else if (key == "fold_lds_hold") {
+        ctx->fold_lds_hold = value != 0;
     } else {
         return fail(HCCL_E_PARA, "unknown knob: " + key);
     }

@@ -5,6 +5,7 @@
 #include <string>
 #include <vector>
 #include "hccl_types.h"
+#include "hcclx.h"
 #include "kernels/launch.h"
 #include "kernels/vops.h"
 
@@ -74,6 +75,9 @@ struct DeviceCtx {
     uint32_t waves_pieces = 0;
     uint32_t moe_scatter_rows = 0;          // MoE dispatch of long rows: entries of a token per wavefront, 1 or 2; 0 = chosen per launch (HCCLX_MOE_SCATTER_ROWS)
     uint64_t store_through_upto = 320ull << 20;   // fold launches with several destinations that write no more than this store through the L2 (HCCLX_STORE_THROUGH_UPTO)
+    // Folds to one place that hold the workgroups of a CU few by LDS that they do not use (the largest chains and trees):
+    // HCCLX_FOLD_LDS_HOLD, 0 = they ask for none, and the largest chains take the shape of the next smaller ones.
+    bool fold_lds_hold = true;
     // Descriptor ring: tables of one-shot launches are written to pinned host memory and copied to the
     // device ring on the launch stream just before the kernel.
     char *h_ring = nullptr;
@@ -86,6 +90,9 @@ struct DeviceCtx {
 
 // Returns the context of the current device, creating it on first use (nullptr + error set on failure).
 DeviceCtx *device_ctx();
+
+// The shape of a chain launch with one destination; *per_cu: non-zero where LDS holds more workgroups than this off a CU.
+WideShape wide_shape_for(const DeviceCtx *ctx, const hcclx_wide_seg_t *segs, uint32_t nseg, int esz, uint32_t *per_cu);
 
 // Reserves `bytes` (multiple of 256) in the descriptor ring.  Blocks the host only when the ring wraps
 // onto a slice whose earlier launches have not finished.

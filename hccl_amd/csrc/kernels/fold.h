@@ -29,15 +29,20 @@ constexpr int kFoldThreads = HCCLX_FOLD_THREADS;
 // Shapes of the wide chain kernel: U vectors per thread, G sources loaded before the first of them is folded in, T threads.
 //   many   several destinations.  U = 2 measured 24 % faster on a 32-rank AllReduce than one vector with sixteen sources
 //          (the same loads outstanding, twice the contiguous run per source); U = 4 costs 5 %.
-//   small, one, large   a single destination.  One source at a time leaves room for more workgroups than G = 8 does (one: 62
-//          registers of bf16 against 174), and fewer of them than would fit read and write HBM faster: the workgroups of a CU
-//          then read for a while together and write together, where many small ones mix the two (LDS that nobody uses holds
-//          the others off).  ReduceScatter among 8 ranks, us, G = 8 and U = 4 : these shapes, same run: small 6 MiB odd 12.9 :
-//          12.4, 16 MiB odd 31.3 : 27.9; one 64 MiB 95.2 : 92.1, 72 MiB 107.7 : 100.8; large 500 MiB bf16 821 : 749, fp32 888 :
-//          782.  Which one: wide_shape_for.
+//   small, three, four, large   a single destination.  One source at a time leaves room for more workgroups than G = 8 does
+//          (U = 4, bf16: 75 registers against 176), and fewer of them than would fit read and write HBM faster: the workgroups
+//          of a CU then read for a while together and write together, where many small ones mix the two.  Three and four are
+//          one shape that asks for so many registers that three or four of its workgroups fill a CU's; one of `large` is
+//          held to a CU by LDS that nobody uses.  ReduceScatter among 8 ranks, us, G = 8 and U = 4 : these shapes, same run:
+//          small 6 MiB odd 12.9 : 12.4, 16 MiB odd 31.3 : 27.9; three or four 64 MiB bf16 95.2 : 89.0, fp32 95.6 : 91.8; large
+//          500 MiB bf16 821 : 749, fp32 888 : 782.  Which one: wide_shape_for.
+// Registers or LDS: both leave a CU's share of the other to kernels on other streams.  The same work side by side, us for all of
+// it, G = 8 and U = 4 : held by LDS : by registers.  Three and four (40 x 8 ranks x 64 MiB bf16) beside a kernel of 64 KiB
+// LDS 11481 : 12237 : 11403, products of 4096^3 7358 : 7162 : 7055, 4096 x 1024 x 7168 6652 : 7122 : 7012, 16384 x 256 x 4096
+// 7061 : 7068 : 7166, softmax 4415 : 4285 : 4191.  Large (20 x 8 x 128 MiB fp32) 11255 : 10991 : 11903, 7371 : 7483 : 7466, 7600 :
+// 6901 : 7583, 7706 : 6800 : 7052, 4328 : 4211 : 4391.  Alone they are equal.
 constexpr int kWideGroup = 8;        // sources whose loads (many) or pointers (the others) are fetched together
-enum WideShape : int { kWideMany, kWideSmall, kWideOne, kWideLarge };
-__host__ __device__ constexpr int wide_vecs(int shape) { return shape == kWideOne ? 4 : shape == kWideLarge ? 8 : 2; }
+__host__ __device__ constexpr int wide_vecs(int shape) { return shape == kWideThree || shape == kWideFour ? 4 : shape == kWideLarge ? 8 : 2; }
 __host__ __device__ constexpr int wide_group(int shape) { return shape == kWideMany ? kWideGroup : 1; }
 // Shapes of the wide tree kernel (one vector per thread):
 //   plain   256 threads
@@ -49,6 +54,16 @@ enum TreeShape : int { kTreePlain, kTreeLarge };
 constexpr uint64_t kTreeLargeFrom = 16ull << 20;
 __host__ __device__ constexpr int tree_threads(int shape, bool half_float) { return shape == kTreeLarge && !half_float ? 512 : kFoldThreads; }
 __host__ __device__ constexpr int wide_threads(int shape) { return shape == kWideLarge ? 512 : kFoldThreads; }
+// Threads of a workgroup of the wide kernels, and the most wavefronts of one that a SIMD takes (its registers are reserved for
+// no more; eight is what any kernel may have).
+__host__ __device__ constexpr int wide_kernel_threads(int mode, int shape, bool half_float)
+{
+    return mode == kFoldTree ? tree_threads(shape, half_float) : wide_threads(shape);
+}
+__host__ __device__ constexpr unsigned wide_most_waves(int mode, int shape)
+{
+    return mode != kFoldChain ? 8 : shape == kWideThree ? 3 : shape == kWideFour ? 4 : 8;
+}
 constexpr uint32_t kFoldDirectSegs = 64;   // up to this many segments the tile prefix is searched in place
 #ifndef HCCLX_TREE16_UNROLL
 #define HCCLX_TREE16_UNROLL 1   // vectors per thread of the tree over up to 16 leaf slots
@@ -1093,7 +1108,8 @@ k_fold_wide_waves(const uint64_t *__restrict__ tile_end, const SegWide *__restri
 }
 
 template <int DT, int OP, int MODE, int SHAPE>
-__global__ void __launch_bounds__(MODE == kFoldTree ? tree_threads(SHAPE, DTypeOf<DT>::kHalfFloat) : wide_threads(SHAPE))
+__global__ void __launch_bounds__(wide_kernel_threads(MODE, SHAPE, DTypeOf<DT>::kHalfFloat))
+__attribute__((amdgpu_waves_per_eu(wide_kernel_threads(MODE, SHAPE, DTypeOf<DT>::kHalfFloat) / 256, wide_most_waves(MODE, SHAPE))))
 k_fold_wide(const uint64_t *__restrict__ tile_end, const SegWide *__restrict__ segs, uint32_t nseg, uint64_t total_tiles,
             uint32_t xcd_remap, uint32_t store_policy, uint32_t uniform_tiles)
 {
@@ -1104,7 +1120,7 @@ k_fold_wide(const uint64_t *__restrict__ tile_end, const SegWide *__restrict__ s
     constexpr bool kTree = MODE == kFoldTree;
     constexpr int U = kTree ? 1 : wide_vecs(SHAPE);
     constexpr int G = wide_group(SHAPE);
-    constexpr int T = kTree ? tree_threads(SHAPE, DTypeOf<DT>::kHalfFloat) : wide_threads(SHAPE);
+    constexpr int T = wide_kernel_threads(MODE, SHAPE, DTypeOf<DT>::kHalfFloat);
     constexpr bool kPairs = kTree && SHAPE == kTreeLarge && DTypeOf<DT>::kHalfFloat;
     constexpr uint64_t TV = static_cast<uint64_t>(T) * U;
     extern __shared__ uint64_t s_end[];
@@ -1193,7 +1209,7 @@ struct FoldLaunch {
     uint64_t total_tiles;
     uint32_t grid;
     int wide_shape = 0;        // the wide kernels: a WideShape or a TreeShape
-    uint32_t per_cu = 0;       // non-zero: no more workgroups of the launch than this share a CU
+    uint32_t per_cu = 0;       // non-zero: LDS holds more workgroups of the launch than this off a CU
     uint32_t xcd_remap;        // the wide kernels: give each XCD a contiguous eighth of the tiles
     uint32_t store_policy;     // kStoreStream / kStoreThrough
     uint32_t uniform_tiles;    // non-zero: every segment has this many tiles, tile t belongs to segment t / uniform_tiles

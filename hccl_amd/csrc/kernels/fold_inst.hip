@@ -63,7 +63,7 @@ static hipError_t launch_waves(const FoldLaunch &l)
 template <int DT, int OP, int MODE, int SHAPE>
 static hipError_t launch_wide_shape(const FoldLaunch &l)
 {
-    constexpr int kThreads = MODE == kFoldTree ? tree_threads(SHAPE, DTypeOf<DT>::kHalfFloat) : wide_threads(SHAPE);
+    constexpr int kThreads = wide_kernel_threads(MODE, SHAPE, DTypeOf<DT>::kHalfFloat);
     const size_t lds = std::max<size_t>(l.nseg * sizeof(uint64_t), lds_for(l.per_cu));
     if (lds > 64 * 1024) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_fold_wide<DT, OP, MODE, SHAPE>),
@@ -97,7 +97,8 @@ static hipError_t launch_wide(const FoldLaunch &l)
     if constexpr (MODE == kFoldChain) {
         switch (l.wide_shape) {
             case kWideSmall: return launch_wide_shape<DT, OP, MODE, kWideSmall>(l);
-            case kWideOne: return launch_wide_shape<DT, OP, MODE, kWideOne>(l);
+            case kWideThree: return launch_wide_shape<DT, OP, MODE, kWideThree>(l);
+            case kWideFour: return launch_wide_shape<DT, OP, MODE, kWideFour>(l);
             case kWideLarge: return launch_wide_shape<DT, OP, MODE, kWideLarge>(l);
             default: return launch_wide_shape<DT, OP, MODE, kWideMany>(l);
         }

@@ -67,4 +67,7 @@ enum FoldMode : int {
     kFoldTree = 2,
 };
 
+// The shapes of the wide chain kernel (fold.h says what they are).
+enum WideShape : int { kWideMany, kWideSmall, kWideThree, kWideFour, kWideLarge };
+
 }  // namespace hcclx

@@ -97,6 +97,9 @@ const char *hcclx_last_error(void);
  *                     launches for which the register kernel is otherwise kept)
  *   "fanout_from"     bytes read and written from which a fold with several destinations is split into fold + fan-out
  *   "store_through_upto"  bytes written up to which multi-destination folds store through the L2
+ *   "fold_lds_hold"   0: folds to one place ask for no LDS beyond their tables (otherwise the largest chains hold 90 KiB of a
+ *                     CU's 160, trees over more than eight sources and from 64 MiB on 37 KiB for each of four workgroups, so
+ *                     that few of their workgroups share a CU; LDS of compute kernels on other streams is then scarcer)
  *   "moe_scatter_rows"  entries of a token per wavefront of the MoE dispatch of long rows (1 or 2; 0 = chosen per launch)
  * Plans made before the call keep the kernels they were made for.  The knobs are plain fields of the device's
  * context: set them while no other thread is planning a launch on that device.  Returns HCCL_E_PARA for an unknown
