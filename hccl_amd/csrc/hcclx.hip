@@ -1194,18 +1194,8 @@ hipError_t dispatch_fold(int dtype, int op, int maxn, int mode, const FoldLaunch
     }
 }
 
-int launch_batch(const DeviceCtx *ctx, const Batch &b, const char *d_table, hipStream_t stream)
+FoldLaunch fold_launch(const DeviceCtx *ctx, const Batch &b, const char *d_table, hipStream_t stream)
 {
-    if (b.phased.tiles != 0) {
-        const hipError_t pe = launch_phased_copy(b.phased.table(d_table), b.phased.grid, stream);
-        if (pe != hipSuccess) return fail_hip(pe, "phased copy kernel launch");
-        return HCCL_SUCCESS;
-    }
-    if (b.blocks.tiles != 0) {
-        const hipError_t be = launch_copy_blocks(b.blocks.table(d_table), b.blocks.blocks.size(), b.blocks.tiles, stream);
-        if (be != hipSuccess) return fail_hip(be, "block copy kernel launch");
-        return HCCL_SUCCESS;
-    }
     FoldLaunch l;
     l.tile_end = reinterpret_cast<const uint64_t *>(d_table);
     l.segs = d_table + align256(b.tile_end.size() * 8);
@@ -1221,7 +1211,37 @@ int launch_batch(const DeviceCtx *ctx, const Batch &b, const char *d_table, hipS
     l.pieces = b.pieces;
     l.waves_fixed = b.waves_fixed;
     l.waves_team = b.waves_team;
+    l.device = ctx->device;
     l.stream = stream;
+    return l;
+}
+
+// What HIP has to be told once about the kernels of these launches.
+int ready_kernels(const DeviceCtx *ctx, const Built &built)
+{
+    for (const Batch &b : built.batches) {
+        if (b.wide.empty()) continue;
+        FoldLaunch l = fold_launch(ctx, b, nullptr, nullptr);
+        l.ready_only = true;
+        const hipError_t e = dispatch_fold(b.dtype, b.op, b.maxn, b.mode, l);
+        if (e != hipSuccess) return fail_hip(e, "fold kernel attributes");
+    }
+    return HCCL_SUCCESS;
+}
+
+int launch_batch(const DeviceCtx *ctx, const Batch &b, const char *d_table, hipStream_t stream)
+{
+    if (b.phased.tiles != 0) {
+        const hipError_t pe = launch_phased_copy(b.phased.table(d_table), b.phased.grid, stream);
+        if (pe != hipSuccess) return fail_hip(pe, "phased copy kernel launch");
+        return HCCL_SUCCESS;
+    }
+    if (b.blocks.tiles != 0) {
+        const hipError_t be = launch_copy_blocks(b.blocks.table(d_table), b.blocks.blocks.size(), b.blocks.tiles, stream);
+        if (be != hipSuccess) return fail_hip(be, "block copy kernel launch");
+        return HCCL_SUCCESS;
+    }
+    const FoldLaunch l = fold_launch(ctx, b, d_table, stream);
     const hipError_t e = b.copy ? fold_dispatch_copy(l) : dispatch_fold(b.dtype, b.op, b.maxn, b.mode, l);
     if (e != hipSuccess) return fail_hip(e, "fold kernel launch");
     return HCCL_SUCCESS;
@@ -1284,6 +1304,8 @@ uint32_t hcclx_dtype_size(int dtype) { return static_cast<uint32_t>(dtype_size(d
 
 static int launch_built(DeviceCtx *ctx, const Built &built, hipStream_t st)
 {
+    const int ready = ready_kernels(ctx, built);
+    if (ready != HCCL_SUCCESS) return ready;
     for (const Batch &b : built.batches) {
         char *h = nullptr;
         char *d = nullptr;
@@ -1300,6 +1322,8 @@ static int launch_built(DeviceCtx *ctx, const Built &built, hipStream_t st)
 
 static int plan_from(DeviceCtx *ctx, Built &built, hcclx_plan_t **plan)
 {
+    const int ready = ready_kernels(ctx, built);
+    if (ready != HCCL_SUCCESS) return ready;
     hcclx_plan *p = new hcclx_plan;
     p->device = ctx->device;
     p->algo_bytes = built.algo_bytes;

@@ -1218,6 +1218,8 @@ struct FoldLaunch {
     uint32_t pieces = 1;       // and this many 1 KiB pieces per source and workgroup
     uint32_t waves_fixed = 0;  // non-zero: every segment of the launch has this many sources
     bool waves_team = false;   // chains: the wavefronts share the fold
+    bool ready_only = false;   // nothing is launched: the kernel is made ready for this launch on `device`
+    int device = 0;
     hipStream_t stream;
 };
 

@@ -6,8 +6,21 @@
 #include "fold.h"
 
 #include <algorithm>
+#include <atomic>
 
 namespace hcclx {
+
+// More than 64 KiB of dynamic LDS a kernel gets only when HIP has been asked for it: once per device, when a launch is built, so
+// that launching (a plan, inside a capture) is nothing but the launch.  `done`: the devices that have been asked.
+constexpr size_t kLdsUnasked = 64 * 1024;
+static hipError_t ask_for_lds(const void *kernel, size_t lds, int device, std::atomic<uint64_t> &done)
+{
+    const uint64_t bit = 1ull << (device & 63);
+    if (lds <= kLdsUnasked || (done.load(std::memory_order_acquire) & bit) != 0) return hipSuccess;
+    const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
+    if (e == hipSuccess) done.fetch_or(bit, std::memory_order_release);
+    return e;
+}
 
 template <int DT, int OP, int MAXN, int MODE>
 static hipError_t launch_one(const FoldLaunch &l)
@@ -65,10 +78,9 @@ static hipError_t launch_wide_shape(const FoldLaunch &l)
 {
     constexpr int kThreads = wide_kernel_threads(MODE, SHAPE, DTypeOf<DT>::kHalfFloat);
     const size_t lds = std::max<size_t>(l.nseg * sizeof(uint64_t), lds_for(l.per_cu));
-    if (lds > 64 * 1024) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_fold_wide<DT, OP, MODE, SHAPE>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
-        if (e != hipSuccess) return e;
+    if (l.ready_only) {
+        static std::atomic<uint64_t> done{0};
+        return ask_for_lds(reinterpret_cast<const void *>(&k_fold_wide<DT, OP, MODE, SHAPE>), lds, l.device, done);
     }
     HCCLX_LAUNCH((k_fold_wide<DT, OP, MODE, SHAPE>), dim3(l.grid), dim3(kThreads), lds, l.stream,
                        l.tile_end, static_cast<const SegWide *>(l.segs), l.nseg, l.total_tiles, l.xcd_remap, l.store_policy, l.uniform_tiles);
@@ -81,10 +93,9 @@ static hipError_t launch_wide_waves(const FoldLaunch &l)
 {
     const bool direct = l.nseg <= kFoldDirectSegs || l.uniform_tiles != 0;
     const size_t lds = static_cast<size_t>(l.waves) * kWaveLanes * 16 + (direct ? 0 : l.nseg * sizeof(uint64_t));
-    if (lds > 64 * 1024) {   // 64 sources and a staged prefix: more than a kernel gets unasked
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_fold_wide_waves<DT, OP, R>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
-        if (e != hipSuccess) return e;
+    if (l.ready_only) {   // (64 sources and a staged prefix)
+        static std::atomic<uint64_t> done{0};
+        return ask_for_lds(reinterpret_cast<const void *>(&k_fold_wide_waves<DT, OP, R>), lds, l.device, done);
     }
     HCCLX_LAUNCH((k_fold_wide_waves<DT, OP, R>), dim3(static_cast<uint32_t>(l.total_tiles)), dim3(kWideWaves * kWaveLanes), lds, l.stream,
                  l.tile_end, static_cast<const SegWide *>(l.segs), l.nseg, l.waves, l.pieces, l.uniform_tiles);

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from oracle import templates as T
-from hccl_amd import api
+from hccl_amd import api, hcclx
 
 from gpu_util import DevBuf, assert_same_bits, payload
 
@@ -183,3 +183,31 @@ def test_a_collective_without_a_plan_for_its_buffers_refuses_to_be_captured():
         del g
     finally:
         w.close()
+
+
+def test_the_first_launch_of_a_plan_of_the_largest_chains_captured():
+    """A plan whose kernel asks for more LDS than HIP gives unasked (9 sources of 144 MiB), launched for the first time inside a
+    capture; replays on other data, with eager work and synchronisations between them."""
+    n, count = 9, (144 << 20) // 4 + 3
+    xs = [torch.empty(count, device="cuda:0") for _ in range(n)]
+    out = torch.empty(count, device="cuda:0")
+    plan = hcclx.Plan([(count, [x.data_ptr() for x in xs], [out.data_ptr()])], T.FP32, T.SUM, wide=True)
+    s = torch.cuda.Stream()
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        g.capture_begin()
+        plan.launch(s.cuda_stream)
+        g.capture_end()
+    for rep in range(3):
+        for k, x in enumerate(xs):
+            x.normal_(generator=torch.Generator(device="cuda:0").manual_seed(100 * rep + k))
+        out.fill_(-1)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        want = xs[0].clone()
+        for x in xs[1:]:
+            want = x + want
+        assert torch.equal(out.view(torch.int32), want.view(torch.int32)), rep
+    plan.close()
