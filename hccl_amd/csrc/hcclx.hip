@@ -971,25 +971,30 @@ int build_wide_batches(const hcclx_wide_seg_t *segs, uint32_t nseg, int dtype, i
 //   many   fewer tiles of `three` than wide_min_tiles, unless they straddle and are 4 MiB or more: eight loads at a time hide more
 //          latency (many : small: 2 MiB bf16 6.9 : 7.5, 16 ranks x 4 MiB 13.9 : 16.0; 6 MiB odd 13.0 : 12.4).
 //   small  straddling below 32 MiB (three or four : small: 16 MiB bf16 31.0 : 27.9, 25 46.0 : 43.8; 40 MiB fp32 59.1 : 62.1).
-//   large  from 128 MiB on (three or four : large: 150 MiB bf16 246 : 229, 12 x 150 fp32 AllReduce 624 : 605, 12 x 1 GiB int32
-//          4395 : 4295; below it the last round of its 64 KiB tiles shows: 72 MiB 100.8 : 105.1), straddling elements of at
-//          least 4 bytes (200 MiB fp32 323 : 315; 400 MiB bf16 691 : 704).
+//   large  from 144 MiB on (the better of three and four : large, fp32: 112 MiB 158 : 159, 128 178 : 183, 144 222 : 215, 192
+//          310 : 296, 256 422 : 388, 5 x 230 236.2 : 235.5, 7 x 170 239 : 235, 12 x 128 275 : 280, 12 x 150 338 : 328, 16 x 128 356 : 353,
+//          16 x 192 552 : 528, 32 x 64 340 : 336; odd 128 185 : 193, 144 222 : 222, 12 x 128 278 : 283, 5 x 256 268 : 265), elements
+//          of 1 and 2 bytes from eight sources on and where they do not straddle (bf16 128 178 : 186, 150 241 : 228, 192 311 : 290,
+//          12 x 150 331 : 317; 5 x 256 275 : 290, 6 x 400 515 : 532, 7 x 256 381 : 389, odd 400 676 : 693; int8 160 252 : 243, 5 x 256
+//          283 : 301).
 //   three, four   otherwise, whichever leaves less of the last round empty (three : four: 25 MiB 40.2 : 38.8, 16 x 40 109.9 :
 //          111.5, 24 x 20 AllReduce 157 : 168, 32 x 16 91.6 : 82.9; two, five and more to a CU: slower).
 WideShape wide_shape_for(const DeviceCtx *ctx, const hcclx_wide_seg_t *segs, uint32_t nseg, int esz, uint32_t *per_cu)
 {
-    constexpr uint64_t kLargeFrom = 128ull << 20;
+    constexpr uint64_t kLargeFrom = 144ull << 20;
     constexpr uint64_t kSmallFrom = 4ull << 20;
     constexpr uint64_t kSmallUpto = 32ull << 20;
     *per_cu = 0;
     if (ctx == nullptr) return kWideMany;
     const uint64_t tile_bytes = 16 * wide_tile_vecs(kWideThree);
     uint64_t bytes = 0;
+    uint64_t read = 0;
     uint64_t tiles = 0;
     bool straddling = false;
     for (uint32_t i = 0; i < nseg; ++i) {
         const uint64_t b = segs[i].count * static_cast<uint64_t>(esz);
         bytes += b;
+        read += b * segs[i].nsrc;
         tiles += (b + tile_bytes - 1) / tile_bytes;
         for (uint32_t k = 0; k < segs[i].nsrc && b != 0; ++k) {
             straddling = straddling || (reinterpret_cast<uint64_t>(segs[i].src[k]) - reinterpret_cast<uint64_t>(segs[i].dst[0])) % 16 != 0;
@@ -997,7 +1002,7 @@ WideShape wide_shape_for(const DeviceCtx *ctx, const hcclx_wide_seg_t *segs, uin
     }
     if (straddling && bytes >= kSmallFrom && bytes < kSmallUpto) return kWideSmall;
     if (bytes / tile_bytes < ctx->wide_min_tiles) return kWideMany;
-    if (ctx->fold_lds_hold && bytes >= kLargeFrom && (!straddling || esz >= 4)) {
+    if (ctx->fold_lds_hold && bytes >= kLargeFrom && (esz >= 4 || (!straddling && read >= 8 * bytes))) {
         *per_cu = 1;
         return kWideLarge;
     }
