@@ -669,18 +669,21 @@ k_moe_gather_pieces(MoeConstPtrs rows, MoeConstPtrs dest, MoeConstPtrs perm, Moe
     st16(to, V::pack(acc));
 }
 
-// Entries of a token that the gather takes at a time.  Two of two (8 x 4096 tokens of 7168 bf16, dispatch and gather, one : two
-// entries at a time, us: 462 : 454, 16 x 695 153.8 : 152.5, 4 x 300 26.3 : 25.4).  Of more entries: four while all wavefronts
-// fit the chip with room to spare and the launch is bound by its round trips (top-8, 8 x 16 tokens 18.8 : 16.0, 16 x 52 26.7 :
-// 25.5; top-4, 8 x 32 15.9 : 14.1; eight at a time 16.0, 25.7 and 14.7), two up to the wavefronts that fit (8 x 64 30.4 : 30.0), and one
-// beyond, where more of them open more rows at once than HBM likes (top-8, 8 x 1024 191 : 199 with four, 8 x 4096 586 : 611;
-// top-4, 4 x 3683 211 : 218).
-inline int gather_entries(const DeviceCtx *ctx, uint32_t topk, uint64_t waves)
+// Entries of a token that the gather takes at a time: four of four and more while the launch is so small that it is bound by its
+// round trips (top-8, one : two : four entries, us: 8 x 16 tokens of 7168 bf16 8.61 : 6.48 : 5.62, 8 x 40 10.69 : 9.06 : 9.28;
+// top-4, 8 x 32 6.63 : 5.67 : 5.56; but top-3, whose fourth is missing, 8 x 24 5.29 : 4.87 : 5.30), then two (8 x 64 12.90 : 12.45 :
+// 12.59, 8 x 96 20.4 : 18.5 : 18.3), and one where the rows are more than the Infinity Cache holds: more of them open more rows at
+// once than HBM likes (top-8, 8 x 256 44.7 : 45.0 : 44.5, 8 x 400 66.6 : 68.6 : 68.4, 8 x 4096 x 4096 398 : 429 : 433; top-4, 4 x
+// 3683 x 4096 93.5 : 99.2 : 99.1).  Top-2, which has no third, keeps two longer (16 x 695 75.5 : 74.6, 8 x 1536 82.1 : 81.8, 8 x
+// 2048 108.4 : 108.8, 8 x 4096 215.8 : 221.3).
+inline int gather_entries(const DeviceCtx *ctx, uint32_t topk, uint64_t waves, uint64_t row_bytes)
 {
+    constexpr uint64_t kTwoUpto = 256ull << 20;
+    constexpr uint64_t kTwoOfTwoUpto = 400ull << 20;
     if (topk == 1) return 1;
-    if (topk == 2) return 2;
     const uint64_t cus = ctx ? static_cast<uint64_t>(ctx->num_cus) : 256;
-    return waves <= 20 * cus ? 4 : waves <= 32 * cus ? 2 : 1;
+    if (topk >= 4 && waves <= 16 * cus) return 4;
+    return row_bytes < (topk == 2 ? kTwoOfTwoUpto : kTwoUpto) ? 2 : 1;
 }
 
 // Which entries share a wavefront, and how rows are stored.  Tokens of up to kWarmTokens in all are usually still in the
@@ -748,6 +751,7 @@ int launch_gather_pieces(int kind, hipStream_t st, const MoeConstPtrs &rows, con
     const uint32_t most = rows_per_launch(vpr, 1);
     if (most == 0) return fail(HCCL_E_PARA, "too much data for one launch");
     const dim3 block(kPieceVecs * kPiecesPerBlock);
+    const uint64_t row_bytes = static_cast<uint64_t>(n) * tokens * topk * vpr * 16;
     for (uint32_t at = 0; at < tokens;) {
         const uint32_t take = tokens - at < most ? tokens - at : most;
         const RowPieces pieces = row_pieces(take, vpr, 1);
@@ -755,7 +759,7 @@ int launch_gather_pieces(int kind, hipStream_t st, const MoeConstPtrs &rows, con
         const MoeConstPtrs ds = moved_on(dest, n, static_cast<uint64_t>(at) * topk * 4);
         const MoeConstPtrs pm = moved_on(perm, n, static_cast<uint64_t>(at) * topk * 4);
         const dim3 grid((pieces.total + kPiecesPerBlock - 1) / kPiecesPerBlock, n);
-        const int k = gather_entries(device_ctx(), topk, static_cast<uint64_t>(pieces.total) * n);
+        const int k = gather_entries(device_ctx(), topk, static_cast<uint64_t>(pieces.total) * n, row_bytes);
         if (kind == HCCL_DATA_TYPE_FP32) {
             launch_gather_k<HCCL_DATA_TYPE_FP32>(k, grid, block, st, rows, ds, pm, to, n, topk, vpr, pieces, esz, sdispls, rdispls);
         } else if (kind == HCCL_DATA_TYPE_FP16) {
