@@ -250,9 +250,12 @@ k_moe_scan_perm(MoeConstPtrs dest, MoePtrs perm, uint32_t n, uint32_t entries, u
 // entries and those in front of chunk c; then the permutation of chunk c as in k_moe_perm.  The workgroups of chunk 0 write
 // their rank's rows of the count and displacement tables and, from a pass over all ranks' destinations, what every rank
 // sends to rank i in front of which.  Bound by the latency of one launch and its rounds of loads.  Two launches : one, us: 8 ranks x 64
-// entries 5.95 : 4.44, x 512 6.16 : 4.61, x 1024 6.5 : 5.2, x 4096 7.6 : 9.4; 16 x 1024 8.3 : 7.3, x 2048 8.9 : 9.7; 64 x 1024
-// 26.3 : 20.5; 2 x 512 5.1 : 3.6, x 4096 6.2 : 7.3.
+// entries 6.28 : 4.60, x 512 6.16 : 4.48, x 1024 6.21 : 4.96; 16 x 1024 8.00 : 6.64; 64 x 1024 25.2 : 18.2; 2 x 512 5.10 : 3.64,
+// x 1024 5.30 : 4.06.
+// No launch has more entries than kOneLaunchEntries: a thread holds that many / kMoeChunk of its rank's destinations and counts no
+// others.  (In a loop over more of them two launches were faster: 8 x 4096 7.6 : 9.4, 16 x 2048 8.9 : 9.7.)
 constexpr uint32_t kOneLaunchEntries = 1024;
+static_assert(kOneLaunchEntries % kMoeChunk == 0, "every thread of a workgroup holds as many entries");
 
 __global__ void __launch_bounds__(kMoeChunk)
 k_moe_route_one(MoeConstPtrs dest, MoePtrs perm, uint32_t n, uint32_t entries, uint64_t row_elems, uint64_t *send_counts,
