@@ -602,11 +602,16 @@ k_moe_scatter_pieces(MoeConstPtrs tokens, MoeConstPtrs dest, MoeConstPtrs perm, 
 // look-ups are in flight together, and their rows too where all K are there.  (A branch per entry makes the compiler wait for
 // every load before the next.)  Where one is dropped or behind the last, those that are left are read one after the other, so
 // that what is dropped costs no bytes.  K by gather_entries.  DT = int8 moves bytes (topk == 1).
-template <int DT, int K>
+// ALL: tokens have K entries (top-2).  There is one round, and no branch between the look-ups and the rows: in the place of a
+// dropped entry the lanes load the row of one that is there, which the caches then hold.  Exchange of 8 x 4096 x 7168 bf16, the
+// other form : this, us: 451.8 : 449.8, 16 x 695 152.6 : 152.1; gather with half of the entries dropped 151.5 : 148.6, all 113.7 : 85.3.
+// Of more entries the other form is the faster one (8 x 96 top-8 41.7 : 41.2, 8 x 16 15.8 : 15.2, 8 x 64 top-3 19.8 : 18.9).
+template <int DT, int K, bool ALL>
 __global__ void __launch_bounds__(kPieceVecs * kPiecesPerBlock)
-k_moe_gather_pieces(MoeConstPtrs rows, MoeConstPtrs dest, MoeConstPtrs perm, MoePtrs out, uint32_t n, uint32_t topk, uint32_t vpr,
+k_moe_gather_pieces(MoeConstPtrs rows, MoeConstPtrs dest, MoeConstPtrs perm, MoePtrs out, uint32_t n, uint32_t any_topk, uint32_t vpr,
                     RowPieces pieces, uint32_t esz, const uint64_t *sdispls, const uint64_t *rdispls)
 {
+    const uint32_t topk = ALL ? K : any_topk;
     using V = Vec16<DT>;
     using C = typename V::C;
     constexpr int NE = V::NE;
@@ -656,7 +661,23 @@ k_moe_gather_pieces(MoeConstPtrs rows, MoeConstPtrs dest, MoeConstPtrs perm, Moe
             ok[k] = (first + k < topk) & (p[k] != kDropped) & (d[k] < n);   // without branches between the look-ups
             all = all & ok[k];
         }
-        if (K > 1 && all) {
+        if constexpr (ALL) {
+            uint32_t there_p = kDropped;
+            uint32_t there_d = 0;
+#pragma unroll
+            for (int k = K - 1; k >= 0; --k) {
+                there_p = ok[k] ? p[k] : there_p;
+                there_d = ok[k] ? d[k] : there_d;
+            }
+            if (there_p == kDropped) continue;   // no entry is there
+            u32x4 raw[K];
+#pragma unroll
+            for (int k = 0; k < K; ++k) raw[k] = row(ok[k] ? d[k] : there_d, ok[k] ? p[k] : there_p);
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                if (ok[k]) add(raw[k]);
+            }
+        } else if (K > 1 && all) {
             u32x4 raw[K];
 #pragma unroll
             for (int k = 0; k < K; ++k) raw[k] = row(d[k], p[k]);
@@ -672,21 +693,20 @@ k_moe_gather_pieces(MoeConstPtrs rows, MoeConstPtrs dest, MoeConstPtrs perm, Moe
     st16(to, V::pack(acc));
 }
 
-// Entries of a token that the gather takes at a time: four of four and more while the launch is so small that it is bound by its
-// round trips (top-8, one : two : four entries, us: 8 x 16 tokens of 7168 bf16 8.61 : 6.48 : 5.62, 8 x 40 10.69 : 9.06 : 9.28;
-// top-4, 8 x 32 6.63 : 5.67 : 5.56; but top-3, whose fourth is missing, 8 x 24 5.29 : 4.87 : 5.30), then two (8 x 64 12.90 : 12.45 :
-// 12.59, 8 x 96 20.4 : 18.5 : 18.3), and one where the rows are more than the Infinity Cache holds: more of them open more rows at
-// once than HBM likes (top-8, 8 x 256 44.7 : 45.0 : 44.5, 8 x 400 66.6 : 68.6 : 68.4, 8 x 4096 x 4096 398 : 429 : 433; top-4, 4 x
-// 3683 x 4096 93.5 : 99.2 : 99.1).  Top-2, which has no third, keeps two longer (16 x 695 75.5 : 74.6, 8 x 1536 82.1 : 81.8, 8 x
-// 2048 108.4 : 108.8, 8 x 4096 215.8 : 221.3).
+// Entries of a token that the gather takes at a time.  Two of two (exchange of the rows, one : two entries, us: 8 x 4096 tokens of
+// 7168 bf16 458.4 : 449.8, 8 x 1024 115.4 : 115.2, 4 x 300 25.9 : 25.2).  Of more, four of four and more while the launch is so
+// small that it is bound by its round trips (top-8, one : two : four: 8 x 16 18.2 : 16.1 : 15.1, 8 x 40 23.8 : 22.3 : 22.5; top-4, 8 x
+// 32 16.5 : 15.2 : 15.0), then two (top-8, 8 x 64 29.5 : 29.2 : 29.4, 8 x 96 42.9 : 41.0 : 41.1, 8 x 128 51.0 : 50.7 : 50.9, 4 x 1000 x 2880
+// 77.3 : 76.7 : 76.6; top-4, 16 x 128 x 4096 37.8 : 37.0 : 36.8), and one where the rows come near to what the Infinity Cache holds:
+// more of them open more rows at once than HBM likes (top-8, 8 x 256 91.0 : 91.3 : 91.8, 8 x 400 134.6 : 136.5 : 137.3, 8 x 4096 x 4096 807 : 825 :
+// 830; top-4, 2 x 2000 97.8 : 99.1 : 99.7, 4 x 3683 x 4096 212.5 : 217.4 : 217.7).
 inline int gather_entries(const DeviceCtx *ctx, uint32_t topk, uint64_t waves, uint64_t row_bytes)
 {
-    constexpr uint64_t kTwoUpto = 256ull << 20;
-    constexpr uint64_t kTwoOfTwoUpto = 400ull << 20;
-    if (topk == 1) return 1;
+    constexpr uint64_t kTwoUpto = 192ull << 20;
+    if (topk <= 2) return static_cast<int>(topk);
     const uint64_t cus = ctx ? static_cast<uint64_t>(ctx->num_cus) : 256;
     if (topk >= 4 && waves <= 16 * cus) return 4;
-    return row_bytes < (topk == 2 ? kTwoOfTwoUpto : kTwoUpto) ? 2 : 1;
+    return row_bytes < kTwoUpto ? 2 : 1;
 }
 
 // Which entries share a wavefront, and how rows are stored.  Tokens of up to kWarmTokens in all are usually still in the
@@ -739,11 +759,13 @@ void launch_gather_k(int k, dim3 grid, dim3 block, hipStream_t st, const MoeCons
                      const uint64_t *sdispls, const uint64_t *rdispls)
 {
     if (k == 4) {
-        HCCLX_LAUNCH((k_moe_gather_pieces<DT, 4>), grid, block, 0, st, rows, dest, perm, out, n, topk, vpr, pieces, esz, sdispls, rdispls);
+        HCCLX_LAUNCH((k_moe_gather_pieces<DT, 4, false>), grid, block, 0, st, rows, dest, perm, out, n, topk, vpr, pieces, esz, sdispls, rdispls);
+    } else if (k == 2 && topk == 2) {
+        HCCLX_LAUNCH((k_moe_gather_pieces<DT, 2, true>), grid, block, 0, st, rows, dest, perm, out, n, topk, vpr, pieces, esz, sdispls, rdispls);
     } else if (k == 2) {
-        HCCLX_LAUNCH((k_moe_gather_pieces<DT, 2>), grid, block, 0, st, rows, dest, perm, out, n, topk, vpr, pieces, esz, sdispls, rdispls);
+        HCCLX_LAUNCH((k_moe_gather_pieces<DT, 2, false>), grid, block, 0, st, rows, dest, perm, out, n, topk, vpr, pieces, esz, sdispls, rdispls);
     } else {
-        HCCLX_LAUNCH((k_moe_gather_pieces<DT, 1>), grid, block, 0, st, rows, dest, perm, out, n, topk, vpr, pieces, esz, sdispls, rdispls);
+        HCCLX_LAUNCH((k_moe_gather_pieces<DT, 1, false>), grid, block, 0, st, rows, dest, perm, out, n, topk, vpr, pieces, esz, sdispls, rdispls);
     }
 }
 
@@ -770,7 +792,7 @@ int launch_gather_pieces(int kind, hipStream_t st, const MoeConstPtrs &rows, con
         } else if (kind == HCCL_DATA_TYPE_BFP16) {
             launch_gather_k<HCCL_DATA_TYPE_BFP16>(k, grid, block, st, rows, ds, pm, to, n, topk, vpr, pieces, esz, sdispls, rdispls);
         } else {
-            HCCLX_LAUNCH((k_moe_gather_pieces<HCCL_DATA_TYPE_INT8, 1>), grid, block, 0, st, rows, ds, pm, to, n, topk, vpr, pieces, esz,
+            HCCLX_LAUNCH((k_moe_gather_pieces<HCCL_DATA_TYPE_INT8, 1, false>), grid, block, 0, st, rows, ds, pm, to, n, topk, vpr, pieces, esz,
                          sdispls, rdispls);
         }
         const hipError_t e = hipGetLastError();
