@@ -109,15 +109,16 @@ class ReduceScatterMesh(Workload):
     """benchmark configuration 2: HcclReduceScatter SUM bf16, 8 ranks x 33,554,432 elements in (64 MiB per rank).
     The selector picks the mesh template; output shard r folds slice r of every rank starting from rank
     r's own data, then ranks ascending (ins_temp_reduce_scatter_mesh_1D.cc:132-154), as one fused pass of the
-    chain kernel that moves four vectors per thread (eight sources, one destination per segment)."""
+    wide chain kernel in the shape for one destination per segment: four vectors per thread, one of the eight sources at a
+    time, four workgroups to a CU."""
     dtype = "bf16"
-    kernel = "hcclx::k_fold_wide<11, 0, 0, 2>"
+    kernel = "hcclx::k_fold_wide<11, 0, 0, 3>"
     profile = "profiles/k_fold_wide_reduce_scatter_bf16_8x64MiB.txt"
 
     def __init__(self, torch, api, T, n=8, recv=4 * 1024 * 1024):
         super().__init__(torch, api, T, n)
         if (n, recv) != (8, 4 * 1024 * 1024):
-            self.profile, self.kernel = None, "hcclx::k_fold_wide<11, 0, 0, 2>"
+            self.profile, self.kernel = None, "hcclx::k_fold_wide<11, 0, 0, 3>"
         self.name = "reduce_scatter_sum_bf16_mesh_%dx%dMiB" % (n, n * recv * 2 >> 20)
         self.recv = recv
         self.x = [_randn_bits16(torch, n * recv, 1000 + r, torch.bfloat16) for r in range(n)]
@@ -158,7 +159,7 @@ class AllReduce(Workload):
     ranks.  One launch folds each slice into the first output (eight inputs read once), a second copies it to the
     other seven, one output at a time."""
     dtype = "f32"
-    kernel = "hcclx::k_fold_wide<4, 0, 0, 2> + hcclx::(anonymous namespace)::k_phased_copy<hcclx::PhasedTable>"
+    kernel = "hcclx::k_fold_wide<4, 0, 0, 3> + hcclx::(anonymous namespace)::k_phased_copy<hcclx::PhasedTable>"
     profile = "profiles/k_fold_wide_k_phased_copy_all_reduce_fp32_8x64MiB.txt"
 
     def __init__(self, torch, api, T, n=8, count=16 * 1024 * 1024, alg=None, step_mode=False, dtype=None, op=None,
@@ -440,7 +441,7 @@ WORKLOADS = {
     "all_reduce_sum_fp32_8x64MiB_two_shot_step_by_step": lambda *a: AllReduce(*a, step_mode=True),
     # communicators of more than 16 ranks: the wide chain kernel (two-shot mesh) and the wide tree kernel (NHR)
     "all_reduce_sum_fp32_32x16MiB": lambda *a: AllReduce(
-        *a, n=32, count=4 * 1024 * 1024, kernel="hcclx::k_fold_wide<4, 0, 0, 2> + k_phased_copy",
+        *a, n=32, count=4 * 1024 * 1024, kernel="hcclx::k_fold_wide<4, 0, 0, 3> + k_phased_copy",
         profile="profiles/k_fold_wide_k_phased_copy_all_reduce_fp32_32x16MiB.txt"),
     "all_reduce_sum_fp32_32x16MiB_nhr": lambda *a: AllReduce(
         *a, n=32, count=4 * 1024 * 1024, alg="InsAllReduceNHR", kernel="hcclx::k_fold_wide<4, 0, 2, 1> + k_phased_copy",
@@ -459,7 +460,7 @@ WORKLOADS = {
     # schedule is a tree per slice, folded by the tree kernel, then handed out one output at a time)
     "all_reduce_max_int32_12x64MiB_rhd": lambda *a: AllReduce(
         *a, n=12, count=16 * 1024 * 1024, dtype=a[2].INT32, op=a[2].MAX, alg="InsAllReduceRHD",
-        kernel="hcclx::k_fold_wide<2, 2, 0, 2> + k_phased_copy",
+        kernel="hcclx::k_fold_wide<2, 2, 0, 3> + k_phased_copy",
         profile="profiles/k_fold_wide_k_phased_copy_all_reduce_rhd_int32_max_12x64MiB.txt"),
     "all_reduce_prod_fp32_12x64MiB_rhd": lambda *a: AllReduce(
         *a, n=12, count=16 * 1024 * 1024, op=a[2].PROD, alg="InsAllReduceRHD",
@@ -481,7 +482,7 @@ EXTRA_WORKLOADS = {
     "copy_calibration_1024MiB": lambda *a: CopyCalibration(*a),
     "all_reduce_max_int32_12x1GiB_nhr": lambda *a: AllReduce(
         *a, n=12, count=256 * 1024 * 1024, dtype=a[2].INT32, op=a[2].MAX, alg="InsAllReduceNHR",
-        kernel="hcclx::k_fold_wide<2, 2, 0, 3> + k_phased_copy",
+        kernel="hcclx::k_fold_wide<2, 2, 0, 4> + k_phased_copy",
         profile="profiles/k_fold_wide_k_phased_copy_all_reduce_nhr_int32_max_12x1GiB.txt"),
     "all_reduce_prod_fp32_12x1GiB_aicpu_nhr": lambda *a: AllReduce(
         *a, n=12, count=256 * 1024 * 1024, op=a[2].PROD, alg="InsAllReduceAicpuReduceNHR",

@@ -33,8 +33,8 @@ struct DeviceCtx {
     // Chain folds whose largest fan-in reaches this go to the wide chain kernel (HCCLX_WIDE_CHAIN_FROM); with 9 to
     // 16 sources it measured 2 to 8 % faster than the kernel that holds all sources in registers, with 8 the same.
     uint32_t wide_chain_from = 9;
-    // The same for chains with a single destination (HCCLX_WIDE_CHAIN_FROM_ONE_DST): there the wide kernel moves
-    // four vectors per thread, and an 8-source ReduceScatter measured 5 % faster on it.
+    // The same for chains with a single destination (HCCLX_WIDE_CHAIN_FROM_ONE_DST): there the wide kernel has
+    // shapes of its own (wide_shape_for), and an 8-source ReduceScatter measured 5 to 10 % faster on it.
     uint32_t wide_chain_from_one_dst = 5;
     // Wide launches whose segments have this many destinations give each XCD a contiguous eighth of the tiles
     // (HCCLX_WIDE_XCD_REMAP_FROM).
