@@ -118,6 +118,16 @@ def test_every_shape_of_a_chain(dtype, op, nsrc, total, straddle, shape):
     run_case(TYPES[dtype], OPS[op], nsrc, total, straddle)
 
 
+@pytest.mark.parametrize("dtype,op", [("fp32", "sum"), ("bf16", "max")])
+def test_the_largest_chains_without_lds_of_their_own(dtype, op):
+    """fold_lds_hold 0: they run in the next smaller shape; what was planned before keeps its kernel."""
+    hcclx.tune("fold_lds_hold", 0)
+    try:
+        run_case(TYPES[dtype], OPS[op], 9, 144 * MIB, False)
+    finally:
+        hcclx.tune("fold_lds_hold", 1)
+
+
 @pytest.mark.parametrize("place", ["first", "last"])
 @pytest.mark.parametrize("dtype,op,nsrc,total,straddle,shape", [c for c in CASES if c[:2] == ("fp32", "min")])
 def test_every_shape_of_a_chain_in_place(dtype, op, nsrc, total, straddle, shape, place):
