@@ -269,17 +269,23 @@ def test_rows_cut_into_pieces(topk, dtype, width, n, tokens):
     test_fused_dispatch_and_gather_combine_equal_the_two_pass_pipeline(topk, dtype, width, n, tokens)
 
 
-# rows of 64 vectors are one piece, so the wavefronts of a gather are tokens x ranks: those that fit 256 CUs 16 deep, and one token
-# more; and 192 MiB of rows (4 x 8192 elements x 384 tokens x 8 ranks)
+# rows of 64 vectors are one piece, so the wavefronts of a gather are tokens x ranks: those that fit 256 CUs 20 and 32 deep, and one token more
 @pytest.mark.parametrize("topk,dtype,width,n,tokens", [(3, T.BFP16, 512, 8, 640), (3, T.BFP16, 512, 8, 641), (5, T.FP16, 512, 8, 1024),
                                                         (5, T.FP32, 256, 8, 1025), (2, T.BFP16, 512, 8, 1025), (8, T.FP32, 256, 1, 1),
-                                                        (7, T.FP16, 520, 1, 9), (1, T.BFP16, 512, 16, 5), (5, T.FP16, 512, 8, 512),
-                                                        (5, T.FP16, 512, 8, 513), (4, T.BFP16, 8192, 8, 384),
-                                                        (2, T.FP32, 260, 1, 7), (2, T.FP16, 4096, 3, 33)])
+                                                        (7, T.FP16, 520, 1, 9), (1, T.BFP16, 512, 16, 5)])
 def test_entries_of_a_token_in_flight_together(topk, dtype, width, n, tokens):
-    """The gather takes four, two or one of a token's entries at a time, by the launch's wavefronts and rows: around the limits, with
+    """The gather takes four, two or one of a token's entries at a time, by the launch's wavefronts: around both limits, with
     entries that four and two do not divide, and (one rank: two of three entries dropped) tokens that keep none.  The order of
     the sum is the oracle's whatever is loaded together, so the results are equal to the bit."""
+    test_fused_dispatch_and_gather_combine_equal_the_two_pass_pipeline(topk, dtype, width, n, tokens)
+
+
+# rows of 64 vectors: the wavefronts that fit 256 CUs 16 deep, and one token more; and 192 MiB of rows (4 x 8192 elements x 384
+# tokens x 8 ranks)
+@pytest.mark.parametrize("topk,dtype,width,n,tokens", [(5, T.FP16, 512, 8, 512), (5, T.FP16, 512, 8, 513), (4, T.BFP16, 8192, 8, 384),
+                                                        (2, T.FP32, 260, 1, 7), (2, T.FP16, 4096, 3, 33)])
+def test_entries_in_flight_together_at_the_limits(topk, dtype, width, n, tokens):
+    """How many entries the gather takes at a time goes by the launch's wavefronts and by its rows: on both sides of the limits."""
     test_fused_dispatch_and_gather_combine_equal_the_two_pass_pipeline(topk, dtype, width, n, tokens)
 
 

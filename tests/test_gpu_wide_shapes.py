@@ -16,36 +16,17 @@ pytestmark = pytest.mark.gpu
 MIB = 1 << 20
 
 
-HALF = (T.FP16, T.BFP16)
-
-
 def step(dtype, op, src, dst):
-    """src (+) dst as the kernels combine: 16-bit floats in fp32 (sums narrowed once, at the end; products every time), max as
-    (s < d) ? d : s, min as (d < s) ? d : s."""
-    if op == T.MAX:
-        return torch.where(src < dst, dst, src)
-    if op == T.MIN:
-        return torch.where(dst < src, dst, src)
-    if op == T.PROD:
-        return (src * dst).to(TORCH_STORAGE[dtype]).float() if dtype in HALF else src * dst
-    return src + dst
+    """src (+) dst as the kernels combine: sums in fp32 for bf16 (narrowed once, at the end), max as (s < d) ? d : s."""
+    return torch.where(src < dst, dst, src) if op == T.MAX else src + dst
 
 
 def chain(xs, dtype, op, flips):
-    wide = (lambda x: x.float()) if dtype in HALF else (lambda x: x)
+    wide = (lambda x: x.float()) if dtype == T.BFP16 else (lambda x: x)
     acc = wide(xs[0])
     for k in range(1, len(xs)):
         acc = step(dtype, op, acc, wide(xs[k])) if flips[k] else step(dtype, op, wide(xs[k]), acc)
     return acc.to(TORCH_STORAGE[dtype])
-
-
-def assert_same(got, want):
-    """Equal to the bit; NaNs where NaNs are."""
-    if got.is_floating_point():
-        bits = {2: torch.int16, 4: torch.int32, 8: torch.int64}[got.element_size()]
-        assert torch.equal(got.isnan(), want.isnan())
-        got, want = (torch.where(v.isnan(), torch.zeros_like(v), v).view(bits) for v in (got, want))
-    assert torch.equal(got, want)
 
 
 @pytest.mark.parametrize("dtype,op", [(T.FP32, T.SUM), (T.BFP16, T.SUM), (T.INT32, T.MAX), (T.FP32, T.MAX)])
@@ -53,7 +34,9 @@ def assert_same(got, want):
                                                (5, 128, False), (5, 129, True)])
 def test_chain_to_one_destination(nsrc, mib, straddle, dtype, op):
     esz = T.DTYPE_SIZE[dtype]
-    lengths = segment_lengths(esz, mib * MIB, straddle)
+    edge = 65536 // esz                       # elements of the largest tile
+    whole = mib * MIB // esz
+    lengths = [edge - 1, whole - 3 * edge - 7, 1, 2 * edge + 3] if straddle else [edge, whole - 2 * edge, edge - 16 // esz]
     total = sum(lengths) + 64
     xs = [device_payload(dtype, total + k, 10 * k + mib) for k in range(nsrc)]
     if op == T.MAX and dtype == T.FP32:       # values that max tells apart only by the order of its operands
@@ -74,8 +57,46 @@ def test_chain_to_one_destination(nsrc, mib, straddle, dtype, op):
     assert hcclx.kernels_launched() == before + 1
     torch.cuda.synchronize()
     want = chain([x[k % 3 if straddle else 0:][:at] for k, x in enumerate(xs)], dtype, op, flips)
-    assert_same(out[:at], want)
+    got = out[:at]
+    if dtype == T.BFP16:
+        got, want = got.view(torch.int16), want.view(torch.int16)
+    elif dtype == T.FP32:
+        assert torch.equal(got.isnan(), want.isnan())
+        got, want = (torch.where(v.isnan(), torch.zeros_like(v), v).view(torch.int32) for v in (got, want))
+    assert torch.equal(got, want)
     assert bool((out[at:] == 77).all())
+
+
+HALF = (T.FP16, T.BFP16)
+
+
+def any_step(dtype, op, src, dst):
+    """src (+) dst as the kernels combine: 16-bit floats in fp32 (sums narrowed once, at the end; products every time), max as
+    (s < d) ? d : s, min as (d < s) ? d : s."""
+    if op == T.MAX:
+        return torch.where(src < dst, dst, src)
+    if op == T.MIN:
+        return torch.where(dst < src, dst, src)
+    if op == T.PROD:
+        return (src * dst).to(TORCH_STORAGE[dtype]).float() if dtype in HALF else src * dst
+    return src + dst
+
+
+def any_chain(xs, dtype, op, flips):
+    wide = (lambda x: x.float()) if dtype in HALF else (lambda x: x)
+    acc = wide(xs[0])
+    for k in range(1, len(xs)):
+        acc = any_step(dtype, op, acc, wide(xs[k])) if flips[k] else any_step(dtype, op, wide(xs[k]), acc)
+    return acc.to(TORCH_STORAGE[dtype])
+
+
+def assert_same(got, want):
+    """Equal to the bit; NaNs where NaNs are."""
+    if got.is_floating_point():
+        bits = {2: torch.int16, 4: torch.int32, 8: torch.int64}[got.element_size()]
+        assert torch.equal(got.isnan(), want.isnan())
+        got, want = (torch.where(v.isnan(), torch.zeros_like(v), v).view(bits) for v in (got, want))
+    assert torch.equal(got, want)
 
 
 TYPES = {"int8": T.INT8, "int16": T.INT16, "int32": T.INT32, "int64": T.INT64, "fp16": T.FP16, "bf16": T.BFP16, "fp32": T.FP32, "fp64": T.FP64}
@@ -98,7 +119,7 @@ def run_case(dtype, op, nsrc, total, straddle, in_place=None):
             x[2 * k::5] = float("nan")
             x[3 * k::11] = float("-inf")
     flips = [op in (T.MAX, T.MIN) and xs[0].is_floating_point() and k % 3 == 1 for k in range(nsrc)]
-    want = chain([x[o:o + whole] for x, o in zip(xs, off)], dtype, op, flips)
+    want = any_chain([x[o:o + whole] for x, o in zip(xs, off)], dtype, op, flips)
     out = xs[in_place] if in_place is not None else torch.full((whole + 64,), 77, device="cuda:0", dtype=TORCH_STORAGE[dtype])
     behind = out[whole:].clone()
     segs, at = [], 0
@@ -192,7 +213,7 @@ def test_wide_trees_of_16_bit_floats_over_all_values(dtype, op):
         torch.cuda.synchronize()
         val = [x.float() for x in xs]
         for d, s in steps:
-            val[d] = step(dtype, op, val[s], val[d])
+            val[d] = any_step(dtype, op, val[s], val[d])
         assert_same(out, val[0].to(TORCH_STORAGE[dtype]))
 
 
