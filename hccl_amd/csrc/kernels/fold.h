@@ -1223,7 +1223,9 @@ struct FoldLaunch {
     hipStream_t stream;
 };
 
-// One translation unit per data type defines these (fold_inst.hip).
+// One translation unit per data type and operation defines this, one per data type those below (fold_inst.hip).
+template <int DT, int OP>
+hipError_t fold_tree(int maxn, const FoldLaunch &l);
 #define HCCLX_DECLARE_FOLD(NAME) hipError_t fold_dispatch_##NAME(int op, int maxn, int mode, const FoldLaunch &l);
 HCCLX_DECLARE_FOLD(i8)
 HCCLX_DECLARE_FOLD(i16)

@@ -2,6 +2,8 @@
 //   -DHCCLX_DT=<HcclDataType enumerator> -DHCCLX_NAME=<suffix> -DHCCLX_ORDERED=<0|1>
 // HCCLX_ORDERED=1 (floating types) also builds the self-first and tree modes; for integers every fold
 // order gives the same bits, so the launcher maps those modes onto the chain kernel.
+// The trees of one operation are a unit of their own, -DHCCLX_TREE_OP=<HcclReduceOp enumerator>: the compiler takes two to five
+// minutes for those of fp16, and units are compiled side by side.
 // With -DHCCLX_COPY the unit holds the byte copy kernel instead (one source, many destinations).
 #include "fold.h"
 
@@ -149,6 +151,18 @@ static hipError_t by_fan(int maxn, const FoldLaunch &l)
     }
 }
 
+#ifdef HCCLX_TREE_OP
+
+template <int DT, int OP>
+hipError_t fold_tree(int maxn, const FoldLaunch &l)
+{
+    static_assert(DT == HCCLX_DT, "the type of the unit");
+    return by_fan<OP, kFoldTree>(maxn, l);
+}
+template hipError_t fold_tree<HCCLX_DT, HCCLX_TREE_OP>(int maxn, const FoldLaunch &l);
+
+#else
+
 template <int MODE>
 static hipError_t by_op(int op, int maxn, const FoldLaunch &l)
 {
@@ -174,12 +188,19 @@ hipError_t HCCLX_CAT(fold_dispatch_, HCCLX_NAME)(int op, int maxn, int mode, con
         return by_op<kFoldSelfFirst>(op, maxn, l);
     }
     if (mode == kFoldTree) {
-        return by_op<kFoldTree>(op, maxn, l);
+        switch (op) {
+            case HCCL_REDUCE_SUM: return fold_tree<HCCLX_DT, HCCL_REDUCE_SUM>(maxn, l);
+            case HCCL_REDUCE_PROD: return fold_tree<HCCLX_DT, HCCL_REDUCE_PROD>(maxn, l);
+            case HCCL_REDUCE_MAX: return fold_tree<HCCLX_DT, HCCL_REDUCE_MAX>(maxn, l);
+            case HCCL_REDUCE_MIN: return fold_tree<HCCLX_DT, HCCL_REDUCE_MIN>(maxn, l);
+            default: return hipErrorInvalidValue;
+        }
     }
 #endif
     return hipErrorInvalidValue;
 }
 
+#endif
 #endif
 
 }  // namespace hcclx
